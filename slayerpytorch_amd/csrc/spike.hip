@@ -1,27 +1,25 @@
 // SRM spike generation: threshold crossing with refractory feedback, sequential in time per
 // neuron, parallel over neurons; plus the fused surrogate-gradient pass of its backward.
 //
-// HBM-bound (12 B per neuron-timestep: read u, write u', write s).  A neuron's row must be
-// walked in time order, so one lane owns one neuron; but lanes that each walk their own row in
-// global memory would touch 64 different cache lines per access.  Instead a 64-lane work-group
-// owns 64 consecutive rows and streams them through LDS in 32-sample time chunks:
-//
-//   load    : 128-byte row segments, lanes along time (coalesced), written into an LDS ring
-//             ring[row][t mod L] that always holds the samples the refractory kernel can
-//             still reach (the current chunk plus ceil((nuSize-1)/32) chunks ahead);
-//   process : lane = row; for each t of the chunk read ring[row][t], compare with theta and,
-//             on a spike, add nu[0..nuSize) onto ring[row][t..t+nuSize) in place - the same
-//             fp32 additions in the same order as the sequential loop, hence bit-identical;
-//   store   : finished samples leave the ring as 128-byte row segments again; the spikes of a
-//             chunk travel as one 32-bit mask per lane and are expanded on the way out.
-//
-// The ring is rotated by the row number (sample t of row r lives at column (t + r) mod L), so
-// both access patterns - a fixed column over 32 rows and 32 consecutive columns of one row -
-// hit 32 different LDS banks.
-//
-// Short refractory kernels (nuSize <= 24, the normal case) take the row-tile kernel further
-// down instead: fewer rows per wavefront, long contiguous runs per row, and a per-lane register
-// window in place of the ring.
+// HBM-bound (12 B per neuron-timestep: read u, write u', write s).  A neuron's row must be walked in time order, but
+// lanes that each walk their own row in global memory would touch 64 different cache lines per access, so rows are
+// staged in LDS as long contiguous runs and walked there.  Three kernels:
+//   spike_rows_kernel   : whole rows (up to 4032 samples), any refractory kernel - nearly everything;
+//   spike_tile_kernel   : long rows in pieces, refractory kernels of up to 24 taps;
+//   spike_stream_kernel : longer rows with 25 to 97 taps, 64 rows per wavefront in 32-sample chunks through an LDS ring:
+//     load    : 128-byte row segments, lanes along time (coalesced), written into ring[row][t mod L] that always
+//               holds the samples the refractory kernel can still reach (the current chunk plus
+//               ceil((nuSize-1)/32) chunks ahead);
+//     process : lane = row; for each t of the chunk read ring[row][t], compare with theta and, on a spike, add
+//               nu[0..nuSize) onto ring[row][t..t+nuSize) in place - the same fp32 additions in the same order as the
+//               sequential loop, hence bit-identical;
+//     store   : finished samples leave the ring as 128-byte row segments again; the spikes of a chunk travel as one
+//               32-bit mask per lane and are expanded on the way out.
+//     The ring is rotated by the row number (sample t of row r lives at column (t + r) mod L), so both access
+//     patterns - a fixed column over 32 rows and 32 consecutive columns of one row - hit 32 different LDS banks.
+// What is beyond all of these runs spike_generic_kernel, one lane per row in global memory.
+#include <type_traits>
+
 #include "common.h"
 
 namespace slayer {
@@ -136,7 +134,7 @@ __global__ __launch_bounds__(64) void spike_stream_kernel(float *__restrict__ s,
 
 // ---- row-tile kernel (nuSize <= NU) --------------------------------------------------------------------
 // The fast path.  A wavefront owns R consecutive rows and moves them through LDS in
-// pieces of Tc samples per row (the whole row when it is short enough), so that global memory
+// pieces of Tc samples per row, so that global memory
 // is read and written as long contiguous runs with 16-byte accesses per lane - the access
 // pattern of a plain copy.  The sequential part then works in LDS, lane = row:
 //  * a refractory kernel without positive taps (the normal case) can only lower the potential, so a sample
@@ -152,29 +150,23 @@ __global__ __launch_bounds__(64) void spike_stream_kernel(float *__restrict__ s,
 // changes no value; a response may reach past the row's end into padding that is never stored.
 // Short tiles keep many wavefronts (and bytes) in flight per CU; the walking wavefront shares its SIMD's issue
 // slots with those that move data, so both walks use all 64 lanes (64 / R per row) to need fewer instructions.
-constexpr int kTileMaxPiece = 352;  // longest row (samples) that travels whole
 // Rows in pieces: samples per piece and row.  With 8-row tiles - tensors of few, long rows - the bytes in flight
 // per compute unit are what the rows in LDS amount to, so those pieces are longer.
 constexpr int kTilePiece16 = 256, kTilePiece8 = 512;
 constexpr int kSpikeRecordMaxT = 16384;  // longest row in pieces whose spikes can be stored shifted (2 KiB of spike bits)
 
-// LAG: samples of a piece that stay behind for the next one (>= NU - 1, whole 16-byte vectors; 32 = one word of
-// candidate bits for rows in pieces).  The samples that leave a piece are the ones LAG before its end, so with
-// several pieces per row LAG = 32 keeps every run of stores on 128-byte boundaries of the row (partial lines
-// are expensive to write).
+// LAG: samples of a piece that stay behind for the next one (one word of candidate bits, at least as many as a
+// response reaches).  The samples that leave a piece are the ones LAG before its end, so LAG = 32 keeps every run of
+// stores on 128-byte boundaries of the row (partial lines are expensive to write).
 // R: rows per tile (16, or 8 when the tensor has too few rows to fill the GPU with 16-row tiles).
-// MODE: how global memory is accessed.  kTileVec: rows are whole 16-byte vectors.  kTileFlat:
-// they are not (T % 4 != 0), but the rows of a tile travel whole and an 8-row tile is one
-// contiguous, 16-byte aligned run of whole vectors, so it is still moved with 16-byte accesses;
-// a vector may then hold the end of one row and the start of the next, and its four samples are
-// placed into (gathered from) LDS one by one.  kTileScalar: anything else, one sample per access.
-constexpr int kTileScalar = 0, kTileVec = 1, kTileFlat = 2;
+// VEC: rows are whole 16-byte vectors, moved as such; otherwise one sample per access.
+constexpr int kTileLag = 32;
 
 // Optional time shift of the spike output (the delayShift that follows spike() in networks with
 // axonal delays, fused into the store of the spikes): s[t] = spike[t - k], k = (int)(delay / Ts),
 // with one delay for all rows or one per neuron of a batch item (row % lutSize).  The membrane
-// potential is not shifted.  Tiles whose rows travel whole read the shifted bits from the tile's masks; rows in
-// pieces keep the spike bits of the whole row in LDS (rows of whole vectors up to kSpikeRecordMaxT samples).
+// potential is not shifted.  Rows in pieces keep the spike bits of the whole row in LDS (rows of whole vectors up to
+// kSpikeRecordMaxT samples).
 struct SpikeDelay {
     const float *lut;   // per-neuron delays, or NULL
     int64_t lutSize;    // neurons per batch item when lut is given
@@ -183,27 +175,24 @@ struct SpikeDelay {
     int on;
 };
 
-template <int NU, int MODE, int LAG, int R>
+template <int NU, bool VEC, int R>
 __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, float *u,
                                                         const float *__restrict__ nu, int64_t rows,
                                                         int T, int nuSize, int Tc, int P, int MP, int MPT,
                                                         int64_t tiles, float theta, float Ts, SpikeDelay dl)
 {
-    static_assert(LAG >= NU - 1 && LAG % 4 == 0, "the window must cover the refractory kernel");
-    constexpr bool VEC = MODE == kTileVec, FLAT = MODE == kTileFlat;
+    constexpr int LAG = kTileLag;
+    static_assert(LAG >= NU - 1, "the window must cover the refractory kernel");
     constexpr int V = VEC ? 4 : 1;      // samples per (row-wise) global access
-    // longest piece this instance stages (LAG = 32 marks the instances for rows in pieces)
-    constexpr int kPiece = (LAG == 32 && VEC) ? (R == 8 ? kTilePiece8 : kTilePiece16) : kTileMaxPiece;
-    constexpr int NB = R * kPiece / (FLAT ? 4 : V) / kWave;  // accesses per lane per piece, at most
+    constexpr int kPiece = VEC && R == 8 ? kTilePiece8 : kTilePiece16;   // longest piece
+    constexpr int NB = R * kPiece / V / kWave;  // accesses per lane per piece, at most
     // vectors per lane that leave in one step, at most: a row's last piece also retires the LAG columns behind it
-    constexpr int NBR = (R * (kPiece + (LAG == 32 ? LAG : 0)) / 4 + kWave - 1) / kWave;
-    // Rows of whole vectors in pieces: a piece is kHalves runs of 64 vectors per row, so vector b of a lane can be
+    constexpr int NBR = (R * (kPiece + LAG) / 4 + kWave - 1) / kWave;
+    // Rows of whole vectors: a piece is kHalves runs of 64 vectors per row, so vector b of a lane can be
     // vector lane + 64 * (b % kHalves) of row b / kHalves in every step - no index arithmetic per vector, the row and
-    // the piece's time travel in scalar offsets.  (Whole rows, 75 vectors at T = 300, would need twice the memory
-    // instructions that way, half of them nearly empty.)
-    constexpr bool STATIC = VEC && LAG == 32;
+    // the piece's time travel in scalar offsets.
     constexpr int kHalves = kPiece / 256;
-    static_assert(!STATIC || (NB == R * kHalves && NBR == NB + R / 8), "static mapping of vectors to lanes");
+    static_assert(!VEC || (NB == R * kHalves && NBR == NB + R / 8), "static mapping of vectors to lanes");
     extern __shared__ __align__(16) float lds[];
     float *tile = lds;                                                    // [R][P], P = 4 (mod 32)
     uint32_t *masks = reinterpret_cast<uint32_t *>(lds + R * P);  // [R][MP]
@@ -252,30 +241,17 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
         monotone = monotone && tap[j] <= 0.0f;
         signedTaps = signedTaps && tap[j] <= 0.0f && tap[j] > -__builtin_inff() && (__builtin_bit_cast(uint32_t, tap[j]) >> 31) != 0u;
     }
-    auto mark = [&](int r, int col, float x) {  // one sample
-        if (x >= theta) atomicOr(cand + r * MP + (col >> 5), 1u << (col & 31));
-    };
     constexpr int G = 32;               // samples per group of the window walk = bits of a spike mask
 
     // A "step" is one piece of one tile.  The global loads of a step are issued one step ahead
     // into x[] and stay in flight while the previous step is walked and retired.
-    float x[NB * (FLAT ? 4 : V)];
+    float x[NB * V];
     auto rows_of = [&](int64_t t) { return static_cast<int>(min(static_cast<int64_t>(R), rows - t * R)); };
-    const float invT = 1.0f / static_cast<float>(T);
     auto issue = [&](int64_t t, int tL) {
         const BufferRsrc bufU = make_buffer(u + t * R * static_cast<int64_t>(T));
-        if constexpr (FLAT) {  // whole rows: the tile is rows_of(t) * T / 4 consecutive vectors
-            const int nVec = (rows_of(t) * T) >> 2;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const float4 q = buffer_load4(bufU, masked_offset(lane + b * kWave < nVec, (lane + b * kWave) * 16), 0);
-                x[4 * b] = q.x; x[4 * b + 1] = q.y; x[4 * b + 2] = q.z; x[4 * b + 3] = q.w;
-            }
-            return;
-        }
         const int n = min(Tc, T - tL);
         const int perRow = n / V;
-        if constexpr (STATIC) {
+        if constexpr (VEC) {
             const int nR = rows_of(t);
             int mine[kHalves];
 #pragma unroll
@@ -294,39 +270,14 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
         const int dr = kWave / perRow, dc = kWave % perRow;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int off = (rc.r * T + tL + rc.c * V) * 4;
-            if constexpr (VEC) {
-                // (masked, not skipped: a fixed number of loads lets the wait for them leave the stores that
-                // are issued behind them in flight)
-                const float4 q = buffer_load4(bufU, masked_offset(lane + b * kWave < total, off), 0);
-                x[4 * b] = q.x; x[4 * b + 1] = q.y; x[4 * b + 2] = q.z; x[4 * b + 3] = q.w;
-            } else if (lane + b * kWave < total) {
-                x[b] = buffer_load(bufU, off, 0);
-            }
+            if (lane + b * kWave < total) x[b] = buffer_load(bufU, (rc.r * T + tL + rc.c) * 4, 0);
             rc.advance(dr, dc, perRow);
         }
     };
     auto commit = [&](int64_t t, int tL) {  // tile[r][LAG + c] = u[row][tL + c]
-        if constexpr (FLAT) {
-            const int nVec = (rows_of(t) * T) >> 2;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                if (lane + b * kWave < nVec) {
-                    int r, c;
-                    divmod_small((lane + b * kWave) << 2, T, invT, r, c);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        tile[r * P + LAG + c] = x[4 * b + e];
-                        if (monotone) mark(r, LAG + c, x[4 * b + e]);
-                        if (++c == T) { c = 0; ++r; }
-                    }
-                }
-            }
-            return;
-        }
         const int n = min(Tc, T - tL);
         const int perRow = n / V;
-        if constexpr (STATIC) {
+        if constexpr (VEC) {
             const int nR = rows_of(t);
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
@@ -348,21 +299,7 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
         const int dr = kWave / perRow, dc = kWave % perRow;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            if (lane + b * kWave < total) {
-                float *dst = tile + rc.r * P + LAG + rc.c * V;
-                if (VEC) {
-                    *reinterpret_cast<float4 *>(dst) = make_float4(x[4 * b], x[4 * b + 1], x[4 * b + 2], x[4 * b + 3]);
-                    if (monotone) {  // (the column is a multiple of 4: the four bits lie in one word)
-                        const uint32_t bits = (x[4 * b] >= theta ? 1u : 0u) | (x[4 * b + 1] >= theta ? 2u : 0u) |
-                                              (x[4 * b + 2] >= theta ? 4u : 0u) | (x[4 * b + 3] >= theta ? 8u : 0u);
-                        const int col = LAG + rc.c * V;
-                        if (bits) atomicOr(cand + rc.r * MP + (col >> 5), bits << (col & 31));
-                    }
-                } else {
-                    *dst = x[b];
-                    if (monotone) mark(rc.r, LAG + rc.c, x[b]);
-                }
-            }
+            if (lane + b * kWave < total) tile[rc.r * P + LAG + rc.c] = x[b];
             rc.advance(dr, dc, perRow);
         }
     };
@@ -397,8 +334,7 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
                                                 : row % dl.lutSize)
                                          : 0];
         }
-        // (whole rows: one tile per work-group, nothing follows, and the walk may use the registers)
-        if constexpr (LAG == 32) issue(tn, tLn);
+        issue(tn, tLn);
 
         // ---- walk: lane = row.  Columns [0, W) become final in this step.
         const int W = last ? n + LAG : n;
@@ -591,17 +527,7 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
                 if (lane < R) rowShift[lane] = max(-(1 << 24), min(1 << 24, delay_steps(rowDelay, dl.Ts)));
                 wave_sync();
             }
-            // the spike bit of the sample `shift` steps before column `col` (0 outside the row)
-            const int nCols = (MP - 1) << 5;
-            auto bits_from = [&](int r, int col) -> uint32_t {
-                const int c2 = col - rowShift[r];
-                if (c2 < 0 || c2 >= nCols) return 0u;
-                const int w = c2 >> 5, sh = c2 & 31;
-                uint32_t m = masks[r * MP + w] >> sh;
-                if (sh > 28 && w + 1 < MP - 1) m |= masks[r * MP + w + 1] << (32 - sh);
-                return m;
-            };
-            // the same from the record of the whole row (rows in pieces): the four bits from bit c2 on
+            // the four spike bits from bit c2 on of the record of the whole row
             const int nBits = T + LAG;
             auto bits_of_row = [&](int r, int c2) -> uint32_t {
                 // no branches: the LDS reads of all vectors of a step go out together.  Bits before LAG and from
@@ -612,52 +538,22 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
                 const uint64_t both = (static_cast<uint64_t>(rm[1]) << 32) | rm[0];
                 return in ? static_cast<uint32_t>(both >> (cc & 31)) : 0u;
             };
-            if constexpr (FLAT) {
-                const int nVec = (nRows * T) >> 2;
-                for (int vi = lane; vi < nVec; vi += kWave) {
-                    int r, c;
-                    divmod_small(vi << 2, T, invT, r, c);
-                    float uu[4], ss[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int col = LAG + c;   // time c of row r
-                        uu[e] = tile[r * P + col];
-                        const uint32_t bit = dl.on ? bits_from(r, col) : masks[r * MP + (col >> 5)] >> (col & 31);
-                        ss[e] = (bit & 1u) ? amplitude : 0.0f;
-                        if (++c == T) { c = 0; ++r; }
-                    }
-                    buffer_store4(bufU, vi * 16, 0, make_float4(uu[0], uu[1], uu[2], uu[3]));
-                    buffer_store4(bufS, vi * 16, 0, make_float4(ss[0], ss[1], ss[2], ss[3]));
-                }
-            } else {
             const int first = (tL == 0) ? LAG : 0;  // before the first sample there is nothing to store
             const int perRow = (W - first) / V;
-            const int total = nRows * perRow;
-            RowCol rc;
-            rc.init(lane, perRow, 1.0f / static_cast<float>(perRow));
-            const int dr = kWave / perRow, dc = kWave % perRow;
             // vector b of this lane in the retire step: row, first column, and whether it exists
             auto where = [&](int b, int &r, int &col) -> bool {
-                bool on;
-                if constexpr (STATIC) {
-                    // as in issue() and commit(); the vectors past 64 * kHalves per row (the LAG columns that a
-                    // row's last piece retires as well) follow, eight per row and lane group
-                    int c;
-                    if (b < NB) {
-                        r = b / kHalves;
-                        c = lane + (b % kHalves) * kWave;
-                    } else {
-                        r = (b - NB) * 8 + (lane >> 3);
-                        c = kHalves * kWave + (lane & 7);
-                    }
-                    on = r < nRows && c < perRow;
-                    col = first + c * 4;
+                // as in issue() and commit(); the vectors past 64 * kHalves per row (the LAG columns that a row's last
+                // piece retires as well) follow, eight per row and lane group
+                int c;
+                if (b < NB) {
+                    r = b / kHalves;
+                    c = lane + (b % kHalves) * kWave;
                 } else {
-                    on = lane + b * kWave < total;
-                    r = rc.r;
-                    col = first + rc.c * V;
-                    rc.advance(dr, dc, perRow);
+                    r = (b - NB) * 8 + (lane >> 3);
+                    c = kHalves * kWave + (lane & 7);
                 }
+                const bool on = r < nRows && c < perRow;
+                col = first + c * 4;
                 if (!on) {
                     r = 0;
                     col = first;
@@ -702,11 +598,10 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
                     int r, col;
                     const bool on = where(b, r, col);
                     const float *src = tile + r * P + col;
-                    // rows in pieces with a shifted output: a shift towards later times only needs spikes that are
-                    // final by now; the rows with a negative shift wait for their last piece
-                    const int shift = record ? rowShift[r] : 0;
-                    const uint32_t m = record ? bits_of_row(r, tL + col - shift)
-                                              : dl.on ? bits_from(r, col) : masks[r * MP + (col >> 5)] >> (col & 31);
+                    // a shift towards later times only needs spikes that are final by now; the rows with a negative
+                    // shift wait for their last piece
+                    const int shift = rowShift[r];
+                    const uint32_t m = bits_of_row(r, tL + col - shift);
                     const int off = masked_offset(on, (r * T + tW + col) * 4);
                     buffer_store4(bufU, off, 0, *reinterpret_cast<const float4 *>(src));
                     buffer_store4(bufS, shift < 0 ? kOutOfRange : off, 0,
@@ -715,17 +610,20 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
                 }
               }
             } else {
+                const int total = nRows * perRow;
+                RowCol rc;
+                rc.init(lane, perRow, 1.0f / static_cast<float>(perRow));
+                const int dr = kWave / perRow, dc = kWave % perRow;
 #pragma unroll 4
                 for (int g0 = lane; g0 < total; g0 += kWave) {
-                    const int col = first + rc.c * V;
+                    const int col = first + rc.c;
                     const int off = (rc.r * T + tW + col) * 4;
                     const float *src = tile + rc.r * P + col;
-                    const uint32_t m = dl.on ? bits_from(rc.r, col) : masks[rc.r * MP + (col >> 5)] >> (col & 31);
+                    const uint32_t m = masks[rc.r * MP + (col >> 5)] >> (col & 31);
                     buffer_store(bufU, off, 0, src[0]);
                     buffer_store(bufS, off, 0, (m & 1u) ? amplitude : 0.0f);
                     rc.advance(dr, dc, perRow);
                 }
-            }
             }
         }
         wave_sync();
@@ -777,13 +675,270 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
         for (int i = lane; i < R * MP; i += kWave)
             if (last || i % MP != 0) cand[i] = 0u;
         wave_sync();
-        if constexpr (LAG == 32) commit(tn, tLn);
-        else if (tn < tiles) {  // (not reached: whole rows are launched with one work-group per tile)
-            issue(tn, tLn);
-            commit(tn, tLn);
-        }
+        commit(tn, tLn);
         t = tn;
         tL = tLn;
+    }
+}
+
+// ---- whole-row kernel (any refractory kernel, any row alignment) -----------------------------------------
+// A wavefront owns R = 64 / PARTS whole rows; PARTS lanes serve a row, lane p its samples p, p + PARTS, ...  The rows
+// travel through LDS with 16-byte accesses (rows that are not whole vectors start on 4-byte boundaries only, which
+// the buffer instructions take; the last samples of such a row go one by one).  A lane keeps one bit per sample of
+// its own, "at or above theta now", in a register: the row's next spike is the smallest sample with a bit set (a
+// minimum over the row's lanes by lane-permuting moves), every visit is a spike, and the lanes add the response to
+// their own samples in LDS, all taps at once, and renew those samples' bits from the sums.  The bits stay exact
+// whatever the signs of the taps, so no tap has to be negative.  The fp32 additions are those of the sequential loop
+// in its order (taps outside the kernel are -0.0f, whose addition changes nothing), hence bit-exact.  Padding behind
+// a row is NaN: never at or above theta.
+// Bound: HBM traffic for short rows; on (12,16,34,34,300) with 11 taps 126-133 us against 143-154 us for the tile
+// kernel (candidate by candidate, every sample written back); not rewriting the blocks of u that no response reached
+// is 15-18 us of that.  Long rows: the chain of LDS round trips from spike to
+// spike, about 0.35 us a spike with one wavefront per SIMD: (4,16,32,32,1450) 262-285 us (tile kernel: 1010 us),
+// (12,512,1,1,350) 13-17 us (25 us); 110 taps on (12,16,32,32,300) 125-140 us (ring kernel: 2400-3400 us).
+template <int PARTS>
+__device__ __forceinline__ uint32_t row_min(uint32_t x)   // minimum over the PARTS lanes of a row
+{
+    auto step = [](uint32_t v, auto perm) {
+        const int o = __builtin_amdgcn_update_dpp(-1, static_cast<int>(v), decltype(perm)::value, 0xf, 0xf, false);
+        return min(v, static_cast<uint32_t>(o));
+    };
+    x = step(x, std::integral_constant<int, 0xb1>{});    // quad_perm [1,0,3,2]
+    x = step(x, std::integral_constant<int, 0x4e>{});    // quad_perm [2,3,0,1]
+    x = step(x, std::integral_constant<int, 0x141>{});   // row_half_mirror
+    if constexpr (PARTS >= 16) x = step(x, std::integral_constant<int, 0x140>{});   // row_mirror
+    if constexpr (PARTS >= 32) {
+        const uint32_t a = min(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 0)),
+                               static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 16)));
+        const uint32_t b = min(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 32)),
+                               static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 48)));
+        x = PARTS == 64 ? min(a, b) : threadIdx.x < 32 ? a : b;
+    }
+    return x;
+}
+
+// The sample that lane k of each row keeps, in all the row's lanes (8 or 16 lanes per row).
+template <int PARTS>
+__device__ __forceinline__ float row_sample(float x, int k)
+{
+    const int in = __builtin_bit_cast(int, x);
+    int q = 0;
+    if constexpr (PARTS == 16) {
+        switch (k) {
+#define SLAYER_ROW_BCAST(n) case n: q = __builtin_amdgcn_update_dpp(0, in, 0x150 + n, 0xf, 0xf, false); break
+            SLAYER_ROW_BCAST(0); SLAYER_ROW_BCAST(1); SLAYER_ROW_BCAST(2); SLAYER_ROW_BCAST(3);
+            SLAYER_ROW_BCAST(4); SLAYER_ROW_BCAST(5); SLAYER_ROW_BCAST(6); SLAYER_ROW_BCAST(7);
+            SLAYER_ROW_BCAST(8); SLAYER_ROW_BCAST(9); SLAYER_ROW_BCAST(10); SLAYER_ROW_BCAST(11);
+            SLAYER_ROW_BCAST(12); SLAYER_ROW_BCAST(13); SLAYER_ROW_BCAST(14); SLAYER_ROW_BCAST(15);
+#undef SLAYER_ROW_BCAST
+        }
+    } else {
+        switch (k % 4) {   // quad_perm: the four lanes of a quad read its lane k % 4
+            case 0: q = __builtin_amdgcn_update_dpp(0, in, 0x00, 0xf, 0xf, false); break;
+            case 1: q = __builtin_amdgcn_update_dpp(0, in, 0x55, 0xf, 0xf, false); break;
+            case 2: q = __builtin_amdgcn_update_dpp(0, in, 0xaa, 0xf, 0xf, false); break;
+            default: q = __builtin_amdgcn_update_dpp(0, in, 0xff, 0xf, 0xf, false); break;
+        }
+        // the quad that does not keep the sample takes it from the other one: lane i of each group of 8 reads lane 7 - i
+        // (row_half_mirror), written only in the quads that need it
+        if (k < 4) q = __builtin_amdgcn_update_dpp(q, q, 0x141, 0xf, 0xa, false);
+        else q = __builtin_amdgcn_update_dpp(q, q, 0x141, 0xf, 0x5, false);
+    }
+    return __builtin_bit_cast(float, q);
+}
+
+template <int PARTS, int ROUNDS, typename Bits>
+__global__ __launch_bounds__(64) void spike_rows_kernel(float *__restrict__ s, float *u, const float *__restrict__ nu,
+                                                        int64_t rows, int T, int nuSize, int P, int NB, int roundsArg,
+                                                        FastDiv byNV, float theta, float Ts, SpikeDelay dl)
+{
+    constexpr int R = kWave / PARTS;
+    constexpr int BATCH = ROUNDS ? ROUNDS : 4;
+    constexpr bool kDenseWalk = PARTS <= 16 && ROUNDS != 0;
+    const int rounds = ROUNDS ? ROUNDS : roundsArg;   // blocks that a response reaches, a multiple of BATCH
+    extern __shared__ __align__(16) float lds[];
+    float *tile = lds;                                                                   // [R][P]
+    uint32_t *spikes = reinterpret_cast<uint32_t *>(lds + R * P);                        // [sizeof(Bits) / 4][R][PARTS]
+    uint32_t *dirtyBlocks = spikes + sizeof(Bits) / 4 * kWave;                           // [R][2]
+    int *rowShift = reinterpret_cast<int *>(dirtyBlocks + 2 * R);                        // [R]
+    float *taps = reinterpret_cast<float *>(rowShift + R);                               // taps[j] = nu[j - (PARTS - 1)]
+
+    const int lane = threadIdx.x;
+    const int cr = lane / PARTS, part = lane % PARTS;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * R;
+    const int nRows = static_cast<int>(min(static_cast<int64_t>(R), rows - row0));
+    const float amplitude = 1.0f / Ts;
+    const BufferRsrc bufU = make_buffer(u + row0 * T), bufS = make_buffer(s + row0 * T);
+    const int nv = T >> 2, total = nRows * nv, rem = T & 3;
+
+    constexpr int kLoads = 10;
+    for (int i0 = lane; i0 < total; i0 += kLoads * kWave) {
+        float4 x[kLoads];
+        int at[kLoads];
+#pragma unroll
+        for (int b = 0; b < kLoads; ++b) {
+            const int i = i0 + b * kWave;
+            const int r = static_cast<int>(fastdiv(static_cast<uint32_t>(i), byNV)), c = i - r * nv;
+            x[b] = buffer_load4(bufU, masked_offset(i < total, (r * T + 4 * c) * 4), 0);
+            at[b] = r * P + 4 * c;
+        }
+#pragma unroll
+        for (int b = 0; b < kLoads; ++b)
+            if (i0 + b * kWave < total) *reinterpret_cast<float4 *>(tile + at[b]) = x[b];
+    }
+    if (rem && cr < nRows && part < rem) tile[cr * P + 4 * nv + part] = buffer_load(bufU, (cr * T + 4 * nv + part) * 4, 0);
+    for (int c = T + part; c < P; c += PARTS) tile[cr * P + c] = __builtin_nanf("");
+    for (int j = lane; j < (rounds + 1) * PARTS; j += kWave) {
+        const int tj = j - (PARTS - 1);
+        taps[j] = (tj >= 0 && tj < nuSize) ? nu[tj] : -0.0f;
+    }
+    if (dl.on && lane < nRows) {
+        const float d = dl.lut ? dl.lut[(row0 + lane) % dl.lutSize] : dl.delay;
+        rowShift[lane] = max(-(1 << 24), min(1 << 24, delay_steps(d, dl.Ts)));
+    }
+    wave_sync();
+
+    // One bit per block of PARTS samples: this lane's sample is at or above theta / has fired; some sample of the
+    // block has changed.
+    float *mine = tile + cr * P + part;
+    Bits above = 0, fired = 0, dirty = 0;
+#pragma unroll 8
+    for (int b = 0; b < NB; ++b) above |= static_cast<Bits>(mine[b * PARTS] >= theta ? 1 : 0) << b;
+    if (cr >= nRows) above = 0;
+    const Bits reach = (static_cast<Bits>(1) << rounds) - 1;
+    const float *tapOf = taps + (PARTS - 1) + part;
+    auto first_of = [](Bits m) { return sizeof(Bits) == 8 ? __builtin_ctzll(m) : __builtin_ctz(static_cast<uint32_t>(m)); };
+    const uint32_t none = static_cast<uint32_t>(NB * PARTS);   // a row without further spikes works on its padding
+    // Going from spike to spike takes a tile about 45 instructions per spike of its busiest row; the walk over every sample
+    // about 8 per sample, whatever fires.  The number of spikes is not known, but the samples at or above theta bound
+    // it: tiles with a row that arrives above theta for more than three fifths of its samples take the latter.
+    // (Pooled potentials on (12,16,32,32,300) firing 14, 31 and 62 % of the time, 50, 81 and 96 % above theta: 197, 308
+    // and 491 us from spike to spike, 164 us sample by sample; firing 6 %, 29 % above: 132 and 168 us.)
+    bool dense = false;
+    if constexpr (kDenseWalk) {
+        int count = __builtin_popcountll(static_cast<uint64_t>(above));
+#pragma unroll
+        for (int off = PARTS / 2; off > 0; off >>= 1) count += __shfl_xor(count, off, kWave);
+        if (__builtin_amdgcn_ballot_w64(count * 5 > T * 3) != 0u) {
+            bool lowers = true;
+            for (int j = lane; j < (rounds + 1) * PARTS; j += kWave)
+                lowers = lowers && taps[j] <= 0.0f && taps[j] > -__builtin_inff() && (__builtin_bit_cast(uint32_t, taps[j]) >> 31) != 0u;
+            dense = __builtin_amdgcn_ballot_w64(!lowers) == 0u;
+        }
+    }
+    if constexpr (kDenseWalk) {
+        if (dense) {
+            // 32 samples at a time in registers, as they lie in the row's lanes; the sample under test is broadcast to
+            // them by lane-permuting moves and the response added as fma(1 or 0, tap, sample) - the addition when the
+            // sample fired, and no change (zeros and their signs included: the taps are negative or -0.0) when not.
+            constexpr int kBlocks = 32 / PARTS;
+            float tq[PARTS][BATCH];   // tq[k][i]: what a spike at lane k's sample adds to this lane's, i blocks on
+#pragma unroll
+            for (int k = 0; k < PARTS; ++k)
+#pragma unroll
+                for (int i = 0; i < BATCH; ++i) tq[k][i] = tapOf[i * PARTS - k];
+            for (int b0 = 0; b0 < NB; b0 += kBlocks) {
+                float w[kBlocks + BATCH - 1];
+#pragma unroll
+                for (int m = 0; m < kBlocks + BATCH - 1; ++m) w[m] = mine[(b0 + m) * PARTS];
+                float hit[2] = {0.0f, 0.0f};   // the spikes as sums of powers of two (one instruction each)
+#pragma unroll
+                for (int k = 0; k < 32; ++k) {
+                    const bool f = row_sample<PARTS>(w[k / PARTS], k % PARTS) >= theta;
+                    const float one = f ? 1.0f : 0.0f;
+                    hit[k / 16] = __builtin_fmaf(one, static_cast<float>(1u << (k % 16)), hit[k / 16]);
+#pragma unroll
+                    for (int i = 0; i < BATCH; ++i) w[k / PARTS + i] = __builtin_fmaf(one, tq[k % PARTS][i], w[k / PARTS + i]);
+                }
+#pragma unroll
+                for (int m = 0; m < kBlocks + BATCH - 1; ++m) mine[(b0 + m) * PARTS] = w[m];
+                const uint32_t hits = static_cast<uint32_t>(hit[0]) | static_cast<uint32_t>(hit[1]) << 16;
+#pragma unroll
+                for (int m = 0; m < kBlocks; ++m) fired |= static_cast<Bits>((hits >> (m * PARTS + part)) & 1u) << (b0 + m);
+            }
+            dirty = ~static_cast<Bits>(0);
+            above = 0;
+        }
+    }
+    while (true) {
+        const uint32_t t = row_min<PARTS>(above != 0 ? static_cast<uint32_t>(first_of(above) * PARTS + part) : none);
+        if (__builtin_amdgcn_ballot_w64(t != none) == 0u) break;
+        const int b = static_cast<int>(t / PARTS), k = static_cast<int>(t % PARTS);
+        float *q = mine + b * PARTS;
+        const float *tp = tapOf - k;
+        Bits now = 0;
+        for (int i0 = 0; i0 < rounds; i0 += BATCH) {
+            float val[BATCH], tv[BATCH];
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) {
+                val[i] = q[(i0 + i) * PARTS];
+                tv[i] = tp[(i0 + i) * PARTS];
+            }
+            uint32_t up = 0u;
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) {
+                const float x = val[i] + tv[i];
+                q[(i0 + i) * PARTS] = x;
+                up |= x >= theta ? 1u << i : 0u;
+            }
+            if (i0 == 0) up &= part > k ? ~0u : ~1u;   // (samples up to the spike are done)
+            now |= static_cast<Bits>(up) << i0;
+        }
+        const Bits hit = reach << b;
+        above = (above & ~hit) | (now << b);
+        dirty |= hit;
+        fired |= static_cast<Bits>(part == k ? 1 : 0) << b;
+    }
+    spikes[lane] = static_cast<uint32_t>(fired);
+    if constexpr (sizeof(Bits) == 8) spikes[kWave + lane] = static_cast<uint32_t>(static_cast<uint64_t>(fired) >> 32);
+    if (part == 0) {
+        dirtyBlocks[2 * cr] = static_cast<uint32_t>(dirty);
+        dirtyBlocks[2 * cr + 1] = static_cast<uint32_t>(static_cast<uint64_t>(dirty) >> 32);
+    }
+    wave_sync();
+
+    // retire.  Samples no response has reached are still in memory as they came: a 64-byte block of u that lies within
+    // one row and holds no changed sample is not written again.
+    const int skew = static_cast<int>((reinterpret_cast<uintptr_t>(u) / 4 + static_cast<uint64_t>(row0) * T) & 15u);
+    auto spike_at = [&](int r, int c) -> bool {   // whether sample c of row r fired (false outside the row)
+        if (c < 0 || c >= T) return false;
+        const int b = c / PARTS;
+        return (spikes[(b >> 5) * kWave + r * PARTS + c % PARTS] >> (b & 31)) & 1u;
+    };
+    constexpr int kStores = 5;
+    for (int i0 = lane; i0 < total; i0 += kStores * kWave) {
+#pragma unroll
+        for (int b2 = 0; b2 < kStores; ++b2) {
+            const int i = i0 + b2 * kWave;
+            const bool on = i < total;
+            const int r = on ? static_cast<int>(fastdiv(static_cast<uint32_t>(i), byNV)) : 0, c = on ? 4 * (i - r * nv) : 0;
+            const int inBlock = (skew + r * T + c) & 15;
+            const int lo = c - inBlock;   // first sample of the vector's first 64-byte block
+            const int hi = lo + (inBlock > 12 ? 31 : 15);   // (an unaligned vector may lie in two)
+            const int loB = lo / PARTS, hiB = hi / PARTS;
+            const uint64_t d = (static_cast<uint64_t>(dirtyBlocks[2 * r + 1]) << 32) | dirtyBlocks[2 * r];
+            const bool clean = lo >= 0 && hi < T && ((static_cast<uint32_t>(d >> loB)) & ((2u << (hiB - loB)) - 1u)) == 0u;
+            float4 sv;
+            if (dl.on) {
+                const int c2 = c - rowShift[r];
+                sv = make_float4(spike_at(r, c2) ? amplitude : 0.0f, spike_at(r, c2 + 1) ? amplitude : 0.0f,
+                                 spike_at(r, c2 + 2) ? amplitude : 0.0f, spike_at(r, c2 + 3) ? amplitude : 0.0f);
+            } else {
+                const int b = c / PARTS;
+                const uint4 w = *reinterpret_cast<const uint4 *>(spikes + (b >> 5) * kWave + r * PARTS + c % PARTS);
+                const uint32_t bit = 1u << (b & 31);
+                sv = make_float4((w.x & bit) ? amplitude : 0.0f, (w.y & bit) ? amplitude : 0.0f,
+                                 (w.z & bit) ? amplitude : 0.0f, (w.w & bit) ? amplitude : 0.0f);
+            }
+            const int off = masked_offset(on, (r * T + c) * 4);
+            buffer_store4(bufU, clean ? kOutOfRange : off, 0, *reinterpret_cast<const float4 *>(tile + r * P + c));
+            buffer_store4(bufS, off, 0, sv);
+        }
+    }
+    if (rem && cr < nRows && part < rem) {
+        const int c = 4 * nv + part, off = (cr * T + c) * 4;
+        buffer_store(bufU, off, 0, tile[cr * P + c]);
+        buffer_store(bufS, off, 0, spike_at(cr, dl.on ? c - rowShift[cr] : c) ? amplitude : 0.0f);
     }
 }
 
@@ -854,8 +1009,69 @@ __global__ __launch_bounds__(256) void spike_bwd_scalar_kernel(float *gradIn, co
 
 namespace slayer {
 
-// Picks and launches the spike kernel.  With a shift of the output (dl.on) only the tile kernel with
-// whole rows qualifies; other shapes return SLAYER_EUNSUPPORTED before anything is launched.
+constexpr int kRowsPiecesFrom = 1600;
+
+// The whole-row kernel for rows whose blocks fit the bit registers; SLAYER_EUNSUPPORTED when they do not (rows beyond
+// 4032 samples).  Lanes per row: 8 for short refractory kernels, 16 for long ones (fewer trips per spike), more while
+// a tile would take over 11 KB of LDS (fewer than 14 tiles per compute unit: (12,16,34,34,496) takes 228 us with 8
+// lanes and 194 us with 16) or the tensor has too few rows for four wavefronts per compute unit.
+static int launch_spike_rows(float *s, float *u, const float *nu, int64_t nNeurons, int64_t T, int64_t nuSize,
+                             float theta, float Ts, hipStream_t st, const SpikeDelay &dl)
+{
+    if (T > 4096 || nuSize > 4096) return SLAYER_EUNSUPPORTED;
+    int parts = nuSize <= 24 ? 8 : 16;
+    int rounds, NB, P;
+    size_t lds;
+    for (;; parts *= 2) {
+        rounds = static_cast<int>((nuSize + 2 * parts - 2) / parts);
+        if (rounds < 2) rounds = 2;
+        if (rounds > 3) rounds = (rounds + 3) & ~3;
+        NB = static_cast<int>(ceil_div(T, parts));
+        P = (NB + rounds) * parts;
+        while (P % 64 != parts % 64) P += parts;   // (the rows of a tile start in different banks)
+        const int R = kWave / parts;
+        lds = (static_cast<size_t>(R) * P + 2 * kWave + 3 * R + (rounds + 1) * parts) * sizeof(float);
+        const bool fits = NB <= 63 && rounds <= 60;
+        if (parts == 64) {
+            if (!fits) return SLAYER_EUNSUPPORTED;
+            break;
+        }
+        if (fits && lds <= 11 * 1024 && ceil_div(nNeurons, R) >= 4 * compute_units()) break;
+    }
+    const int R = kWave / parts;
+    const int64_t groups = ceil_div(nNeurons, R);
+    if (groups >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
+    const FastDiv byNV = make_fastdiv(static_cast<uint32_t>(T >= 4 ? T / 4 : 1));
+    const dim3 grid(static_cast<unsigned>(groups));
+    const bool small = NB <= 31 && rounds <= 31;
+#define SLAYER_SPIKE_ROWS(PV, RV, BV)                                                                                  \
+    hipLaunchKernelGGL((spike_rows_kernel<PV, RV, BV>), grid, dim3(kWave), lds, st, s, u, nu, nNeurons, static_cast<int>(T), \
+                       static_cast<int>(nuSize), P, NB, rounds, byNV, theta, Ts, dl)
+#define SLAYER_SPIKE_ROWS_OF(PV)                                                                                        \
+    do {                                                                                                                \
+        if (small) {                                                                                                    \
+            if (rounds == 2) SLAYER_SPIKE_ROWS(PV, 2, uint32_t);                                                        \
+            else if (rounds == 3) SLAYER_SPIKE_ROWS(PV, 3, uint32_t);                                                   \
+            else SLAYER_SPIKE_ROWS(PV, 0, uint32_t);                                                                    \
+        } else {                                                                                                        \
+            if (rounds == 2) SLAYER_SPIKE_ROWS(PV, 2, uint64_t);                                                        \
+            else if (rounds == 3) SLAYER_SPIKE_ROWS(PV, 3, uint64_t);                                                   \
+            else SLAYER_SPIKE_ROWS(PV, 0, uint64_t);                                                                    \
+        }                                                                                                               \
+    } while (0)
+    switch (parts) {
+        case 8: SLAYER_SPIKE_ROWS_OF(8); break;
+        case 16: SLAYER_SPIKE_ROWS_OF(16); break;
+        case 32: SLAYER_SPIKE_ROWS_OF(32); break;
+        default: SLAYER_SPIKE_ROWS_OF(64); break;
+    }
+#undef SLAYER_SPIKE_ROWS_OF
+#undef SLAYER_SPIKE_ROWS
+    return launch_status();
+}
+
+// Picks and launches the spike kernel.  A shift of the output (dl.on) is done by the whole-row kernel and by the tile
+// kernel on rows of whole vectors; other shapes return SLAYER_EUNSUPPORTED before anything is launched.
 static int launch_get_spikes(float *s, float *u, const float *nu, int64_t nNeurons, int64_t T, int64_t nuSize,
                              float theta, float Ts, hipStream_t st, const SpikeDelay &dl)
 {
@@ -863,93 +1079,73 @@ static int launch_get_spikes(float *s, float *u, const float *nu, int64_t nNeuro
     const int64_t groups = ceil_div(nNeurons, kWave);
     const bool stream_ok = !generic_forced() && T < (1LL << 30) && groups < (1LL << 31);
     const bool window_ok = stream_ok && T <= kBufferMaxT;
-#define SLAYER_SPIKE_TILE_LAUNCH(NU, LAGV, RV)                                                           \
-    do {                                                                                                \
-        if (vec)                                                                                        \
-            hipLaunchKernelGGL((spike_tile_kernel<NU, kTileVec, LAGV, RV>), dim3(grid), dim3(kWave),    \
-                               lds, st, s, u, nu, nNeurons, static_cast<int>(T),                        \
-                               static_cast<int>(nuSize), Tc, P, MP, MPT, tiles, theta, Ts, dl);         \
-        else if (flat && RV == 8)                                                                       \
-            hipLaunchKernelGGL((spike_tile_kernel<NU, (RV == 8 ? kTileFlat : kTileScalar), LAGV, RV>),  \
-                               dim3(grid), dim3(kWave), lds, st, s, u, nu, nNeurons,                    \
-                               static_cast<int>(T), static_cast<int>(nuSize), Tc, P, MP, MPT, tiles,    \
-                               theta, Ts, dl);                                                          \
-        else                                                                                            \
-            hipLaunchKernelGGL((spike_tile_kernel<NU, kTileScalar, LAGV, RV>), dim3(grid), dim3(kWave), \
-                               lds, st, s, u, nu, nNeurons, static_cast<int>(T),                        \
-                               static_cast<int>(nuSize), Tc, P, MP, MPT, tiles, theta, Ts, dl);         \
-        return launch_status();                                                                         \
-    } while (0)
-#define SLAYER_SPIKE_TILE_LAG(NU, LAGV)                                                                  \
-    do {                                                                                                \
-        /* Rows that travel whole: 8-row tiles, one work-group per tile - many short-lived groups per   \
-           CU overlap the memory phases of some with the walks of others better than a loop does.       \
-           Rows in pieces: the group loops over the pieces; 16 rows per tile and pieces of 256 samples  \
-           unless that would leave wavefront slots of the GPU empty: then 8 rows and, for rows of whole \
-           vectors, pieces of 512 samples, which doubles the bytes in flight per wavefront. */          \
-        int Tc = whole ? static_cast<int>(T) : kTilePiece16;                                            \
-        int cols, P, MP;                                                                                \
-        auto layout = [&]() {                                                                           \
-            cols = (LAGV + Tc + 31) & ~31; /* the walk goes in groups of 32 columns */                  \
-            /* 4 (mod 8): rows are 16-byte aligned and 8 of them start in different banks; a refractory \
-               response that is added in place may reach NU - 1 columns past the last one */           \
-            P = cols + 4;                                                                               \
-            while (P - (LAGV + Tc) < NU - 1) P += 8;                                                    \
-            MP = cols / 32 + 1;                                                                         \
-        };                                                                                              \
-        layout();                                                                                       \
-        const int64_t slots16 = static_cast<int64_t>(cus) * (160 * 1024 / ((16LL * P + 32 * MP + 16) * 4)); \
-        const int rowsPerTile = (!whole && ceil_div(nNeurons, 16) >= slots16) ? 16 : 8;                 \
-        if (!whole && rowsPerTile == 8 && vec) {                                                        \
-            Tc = kTilePiece8;                                                                           \
-            layout();                                                                                   \
-        }                                                                                               \
-        /* shifted spikes of rows in pieces: the spike bits of whole rows stay in LDS */                \
-        const int MPT = (dl.on && !whole) ? static_cast<int>((T + LAGV + 31) / 32 + 1) : 0;             \
-        auto lds_bytes = [&]() {                                                                        \
-            /* tile, spike and candidate bits, row shifts, whole rows' spike bits, the padded kernel */  \
-            return (static_cast<size_t>(rowsPerTile) * P + 2 * rowsPerTile * MP + rowsPerTile +         \
-                    static_cast<size_t>(rowsPerTile) * MPT + 48) * sizeof(float);                       \
-        };                                                                                              \
-        /* eight wavefronts per compute unit are what the 8-row tiles of a small tensor need to be      \
-           resident all at once: shorter pieces if the tile does not fit an eighth of the LDS */        \
-        while (!whole && rowsPerTile == 8 && vec && Tc > kTilePiece16 && lds_bytes() > 160 * 1024 / 8) { \
-            Tc -= 32;                                                                                   \
-            layout();                                                                                   \
-        }                                                                                               \
-        const size_t lds = lds_bytes();                                                                 \
-        const int64_t tiles = ceil_div(nNeurons, rowsPerTile);                                          \
-        const int64_t resident = static_cast<int64_t>(cus) * (160 * 1024 / static_cast<int64_t>(lds));  \
-        if (tiles >= (1LL << 31)) return SLAYER_EUNSUPPORTED;                                           \
-        const unsigned grid = static_cast<unsigned>((whole || tiles < resident) ? tiles : resident);    \
-        if (rowsPerTile == 16) SLAYER_SPIKE_TILE_LAUNCH(NU, LAGV, 16);                                  \
-        SLAYER_SPIKE_TILE_LAUNCH(NU, LAGV, 8);                                                          \
-    } while (0)
-#define SLAYER_SPIKE_TILE(NU)                                                                            \
-    do {                                                                                                \
-        if (whole) SLAYER_SPIKE_TILE_LAG(NU, ((NU + 2) & ~3));                                          \
-        SLAYER_SPIKE_TILE_LAG(NU, 32);                                                                  \
-    } while (0)
-    // a shifted output: rows that travel whole, or rows of whole vectors whose spike bits fit into LDS
-    if (dl.on && !(window_ok && nuSize <= 24 &&
-                   (T <= kTileMaxPiece || (T <= kSpikeRecordMaxT && T % 4 == 0 && aligned16(s) && aligned16(u)))))
-        return SLAYER_EUNSUPPORTED;
+    const bool vec = T % 4 == 0 && aligned16(s) && aligned16(u);
+    // Long rows of whole vectors with a short kernel, and enough of them to fill the GPU, go in pieces: 16384 rows of
+    // 2000 samples take 98 us that way and 107 us whole (of 1500: 79 and 80; 2048 rows of 2000: 41 and 24).
+    const bool pieces = vec && nuSize <= 24 && T > kRowsPiecesFrom && nNeurons >= 8192 && (!dl.on || T <= kSpikeRecordMaxT);
+    if (window_ok && !pieces) {
+        const int status = launch_spike_rows(s, u, nu, nNeurons, T, nuSize, theta, Ts, st, dl);
+        if (status != SLAYER_EUNSUPPORTED) return status;
+    }
+    // a shifted output of rows in pieces: rows of whole vectors whose spike bits fit into LDS
+    if (dl.on && !(window_ok && nuSize <= 24 && vec && T <= kSpikeRecordMaxT)) return SLAYER_EUNSUPPORTED;
     if (window_ok && nuSize <= 24) {
-        // short rows travel whole; long rows in pieces
-        const bool whole = T <= kTileMaxPiece;
-        const bool vec = (T % 4 == 0) && aligned16(s) && aligned16(u);
-        // whole rows that are not whole vectors, in a tensor that is: 8-row tiles are aligned runs
-        const bool flat = whole && !vec && T >= 4 && (nNeurons * T) % 4 == 0 && aligned16(s) && aligned16(u);
+        // 16 rows per tile and pieces of 256 samples unless that would leave wavefront slots of the GPU empty: then 8
+        // rows and, for rows of whole vectors, pieces of 512 samples, which doubles the bytes in flight per wavefront
         const int cus = compute_units();
+        int Tc = kTilePiece16, P = 0, MP = 0;
+        auto layout = [&]() {
+            const int cols = (kTileLag + Tc + 31) & ~31;  // the walk goes in groups of 32 columns
+            // 4 (mod 8): rows are 16-byte aligned and 8 of them start in different banks; a refractory response that
+            // is added in place may reach 23 columns past the last one
+            P = cols + 4;
+            while (P - (kTileLag + Tc) < 23) P += 8;
+            MP = cols / 32 + 1;
+        };
+        layout();
+        const int64_t slots16 = static_cast<int64_t>(cus) * (160 * 1024 / ((16LL * P + 32 * MP + 16) * 4));
+        const int rowsPerTile = ceil_div(nNeurons, 16) >= slots16 ? 16 : 8;
+        if (rowsPerTile == 8 && vec) {
+            Tc = kTilePiece8;
+            layout();
+        }
+        // shifted spikes: the spike bits of whole rows stay in LDS
+        const int MPT = dl.on ? static_cast<int>((T + kTileLag + 31) / 32 + 1) : 0;
+        auto lds_bytes = [&]() {
+            // tile, spike and candidate bits, row shifts, whole rows' spike bits, the padded kernel
+            return (static_cast<size_t>(rowsPerTile) * P + 2 * rowsPerTile * MP + rowsPerTile +
+                    static_cast<size_t>(rowsPerTile) * MPT + 48) * sizeof(float);
+        };
+        // eight wavefronts per compute unit are what the 8-row tiles of a small tensor need to be resident all at once:
+        // shorter pieces if the tile does not fit an eighth of the LDS
+        while (rowsPerTile == 8 && vec && Tc > kTilePiece16 && lds_bytes() > 160 * 1024 / 8) {
+            Tc -= 32;
+            layout();
+        }
+        const size_t lds = lds_bytes();
+        const int64_t tiles = ceil_div(nNeurons, rowsPerTile);
+        const int64_t resident = static_cast<int64_t>(cus) * (160 * 1024 / static_cast<int64_t>(lds));
+        if (tiles >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
+        const dim3 grid(static_cast<unsigned>(tiles < resident ? tiles : resident));
+#define SLAYER_SPIKE_TILE_LAUNCH(NU, VECV, RV)                                                                        \
+    hipLaunchKernelGGL((spike_tile_kernel<NU, VECV, RV>), grid, dim3(kWave), lds, st, s, u, nu, nNeurons,             \
+                       static_cast<int>(T), static_cast<int>(nuSize), Tc, P, MP, MPT, tiles, theta, Ts, dl)
+#define SLAYER_SPIKE_TILE(NU)                                                 \
+    do {                                                                      \
+        if (vec && rowsPerTile == 16) SLAYER_SPIKE_TILE_LAUNCH(NU, true, 16); \
+        else if (vec) SLAYER_SPIKE_TILE_LAUNCH(NU, true, 8);                  \
+        else if (rowsPerTile == 16) SLAYER_SPIKE_TILE_LAUNCH(NU, false, 16);  \
+        else SLAYER_SPIKE_TILE_LAUNCH(NU, false, 8);                          \
+        return launch_status();                                               \
+    } while (0)
         if (nuSize <= 4) SLAYER_SPIKE_TILE(4);
         if (nuSize <= 8) SLAYER_SPIKE_TILE(8);
         if (nuSize <= 12) SLAYER_SPIKE_TILE(12);
         if (nuSize <= 16) SLAYER_SPIKE_TILE(16);
         SLAYER_SPIKE_TILE(24);
-    }
 #undef SLAYER_SPIKE_TILE
-#undef SLAYER_SPIKE_TILE_LAG
 #undef SLAYER_SPIKE_TILE_LAUNCH
+    }
     if (stream_ok && nuSize <= 33) {
         hipLaunchKernelGGL(spike_stream_kernel<64>, dim3(static_cast<unsigned>(groups)), dim3(kWave), 0,
                            st, s, u, nu, nNeurons, static_cast<int>(T), static_cast<int>(nuSize), theta,

@@ -628,6 +628,33 @@ def test_spikes_bit_exact(impl, shape, nuSize):
     assert want_s.sum() > 0 or shape[-1] < 8
 
 
+@pytest.mark.parametrize("rows,T,nuSize", [
+    # whole rows: every number of lanes per row (8 to 64, by taps, row length and number of rows), rows that start off
+    # 16-byte boundaries, one to three samples behind the last vector, the last block of bits full and nearly empty
+    (9000, 40, 11), (9000, 173, 11), (9000, 250, 11), (9000, 301, 24), (8200, 303, 40), (4100, 497, 5), (4099, 248, 25),
+    (2100, 1002, 24), (2100, 1007, 64), (37, 1450, 110), (5, 1984, 11), (5, 2016, 12), (3, 2017, 300), (2, 4030, 16),
+    (3, 4032, 111), (1, 3, 2), (70, 1, 1), (7, 2, 300),
+    # just beyond: the ring and the generic kernel, and rows in pieces
+    (3, 4033, 11), (3, 4036, 40), (3, 4033, 110), (8192, 1604, 11), (8195, 2000, 24), (8192, 1600, 11)])
+@pytest.mark.parametrize("kind", ["lowering", "raising", "smooth"])
+def test_spikes_whole_rows_bit_exact(rows, T, nuSize, kind):
+    rng = np.random.default_rng(rows + T + nuSize)
+    u = (rng.standard_normal((1, rows, 1, 1, T)) * 6).astype(np.float32)
+    nu = (-rng.random(nuSize) * 12).astype(np.float32)
+    if kind == "raising":       # taps of both signs, a NaN and an infinity among the samples
+        nu = (rng.standard_normal(nuSize) * 0.5 - 0.3).astype(np.float32)
+        u.reshape(-1)[T // 2] = np.nan
+        u.reshape(-1)[-1] = np.inf
+    if kind == "smooth":        # above the threshold for runs of samples, whole rows without a spike
+        u = (np.sin(np.arange(T) / 9.0) * 14 * (np.arange(rows) % 3 != 1)[:, None]).astype(np.float32).reshape(u.shape)
+    want_s, want_u = O.get_spikes(u, nu, 10.0, 1.0)
+    ud = dev(u)
+    s = slayerCuda.getSpikes(ud, dev(nu), 10.0, 1.0)
+    assert np.array_equal(bits(host(s)), bits(want_s))
+    same = (bits(host(ud)) == bits(want_u)) | (np.isnan(host(ud)) & np.isnan(want_u))
+    assert same.all()
+
+
 def test_spikes_dense_firing_and_positive_feedback(impl):
     # every sample above threshold, and a refractory kernel that pushes u up (runaway firing)
     rng = np.random.default_rng(3)
@@ -1030,7 +1057,8 @@ def test_empty_tensors():
 # ------------------------------------------------------------------ spike with the shift fused in
 @pytest.mark.parametrize("shape", [(3, 5, 4, 4, 300), (2, 3, 2, 2, 352), (2, 7, 1, 1, 100), (2, 3, 1, 1, 7),
                                    (4, 3, 2, 2, 350), (1, 9, 1, 1, 33), (2, 4, 1, 1, 2000), (3, 21, 1, 1, 1000),
-                                   (1, 9, 1, 1, 356), (2, 40, 1, 1, 512), (1, 3, 1, 1, 2002)])
+                                   (1, 9, 1, 1, 356), (2, 40, 1, 1, 512), (1, 3, 1, 1, 2002), (2, 4100, 1, 1, 1604),
+                                   (3, 2, 1, 1, 4037)])
 @pytest.mark.parametrize("delay", ["scalar", "negative", "zero", "huge", "table", "one-element", "far", "far-negative",
                                    "long-table"])
 def test_spike_delayed_equals_spike_then_shift(shape, delay, impl):
