@@ -540,6 +540,276 @@ __global__ __launch_bounds__(64, 2) void loihi_lines_kernel(float *__restrict__ 
     }
 }
 
+// ---- pipelined kernel: spikes, or spikes and voltage -----------------------------------------------------
+// The lines kernel's tiles and lines (64 rows, one 128-byte line per row and piece, the line that two rows share going
+// out once and whole), with the work of a piece cut into four stages that the four wavefronts of a work-group run on
+// four consecutive pieces at the same time, one barrier per piece:
+//   load    : lines from memory, kAhead pieces in flight in registers, into the piece's slot in LDS; samples outside
+//             the row, and sample 0, become zeros, which leave a neuron at rest as it is;
+//   current : lane = row, in place in the slot;
+//   voltage : lane = row; spikes as bits, the voltage in place in the slot (if wanted), the first line of every row kept
+//             aside for the row above;
+//   store   : voltage and spikes as whole lines.
+// What sets the pace of a small tensor is the chain of dependent instructions from one voltage to the next, which now
+// shares its wavefront with nothing else: 44 or 16384 rows of 1450 samples take 57 us with the voltage and 42 us without
+// (173 and 159 us in one wavefront per tile), 4096 rows of 300 take 19 and 15 us (45 and 42 us).  On a large tensor
+// memory sets the pace ((8,16,32,32,300): 75 and 55 us; 82 and 59 us).  With the voltage, which stage a wavefront runs
+// depends on its work-group, so that the stages on a compute unit mix over its SIMDs (65536 rows of 1450: 242 us, 262 us
+// without that).
+//
+// Decay: sign(x) * ((|x| * keep) >> 12) = x + ((x * -decay + (x < 0 ? 4095 : 0)) >> 12) while |x| * keep and
+// x * decay + 4095 fit their 32 bits; below 2^20 the upper twelve bits of x are that 4095 or 0.  A piece that leaves
+// this range is computed again in wrap-around arithmetic.
+constexpr int kPipeRows = 64, kPipePitch = 36, kAhead = 3;
+
+// the LDS part of __syncthreads(): loads and stores of global memory stay in flight
+__device__ __forceinline__ void pipe_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__device__ __forceinline__ int loihi_loss(int x, int minusDecay)   // what the decay adds to x
+{
+    int scaled;
+    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(scaled) : "v"(x), "v"(minusDecay), "v"(static_cast<uint32_t>(x) >> 20));
+    return scaled >> 12;
+}
+
+// REF1: a refractory delay of 1 (no step is ever refractory).  VOLT: the voltage is wanted.
+template <bool ELEM, bool REF1, bool VOLT>
+__global__ __launch_bounds__(256) void loihi_pipe_kernel(float *__restrict__ s, float *__restrict__ v,
+                                                         const float *__restrict__ w, int64_t rows, int T, int pieces,
+                                                         int smallI, int smallV, LoihiParams p)
+{
+    constexpr int G = 32, R = kPipeRows, P = kPipePitch;
+    __shared__ __align__(16) int slots[4][R * P];        // input, then current, then voltage of a piece
+    __shared__ __align__(16) int head[VOLT ? R * P : 4]; // voltages of every row's first line
+    __shared__ uint32_t firedBits[2][R], outBits[2][R], headFired[R], headOut[R];
+
+    const int lane = threadIdx.x & 63;
+    const int stage = __builtin_amdgcn_readfirstlane((static_cast<int>(threadIdx.x >> 6) + (VOLT ? static_cast<int>(blockIdx.x >> 8) : 0)) & 3);
+    const int64_t tile = blockIdx.x;
+    const int64_t base = tile * R * static_cast<int64_t>(T);
+    const int nRows = static_cast<int>(min(static_cast<int64_t>(R), rows - tile * R));
+    const int o0 = static_cast<int>((reinterpret_cast<uintptr_t>(w + base) >> 2) & 31);  // row 0 starts so many samples into a line
+    const int subRow = lane >> 3, col = (lane & 7) * 4;   // load and store: 8 rows per access
+    const int steps = pieces + 3;
+
+    if (stage == 0) {
+        const BufferRsrc bufW = make_buffer(w + base);
+        float4 x[kAhead][8];
+        auto issue = [&](float4 (&q)[8], int j) {
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const int r = b * 8 + subRow;
+                const int time = G * j - ((o0 + r * T) & 31) + col;
+                // (any sample of the vector inside the row)
+                q[b] = buffer_load4<kCached>(bufW, masked_offset(r < nRows && time + 3 >= 0 && time < T, (r * T + time) * 4), 0);
+            }
+        };
+        auto commit = [&](float4 (&q)[8], int j) {
+            const bool inside = j >= 1 && G * (j + 1) <= T;
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const int r = b * 8 + subRow;
+                float4 y = q[b];
+                if (!inside) {
+                    const int time = G * j - ((o0 + r * T) & 31) + col;
+                    y.x = time >= 1 && time < T ? y.x : 0.0f;
+                    y.y = time + 1 >= 1 && time + 1 < T ? y.y : 0.0f;
+                    y.z = time + 2 >= 1 && time + 2 < T ? y.z : 0.0f;
+                    y.w = time + 3 >= 1 && time + 3 < T ? y.w : 0.0f;
+                }
+                *reinterpret_cast<float4 *>(&slots[j & 3][r * P + col]) = y;
+            }
+        };
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a) issue(x[a], a);
+        for (int i0 = 0; i0 < steps; i0 += kAhead) {
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                if (i0 + a < steps) {
+                    if (i0 + a < pieces) commit(x[a], i0 + a);
+                    issue(x[a], i0 + a + kAhead);   // (beyond the rows: masked)
+                    pipe_barrier();
+                }
+            }
+        }
+    } else if (stage == 1) {
+        int c = 0;
+        const int minusDecay = static_cast<int>(p.keepI) - 4096;
+        const float most = static_cast<float>(smallI >> p.weightShift);
+        for (int i = 0; i < steps; ++i) {
+            const int j = i - 1;
+            if (j >= 0 && j < pieces) {
+                int4 *mine = reinterpret_cast<int4 *>(&slots[j & 3][lane * P]);
+                int in[G];
+#pragma unroll
+                for (int k = 0; k < G; k += 4) {
+                    const int4 q = mine[k / 4];
+                    in[k] = q.x; in[k + 1] = q.y; in[k + 2] = q.z; in[k + 3] = q.w;
+                }
+                const int before = c;
+                int lo = c, hi = c;
+                float top = 0.0f;
+                int out[G];
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const float x = __builtin_bit_cast(float, in[k]);
+                    top = fmaxf(top, fabsf(x));
+                    const int wi = static_cast<int>(static_cast<uint32_t>(cvt_trunc_sat(x)) << p.weightShift);
+                    c = static_cast<int>(static_cast<uint32_t>(c) + static_cast<uint32_t>(wi) + static_cast<uint32_t>(loihi_loss(c, minusDecay)));
+                    lo = min(lo, c);
+                    hi = max(hi, c);
+                    out[k] = c;
+                }
+                if (__builtin_amdgcn_ballot_w64(lo <= -smallI || hi >= smallI || !(top < most)) != 0u) {
+                    c = before;
+#pragma unroll
+                    for (int k = 0; k < G; ++k) {
+                        c = static_cast<int>(loihi_decay(c, p.keepI) +
+                                             (static_cast<uint32_t>(cvt_trunc_sat(__builtin_bit_cast(float, in[k]))) << p.weightShift));
+                        out[k] = c;
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < G; k += 4) mine[k / 4] = make_int4(out[k], out[k + 1], out[k + 2], out[k + 3]);
+            }
+            pipe_barrier();
+        }
+    } else if (stage == 2) {
+        int volt = 0, countdown = 0;
+        uint32_t prev = 0;
+        const int minusDecay = static_cast<int>(p.keepV) - 4096;
+        for (int i = 0; i < steps; ++i) {
+            const int j = i - 2;
+            if (j >= 0 && j < pieces) {
+                int4 *mine = reinterpret_cast<int4 *>(&slots[j & 3][lane * P]);
+                int cur[G], out[G];
+#pragma unroll
+                for (int k = 0; k < G; k += 4) {
+                    const int4 q = mine[k / 4];
+                    cur[k] = q.x; cur[k + 1] = q.y; cur[k + 2] = q.z; cur[k + 3] = q.w;
+                }
+                const int before = volt, beforeCount = countdown;
+                int lo = volt, hi = volt;
+                uint32_t fired = 0;   // the first sample's bit ends up at the top
+                // the voltage after one step that reached `now`, and the step's spike
+                auto settle = [&](int now) {
+                    if constexpr (REF1) {
+                        const int d = static_cast<int>(static_cast<uint32_t>(p.theta) - static_cast<uint32_t>(now));   // negative: above theta
+                        fired = __builtin_amdgcn_alignbit(fired, static_cast<uint32_t>(d), 31);
+                        volt = now & ~(d >> 31);
+                    } else {
+                        countdown = max(countdown - 1, 0);
+                        const bool quiet = countdown == 0, spike = quiet & (now > p.theta);
+                        volt = (quiet & !spike) ? now : 0;
+                        countdown = spike ? p.refDelay : countdown;
+                        fired = (fired << 1) | (spike ? 1u : 0u);
+                    }
+                };
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const int now = static_cast<int>(static_cast<uint32_t>(volt) + static_cast<uint32_t>(cur[k]) + static_cast<uint32_t>(loihi_loss(volt, minusDecay)));
+                    lo = min(lo, now);
+                    hi = max(hi, now);
+                    settle(now);
+                    if (VOLT) out[k] = volt;
+                }
+                if (__builtin_amdgcn_ballot_w64(lo <= -smallV || hi >= smallV) != 0u) {
+                    volt = before;
+                    countdown = beforeCount;
+                    fired = 0;
+#pragma unroll
+                    for (int k = 0; k < G; ++k) {
+                        const int now = static_cast<int>(loihi_decay(volt, p.keepV) + static_cast<uint32_t>(cur[k]));
+                        if constexpr (REF1) {   // (the difference in settle() could wrap around here)
+                            const bool spike = now > p.theta;
+                            fired = (fired << 1) | (spike ? 1u : 0u);
+                            volt = spike ? 0 : now;
+                        } else {
+                            settle(now);
+                        }
+                        if (VOLT) out[k] = volt;
+                    }
+                }
+                fired = __builtin_bitreverse32(fired);
+                const uint32_t late = loihi_delayed(fired, prev, p.delay);
+                prev = fired;
+                firedBits[j & 1][lane] = fired;
+                outBits[j & 1][lane] = late;
+                if (VOLT) {
+#pragma unroll
+                    for (int k = 0; k < G; k += 4) mine[k / 4] = make_int4(out[k], out[k + 1], out[k + 2], out[k + 3]);
+                }
+                if (j == 0) {
+                    headFired[lane] = fired;
+                    headOut[lane] = late;
+                    if (VOLT) {
+#pragma unroll
+                        for (int k = 0; k < G; k += 4)
+                            *reinterpret_cast<int4 *>(&head[lane * P + k]) = make_int4(out[k], out[k + 1], out[k + 2], out[k + 3]);
+                    }
+                }
+            }
+            pipe_barrier();
+        }
+    } else {
+        const BufferRsrc bufS = make_buffer(s + base);
+        const BufferRsrc bufV = make_buffer(VOLT ? v + base : s + base);
+        const float marker = static_cast<float>(static_cast<int>(p.vDecay));   // reported in place of the voltage at a spike
+        for (int i = 0; i < steps; ++i) {
+            const int j = i - 3;
+            if (j >= 0) {
+                const bool inside = j >= 1 && G * (j + 1) <= T;
+#pragma unroll
+                for (int b = 0; b < 8; ++b) {
+                    const int r = b * 8 + subRow;
+                    const int skew = (o0 + r * T) & 31;
+                    const int time = G * j - skew + col;
+                    bool ok = r < nRows && time >= 0 && time < T;
+                    uint32_t mOut = outBits[j & 1][r], mFired = firedBits[j & 1][r];
+                    int4 q = make_int4(0, 0, 0, 0);
+                    if (VOLT) q = *reinterpret_cast<const int4 *>(&slots[j & 3][r * P + col]);
+                    if (!inside) {
+                        // a row's first line, when shared, goes out with the last line of the row above ..
+                        if (j == 0 && r > 0 && skew > 0) ok = false;
+                        // .. whose last line therefore extends into the row below
+                        const int left = T - (G * j - skew);   // samples of this row from the line's start on
+                        if (left > 0 && left < G) {
+                            const uint32_t own = (1u << left) - 1u;
+                            const bool below = r + 1 < nRows;
+                            const int rb = below ? r + 1 : r;
+                            if (below && time >= T) ok = true;
+                            mOut = (mOut & own) | (below ? headOut[rb] & ~own : 0u);
+                            mFired = (mFired & own) | (below ? headFired[rb] & ~own : 0u);
+                            if (VOLT && time + 3 >= T) {
+                                const int *h = &head[rb * P + col];
+                                if (!ELEM || time >= T) q.x = h[0];
+                                if (!ELEM || time + 1 >= T) q.y = h[1];
+                                if (!ELEM || time + 2 >= T) q.z = h[2];
+                                q.w = h[3];
+                            }
+                        }
+                    }
+                    const int off = masked_offset(ok, (r * T + time) * 4);
+                    mOut >>= col;
+                    mFired >>= col;
+                    if (VOLT)
+                        buffer_store4(bufV, off, 0,
+                                      make_float4((mFired & 1u) ? marker : static_cast<float>(q.x), (mFired & 2u) ? marker : static_cast<float>(q.y),
+                                                  (mFired & 4u) ? marker : static_cast<float>(q.z), (mFired & 8u) ? marker : static_cast<float>(q.w)));
+                    buffer_store4(bufS, off, 0, make_float4((mOut & 1u) ? 1.0f : 0.0f, (mOut & 2u) ? 1.0f : 0.0f,
+                                                            (mOut & 4u) ? 1.0f : 0.0f, (mOut & 8u) ? 1.0f : 0.0f));
+                }
+            }
+            pipe_barrier();
+        }
+    }
+}
+
 }  // namespace slayer
 
 namespace slayer {
@@ -594,6 +864,40 @@ static int launch_loihi(float *s, float *v, float *u, const float *w, int64_t nN
             const int64_t fit = static_cast<int64_t>(compute_units()) * (160 * 1024 / ldsBytes);
             return dim3(static_cast<unsigned>(lineTiles < fit ? lineTiles : fit));
         };
+        // Spikes alone or with the voltage (what the layers ask for).  Large tensors stay with one wavefront per tile where
+        // that is the better one: refractory delays above 1, whose longer step the voltage stage takes alone (131072 rows
+        // of 300, spikes alone: 59 us against 63-70 us), and spikes alone on long rows (65536 rows of 1450: 171 us
+        // against 180 us).
+        const bool large = nNeurons > 2 * kPipeRows * static_cast<int64_t>(compute_units());
+        if (wide && T >= 64 && !(large && (refDelay > 1 || (!v && T > 1000))) && (elem || (vec && samePhase)) && theta >= 0 && theta < (1 << 30) && iDecay <= 4096u && vDecay <= 4096u) {
+            // magnitudes below which the decay is exact without wrap-around
+            auto small = [](uint32_t decay) {
+                const uint32_t keep = 4096u - decay;
+                uint32_t most = 1u << 20;
+                if (keep && 0xffffffffu / keep < most) most = 0xffffffffu / keep;
+                if (decay && (0x7fffffffu - 4095u) / decay < most) most = (0x7fffffffu - 4095u) / decay;
+                return static_cast<int>(most);
+            };
+            const int64_t groups = ceil_div(nNeurons, kPipeRows);
+            if (groups >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
+            const int pieces = static_cast<int>((T + 31 + 31) / 32);   // enough for the most skewed row
+            const dim3 nb(static_cast<unsigned>(groups));
+#define SLAYER_LOIHI_PIPE(ELEM_, REF1_, VOLT_)                                                                           \
+    hipLaunchKernelGGL((loihi_pipe_kernel<ELEM_, REF1_, VOLT_>), nb, dim3(256), 0, st, s, v, w, nNeurons,               \
+                       static_cast<int>(T), pieces, small(iDecay), small(vDecay), p)
+#define SLAYER_LOIHI_PIPE_REF(ELEM_, VOLT_)                  \
+    do {                                                     \
+        if (refDelay == 1) SLAYER_LOIHI_PIPE(ELEM_, true, VOLT_); \
+        else SLAYER_LOIHI_PIPE(ELEM_, false, VOLT_);         \
+    } while (0)
+            if (elem && v) SLAYER_LOIHI_PIPE_REF(true, true);
+            else if (elem) SLAYER_LOIHI_PIPE_REF(true, false);
+            else if (v) SLAYER_LOIHI_PIPE_REF(false, true);
+            else SLAYER_LOIHI_PIPE_REF(false, false);
+#undef SLAYER_LOIHI_PIPE_REF
+#undef SLAYER_LOIHI_PIPE
+            return launch_status();
+        }
 #define SLAYER_LOIHI_LINES(R_, LPP_, MERGE_, ELEM_, OUTS_)                                                           \
     do {                                                                                                             \
         int64_t lineTiles;                                                                                           \

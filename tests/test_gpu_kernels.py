@@ -966,6 +966,25 @@ def test_loihi_parameters_wraparound_and_truncation(impl, params):
         assert np.array_equal(bits(host(a)), bits(b)), name
 
 
+@pytest.mark.parametrize("rows,T", [(1, 64), (3, 68), (64, 65), (65, 100), (63, 127), (129, 96), (130, 350), (200, 1450), (1000, 33 * 32),
+                                    (40000, 67), (40001, 64)])
+@pytest.mark.parametrize("refDelay,delay", [(1, 0), (1, 1), (2, 31), (17, 3)])
+@pytest.mark.parametrize("scale", [1, 40])
+def test_loihi_stages_bit_exact(rows, T, refDelay, delay, scale):
+    """Spikes alone and spikes with the voltage (the layers' calls): tiles of 64 rows with lines that two rows share, one
+    row, partial tiles, rows off 16-byte boundaries, states inside and outside the range of the short arithmetic."""
+    rng = np.random.default_rng(rows + T + refDelay)
+    w = (loihi_input(rng, (1, rows, T), p=0.3) * scale).astype(np.float32)
+    w[:, ::3] = np.abs(w[:, ::3])
+    want_s, want_v, _ = O.loihi_get_spikes(w, 0, 80 * 64, 1024, 128, refDelay)
+    late = O.shift(want_s.reshape(1, rows, 1, 1, T), float(delay), 1.0).reshape(w.shape)
+    s, v, _ = slayerLoihiCuda.getSpikesDelayed(dev(w), 0, 80 * 64, 1024, 128, refDelay, delay, voltage=True, current=False)
+    assert np.array_equal(bits(host(s)), bits(late)) and np.array_equal(bits(host(v)), bits(want_v))
+    s, _, _ = slayerLoihiCuda.getSpikesDelayed(dev(w), 0, 80 * 64, 1024, 128, refDelay, delay, voltage=False, current=False)
+    assert np.array_equal(bits(host(s)), bits(late))
+    assert want_s.sum() > 0
+
+
 @pytest.mark.parametrize("scale", [1, 6, 30, 200])
 @pytest.mark.parametrize("params", [(0, 80 * 64, 1024, 128, 2), (2, 3000 * 64, 64, 16, 1), (3, 100000 * 64, 0, 0, 3),
                                     (1, 5000, 4096, 4096, 1), (0, 5000, 5000, 4097, 1)])
