@@ -47,12 +47,25 @@ struct GatherArgs {
     int KH, KW, Cg, Og;
     int mulH, mulW, offH, offW, stepH, stepW;  // source row numerator = a*mulH + offH + i*stepH
     FastDiv divH, divW;                        // ... divided by the stride in the gradient
-    int P;                                     // vectors per destination channel plane = DH*DW*T/VEC
+    int P;                                     // vectors per destination channel plane = DH*DW*ceil(T/VEC)
     int chunks;                                // work-groups per (n, group, m-block)
     FastDiv byChunks, byMBlocks, byGroups, byTV, byDW;
 };
 
 constexpr int kTapChunk = 256;  // taps of weights held in LDS at a time
+
+// Rows that are not whole vectors: vector tv of a row starts at sample 4 tv, the last one at T - 4.  It overlaps the
+// one before, whose samples it computes again, by the same operations, and stores again with the same value: every
+// load and store is a whole vector within its row whatever T >= 4 is.  Rows (and tensors) then start at any multiple
+// of four bytes, which is all the alignment that the 16-byte buffer accesses ask for.  These kernels are bound by their
+// loads, of which one sample per access issues four times as many.  Measured, one sample -> one vector per access, with
+// rows of 1450 samples and a batch of 4: 2x2 pooling forward / input gradient 145 -> 93 / 149 -> 68 us, 2 -> 16 channels
+// 5x5 on 32x32 pixels 290 -> 155 us; rows of 173 samples, batch of 5, 29x37 pixels: 2 -> 16 channels 64 -> 31 us.
+template <int VEC>
+__device__ __forceinline__ int vec_start(int tv, int T)
+{
+    return VEC == 4 ? min(tv * 4, T - 4) : tv;
+}
 
 template <int VEC> struct TimeVec;
 template <> struct TimeVec<4> {
@@ -114,7 +127,7 @@ __global__ __launch_bounds__(256) void synapse_gather_kernel(GatherArgs g)
     const BufferRsrc srcB = make_buffer(g.src + (static_cast<int64_t>(n) * g.SC + static_cast<int64_t>(grp) * g.Qg) * srcPlane);
     const int rowBytes = g.SW * g.T * 4, pixBytes = g.T * 4;
     const int planeBytes = static_cast<int>(srcPlane) * 4;
-    const int laneBytes = tv * VEC * 4;
+    const int laneBytes = vec_start<VEC>(tv, g.T) * 4;
     const int yNum0 = a * g.mulH + g.offH, xNum0 = b * g.mulW + g.offW;
     // unstrided sources: position and byte offset of the lane before any tap offset, and a buffer
     // that starts at the smallest tap offset
@@ -216,7 +229,7 @@ __global__ __launch_bounds__(256) void synapse_gather_kernel(GatherArgs g)
     const int dstPlaneBytes = static_cast<int>(dstPlane) * 4;
 #pragma unroll
     for (int m = 0; m < MB; ++m)
-        acc[m].store(dstB, masked_offset(live && mb0 + m < g.Mg, (mb0 + m) * dstPlaneBytes + p * VEC * 4));
+        acc[m].store(dstB, masked_offset(live && mb0 + m < g.Mg, (mb0 + m) * dstPlaneBytes + static_cast<int>(pix) * pixBytes + laneBytes));
 }
 
 
@@ -252,7 +265,7 @@ __global__ __launch_bounds__(256) void synapse_gather_row_kernel(GatherArgs g)
     const int p = chunk * 256 + static_cast<int>(threadIdx.x);
     const bool live = p < g.P;
     const uint32_t pg = fastdiv(static_cast<uint32_t>(live ? p : 0), g.byTV);
-    const int tv = (live ? p : 0) - static_cast<int>(pg * g.byTV.d);
+    const int t4 = vec_start<4>((live ? p : 0) - static_cast<int>(pg * g.byTV.d), g.T) * 4;
     const int a = static_cast<int>(fastdiv(pg, g.byDW));
     const int b0 = (static_cast<int>(pg) - a * static_cast<int>(g.byDW.d)) * PX;
 
@@ -267,7 +280,7 @@ __global__ __launch_bounds__(256) void synapse_gather_row_kernel(GatherArgs g)
     int colOff[E];
 #pragma unroll
     for (int e = 0; e < E; ++e)
-        colOff[e] = masked_offset(live && static_cast<unsigned>(x0 + e) < static_cast<unsigned>(g.SW), (x0 + e) * pixBytes + tv * 16);
+        colOff[e] = masked_offset(live && static_cast<unsigned>(x0 + e) < static_cast<unsigned>(g.SW), (x0 + e) * pixBytes + t4);
 
     TimeVec<4> acc[PX][MB];
 #pragma unroll
@@ -339,7 +352,7 @@ __global__ __launch_bounds__(256) void synapse_gather_row_kernel(GatherArgs g)
 #pragma unroll
         for (int m = 0; m < MB; ++m)
             acc[px][m].store(dstB, masked_offset(live && b0 + px < g.DW && mb0 + m < g.Mg,
-                                                 (mb0 + m) * dstPlaneBytes + ((a * g.DW + b0 + px) * g.T) * 4 + tv * 16));
+                                                 (mb0 + m) * dstPlaneBytes + ((a * g.DW + b0 + px) * g.T) * 4 + t4));
 }
 
 
@@ -350,7 +363,7 @@ __global__ __launch_bounds__(256) void synapse_gather_row_kernel(GatherArgs g)
 struct WindowArgs {
     const float *gradOut, *w;
     float *gradIn;
-    int H, W, OH, OW, T, KW, P;  // P = H*W*T/VEC vectors per batch item
+    int H, W, OH, OW, T, KW, P;  // P = H*W*ceil(T/VEC) vectors per batch item
     int chunks;
     FastDiv byChunks, byTV, byW, bySH, bySW;
 };
@@ -363,7 +376,7 @@ __global__ __launch_bounds__(256) void synapse_window_bwd_kernel(WindowArgs g)
     const int p = static_cast<int>(blk - n * g.byChunks.d) * 256 + static_cast<int>(threadIdx.x);
     if (p >= g.P) return;
     const uint32_t pix = fastdiv(static_cast<uint32_t>(p), g.byTV);
-    const int tv = p - static_cast<int>(pix * g.byTV.d);
+    const int t = vec_start<VEC>(p - static_cast<int>(pix * g.byTV.d), g.T);
     const int y = static_cast<int>(fastdiv(pix, g.byW)), x = static_cast<int>(pix) - y * g.W;
     const int a = static_cast<int>(fastdiv(static_cast<uint32_t>(y), g.bySH));
     const int b = static_cast<int>(fastdiv(static_cast<uint32_t>(x), g.bySW));
@@ -372,10 +385,10 @@ __global__ __launch_bounds__(256) void synapse_window_bwd_kernel(WindowArgs g)
     const BufferRsrc src = make_buffer(g.gradOut + static_cast<int64_t>(n) * g.OH * g.OW * g.T);
     const BufferRsrc dst = make_buffer(g.gradIn + static_cast<int64_t>(n) * g.H * g.W * g.T);
     TimeVec<VEC> v, out;
-    v.load(src, masked_offset(inside, ((a * g.OW + b) * g.T + tv * VEC) * 4));
+    v.load(src, masked_offset(inside, ((a * g.OW + b) * g.T + t) * 4));
     out.zero();
     out.fma(inside ? g.w[i * g.KW + j] : 0.f, v);
-    out.store(dst, p * VEC * 4);
+    out.store(dst, (static_cast<int>(pix) * g.T + t) * 4);
 }
 
 // ---- weight gradient -----------------------------------------------------------------------------
@@ -679,6 +692,13 @@ struct GatherMfmaArgs {
     int chansPerPass, passes, WX, xBias, rows;   // patch: chansPerPass x KH x WX rows; xBias: patch column of tap 0 of pixel 0
     int oGroups;                                 // blocks of 16 * OT destination channels per group
     int blocksPerRow, steps, pairs, slices, pairsPerSlice;
+    // Sample at which the last step may start.  Rows of whole vectors: wherever it starts, its missing vectors are
+    // masked.  Other rows: T - 32, so that every vector of every step lies within its row; the samples that the last
+    // step shares with the one before are computed and stored twice, with the same values.  (16 -> 32 channels 3x3 on
+    // 16x16 pixels, 4 x 1450 samples, against the vector kernel with one sample per access, which such rows took
+    // before: forward 283 -> 155 us, input gradient 334 -> 194 us; like every product on the matrix cores here, a
+    // non-finite sample may give NaN where that kernel gave an infinity.)
+    int tLast;
     FastDiv byOGroups, byGroups, byKK, byKW, bySteps, byBlocks, byBlocksPerRow, byPatch, byWX;
 };
 
@@ -783,8 +803,8 @@ __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs
         return n;
     };
     auto issue = [&](float4 (&R)[NS], int st, int pass, bool more) {
-        const int uniform = (st << 7) + pass * g.chansPerPass * planeBytes;
-        const bool live = more && (st << 5) + (u << 2) < g.T;
+        const int t0 = min(st << 5, g.tLast), uniform = t0 * 4 + pass * g.chansPerPass * planeBytes;
+        const bool live = more && t0 + (u << 2) < g.T;
 #pragma unroll
         for (int m = 0; m < NS; ++m) R[m] = buffer_load4<0>(srcB, live ? sOff[m] : kOutOfRange, uniform);
     };
@@ -841,10 +861,10 @@ __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs
     // the 16 -> 32 channel layer)
     auto store = [&](int pix, int st) {
         if (pix < 0) return;
-        const int uniform = pix + (st << 7);
+        const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
-            const bool live = (st << 5) + hf * 16 + (h << 2) < g.T;
+            const bool live = t0 + hf * 16 + (h << 2) < g.T;
 #pragma unroll
             for (int ot = 0; ot < OT; ++ot)
                 buffer_store4<0>(dstB, live ? oOff[ot] : kOutOfRange, uniform + hf * 64,
@@ -895,7 +915,7 @@ __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs
                 using I0 = std::integral_constant<int, 0>;
                 using I1 = std::integral_constant<int, 1>;
                 using I2 = std::integral_constant<int, 2>;
-                if ((stCur << 5) + 16 < g.T) {
+                if (min(stCur << 5, g.tLast) + 16 < g.T) {
                     if (buf == 0) multiply(I0{}, I2{}, passCur);
                     else multiply(I1{}, I2{}, passCur);
                 } else {
@@ -1049,8 +1069,8 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
         return n;
     };
     auto issue = [&](float4 (&R)[NS], int st, int pass, bool more) {
-        const int uniform = (st << 7) + pass * g.chansPerPass * planeBytes;
-        const bool live = more && (st << 5) + (u << 2) < g.T;
+        const int t0 = min(st << 5, g.tLast), uniform = t0 * 4 + pass * g.chansPerPass * planeBytes;
+        const bool live = more && t0 + (u << 2) < g.T;
 #pragma unroll
         for (int m = 0; m < NS; ++m) R[m] = buffer_load4<0>(srcB, live ? sOff[m] : kOutOfRange, uniform);
     };
@@ -1137,10 +1157,10 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
     };
     auto store = [&](int pix, int st) {
         if (pix < 0) return;
-        const int uniform = pix + (st << 7);
+        const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
-            const bool live = (st << 5) + hf * 16 + (h << 2) < g.T;
+            const bool live = t0 + hf * 16 + (h << 2) < g.T;
 #pragma unroll
             for (int ot = 0; ot < OT; ++ot)
                 buffer_store4<0>(dstB, live ? oOff[ot] : kOutOfRange, uniform + hf * 64,
@@ -1187,7 +1207,7 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
                 using I0 = std::integral_constant<int, 0>;
                 using I1 = std::integral_constant<int, 1>;
                 using I2 = std::integral_constant<int, 2>;
-                if ((stCur << 5) + 16 < g.T) {
+                if (min(stCur << 5, g.tLast) + 16 < g.T) {
                     if (DOUBLE && buf != 0) multiply(I1{}, I2{}, passCur, 1);
                     else multiply(I0{}, I2{}, passCur, 0);
                 } else {
@@ -1244,6 +1264,7 @@ struct WgradLdsArgs {
     int WX, rows;              // patch width in input pixels, patch rows = channels * KH * WX
     int blocksPerRow, steps;   // pixel blocks per output row, steps of 32 samples per row
     int pairs, slices, pairsPerSlice, nW;
+    int tLast;                 // sample at which the last step may start (rows that are not whole vectors: T - 32)
     FastDiv byColGroups, byOGroups, byGroups, byKK, byKW, bySteps, byBlocks, byBlocksPerRow, byPatch, byWX;
 };
 
@@ -1341,8 +1362,8 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
     // exactly this batch in flight on every path.  `plain`: every sample of the step exists, so the block's
     // offsets are used as they are.
     auto issue = [&](float4 (&R)[NS], float4 (&A)[2][MT], int st, bool more) {
-        const int tBytes = st << 7;
-        if (more && (st << 5) + 32 <= s.T) {
+        const int t0 = min(st << 5, g.tLast), tBytes = t0 * 4;
+        if (more && t0 + 32 <= s.T) {
 #pragma unroll
             for (int m = 0; m < NS; ++m) R[m] = buffer_load4<0>(inB, sOff[m], tBytes);
 #pragma unroll
@@ -1351,8 +1372,8 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
                 A[1][mt] = buffer_load4<0>(goB, aOff[mt], tBytes + 64);
             }
         } else {
-            const bool liveU = more && (st << 5) + (u << 2) < s.T;
-            const bool liveH0 = more && (st << 5) + (h << 2) < s.T, liveH1 = more && (st << 5) + 16 + (h << 2) < s.T;
+            const bool liveU = more && t0 + (u << 2) < s.T;
+            const bool liveH0 = more && t0 + (h << 2) < s.T, liveH1 = more && t0 + 16 + (h << 2) < s.T;
 #pragma unroll
             for (int m = 0; m < NS; ++m) R[m] = buffer_load4<0>(inB, liveU ? sOff[m] : kOutOfRange, tBytes);
 #pragma unroll
@@ -1360,6 +1381,21 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
                 A[0][mt] = buffer_load4<0>(goB, liveH0 ? aOff[mt] : kOutOfRange, tBytes);
                 A[1][mt] = buffer_load4<0>(goB, liveH1 ? aOff[mt] : kOutOfRange, tBytes + 64);
             }
+        }
+    };
+    // the first `seen` samples of the last step of a row that is not whole vectors belong to the step before: zeros in
+    // both operands (2 -> 16 channels 5x5, 4 x 1450 samples of 32x32 pixels: 375 us with the vector kernel, which such
+    // rows took before, 143 us here)
+    auto forget = [&](float4 (&R)[NS], float4 (&A)[2][MT], int seen) {
+        auto keep = [&](float4 &v, int t) {
+            v = make_float4(t >= seen ? v.x : 0.f, t + 1 >= seen ? v.y : 0.f, t + 2 >= seen ? v.z : 0.f, t + 3 >= seen ? v.w : 0.f);
+        };
+#pragma unroll
+        for (int m = 0; m < NS; ++m) keep(R[m], u << 2);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            keep(A[0][mt], h << 2);
+            keep(A[1][mt], 16 + (h << 2));
         }
     };
     // registers -> patch; a wavefront notes whether any of its samples has more than the upper 16 bits
@@ -1445,6 +1481,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
             if (!first) multiply(A, buf);
             __builtin_amdgcn_sched_barrier(0);
             if (!more) break;
+            if ((st << 5) > g.tLast) forget(R, An, (st << 5) - g.tLast);
             buf = kWgBuf - buf;
             stage(R, buf);
 #pragma unroll
@@ -1560,13 +1597,13 @@ static void launch_gather_mb(const GatherArgs &g, bool strided, unsigned blocks,
         hipLaunchKernelGGL((synapse_gather_kernel<MB, VEC, BACKWARD, false>), dim3(blocks), dim3(256), 0, st, g);
 }
 
-// The matrix-core gather: unit stride in the gradient (forward: any stride), rows of whole vectors, passes of
-// whole source channels that fill most of the 36 tap steps, at least 16 destination channels, patch and weights
+// The matrix-core gather: unit stride in the gradient (forward: any stride), rows of whole vectors or at least one
+// step, passes of whole source channels that fill most of the 36 tap steps, at least 16 destination channels, patch and weights
 // within LDS.  Returns SLAYER_EUNSUPPORTED (nothing launched) when the geometry does not qualify.
 template <bool BACKWARD>
 static int launch_gather_mfma(const GatherArgs &a, const SynGeom &s, bool strided, hipStream_t st)
 {
-    if (strided || a.Mg < 16) return SLAYER_EUNSUPPORTED;
+    if (strided || a.Mg < 16 || (a.T % 4 != 0 && a.T < 32)) return SLAYER_EUNSUPPORTED;
     const int KK = a.KH * a.KW;
     if (KK > 4 * kGmSteps) return SLAYER_EUNSUPPORTED;
     int chans = 4 * kGmSteps / KK;
@@ -1590,6 +1627,7 @@ static int launch_gather_mfma(const GatherArgs &a, const SynGeom &s, bool stride
     g.oGroups = static_cast<int>(ceil_div(a.Mg, 16 * OT));
     g.blocksPerRow = static_cast<int>(ceil_div(a.DW, kGmPix));
     g.steps = (a.T + 31) / 32;
+    g.tLast = a.T % 4 == 0 ? (g.steps - 1) * 32 : a.T - 32;
     const int64_t pairs = static_cast<int64_t>(s.N) * a.DH * g.blocksPerRow * g.steps;
     if (pairs < 1 || pairs >= (1LL << 30)) return SLAYER_EUNSUPPORTED;
     g.pairs = static_cast<int>(pairs);
@@ -1684,19 +1722,19 @@ static int launch_gather(float *dst, const float *src, const float *w, const Syn
     }
     const int64_t dstElems = static_cast<int64_t>(s.N) * g.DC * g.DH * g.DW * g.T;
     if (dstElems == 0) return SLAYER_OK;
-    const bool vec = s.T % 4 == 0 && aligned16(src) && aligned16(dst);
-    const int VEC = vec ? 4 : 1;
+    const bool vec = s.T >= 4;      // (any row length and alignment from there on: vec_start)
+    const int VEC = vec ? 4 : 1, TV = (s.T + VEC - 1) / VEC;
     if (BACKWARD && s.C == 1 && s.O == 1 && s.sH == s.KH && s.sW == s.KW && s.pH == 0 && s.pW == 0 && s.dH == 1 &&
         s.dW == 1 && s.OH > 0 && s.OW > 0 && !generic_forced()) {
         WindowArgs a{};
         a.gradOut = src; a.w = w; a.gradIn = dst;
         a.H = s.H; a.W = s.W; a.OH = s.OH; a.OW = s.OW; a.T = s.T; a.KW = s.KW;
-        a.P = s.H * s.W * (s.T / VEC);
+        a.P = s.H * s.W * TV;
         a.chunks = static_cast<int>(ceil_div(a.P, 256));
         const int64_t nBlocks = static_cast<int64_t>(s.N) * a.chunks;
         if (nBlocks >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
         a.byChunks = make_fastdiv(static_cast<uint32_t>(a.chunks));
-        a.byTV = make_fastdiv(static_cast<uint32_t>(s.T / VEC));
+        a.byTV = make_fastdiv(static_cast<uint32_t>(TV));
         a.byW = make_fastdiv(static_cast<uint32_t>(s.W));
         a.bySH = make_fastdiv(static_cast<uint32_t>(s.sH));
         a.bySW = make_fastdiv(static_cast<uint32_t>(s.sW));
@@ -1714,7 +1752,7 @@ static int launch_gather(float *dst, const float *src, const float *w, const Syn
     if (MB <= 2 && vec && !strided && g.mulW == 1 && g.stepW == (BACKWARD ? -1 : 1) && (g.KW == 3 || g.KW == 5 || g.KW == 7) &&
         static_cast<int64_t>(g.Qg) * g.KH * g.KW >= 32 && !generic_forced()) {
         const int pixelGroups = static_cast<int>(ceil_div(g.DW, kGatherRowPx));
-        g.P = g.DH * pixelGroups * (g.T / 4);
+        g.P = g.DH * pixelGroups * TV;
         g.chunks = static_cast<int>(ceil_div(g.P, 256));
         g.mBlocks = static_cast<int>(ceil_div(g.Mg, MB));
         const int64_t blocks = static_cast<int64_t>(s.N) * s.groups * g.mBlocks * g.chunks;
@@ -1722,7 +1760,7 @@ static int launch_gather(float *dst, const float *src, const float *w, const Syn
         g.byChunks = make_fastdiv(static_cast<uint32_t>(g.chunks));
         g.byMBlocks = make_fastdiv(static_cast<uint32_t>(g.mBlocks));
         g.byGroups = make_fastdiv(static_cast<uint32_t>(s.groups));
-        g.byTV = make_fastdiv(static_cast<uint32_t>(g.T / 4));
+        g.byTV = make_fastdiv(static_cast<uint32_t>(TV));
         g.byDW = make_fastdiv(static_cast<uint32_t>(pixelGroups));
         const dim3 nb(static_cast<unsigned>(blocks));
 #define SLAYER_GATHER_ROW(MBV)                                                                                          \
@@ -1736,7 +1774,7 @@ static int launch_gather(float *dst, const float *src, const float *w, const Syn
 #undef SLAYER_GATHER_ROW
         return launch_status();
     }
-    g.P = g.DH * g.DW * (g.T / VEC);
+    g.P = g.DH * g.DW * TV;
     g.chunks = static_cast<int>(ceil_div(g.P, 256));
     g.mBlocks = static_cast<int>(ceil_div(g.Mg, MB));
     const int64_t blocks = static_cast<int64_t>(s.N) * s.groups * g.mBlocks * g.chunks;
@@ -1744,7 +1782,7 @@ static int launch_gather(float *dst, const float *src, const float *w, const Syn
     g.byChunks = make_fastdiv(static_cast<uint32_t>(g.chunks));
     g.byMBlocks = make_fastdiv(static_cast<uint32_t>(g.mBlocks));
     g.byGroups = make_fastdiv(static_cast<uint32_t>(s.groups));
-    g.byTV = make_fastdiv(static_cast<uint32_t>(g.T / VEC));
+    g.byTV = make_fastdiv(static_cast<uint32_t>(TV));
     g.byDW = make_fastdiv(static_cast<uint32_t>(g.DW));
     const unsigned nb = static_cast<unsigned>(blocks);
 #define SLAYER_GATHER(MBV)                                                        \
@@ -1806,8 +1844,9 @@ static MfmaPlan plan_wgrad_mfma(const SynGeom &s)
     MfmaPlan p{};
     const int Og = s.O / s.groups, CK = (s.C / s.groups) * s.KH * s.KW;
     const int64_t pixels = static_cast<int64_t>(s.OH) * s.OW;
-    // worth it when the 16 x 16 tiles are reasonably full and rows are whole 16-byte vectors
-    p.use = s.T % 4 == 0 && s.T >= 16 && Og >= 8 && CK >= 8 && pixels > 0 && s.N > 0;
+    // worth it when the 16 x 16 tiles are reasonably full (rows that are not whole 16-byte vectors: only where the
+    // patch fits, plan_wgrad_lds, and the row is at least one step)
+    p.use = (s.T % 4 == 0 ? s.T >= 16 : s.T >= 32) && Og >= 8 && CK >= 8 && pixels > 0 && s.N > 0;
     if (!p.use) return p;
     const int oTiles = static_cast<int>(ceil_div(Og, 16)), cTiles = static_cast<int>(ceil_div(CK, 16));
     // two tiles of output channels at most: 4 x 6 tiles (one wavefront per SIMD) measured 132 us on
@@ -1963,6 +2002,7 @@ static int launch_wgrad_lds(const float *gradOut, const float *in, float *worksp
     g.oGroups = m.oGroups; g.colGroups = m.colGroups;
     g.WX = p.WX; g.rows = p.rows; g.blocksPerRow = p.blocksPerRow; g.steps = p.steps;
     g.pairs = p.pairs; g.slices = p.slices; g.pairsPerSlice = p.pairsPerSlice; g.nW = nW;
+    g.tLast = s.T % 4 == 0 ? (p.steps - 1) * 32 : s.T - 32;
     g.byColGroups = make_fastdiv(static_cast<uint32_t>(m.colGroups));
     g.byOGroups = make_fastdiv(static_cast<uint32_t>(m.oGroups));
     g.byGroups = make_fastdiv(static_cast<uint32_t>(s.groups));
@@ -2086,8 +2126,8 @@ extern "C" int slayer_synapse_conv_grad_weight_f32(float *gradW, const float *gr
         WgradPlan p = plan_wgrad(s, vecT);
         const bool vec = vecT && aligned16(gradOut) && aligned16(in);
         const MfmaPlan m = plan_wgrad_mfma(s);
-        if (m.use && vec && !generic_forced()) {
-            const LdsPlan l = plan_wgrad_lds(s, m);
+        const LdsPlan l = plan_wgrad_lds(s, m);
+        if ((l.use || (m.use && vec)) && !generic_forced()) {
             rows = l.use ? launch_wgrad_lds(gradOut, in, workspace, s, m, l, nW, st)
                          : launch_wgrad_mfma(gradOut, in, workspace, s, m, nW, st);
             if (rows < 0) return -rows;

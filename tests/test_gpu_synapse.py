@@ -207,7 +207,7 @@ def test_random_geometries_against_conv3d():
 
 
 def test_unaligned_storage():
-    """Tensors that start 4 bytes into an allocation take the one-sample-per-lane kernels."""
+    """Tensors that start 4 bytes into an allocation."""
     case = (1, 3, 6, 7, 8, 4, (3, 3), 1, 1, 1, 1)
     x, w, a = make(case, 6)
     shape = O.synapse_geom(x.shape, w.shape, *a)[1]
@@ -227,6 +227,47 @@ def test_unaligned_storage():
     close(host(synapse.convGradWeight(off(go), off(x), w.shape, *a)),
           O.synapse_conv_grad_weight(go, x, w.shape, *a).astype(np.float64),
           O.synapse_conv_grad_weight(np.abs(go), np.abs(x), w.shape, *a))
+
+
+# layers of every kernel that takes rows of any length and alignment: (C, H, W, O, K, stride, padding)
+RAGGED_LAYERS = {
+    "vector ALUs": (3, 6, 7, 8, (3, 3), 1, 1),
+    "few channels": (8, 7, 9, 2, (3, 3), 1, 1),
+    "strided": (2, 9, 8, 5, (3, 2), 2, 1),
+    "pool": (1, 9, 7, 1, (2, 2), 2, 0),
+    "matrix cores": (16, 5, 9, 32, (3, 3), 1, 1),
+    "matrix cores, two passes": (32, 4, 10, 64, (3, 3), 1, 1),
+    "wide filter": (2, 8, 9, 16, (5, 5), 1, 1),
+}
+
+
+@pytest.mark.parametrize("T", [3, 4, 5, 7, 13, 31, 32, 33, 35, 61, 63, 66, 97, 173])
+@pytest.mark.parametrize("layer", RAGGED_LAYERS, ids=[k.replace(" ", "-") for k in RAGGED_LAYERS])
+def test_rows_of_any_length_and_alignment(layer, T, impl):
+    """Rows that are not whole vectors (last vector and last step overlap the ones before; below 32 samples the matrix-core
+    kernels leave them to the vector ones), inputs that start 4, 8 and 12 bytes after a 16-byte boundary: forward pass and both
+    gradients against the oracle."""
+    C, H, W, Oc, K, stride, pad = RAGGED_LAYERS[layer]
+    for k, dense in enumerate((True, False)):
+        x, w, a = make((2, C, H, W, T, Oc, K, stride, pad, 1, 1), T)
+        if not dense:
+            x = (x > 1.0).astype(np.float32)
+        shape = O.synapse_geom(x.shape, w.shape, *a)[1]
+        go = np.random.default_rng(T + 1).standard_normal(shape).astype(np.float32)
+
+        def off(arr, n):
+            view = torch.empty(arr.size + n, dtype=torch.float32, device="cuda")[n:].view(arr.shape)
+            view.copy_(torch.from_numpy(arr))
+            return view
+
+        close(host(synapse.conv(off(x, 3 * k), dev(w), *a)), O.synapse_conv(x, w, *a).astype(np.float64),
+              O.synapse_conv(np.abs(x), np.abs(w), *a))
+        close(host(synapse.convGradInput(off(go, 1 + k), dev(w), x.shape, *a)),
+              O.synapse_conv_grad_input(go, w, x.shape, *a).astype(np.float64),
+              O.synapse_conv_grad_input(np.abs(go), np.abs(w), x.shape, *a))
+        close(host(synapse.convGradWeight(off(go, k), off(x, 2), w.shape, *a)),
+              O.synapse_conv_grad_weight(go, x, w.shape, *a).astype(np.float64),
+              O.synapse_conv_grad_weight(np.abs(go), np.abs(x), w.shape, *a))
 
 
 def test_adjoint_identity_full_size():
