@@ -572,26 +572,26 @@ static int launch_fir(float *out, const float *in, const float *filt, int64_t ro
 
     const bool vec = (T % 4 == 0) && aligned16(out) && aligned16(in) && (!GATED || aligned16(gate.u));
     // The correlation's input is a gradient, i.e. dense: from 34 taps on, where the chain kernels are bound by
-    // FMA issue, it runs on the matrix cores (the gated one too when its rows fit that kernel's linear layout).
+    // FMA issue, it runs on the matrix cores.
     // The convolution does not: its input is mostly spike trains, which the tiled kernel's event-driven path
     // serves at the speed of a copy and with the bits of the chain.
-    if (!CAUSAL && !generic_forced() && launch_fir_corr_mfma(out, in, filt, rows, T, F, Ts, gate, stream))
+    if (!CAUSAL && !generic_forced() && launch_fir_corr_mfma(out, in, filt, rows, T, F, Ts, gate, true, stream))
         return launch_status();
-    {
-    FirPlan p;
-    // Longer filters on rows of whole vectors: the tiled kernel whose dense tiles run on the matrix cores (its
-    // sparse tiles, spike trains, keep the event-driven path and the bits of the chain).
-    if (!generic_forced() && vec && plan_fir_mfma(rows, T, F, p) && ceil_div(rows, p.R) < (1LL << 31)) {
-        switch ((F + 14) / 16 + 1) {
-            case 4: launch_tiled<CAUSAL, true, 16, GATED, 4>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
-            case 5: launch_tiled<CAUSAL, true, 16, GATED, 5>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
-            case 6: launch_tiled<CAUSAL, true, 16, GATED, 6>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
-            case 7: launch_tiled<CAUSAL, true, 16, GATED, 7>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
-            case 8: launch_tiled<CAUSAL, true, 16, GATED, 8>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
-            default: launch_tiled<CAUSAL, true, 16, GATED, 9>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
+    if constexpr (CAUSAL) {
+        FirPlan p;
+        // Longer filters on rows of whole vectors: the tiled kernel whose dense tiles run on the matrix cores (its
+        // sparse tiles, spike trains, keep the event-driven path and the bits of the chain).
+        if (!generic_forced() && vec && plan_fir_mfma(rows, T, F, p) && ceil_div(rows, p.R) < (1LL << 31)) {
+            switch ((F + 14) / 16 + 1) {
+                case 4: launch_tiled<true, true, 16, false, 4>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
+                case 5: launch_tiled<true, true, 16, false, 5>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
+                case 6: launch_tiled<true, true, 16, false, 6>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
+                case 7: launch_tiled<true, true, 16, false, 7>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
+                case 8: launch_tiled<true, true, 16, false, 8>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
+                default: launch_tiled<true, true, 16, false, 9>(p, out, in, filt, rows, T, F, Ts, gate, stream); break;
+            }
+            return launch_status();
         }
-        return launch_status();
-    }
     }
     // Register-only kernel for short filters (the op is then a stream).
     const int64_t directMax = 33;
@@ -654,4 +654,20 @@ extern "C" int slayer_spike_bwd_corr_f32(float *gradIn, const float *gradOut, co
     return slayer::launch_fir<false, true>(gradIn, gradOut, filt, nNeurons, T, F, Ts,
                                            slayer::FirGate{u, theta, tau, scale / tau},
                                            static_cast<hipStream_t>(stream));
+}
+
+extern "C" int slayer_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradOut, const float *u, const float *filt,
+                                                 int64_t nNeurons, int64_t T, int64_t F, int64_t delaySteps, float theta,
+                                                 float tau, float scale, float Ts, void *stream)
+{
+    if (tau == 0.0f || nNeurons < 0 || T < 0 || F < 0 || delaySteps < 0) return SLAYER_EINVAL;
+    if (nNeurons == 0 || T == 0) return SLAYER_OK;
+    if (!gradIn || !gradOut || !u || (F > 0 && !filt)) return SLAYER_EINVAL;
+    const slayer::FirGate gate{u, theta, tau, scale / tau};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (slayer::generic_forced()) return SLAYER_EUNSUPPORTED;
+    if (delaySteps == 0 ? !slayer::launch_fir_corr_mfma(gradIn, gradOut, filt, nNeurons, T, F, Ts, gate, false, st)
+                        : !slayer::launch_fir_corr_walk(gradIn, gradOut, filt, nNeurons, T, F, delaySteps, Ts, gate, st))
+        return SLAYER_EUNSUPPORTED;
+    return slayer::launch_status();
 }

@@ -14,9 +14,14 @@ struct FirGate {
     float theta, tau, gain;
 };
 
-// Matrix-core correlation (fir_mfma.hip).  Returns false, launching nothing, for shapes it does not serve.
+// Matrix-core correlation (fir_mfma.hip).  Returns false, launching nothing, for shapes it does not serve; with
+// chainBits, rows that are not whole aligned vectors are among those.
 bool launch_fir_corr_mfma(float *out, const float *in, const float *filt, int64_t rows, int64_t T, int64_t F, float Ts,
-                          const FirGate &gate, hipStream_t stream);
+                          const FirGate &gate, bool chainBits, hipStream_t stream);
+
+// ... and its kernel for rows of any length and alignment, whose samples are in[t + shift] (zero from T on).
+bool launch_fir_corr_walk(float *out, const float *in, const float *filt, int64_t rows, int64_t T, int64_t F, int64_t shift,
+                          float Ts, const FirGate &gate, hipStream_t stream);
 
 // Filter lengths that the matrix-core paths serve (the correlation kernel of fir_mfma.hip and the dense tiles of
 // the tiled kernel of fir.hip).

@@ -10,17 +10,13 @@
 //
 // of a banded Toeplitz matrix made of the filter (zero where k - i is not a tap) and the rows' samples.
 //
-// A work-group is ONE wavefront that walks over tiles of 16 consecutive rows.  It copies a tile into LDS with
-// 16-byte loads that run through the rows' memory front to back, walks the blocks - the window of samples lives in
-// registers and moves on by what one step consumes, so each step reads only the new samples from LDS (the walk is
-// unrolled by the window size) - writes every output block over input that has left the window, and copies the rows
-// back out the way they came in.  The next tile's samples are on their way into registers during the walk.  No
-// barriers: the wavefronts of a compute unit overlap each other's memory and matrix work.
+// A work-group is ONE wavefront that walks over the chunks of 16 consecutive rows; the window of samples lives in
+// registers and moves on by what one step consumes, so each step reads only new samples (the walk is unrolled by the
+// window size).  No barriers: the wavefronts of a compute unit overlap each other's memory and matrix work.
 //
-// Two kernels.  fir_mfma_split_kernel: tiles of 16 whole rows kept in LDS exactly as they lie in memory, for rows
-// whose length spreads them over the LDS banks as it is (T / 4 odd); the product runs on bf16 instructions over a
-// three-way split of both operands.  fir_mfma_kernel: every other row length (padded rows, or tiles of the time axis
-// with halo), fp32 instructions, plain correlation only.
+// Two kernels.  fir_mfma_split_kernel: tiles of 16 whole rows kept in LDS exactly as they lie in memory, copied with
+// 16-byte accesses that run through the rows' memory front to back, for short aligned rows whose length spreads them over
+// the LDS banks as it is (T / 4 odd).  fir_walk_kernel: rows of any length and alignment, straight from and to memory.
 //
 // The matrix instructions sum their products in their own order, so results agree with the sequential chain to
 // rounding (a few 1e-7 of sum |x| |filt|), not bit for bit.  A structural zero times a non-finite sample would
@@ -31,204 +27,20 @@
 
 namespace slayer {
 
-constexpr int kMfmaLdsBytes = 160 * 1024 / 8;  // per wavefront: 8 of them on a compute unit
+constexpr int kMfmaMaxBlocks = 19;   // blocks of 16 samples per row of a tile: 8 tiles in a compute unit's 160 KB of LDS
 
 struct MfmaFirArgs {
     float *out;
     const float *in, *filt;
     int64_t rows;
     int T, F;
-    int nb;         // output blocks per tile of the time axis
-    int timeTiles;  // tiles per row
-    int pitch;      // floats per row in LDS; pitch / 4 is odd, which spreads the 16 rows over the banks
-    int nv;         // 16-byte vectors per lane and tile that are in use (<= NV; whole rows: nv KiB of LDS)
+    int nv;         // 16-byte vectors per lane and tile that are in use (<= NV; nv KiB of LDS)
     uint32_t nItems;
     float Ts;
-    FirGate gate;  // GATED (whole rows only): the samples are in * gain * exp(-|u - theta| / tau), applied on the way into LDS
+    FirGate gate;  // GATED: the samples are in * gain * exp(-|u - theta| / tau), applied on the way into LDS
 };
 
-// ---- fp32 instructions, rows padded in LDS or cut into time tiles ------------------------------------------------
-// v_mfma_f32_16x16x4_f32 takes 4 of the k per instruction: a lane (c = lane % 16, h = lane / 16) supplies
-// X[.. + 4h + v] of row c for instruction v = 0..3, which are the four components of ONE 16-byte LDS read, and
-// filt[16d + 4h + v - i] for i = lane % 16 and each of the D = F/16 + 1..2 blocks of the window, which it keeps in
-// 4 D registers.  Its accumulator then holds outputs 4h..4h+3 of row c.
-// NV: 16-byte vectors per lane and tile, NV * 64 >= 16 rows * (staged blocks * 4)
-template <int D, int NV>
-__global__ __launch_bounds__(64, 2) void fir_mfma_kernel(MfmaFirArgs p)
-{
-    extern __shared__ __align__(16) float X[];
-    constexpr int W = D + 1;  // window slots: the D blocks of a tile and the block the next tile adds
-    const int lane = threadIdx.x;
-    const int c = lane & 15, h = lane >> 4;
-    const int T = p.T, F = p.F, P = p.pitch;
-    const int nBlk = (T + 15) >> 4;
-    const int nInMax = p.nb + (p.timeTiles > 1 ? D - 1 : 0);  // staged blocks per row
-    const int lenIn = 4 * nInMax, lenOut = 4 * p.nb;          // 16-byte vectors per row coming in / going out
-
-    // the lane's column of the Toeplitz factor; the range check of a buffer that ends with the filter turns
-    // every index that is not a tap into a zero
-    const BufferRsrc bufF = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.filt), 0, F * 4, 0x00020000);
-    float a[D][4];
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int tap = 16 * d + 4 * h + v - c;
-            a[d][v] = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(bufF, masked_offset(tap >= 0 && tap < F, tap * 4), 0, 0));
-        }
-
-    struct Tile {
-        int64_t row0;
-        int nRows, t0, nb, nIn;
-    };
-    auto tile_of = [&](uint32_t i) {
-        // tiles that share halo blocks (time tiles of the same rows) and memory lines (neighbouring rows) run on
-        // the same die (the grid is a multiple of 8 wavefronts)
-        const uint32_t item = xcd_contiguous(i, p.nItems);
-        const uint32_t rowGroup = item / static_cast<uint32_t>(p.timeTiles);
-        const int timeTile = static_cast<int>(item - rowGroup * static_cast<uint32_t>(p.timeTiles));
-        Tile q;
-        q.row0 = static_cast<int64_t>(rowGroup) * 16;
-        q.nRows = static_cast<int>(min(static_cast<int64_t>(16), p.rows - q.row0));
-        const int b0 = timeTile * p.nb;
-        q.t0 = 16 * b0;
-        q.nb = min(p.nb, nBlk - b0);
-        q.nIn = min(nInMax, nBlk - b0);
-        return q;
-    };
-    // vector e = lane + 64 k of a tile is vector e % lenIn of row e / lenIn; samples outside the row read as zeros
-    float4 pre[NV];
-    // the lane index behind a barrier for the optimiser: the (row, vector) sequences below do not depend on the
-    // tile, and kept across the walk they would cost 2 registers per vector
-    auto lane_again = [&]() {
-        int l = lane;
-        asm volatile("" : "+v"(l));
-        return l;
-    };
-    // (a fixed number of loads and stores per tile, masked where a tile is short: the wait for a tile's loads can
-    // then leave exactly the younger stores of the tile before in flight)
-    auto fetch = [&](const Tile &q) {
-        const BufferRsrc bufIn = make_buffer(p.in + q.row0 * T);
-        RowCol rc;
-        rc.init(lane_again(), lenIn, 1.0f / static_cast<float>(lenIn));
-        const int dr = kWave / lenIn, dc = kWave % lenIn;
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const int t = q.t0 + (rc.c << 2);
-            pre[k] = buffer_load4(bufIn, masked_offset(rc.r < q.nRows && t < T, (rc.r * T + t) * 4), 0);
-            rc.advance(dr, dc, lenIn);
-        }
-    };
-    auto stage = [&]() {  // the fetched vectors into LDS; true if a sample is not finite
-        bool bad = false;
-        RowCol rc;
-        rc.init(lane_again(), lenIn, 1.0f / static_cast<float>(lenIn));
-        const int dr = kWave / lenIn, dc = kWave % lenIn;
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const float4 x = pre[k];
-            // infinite or NaN (or four samples that add up to more than fp32 holds, which only costs time)
-            bad |= ((x.x + x.y) + (x.z + x.w)) * 0.0f != 0.0f;
-            if (rc.r < 16) *reinterpret_cast<float4 *>(X + rc.r * P + (rc.c << 2)) = x;
-            rc.advance(dr, dc, lenIn);
-        }
-        return __builtin_amdgcn_ballot_w64(bad) != 0;
-    };
-
-    // 64 bytes of zeros behind the 16 rows
-    const int zeroOff = 16 * P;
-    if (lane < 4) *reinterpret_cast<float4 *>(X + zeroOff + 4 * lane) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-
-    uint32_t i = blockIdx.x;
-    if (i >= p.nItems) return;
-    Tile cur = tile_of(i);
-    fetch(cur);
-    {
-        // stores that the range check drops, as many as a tile's: the first trip then finds the same instructions in
-        // flight as the later ones - a tile's loads, then the stores of the tile before - so that one count serves all
-        const BufferRsrc none = make_buffer(p.out, 0);
-#pragma unroll
-        for (int k = 0; k < NV; ++k) buffer_store4(none, (lane + kWave * k) * 16, 0, make_float4(static_cast<float>(k), 0.0f, 0.0f, 0.0f));
-    }
-    for (;;) {
-        const bool chains = stage();
-        wave_sync();
-        const uint32_t iNext = i + gridDim.x;
-        const bool more = iNext < p.nItems;
-        // (the next tile's loads behind every wait of stage(): moved up between them, as the compiler likes to do to
-        // reuse the registers one by one, each of those waits would also wait for the stores of the tile before)
-        // (behind the last tile: a tile without rows, whose loads are all masked)
-        Tile next = tile_of(more ? iNext : i);
-        if (!more) next.nRows = 0;
-        fetch(next);
-        if (chains) {
-            // a non-finite sample: the tile's outputs as sequential chains over the valid taps
-            const int width = min(16 * cur.nb, T - cur.t0);
-            for (int e = lane; e < cur.nRows * width; e += kWave) {
-                const int r = e / width, t = cur.t0 + (e - r * width);
-                const float *x = p.in + (cur.row0 + r) * T;
-                const int taps = min(T - t, F);
-                float acc = 0.0f;
-                for (int k = 0; k < taps; ++k) acc = __builtin_fmaf(x[t + k], p.filt[k], acc);
-                p.out[(cur.row0 + r) * T + t] = acc * p.Ts;
-            }
-        } else {
-            // walk: step j makes output block j from input blocks j .. j + D - 1 and writes it over input block j
-            float *col = X + c * P + 4 * h;
-            const float *zeros = X + zeroOff + 4 * h;
-            const int nIn = cur.nIn;
-            // block q of the lane's row; behind the row, 16 bytes of zeros (choosing the address instead of masking
-            // the data leaves nothing to do when the read returns, so it can stay in flight during the step)
-            auto block = [&](int q) { return *reinterpret_cast<const float4 *>(q < nIn ? col + 16 * q : zeros); };
-            float4 w[W];
-#pragma unroll
-            for (int d = 0; d < D; ++d) w[d] = block(d);
-            for (int j0 = 0; j0 < cur.nb; j0 += W) {
-#pragma unroll
-                for (int u = 0; u < W; ++u) {
-                    const int j = j0 + u;
-                    if (j < cur.nb) {
-                        w[(u + D) % W] = block(j + D);  // the block the next step adds
-                        __builtin_amdgcn_sched_barrier(0);  // (issued here, not after the step's matrix work)
-                        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                        for (int d = 0; d < D; ++d) {
-                            const float4 &x = w[(u + d) % W];
-                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[d][0], x.x, acc, 0, 0, 0);
-                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[d][1], x.y, acc, 0, 0, 0);
-                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[d][2], x.z, acc, 0, 0, 0);
-                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[d][3], x.w, acc, 0, 0, 0);
-                        }
-                        *reinterpret_cast<float4 *>(col + 16 * j) =
-                            make_float4(acc.x * p.Ts, acc.y * p.Ts, acc.z * p.Ts, acc.w * p.Ts);
-                    }
-                }
-            }
-        }
-        wave_sync();
-        // rows back out
-        const BufferRsrc bufOut = make_buffer(p.out + cur.row0 * T);
-        RowCol rc;
-        rc.init(lane_again(), lenOut, 1.0f / static_cast<float>(lenOut));
-        const int dr = kWave / lenOut, dc = kWave % lenOut;
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const int t = cur.t0 + (rc.c << 2);
-            const bool on = !chains && rc.r < cur.nRows && rc.c < 4 * cur.nb && t < T;
-            const float4 y = *reinterpret_cast<const float4 *>(X + min(rc.r, 15) * P + (rc.c << 2));
-            buffer_store4(bufOut, masked_offset(on, (rc.r * T + t) * 4), 0, y);
-            rc.advance(dr, dc, lenOut);
-            if (k % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // a few vectors at a time: they occupy registers
-        }
-        if (!more) break;
-        wave_sync();
-        i = iNext;
-        cur = next;
-    }
-}
-
-// ---- the same product from bf16 instructions on a three-way split of both operands -------------------------------
+// ---- bf16 instructions on a three-way split of both operands ------------------------------------------------------
 // v_mfma_f32_16x16x32_bf16 multiplies 8 pairs in the time the fp32 instruction takes for one.  An fp32 number is,
 // to 2^-24 of its size, the sum of three bf16 numbers: its upper 16 bits, the upper 16 bits of what is left, and
 // the same again (8 + 8 + 8 significant bits, each cut, not rounded, so that all three have the number's sign and no
@@ -440,42 +252,178 @@ __global__ __launch_bounds__(64, 2) void fir_mfma_split_kernel(MfmaFirArgs p)
     }
 }
 
-struct MfmaFirPlan {
-    int nb, timeTiles, pitch;
+// ---- the same product for rows of any length and alignment, gated or not -------------------------------------------
+// One wavefront walks over 16 rows chunk by chunk (32 samples), as above, but the samples come straight from memory
+// into the lane that multiplies them, two chunks ahead, and the outputs leave straight from the accumulators, either way 64
+// contiguous bytes per row and instruction (a lane holds samples 4h .. 4h + 3 and 16 + 4h .. of a chunk): no LDS, so a row may have any length, and
+// 16-byte accesses at any multiple of four bytes, so it may start anywhere.  Chunks that reach past the end of the row are
+// loaded (and the last outputs stored) sample by sample.  A long row is cut into segments where there are few rows;
+// a segment reads the NC - 1 chunks behind its own.  GATED: `shift` delays the gate against the samples, i.e. the samples
+// are in[t + shift] (zero from T on): the adjoint of a delay that follows the spike function.
+// An item (16 rows, one segment) in which a sample is not finite is noted and computed again as chains after the walk.
+// Measured, against the kernels that these rows took before (chains on the vector ALUs for rows that are not whole
+// vectors, fp32 matrix instructions for the others): gated, 110 taps, rows of 1450 samples: 65536 rows 580 -> 340 us, 8192
+// rows 79 -> 40, 44 rows 13.4 -> 9.5; plain, 77 taps: (16384, 2000) 92 -> 46 us, (60000, 512) 84 -> 48, (25, 500) 11.2 ->
+// 7.6.  Error against double precision (2-norm): 2.5e-7 -> 1.1e-7.  Bound by the pieces of many rows that it reads and writes
+// (3.4 TB/s; 4.1 where rows start on memory lines, 5.6 on tensors in the last-level cache): 77 taps take as long as 110, and
+// a gate with half the instructions changed nothing.
+struct WalkArgs {
+    float *out;
+    const float *in, *filt;
+    int64_t rows;
+    int T, F, shift;
+    int segChunks, segs;    // chunks per segment, segments per row
+    uint32_t nItems;
+    FastDiv bySegs;
+    float Ts;
+    FirGate gate;
 };
 
-// Blocks per time tile: whole rows if 16 of them fit into a wavefront's share of LDS, else the fewest tiles.
-static MfmaFirPlan plan_mfma(int nBlk, int D, int ldsBytes)
+template <int NCE, int NC, bool GATED>
+__global__ __launch_bounds__(64, 2) void fir_walk_kernel(WalkArgs p)
 {
-    for (int timeTiles = 1; timeTiles <= nBlk; ++timeTiles) {
-        const int nb = static_cast<int>(ceil_div(nBlk, timeTiles));
-        if (static_cast<int>(ceil_div(nBlk, nb)) != timeTiles) continue;
-        const int staged = nb + (timeTiles > 1 ? D - 1 : 0);
-        int pitch = 16 * staged;
-        if ((pitch / 4) % 2 == 0) pitch += 4;
-        if ((16 * pitch + 16) * 4 <= ldsBytes) return MfmaFirPlan{nb, timeTiles, pitch};
-        if (nb <= D) break;  // more halo than tile
-    }
-    return MfmaFirPlan{0, 0, 0};
-}
+    const int lane = threadIdx.x;
+    const int c = lane & 15, h = lane >> 4;
+    const int T = p.T, F = p.F, nCh = (T + 31) >> 5;
 
-template <int NV>
-static void launch_mfma(int D, dim3 grid, size_t lds, hipStream_t st, const MfmaFirArgs &args)
-{
-#define SLAYER_FIR_MFMA(DD)                                                                                            \
-    case DD:                                                                                                           \
-        hipLaunchKernelGGL((fir_mfma_kernel<DD, NV>), grid, dim3(64), lds, st, args);                                 \
-        break
-    switch (D) {
-        SLAYER_FIR_MFMA(4);
-        SLAYER_FIR_MFMA(5);
-        SLAYER_FIR_MFMA(6);
-        SLAYER_FIR_MFMA(7);
-        SLAYER_FIR_MFMA(8);
-        default:
-            SLAYER_FIR_MFMA(9);
+    const BufferRsrc bufF = make_buffer(p.filt, F * 4);
+    SplitPlanes aE[NCE], aO[NC];
+    bool badTap = false;
+#pragma unroll
+    for (int s = 0; s < NC; ++s) {
+        float fe[8], fo[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int tap = 32 * s + 4 * h + e + (e < 4 ? 0 : 12) - c;
+            fe[e] = buffer_load<kCached>(bufF, masked_offset(tap >= 0 && tap < F, tap * 4), 0);
+            fo[e] = buffer_load<kCached>(bufF, masked_offset(tap >= 16 && tap - 16 < F, (tap - 16) * 4), 0);
+            badTap |= fe[e] * 0.0f != 0.0f || fo[e] * 0.0f != 0.0f;
+        }
+        if (s < NCE) aE[s] = split_bf16(fe);
+        aO[s] = split_bf16(fo);
     }
-#undef SLAYER_FIR_MFMA
+    const bool chainsAlways = __builtin_amdgcn_ballot_w64(badTap) != 0;
+
+    for (uint32_t i = blockIdx.x; i < p.nItems; i += gridDim.x) {
+        const uint32_t item = xcd_contiguous(i, p.nItems);
+        const uint32_t rowGroup = fastdiv(item, p.bySegs);
+        const int seg = static_cast<int>(item - rowGroup * p.bySegs.d);
+        const int64_t row0 = static_cast<int64_t>(rowGroup) * 16;
+        const int nRows = static_cast<int>(min(static_cast<int64_t>(16), p.rows - row0));
+        const int mBegin = seg * p.segChunks, mEnd = min(nCh, mBegin + p.segChunks);
+        const BufferRsrc bufIn = make_buffer(p.in + row0 * T), bufOut = make_buffer(p.out + row0 * T);
+        const BufferRsrc bufU = make_buffer((GATED ? p.gate.u : p.in) + row0 * T);
+        const int laneOff = masked_offset(c < nRows, (c * T + 4 * h) * 4);   // sample 4 h of the lane's row
+
+        struct Raw {
+            float4 x0, x1, u0, u1;
+        };
+        auto load = [&](Raw &r, int s) {
+            const int t0 = 32 * s;
+            if (t0 + 32 + p.shift <= T) {
+                r.x0 = buffer_load4<kCached>(bufIn, laneOff, (t0 + p.shift) * 4);
+                r.x1 = buffer_load4<kCached>(bufIn, laneOff, (t0 + p.shift) * 4 + 64);
+                if (GATED) {
+                    r.u0 = buffer_load4<kCached>(bufU, laneOff, t0 * 4);
+                    r.u1 = buffer_load4<kCached>(bufU, laneOff, t0 * 4 + 64);
+                }
+            } else if (t0 >= T) {
+                r.x0 = r.x1 = r.u0 = r.u1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            } else {
+                float x[8], u[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int k = t0 + e + (e < 4 ? 0 : 12), t = k + 4 * h;
+                    const bool row = laneOff != kOutOfRange;
+                    x[e] = buffer_load<kCached>(bufIn, masked_offset(row && t + p.shift < T, laneOff + (k + p.shift) * 4), 0);
+                    u[e] = GATED ? buffer_load<kCached>(bufU, masked_offset(row && t < T, laneOff + k * 4), 0) : 0.0f;
+                }
+                r.x0 = make_float4(x[0], x[1], x[2], x[3]);
+                r.x1 = make_float4(x[4], x[5], x[6], x[7]);
+                r.u0 = make_float4(u[0], u[1], u[2], u[3]);
+                r.u1 = make_float4(u[4], u[5], u[6], u[7]);
+            }
+        };
+        bool bad = false;
+        auto enter = [&](const Raw &r) {
+            float x[8] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w};
+            if (GATED) {
+                const float u[8] = {r.u0.x, r.u0.y, r.u0.z, r.u0.w, r.u1.x, r.u1.y, r.u1.z, r.u1.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] *= spike_pdf(u[e], p.gate.theta, p.gate.tau, p.gate.gain);
+            }
+            bad |= (((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]))) * 0.0f != 0.0f;
+            return split_bf16(x);
+        };
+        auto store = [&](int t0, const f32x4 &a, const f32x4 &b) {   // outputs t0 + 4 h .. + 3 of the lane's row
+            const float y[4] = {(a.x + b.x) * p.Ts, (a.y + b.y) * p.Ts, (a.z + b.z) * p.Ts, (a.w + b.w) * p.Ts};
+            // (cached: the two blocks of a chunk, and neighbouring chunks, complete each other's memory lines)
+            if (t0 + 16 <= T) {
+                buffer_store4<kCached>(bufOut, laneOff, t0 * 4, make_float4(y[0], y[1], y[2], y[3]));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    buffer_store<kCached>(bufOut, masked_offset(laneOff != kOutOfRange && t0 + 4 * h + e < T, laneOff + (t0 + e) * 4), 0, y[e]);
+            }
+        };
+
+        SplitPlanes w[NC];
+        Raw raw[2];
+        {
+            Raw r[NC];
+#pragma unroll
+            for (int s = 0; s < NC; ++s) load(r[s], mBegin + s);
+            load(raw[0], mBegin + NC);
+#pragma unroll
+            for (int s = 0; s < NC; ++s) w[s] = enter(r[s]);
+        }
+        for (int m0 = mBegin; m0 < mEnd; m0 += 2 * NC) {
+#pragma unroll
+            for (int v = 0; v < 2 * NC; ++v) {
+                const int m = m0 + v, u = v % NC;
+                if (m < mEnd) {
+                    load(raw[(v + 1) & 1], m + NC + 1);   // (enters the window one step after the next)
+                    __builtin_amdgcn_sched_barrier(0);
+                    f32x4 e0 = {0.0f, 0.0f, 0.0f, 0.0f}, e1 = e0, o0 = e0, o1 = e0;
+#pragma unroll
+                    for (int s = 0; s < NC; ++s) {
+                        const SplitPlanes &x = w[(u + s) % NC];
+                        if (s < NCE) e1 = mfma_bf16(aE[s].lo, x.hi, e1);
+                        o1 = mfma_bf16(aO[s].lo, x.hi, o1);
+                        if (s < NCE) e1 = mfma_bf16(aE[s].hi, x.lo, e1);
+                        o1 = mfma_bf16(aO[s].hi, x.lo, o1);
+                        if (s < NCE) e1 = mfma_bf16(aE[s].mid, x.mid, e1);
+                        o1 = mfma_bf16(aO[s].mid, x.mid, o1);
+                        if (s < NCE) e1 = mfma_bf16(aE[s].mid, x.hi, e1);
+                        o1 = mfma_bf16(aO[s].mid, x.hi, o1);
+                        if (s < NCE) e1 = mfma_bf16(aE[s].hi, x.mid, e1);
+                        o1 = mfma_bf16(aO[s].hi, x.mid, o1);
+                        if (s < NCE) e0 = mfma_bf16(aE[s].hi, x.hi, e0);
+                        o0 = mfma_bf16(aO[s].hi, x.hi, o0);
+                    }
+                    store(32 * m, e0, e1);
+                    store(32 * m + 16, o0, o1);
+                    w[u] = enter(raw[v & 1]);
+                }
+            }
+        }
+        if (chainsAlways || __builtin_amdgcn_ballot_w64(bad) != 0) {
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");   // the walk's stores are done before the same samples are written again
+            const int tA = 32 * mBegin, n = min(T, 32 * mEnd) - tA;
+            for (int e = lane; e < nRows * n; e += kWave) {
+                const int r = e / n, t = tA + e - r * n;
+                const float *x = p.in + (row0 + r) * T;
+                const float *gu = GATED ? p.gate.u + (row0 + r) * T : nullptr;
+                const int taps = min(T - t, F);
+                float acc = 0.0f;
+                for (int k = 0; k < taps; ++k) {
+                    const float v = t + k + p.shift < T ? x[t + k + p.shift] : 0.0f;
+                    acc = __builtin_fmaf(GATED ? v * spike_pdf(gu[t + k], p.gate.theta, p.gate.tau, p.gate.gain) : v, p.filt[k], acc);
+                }
+                p.out[(row0 + r) * T + t] = acc * p.Ts;
+            }
+        }
+    }
 }
 
 template <bool GATED>
@@ -494,41 +442,86 @@ static void launch_split(int nce, int nc, int nv, dim3 grid, size_t lds, hipStre
 #undef SLAYER_SPLIT_NV
 }
 
-bool launch_fir_corr_mfma(float *out, const float *in, const float *filt, int64_t rows, int64_t T, int64_t F, float Ts,
-                          const FirGate &gate, hipStream_t stream)
+// Segments of a row so that the walks of the wavefronts resident at once end together: the fewest chunks that any of
+// them passes, counting what a segment reads beyond its own and about eight chunks' time for its start.
+static int walk_segments(int64_t rowGroups, int nCh, int nc, int64_t resident)
 {
-    if (F < kFirMfmaMinTaps || F > kFirMfmaMaxTaps || T % 4 != 0 || T < 16 || T > kBufferMaxT) return false;
-    if (!aligned16(out) || !aligned16(in) || (gate.u && !aligned16(gate.u))) return false;
-    const int D = static_cast<int>((F + 14) / 16 + 1);
-    const int nBlk = static_cast<int>(ceil_div(T, 16));
-    MfmaFirPlan plan = plan_mfma(nBlk, D, kMfmaLdsBytes);
-    if (plan.nb < 1) return false;
-    // whole rows whose length spreads the 16 rows over the LDS banks as it is: the tile as it lies in memory
-    const bool asInMemory = plan.timeTiles == 1 && (T / 4) % 2 == 1;
-    // the gated correlation only in that layout (elsewhere it measured no faster than the tiled kernel)
-    if (gate.u && !asInMemory) return false;
-    if (asInMemory) plan.pitch = static_cast<int>(T);
-    const int64_t items = ceil_div(rows, 16) * plan.timeTiles;
-    if (items >= (1LL << 31) || 16 * T >= (1LL << 28)) return false;
+    int best = 1;
+    int64_t bestCost = -1;
+    for (int segs = 1; segs <= nCh && segs <= 64; ++segs) {
+        const int64_t cost = ceil_div(rowGroups * segs, resident) * (ceil_div(nCh, segs) + nc + 8);
+        if (bestCost < 0 || cost < bestCost) {
+            best = segs;
+            bestCost = cost;
+        }
+    }
+    return best;
+}
+
+template <bool GATED>
+static void launch_walk(int nce, int nc, dim3 grid, hipStream_t st, const WalkArgs &a)
+{
+    if (nc == 3 && nce == 2) hipLaunchKernelGGL((fir_walk_kernel<2, 3, GATED>), grid, dim3(64), 0, st, a);
+    else if (nc == 3) hipLaunchKernelGGL((fir_walk_kernel<3, 3, GATED>), grid, dim3(64), 0, st, a);
+    else if (nc == 4 && nce == 3) hipLaunchKernelGGL((fir_walk_kernel<3, 4, GATED>), grid, dim3(64), 0, st, a);
+    else if (nc == 4) hipLaunchKernelGGL((fir_walk_kernel<4, 4, GATED>), grid, dim3(64), 0, st, a);
+    else if (nce == 4) hipLaunchKernelGGL((fir_walk_kernel<4, 5, GATED>), grid, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((fir_walk_kernel<5, 5, GATED>), grid, dim3(64), 0, st, a);
+}
+
+// Aligned rows of at most 304 samples whose length spreads 16 of them over the LDS banks as it is (T / 4 odd): tiles.
+static bool fits_tiles(int64_t T, const void *out, const void *in, const void *u)
+{
+    return T % 8 == 4 && T <= 16 * kMfmaMaxBlocks && aligned16(out) && aligned16(in) && aligned16(u);
+}
+
+bool launch_fir_corr_walk(float *out, const float *in, const float *filt, int64_t rows, int64_t T, int64_t F, int64_t shift,
+                          float Ts, const FirGate &gate, hipStream_t stream)
+{
+    // (rows that the tiles take without a shift are shifted apart, so that a delay's gradient has the same bits either way)
+    if (shift > 0 && fits_tiles(T, out, in, gate.u)) return false;
+    if (F < kFirMfmaMinTaps || F > kFirMfmaMaxTaps || T < 16 || T > kBufferMaxT || shift < 0 || shift > T) return false;
+    const int nCh = static_cast<int>(ceil_div(T, 32));
+    const int nce = static_cast<int>((15 + F + 31) / 32), nc = static_cast<int>((31 + F + 31) / 32);
+    const int64_t rowGroups = ceil_div(rows, 16), resident = static_cast<int64_t>(compute_units()) * 8;
+    if (rowGroups >= (1LL << 24)) return false;
+    int segs = walk_segments(rowGroups, nCh, nc, resident);
+    const int segChunks = static_cast<int>(ceil_div(nCh, segs));
+    segs = static_cast<int>(ceil_div(nCh, segChunks));
+    const int64_t items = rowGroups * segs;
+    const int64_t waves = items < resident ? items : resident;   // (resident: a multiple of 8, one range of items per die)
+    const WalkArgs a{out, in, filt, rows, static_cast<int>(T), static_cast<int>(F), static_cast<int>(shift), segChunks, segs,
+                     static_cast<uint32_t>(items), make_fastdiv(static_cast<uint32_t>(segs)), Ts, gate};
+    const dim3 grid(static_cast<unsigned>(waves));
+    if (gate.u) launch_walk<true>(nce, nc, grid, stream, a);
+    else launch_walk<false>(nce, nc, grid, stream, a);
+    return true;
+}
+
+bool launch_fir_corr_mfma(float *out, const float *in, const float *filt, int64_t rows, int64_t T, int64_t F, float Ts,
+                          const FirGate &gate, bool chainBits, hipStream_t stream)
+{
+    // Tiles of whole rows in LDS as they lie in memory, for aligned rows whose length spreads the 16 rows over the banks
+    // as it is and that are short enough for eight tiles on a compute unit: the walk over rows in memory reads its first
+    // chunks and its ragged last ones again, which counts on short rows (rows of 300 samples: 110 taps gated 111 us here,
+    // 153 us there; 77 taps 112 and 157 us).  Everything else walks, but for rows that are not whole aligned vectors where
+    // the caller has been promised the bits of the chain for them (chainBits).
+    if (chainBits && !(T % 4 == 0 && aligned16(out) && aligned16(in) && aligned16(gate.u))) return false;
+    const bool tiles = F >= kFirMfmaMinTaps && F <= kFirMfmaMaxTaps && T >= 16 && fits_tiles(T, out, in, gate.u) &&
+                       ceil_div(rows, 16) < (1LL << 31);
+    if (!tiles) return launch_fir_corr_walk(out, in, filt, rows, T, F, 0, Ts, gate, stream);
+    const int nv = static_cast<int>(ceil_div(T, 16));
+    const int64_t items = ceil_div(rows, 16);
     // wavefronts resident at once (8 per compute unit); each walks over its share of the tiles
     const int64_t resident = static_cast<int64_t>(compute_units()) * 8;
     const int64_t trips = ceil_div(items, resident);
     const int64_t waves = ceil_div(ceil_div(items, trips), 8) * 8;  // a multiple of 8: one range of tiles per die
-    const int nv = plan.nb + (plan.timeTiles > 1 ? D - 1 : 0);      // vectors per lane = staged blocks per row
-    MfmaFirArgs args{out, in, filt, rows, static_cast<int>(T), static_cast<int>(F), plan.nb, plan.timeTiles, plan.pitch,
-                     nv, static_cast<uint32_t>(items), Ts, gate};
+    MfmaFirArgs args{out, in, filt, rows, static_cast<int>(T), static_cast<int>(F), nv, static_cast<uint32_t>(items), Ts, gate};
     const dim3 grid(static_cast<unsigned>(waves));
-    // (rows as they lie in memory: every lane writes its nv vectors, nv KiB)
-    const size_t lds = asInMemory ? static_cast<size_t>(nv) * 1024 : (static_cast<size_t>(16) * plan.pitch + 16) * sizeof(float);
-    if (asInMemory) {
-        const int nce = static_cast<int>((15 + F + 31) / 32), nc = static_cast<int>((31 + F + 31) / 32);
-        if (gate.u) launch_split<true>(nce, nc, nv, grid, lds, stream, args);
-        else launch_split<false>(nce, nc, nv, grid, lds, stream, args);
-    } else {
-        if (nv <= 12) launch_mfma<12>(D, grid, lds, stream, args);
-        else if (nv <= 16) launch_mfma<16>(D, grid, lds, stream, args);
-        else launch_mfma<20>(D, grid, lds, stream, args);
-    }
+    const size_t lds = static_cast<size_t>(nv) * 1024;
+    const int nce = static_cast<int>((15 + F + 31) / 32), nc = static_cast<int>((31 + F + 31) / 32);
+    if (gate.u) launch_split<true>(nce, nc, nv, grid, lds, stream, args);
+    else launch_split<false>(nce, nc, nv, grid, lds, stream, args);
     return true;
 }
 

@@ -17,7 +17,7 @@ Python numbers or 0-dim tensors, as with pybind11's float conversion.  Outputs a
 with ``torch.empty_like``; kernels are enqueued on PyTorch's current stream of the tensor's
 device and never synchronise with the host.
 
-``spikeBackward``, ``spikeBackwardCorr``, ``pspSpike``, ``getSpikesDelayed``, ``spikeBackwardDelayed``,
+``spikeBackward``, ``spikeBackwardCorr``, ``spikeBackwardDelayedCorr``, ``pspSpike``, ``getSpikesDelayed``, ``spikeBackwardDelayed``,
 ``delayGrad`` and the ``sign`` argument
 of ``shift`` have no counterpart in the reference extension: they are the fused forms of the
 elementwise chains in ``_spikeFunction.backward`` / ``_delayFunction.backward``
@@ -30,8 +30,8 @@ import torch
 
 from . import _lib
 
-__all__ = ["getSpikes", "conv", "corr", "shift", "spikeBackward", "spikeBackwardCorr", "pspSpike", "delayGrad",
-           "getSpikesDelayed", "spikeBackwardDelayed", "spikeLoss", "pspAlpha", "spikeBackwardPspAlpha",
+__all__ = ["getSpikes", "conv", "corr", "shift", "spikeBackward", "spikeBackwardCorr", "spikeBackwardDelayedCorr",
+           "pspSpike", "delayGrad", "getSpikesDelayed", "spikeBackwardDelayed", "spikeLoss", "pspAlpha", "spikeBackwardPspAlpha",
            "pspSpikeBackwardAlpha"]
 
 
@@ -376,9 +376,7 @@ def pspSpike(input, srmKernel, refKernel, theta, Ts):
     return spike, u
 
 
-def spikeBackwardCorr(gradOutput, membranePotential, filter, theta, tau, scale, Ts):
-    """``corr(spikeBackward(gradOutput, membranePotential, theta, tau, scale), filter, Ts)`` in one
-    kernel, without the intermediate tensor (the backward pass of the Loihi neuron)."""
+def _check_corr(gradOutput, membranePotential, filter):
     _check_input(gradOutput, "gradOutput")
     _check_input(membranePotential, "membranePotential")
     _check_input(filter, "filter")
@@ -386,6 +384,12 @@ def spikeBackwardCorr(gradOutput, membranePotential, filter, theta, tau, scale, 
     _check_device(gradOutput, filter, "gradOutput", "filter")
     if gradOutput.shape != membranePotential.shape:
         raise RuntimeError("gradOutput and membranePotential must have the same shape")
+
+
+def spikeBackwardCorr(gradOutput, membranePotential, filter, theta, tau, scale, Ts):
+    """``corr(spikeBackward(gradOutput, membranePotential, theta, tau, scale), filter, Ts)`` in one
+    kernel, without the intermediate tensor (the backward pass of the Loihi neuron)."""
+    _check_corr(gradOutput, membranePotential, filter)
     theta, tau, scale, Ts = _scalar(theta, "theta"), _scalar(tau, "tau"), _scalar(scale, "scale"), _scalar(Ts, "Ts")
     lib = _lib.load()
     gradInput = torch.empty_like(gradOutput)
@@ -396,6 +400,27 @@ def spikeBackwardCorr(gradOutput, membranePotential, filter, theta, tau, scale, 
                                                  stream),
                    "slayer_spike_bwd_corr_f32")
     return gradInput
+
+
+def spikeBackwardDelayedCorr(gradOutput, membranePotential, filter, delaySteps, theta, tau, scale, Ts):
+    """:func:`spikeBackwardCorr` of ``shift(gradOutput, delaySteps, 1.0, sign=-1.0)``: the backward pass of a
+    Loihi neuron whose spikes leave ``delaySteps >= 0`` samples late.  One kernel, on the matrix cores, for
+    rows of any length from 16 samples on and 34 to 129 taps; the two calls elsewhere."""
+    _check_corr(gradOutput, membranePotential, filter)
+    theta, tau, scale, Ts = _scalar(theta, "theta"), _scalar(tau, "tau"), _scalar(scale, "scale"), _scalar(Ts, "Ts")
+    lib = _lib.load()
+    gradInput = torch.empty_like(gradOutput)
+    nNeurons, T = _rows(gradOutput)
+    with _on_device_of(gradOutput) as stream:
+        status = lib.slayer_spike_bwd_delayed_corr_f32(_ptr(gradInput), _ptr(gradOutput), _ptr(membranePotential),
+                                                       _ptr(filter), nNeurons, T, filter.numel(), int(delaySteps),
+                                                       theta, tau, scale, Ts, stream)
+    if status != 2:     # (2: rows that the fused kernel does not serve)
+        _lib.check(status, "slayer_spike_bwd_delayed_corr_f32")
+        return gradInput
+    if delaySteps:
+        gradOutput = shift(gradOutput, float(delaySteps), 1.0, sign=-1.0)
+    return spikeBackwardCorr(gradOutput, membranePotential, filter, theta, tau, scale, Ts)
 
 
 def delayGrad(output, gradOutput, Ts):

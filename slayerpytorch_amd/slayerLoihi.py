@@ -163,9 +163,7 @@ class _spike(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gradOutput):
         voltage, srmKernel = ctx.saved_tensors
-        gradOutput = gradOutput.contiguous()
-        if ctx.delaySteps:   # adjoint of the fused delay: the gradient moves back by as many samples
-            gradOutput = slayerCuda.shift(gradOutput, float(ctx.delaySteps), 1.0, sign=-1.0)
-        # surrogate gradient and correlation with the PSP kernel in one kernel
-        return slayerCuda.spikeBackwardCorr(gradOutput, voltage, srmKernel, ctx.theta,
-                                            ctx.pdfTimeConstant, ctx.pdfScale, ctx.Ts), None, None, None, None
+        # surrogate gradient and correlation with the PSP kernel in one kernel, which also moves the gradient back by
+        # as many samples as the spikes left late
+        return slayerCuda.spikeBackwardDelayedCorr(gradOutput.contiguous(), voltage, srmKernel, ctx.delaySteps, ctx.theta,
+                                                   ctx.pdfTimeConstant, ctx.pdfScale, ctx.Ts), None, None, None, None

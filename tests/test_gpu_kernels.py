@@ -722,6 +722,39 @@ def test_spike_bwd_corr_is_the_two_ops_in_one(impl, shape, Fl):
         assert np.array_equal(bits(got), bits(two)), "fused kernel differs from spikeBackward followed by corr"
 
 
+@pytest.mark.parametrize("T,Fl", [(16, 34), (17, 50), (31, 77), (32, 110), (33, 129), (35, 49), (64, 65), (97, 110), (173, 82),
+                                  (300, 110), (305, 77), (513, 113), (1450, 110)])
+@pytest.mark.parametrize("rows", [1, 19, 32])
+def test_spike_bwd_delayed_corr(T, Fl, rows):
+    """Rows of any length (whole chunks of 32 samples, a last chunk of 1 to 31, one chunk, segments of a long row), inputs that
+    start anywhere, delays up to the whole row: every element within 2e-6 of the sum of its terms' magnitudes of the exact sum
+    (the 1e-6 that split operands are held to elsewhere, and 1e-6 for the gate's rounding);
+    an infinite gradient or potential reaches what it reaches in shift, spikeBackward and corr."""
+    rng = np.random.default_rng(T + Fl + rows)
+    theta, tau, scale, Ts = 10.0, 5.0, 1.5, 0.5
+    f = rng.standard_normal(Fl).astype(np.float32)
+    for n, delay in enumerate([0, 1, 3, 31, T]):
+        if delay > T:
+            continue
+        v = (rng.standard_normal((rows, T)) * 20 + 8).astype(np.float32)
+        g = rng.standard_normal((rows, T)).astype(np.float32)
+        gd, vd = torch.empty(rows * T + 3, device="cuda")[n % 4:][:rows * T].view(rows, T), dev(v)
+        gd.copy_(torch.from_numpy(g))
+        got = host(slayerCuda.spikeBackwardDelayedCorr(gd, vd, dev(f), delay, theta, tau, scale, Ts)).astype(np.float64)
+        moved = np.concatenate([g[:, delay:], np.zeros((rows, delay), np.float32)], axis=1)
+        w = moved.astype(np.float64) * (scale / tau) * np.exp(-np.abs(v.astype(np.float64) - theta) / tau)
+        exact, mag, _ = sum_bounds(w, f)
+        assert np.all(np.abs(got - Ts * exact) <= 2e-6 * Ts * mag + 1e-37), (delay, np.max(np.abs(got - Ts * exact) / (Ts * mag + 1e-37)))
+        if rows > 1:
+            g[rows // 2, T // 2], v[0, T // 3] = -np.inf, np.inf
+            got = host(slayerCuda.spikeBackwardDelayedCorr(dev(g), dev(v), dev(f), delay, theta, tau, scale, Ts))
+            moved = np.concatenate([g[:, delay:], np.zeros((rows, delay), np.float32)], axis=1)
+            want = O.corr(O.spike_bwd(moved, v, theta, tau, scale), f, Ts, fused=True)
+            fin = np.isfinite(want)
+            assert np.array_equal(got[~fin], want[~fin], equal_nan=True) and np.array_equal(np.isfinite(got), fin)
+            assert rel_err(np.where(fin, got, 0), np.where(fin, want, 0)) <= REL_TOL
+
+
 def spikes_follow_filtered_input(s, u, a, srm, nu, theta, Ts):
     """Checks (s, u) = getSpikes(psp) for SOME psp that agrees with Ts * conv(a, srm) to rounding, without knowing
     that psp's bits (a filter summed on the matrix cores): exactly, every sample without a spike ended below the
