@@ -377,12 +377,8 @@ class _poolLayer(nn.Conv3d):
 
     def forward(self, input):
         kH, kW = self.weight.shape[2], self.weight.shape[3]
-        if input.shape[2] % kH != 0:
-            input = torch.cat((input, input.new_zeros((input.shape[0], input.shape[1], input.shape[2] % kH,
-                                                       input.shape[3], input.shape[4]))), 2)
-        if input.shape[3] % kW != 0:
-            input = torch.cat((input, input.new_zeros((input.shape[0], input.shape[1], input.shape[2],
-                                                       input.shape[3] % kW, input.shape[4]))), 3)
+        if input.shape[2] % kH != 0 or input.shape[3] % kW != 0:
+            input = F.pad(input, (0, 0, 0, input.shape[3] % kW, 0, input.shape[2] % kH))
         N, C, H, W, T = input.shape
         weight = self.weight if self.preHookFx is None else self.preHookFx(self.weight)
         result = synapse.synapseConv(input.reshape(N, 1, C * H, W, T), weight, self.stride[:2], self.padding[:2],

@@ -52,6 +52,8 @@ def _check_device(x, y, xname, yname):
 
 
 def _scalar(x, name):
+    if type(x) is float:
+        return x
     if isinstance(x, torch.Tensor):
         if x.numel() != 1:
             raise TypeError("%s must be a number or a one-element tensor" % name)

@@ -79,9 +79,10 @@ class spikeLoss(torch.nn.Module):
             inRegion[startID:stopID] = 1
             actualSpikes = torch.sum(out[..., startID:stopID], 4, keepdim=True) * Ts
             # the count error in double precision, rounded to fp32 at the end, as the reference's numpy does
+            # (the two counts are filled in on the device: a copy from the host would wait for the whole forward pass)
             desiredSpikes = torch.where(desiredClass.to(out.device) == True,            # noqa: E712
-                                        torch.as_tensor(float(count[True]), dtype=torch.float64, device=out.device),
-                                        torch.as_tensor(float(count[False]), dtype=torch.float64, device=out.device))
+                                        torch.full((), float(count[True]), dtype=torch.float64, device=out.device),
+                                        torch.full((), float(count[False]), dtype=torch.float64, device=out.device))
             errorSpikeCount = (actualSpikes.double() - desiredSpikes) / (stopID - startID) * numSpikesScale
             spikeDesired = out * inRegion                 # the output's own spikes inside the region
             countError = (errorSpikeCount * inRegion.double()).to(out.dtype)

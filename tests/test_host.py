@@ -261,3 +261,42 @@ def test_synapse_geometries_beyond_the_kernels_fall_back_to_torch():
     assert t.shape == x.shape
     with pytest.raises(RuntimeError, match="CUDA"):
         synapse.synapseConv(torch.zeros((1, 2, 5, 5, 4)), torch.zeros((3, 2, 3, 3)), 1, 1)
+
+
+def test_plans_are_kept_for_whole_numbers_only():
+    """A layer's plan is kept by its sizes: what was refused before an equal one was kept is refused after, a list, an array or
+    a changed tensor is worked out anew, and a geometry beyond the limits raises every time."""
+    from slayerpytorch_amd import synapse
+    a, w = (1, 2, 9, 9, 8), (4, 2, 3, 3)
+    for _ in range(2):
+        assert synapse.outShape(a, w, 2, 1) == synapse.outShape(list(a), list(w), [2, 2], (1, 1)) == (1, 4, 5, 5, 8)
+        assert synapse.outShape(torch.Size(a), w + (1,), (2, 2), 1) == (1, 4, 5, 5, 8)
+        with pytest.raises(TypeError):
+            synapse.outShape(a, w, 2.0, 1)
+        with pytest.raises(RuntimeError):
+            synapse.outShape(a, (4, 3, 3, 3))
+        with pytest.raises(RuntimeError):
+            synapse.outShape((1, 64, 4096, 4096, 4), (6, 64, 3, 3))
+    stride = torch.tensor(1)
+    assert synapse.outShape(a, w, (stride, 1)) == (1, 4, 7, 7, 8)
+    stride.fill_(2)
+    assert synapse.outShape(a, w, (stride, 1)) == (1, 4, 4, 7, 8)
+
+
+def test_pool_layer_extends_odd_extents_by_zeros():
+    """The pooled tensor and its gradient for odd heights and widths, against the extension that the layer stands for."""
+    from slayerpytorch_amd import slayer, synapse
+    layer = slayer._poolLayer(1.0, 2)
+    seen = []
+    keep, synapse.synapseConv = synapse.synapseConv, lambda x, *rest: seen.append(x) or x
+    try:
+        for H, W in [(5, 4), (4, 5), (5, 7), (4, 6)]:
+            x = torch.randn(2, 3, H, W, 6, requires_grad=True)
+            layer(x)
+            got = seen.pop().reshape(2, 3, H + H % 2, W + W % 2, 6)
+            assert torch.equal(got[:, :, :H, :W], x) and not got[:, :, H:].any() and not got[:, :, :, W:].any()
+            g = torch.randn_like(got)
+            got.backward(g)
+            assert torch.equal(x.grad, g[:, :, :H, :W])
+    finally:
+        synapse.synapseConv = keep
