@@ -14,7 +14,7 @@
 // source patch in LDS (from global memory for patches that do not fit, and a vector kernel for
 // small or unaligned shapes); pooling has a streaming input gradient.  The forward gather and the
 // weight gradient multiply with bf16 matrix instructions over operands split into three bf16 parts
-// (fir_core.h); the input gradient, whose source is a gradient tensor, with the fp32 instruction.
+// (fir_core.h); so does the input gradient where a patch fits LDS as split planes, else with the fp32 instruction.
 // Work-groups that read the same rows are kept on the same die (xcd_contiguous).
 #include <atomic>
 #include <type_traits>
@@ -699,6 +699,7 @@ struct GatherMfmaArgs {
     // before: forward 283 -> 155 us, input gradient 334 -> 194 us; like every product on the matrix cores here, a
     // non-finite sample may give NaN where that kernel gave an infinity.)
     int tLast;
+    int band;                                    // pixel blocks per band (whole rows; planes kernel)
     FastDiv byOGroups, byGroups, byKK, byKW, bySteps, byBlocks, byBlocksPerRow, byPatch, byWX;
 };
 
@@ -1234,6 +1235,280 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
     }
 }
 
+// ---- the same from a patch that is split once, when it is staged -----------------------------------------------------
+// The kernel above reads the patch one dword per tap and sample and splits it in registers, up to KH x KW times per sample
+// and number of channel tiles: its vector and LDS instructions, not its products, set its time.  Where a pass is 16 source
+// channels and the filter has at most ten taps under 30 patch positions (3x3 over eight neighbouring pixels), the staging
+// lanes split every sample once into three planes of bf16 and write them in the layout of the instruction's first operand,
+// channels innermost: a group of 32 reduction indices is two taps of 16 channels, lane (r, h) takes channels 8 (h % 2) .. + 7
+// of sample r at tap h / 2 with one 16-byte read per plane.  A staging lane holds eight channels x four samples of one
+// position.  Sample 4 u + e of octet o of a plane lies at e * 256 + ((8 o + u) ^ (4 e)) * 16: the 16 lanes of a write
+// (u, o) and the 16 lanes of a read (r = 4 u + e) both fall on 16 different 16-byte columns.
+// One patch: the next one travels in registers during the products and is written between two barriers.  Bound by LDS reads
+// (a wavefront reads 60 KB per trip with two channel tiles) and matrix instructions together, 3840 cycles per trip each.
+// 3x3, (12, 300), split kernel / fp32 instructions before -> now: 16 -> 32 channels on 16x16 pixels forward 101 -> 80 us,
+// input gradient 126 -> 102; 32 -> 64 on 8x8: 85 -> 67, 109 -> 87.  Batch of 64: 643 -> 470, 634 -> 598, 427 -> 336, 529 ->
+// 464.  Error against double precision unchanged (forward 1.7e-7) or smaller (gradient 2.9e-7 -> 2.4e-7).
+constexpr int kGpPos = 30;                        // patch positions (filter rows x patch columns)
+constexpr int kGpPosBytes = 3 * 1024;             // 3 planes x 32 samples x 16 channels; position kGpPos holds zeros
+constexpr int kGpPatch = (kGpPos + 1) * kGpPosBytes;
+constexpr int kGpChans = 16;
+
+template <int OT, bool BACKWARD>
+__global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaArgs g)
+{
+    extern __shared__ __align__(16) float lds[];
+    char *const ldsBytes = reinterpret_cast<char *>(lds);
+    constexpr int NG = kGsGroups;
+    typedef const uint4_ext __attribute__((address_space(3))) *LdsUint4;
+    const uint32_t ldsBase = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char *)ldsBytes));
+    uint32_t rest = xcd_contiguous(blockIdx.x, gridDim.x);
+    uint32_t qq = fastdiv(rest, g.byOGroups);
+    const int og = static_cast<int>(rest - qq * g.byOGroups.d);
+    rest = qq; qq = fastdiv(rest, g.byGroups);
+    const int grp = static_cast<int>(rest - qq * g.byGroups.d);
+    const int slice = static_cast<int>(qq);
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, h = lane >> 4;
+    const int KK = g.KH * g.KW;
+    const int64_t srcPlane = static_cast<int64_t>(g.SH) * g.SW * g.T, dstPlane = static_cast<int64_t>(g.DH) * g.DW * g.T;
+    const int rowBytes = g.SW * g.T * 4, pixBytes = g.T * 4, planeBytes = static_cast<int>(srcPlane) * 4;
+    BufferRsrc srcB = make_buffer(g.src), dstB = make_buffer(g.dst);   // (of the batch item at hand: set by place())
+
+    // weights: unit (pass, ot), group G, part, lane (r, h): channels 8 (h % 2) .. + 7 of the pass at tap 2 G + h / 2, for
+    // destination channel 16 (og OT + ot) + r
+    uint4_ext *const wl = reinterpret_cast<uint4_ext *>(ldsBytes + kGpPatch);
+    uint32_t *const flags = reinterpret_cast<uint32_t *>(ldsBytes + kGpPatch + g.passes * OT * kGsUnitBytes);   // [8]
+    for (int e = tid; e < g.passes * OT * NG * 64; e += 512) {
+        const int l = e & 63, G = (e >> 6) % NG, po = (e >> 6) / NG;
+        const int ot = po % OT, pass = po / OT;
+        const int m = (og * OT + ot) * 16 + (l & 15), ij = 2 * G + (l >> 5), q0 = pass * kGpChans + ((l >> 4) & 1) * 8;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v[j] = 0.f;
+            if (ij < KK && m < g.Mg) {
+                const int64_t idx = BACKWARD ? (static_cast<int64_t>(grp * g.Og + q0 + j) * g.Cg + m) * KK + ij
+                                             : (static_cast<int64_t>(grp * g.Og + m) * g.Cg + q0 + j) * KK + ij;
+                v[j] = g.w[idx];
+            }
+        }
+        const SplitPlanes sp = split_bf16(v);
+        uint4_ext *unit = wl + (po * NG + G) * 3 * 64 + l;
+        unit[0] = sp.hi;
+        unit[64] = sp.mid;
+        unit[128] = sp.lo;
+    }
+    if (tid < kGpPosBytes / 16) reinterpret_cast<uint4_ext *>(ldsBytes + kGpPos * kGpPosBytes)[tid] = uint4_ext{0u, 0u, 0u, 0u};
+
+    // LDS address of this lane's operand of group G for samples 16 hf + r (plane `hi`; the others lie 1 and 2 KB on)
+    uint32_t aTab[NG][2];
+#pragma unroll
+    for (int G = 0; G < NG; ++G) {
+        const int ij = 2 * G + (h >> 1);
+        const int i = static_cast<int>(fastdiv(static_cast<uint32_t>(ij), g.byKW)), j = ij - i * g.KW;
+        const int pos = ij < KK ? i * g.WX + wave * g.mulW + j * g.stepW + g.xBias : kGpPos;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+            aTab[G][hf] = ldsBase + static_cast<uint32_t>(pos * kGpPosBytes + (r & 3) * 256 +
+                                                          ((((h & 1) * 8 + (r >> 2) + 4 * hf) ^ (4 * (r & 3))) << 4));
+    }
+    const uint32_t wAddr = ldsBase + kGpPatch + lane * 16;
+
+    int oOff[OT];
+#pragma unroll
+    for (int ot = 0; ot < OT; ++ot) {
+        const int m = (og * OT + ot) * 16 + r;
+        oOff[ot] = masked_offset(m < g.Mg, m * static_cast<int>(dstPlane) * 4 + h * 16);
+    }
+
+    // This lane copies samples 4 u .. 4 u + 3 of channels 8 oct .. + 7 of patch position tid / 16
+    constexpr int NS = 8;
+    const int u = tid & 7, oct = (tid >> 3) & 1, pos = tid >> 4;
+    const bool stages = pos < kGpPos;
+
+    const int p0 = slice * g.pairsPerSlice, p1 = min(g.pairs, p0 + g.pairsPerSlice);
+    const int py = static_cast<int>(fastdiv(static_cast<uint32_t>(pos), g.byWX)), px = pos - py * g.WX;
+    int sOff = kOutOfRange;
+    int pixNext = 0;          // byte offset of this wavefront's destination pixel in a channel plane, or -1
+    auto place = [&](int blockOfAll) {
+        const int n = static_cast<int>(fastdiv(static_cast<uint32_t>(blockOfAll), g.byBlocks));
+        const int block = blockOfAll - n * static_cast<int>(g.byBlocks.d);
+        srcB = make_buffer(g.src + (static_cast<int64_t>(n) * g.SC + static_cast<int64_t>(grp) * g.Qg) * srcPlane);
+        const int a = static_cast<int>(fastdiv(static_cast<uint32_t>(block), g.byBlocksPerRow));
+        const int b0 = (block - a * g.blocksPerRow) * kGmPix;
+        const int nv = min(kGmPix, g.DW - b0);
+        const int xLimit = (nv - 1) * g.mulW + (g.KW - 1) * (g.stepW < 0 ? -g.stepW : g.stepW) + 1;
+        const int y = a * g.mulH + g.offH + py * g.stepH, xx = b0 * g.mulW + g.offW - g.xBias + px;
+        const bool ok = py < g.KH && px < xLimit && static_cast<unsigned>(y) < static_cast<unsigned>(g.SH) &&
+                        static_cast<unsigned>(xx) < static_cast<unsigned>(g.SW);
+        sOff = masked_offset(ok, oct * 8 * planeBytes + y * rowBytes + xx * pixBytes + u * 16);
+        const int b = b0 + wave;
+        pixNext = b < g.DW ? (a * g.DW + b) * pixBytes : -1;
+        return n;
+    };
+    auto issue = [&](float4 (&R)[NS], int st, int pass, bool more) {
+        const int t0 = min(st << 5, g.tLast), uniform = t0 * 4 + pass * kGpChans * planeBytes;
+        const bool live = more && t0 + (u << 2) < g.T;
+#pragma unroll
+        for (int c = 0; c < NS; ++c) R[c] = buffer_load4<0>(srcB, live ? sOff : kOutOfRange, uniform + c * planeBytes);
+    };
+    // registers -> planes; a wavefront notes whether any of its samples has more than the upper 16 bits
+    const int stageAddr = pos * kGpPosBytes;
+    auto stage = [&](const float4 (&R)[NS]) {
+        uint32_t low = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float v[8];
+#pragma unroll
+            for (int c = 0; c < NS; ++c) {
+                v[c] = e == 0 ? R[c].x : e == 1 ? R[c].y : e == 2 ? R[c].z : R[c].w;
+                low |= __builtin_bit_cast(uint32_t, v[c]);
+            }
+            const SplitPlanes sp = split_bf16(v);
+            if (stages) {
+                uint4_ext *at = reinterpret_cast<uint4_ext *>(ldsBytes + stageAddr + e * 256 + (((oct * 8 + u) ^ (4 * e)) << 4));
+                at[0] = sp.hi;
+                at[64] = sp.mid;
+                at[128] = sp.lo;
+            }
+        }
+        const bool any = __builtin_amdgcn_ballot_w64((low & 0xffffu) != 0u) != 0;
+        if (lane == 0) flags[wave] = any ? 1u : 0u;
+    };
+
+    f32x4 acc[2][OT];
+    auto clear = [&]() {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int ot = 0; ot < OT; ++ot) acc[hf][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    // the products of one pass; PARTS = 1 when the patch holds bf16 numbers only (three products instead of six);
+    // HALVES = 1 when the second half of the step lies past the end of the row.  Operands are read one group ahead.
+    auto multiply = [&](auto partsTag, auto halvesTag, int pass) {
+        constexpr int PARTS = decltype(partsTag)::value, HALVES = decltype(halvesTag)::value;
+        const uint32_t wp = wAddr + pass * OT * kGsUnitBytes;
+        uint4_ext wq[2][OT][3], x[2][HALVES][PARTS];
+        auto fetch = [&](int set, int G) {
+#pragma unroll
+            for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+                for (int part = 0; part < 3; ++part)
+                    wq[set][ot][part] = *reinterpret_cast<LdsUint4>(static_cast<size_t>(wp + ((ot * NG + G) * 3 + part) * 1024));
+#pragma unroll
+            for (int hf = 0; hf < HALVES; ++hf)
+#pragma unroll
+                for (int part = 0; part < PARTS; ++part)
+                    x[set][hf][part] = *reinterpret_cast<LdsUint4>(static_cast<size_t>(aTab[G][hf] + part * 1024));
+        };
+        fetch(0, 0);
+#pragma unroll
+        for (int G = 0; G < NG; ++G) {
+            const int set = G & 1;
+            if (G + 1 < NG) fetch(set ^ 1, G + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#define SLAYER_PLANES_MUL(XP, WP)                                                                                      \
+    _Pragma("unroll") for (int hf = 0; hf < HALVES; ++hf) _Pragma("unroll") for (int ot = 0; ot < OT; ++ot)            \
+        acc[hf][ot] = mfma_bf16(x[set][hf][XP], wq[set][ot][WP], acc[hf][ot]);
+            SLAYER_PLANES_MUL(0, 2)
+            if constexpr (PARTS == 3) {
+                SLAYER_PLANES_MUL(2, 0)
+                SLAYER_PLANES_MUL(1, 1)
+            }
+            SLAYER_PLANES_MUL(0, 1)
+            if constexpr (PARTS == 3) {
+                SLAYER_PLANES_MUL(1, 0)
+            }
+            SLAYER_PLANES_MUL(0, 0)
+#undef SLAYER_PLANES_MUL
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto store = [&](int pix, int st) {
+        if (pix < 0) return;
+        const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            const bool live = t0 + hf * 16 + (h << 2) < g.T;
+#pragma unroll
+            for (int ot = 0; ot < OT; ++ot)
+                buffer_store4<0>(dstB, live ? oOff[ot] : kOutOfRange, uniform + hf * 64,
+                                 make_float4(acc[hf][ot][0], acc[hf][ot][1], acc[hf][ot][2], acc[hf][ot][3]));
+        }
+    };
+
+    {
+        // Trip k loads (pair, pass) number k of the range into registers, multiplies number k - 1 from the patch and then,
+        // after a barrier, writes the registers to the patch; the first trip only loads.  Pairs are numbered with the
+        // pixel block of a band fastest, then the step, then the band, then the batch item.
+        const int perItem = static_cast<int>(g.byBlocks.d);   // pixel blocks of a batch item
+        int item = p0 / (perItem * g.steps), left = p0 - item * perItem * g.steps;
+        int first0 = left / (g.band * g.steps) * g.band;          // first pixel block of the band
+        left -= first0 * g.steps;
+        int inBand = min(g.band, perItem - first0);               // pixel blocks of the band
+        int st = left / inBand, at = left - st * inBand, pass = 0;
+        int stCur = 0, passCur = 0, pixCur = -1, nCur = -1, nNext = -1;
+        float4 R[NS];
+        bool first = true;
+        const int trips = (p1 - p0) * g.passes;
+        clear();
+#pragma nounroll
+        for (int k = 0;; ++k) {
+            const bool more = k < trips;
+            bool moved = first;
+            if (more && !first) {
+                if (++pass == g.passes) {
+                    pass = 0;
+                    moved = true;
+                    if (++at == inBand) {
+                        at = 0;
+                        if (++st == g.steps) {
+                            st = 0;
+                            first0 += inBand;
+                            if (first0 == perItem) {
+                                first0 = 0;
+                                ++item;
+                            }
+                            inBand = min(g.band, perItem - first0);
+                        }
+                    }
+                }
+            }
+            if (more && moved) nNext = place(item * perItem + first0 + at);
+            issue(R, st, pass, more);
+            __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the matrix work
+            if (!first) {
+                using I1 = std::integral_constant<int, 1>;
+                using I2 = std::integral_constant<int, 2>;
+                using I3 = std::integral_constant<int, 3>;
+                const bool all = __builtin_amdgcn_ballot_w64(lane < 8 && flags[lane & 7] != 0u) != 0;
+                if (min(stCur << 5, g.tLast) + 16 < g.T) {
+                    if (all) multiply(I3{}, I2{}, passCur);
+                    else multiply(I1{}, I2{}, passCur);
+                } else {
+                    if (all) multiply(I3{}, I1{}, passCur);
+                    else multiply(I1{}, I1{}, passCur);
+                }
+                if (passCur == g.passes - 1) {
+                    if (nCur >= 0) {
+                        dstB = make_buffer(g.dst + (static_cast<int64_t>(nCur) * g.DC + static_cast<int64_t>(grp) * g.Mg) * dstPlane);
+                        store(pixCur, stCur);
+                    }
+                    clear();
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (!more) break;
+            __syncthreads();           // every wavefront has read the patch
+            stage(R);
+            stCur = st; passCur = pass; pixCur = pixNext; nCur = nNext;
+            __syncthreads();
+            first = false;
+        }
+    }
+}
+
 // ---- weight gradient on the matrix cores, input patch of a block of pixels in LDS -------------------
 // The kernel above fetches every input row once per tap that uses it (the working set of four
 // wavefronts does not stay in the 32 KB L1), 64 bytes at a time: it is bound by the number of cache
@@ -1649,9 +1924,36 @@ static int launch_gather_mfma(const GatherArgs &a, const SynGeom &s, bool stride
     g.byWX = make_fastdiv(static_cast<uint32_t>(g.WX));
     const int64_t blocks = base * g.slices;
     if (blocks >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
+    if (chans == kGpChans && KK <= 2 * kGsGroups && static_cast<int64_t>(a.KH) * WX <= kGpPos) {
+        // Bands of pixel blocks that are taken through all steps: consecutive steps share memory lines (a step is one line
+        // long, rows start anywhere), consecutive blocks share patch rows and columns.  Source and destination that fit
+        // the 256 MB last-level cache together: the whole image, step by step (16 -> 32 channels 3x3 on 16x16 pixels,
+        // (12, 300): forward 80 us, in bands of four rows 86).  Larger ones: four rows (batch of 64: forward whole 626 us,
+        // 8 rows 555, 4 rows 470, 2 rows 505, 1 row 551; input gradient 648, 638, 598, 638, 678).
+        const int64_t bytes = 4LL * s.N * a.T * (static_cast<int64_t>(a.SC) * a.SH * a.SW + static_cast<int64_t>(a.DC) * a.DH * a.DW);
+        g.band = g.blocksPerRow * (bytes > (256LL << 20) && a.DH > 4 ? 4 : a.DH);
+        const int ldsBytes = kGpPatch + passes * OT * kGsUnitBytes + 64;
+        // more LDS than a kernel may use without asking; asked once per device (a host-side setting, no allocation)
+        static std::atomic<bool> raised[2][64];
+        int device = 0;
+        hipError_t err = hipGetDevice(&device);
+        if (err == hipSuccess && (device < 0 || device >= 64)) err = hipErrorInvalidDevice;
+        if (err == hipSuccess && !raised[OT - 1][device].load(std::memory_order_acquire)) {
+            const void *fn = OT == 2 ? reinterpret_cast<const void *>(&synapse_gather_planes_kernel<2, BACKWARD>)
+                                     : reinterpret_cast<const void *>(&synapse_gather_planes_kernel<1, BACKWARD>);
+            err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kGpPatch + 4 * kGsUnitBytes + 64);
+            if (err == hipSuccess) raised[OT - 1][device].store(true, std::memory_order_release);
+        }
+        if (err != hipSuccess) return note_hip_error(err);
+        const dim3 grid(static_cast<unsigned>(blocks));
+        if (OT == 2) hipLaunchKernelGGL((synapse_gather_planes_kernel<2, BACKWARD>), grid, dim3(512), ldsBytes, st, g);
+        else hipLaunchKernelGGL((synapse_gather_planes_kernel<1, BACKWARD>), grid, dim3(512), ldsBytes, st, g);
+        return launch_status();
+    }
     if constexpr (BACKWARD) {
         // The source is a gradient tensor: numbers with all their bits, which the bf16 kernel would have to split in
-        // registers, tap by tap (137 us against 120 us on the 16 -> 32 channel layer): the fp32 instructions stay.
+        // registers, tap by tap (137 us against 120 us on the 16 -> 32 channel layer): the fp32 instructions stay for
+        // geometries that the planes do not take.
         const int ldsBytes = 2 * kGmBuf + passes * OT * 64 * kGmSteps * 4;
         // more LDS than a kernel may use without asking; asked once per device (a host-side setting, no allocation)
         static std::atomic<bool> raised[2][64];

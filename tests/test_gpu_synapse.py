@@ -270,6 +270,22 @@ def test_rows_of_any_length_and_alignment(layer, T, impl):
               O.synapse_conv_grad_weight(np.abs(go), np.abs(x), w.shape, *a))
 
 
+@pytest.mark.parametrize("H,T", [(19, 300), (6, 1001)])
+def test_tensors_beyond_the_last_level_cache_are_taken_in_bands(H, T):
+    """Large tensors are walked in bands of four rows of pixels (the last one shorter), small ones image by image: the same
+    products in the same order per element, so every image of a large batch has the bits it has alone."""
+    N = 1 + (1 << 28) // (4 * T * (16 + 32) * H * 16)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    w = torch.randn((32, 16, 3, 3), device="cuda", generator=gen)
+    x = torch.randn((N, 16, H, 16, T), device="cuda", generator=gen)
+    y = synapse.conv(x, w, 1, 1)
+    gx = synapse.convGradInput(y, w, x.shape, 1, 1)
+    for n in (0, 1, N // 2, N - 1):
+        one = x[n:n + 1].contiguous()
+        assert torch.equal(y[n:n + 1], synapse.conv(one, w, 1, 1))
+        assert torch.equal(gx[n:n + 1], synapse.convGradInput(y[n:n + 1].contiguous(), w, one.shape, 1, 1))
+
+
 def test_adjoint_identity_full_size():
     """<conv(x), g> == <x, gradInput(g)> == <w, gradWeight(g, x)> on the benchmark's first layer
     (12, 2, 34, 34, 300) -> 16 channels: a size-independent check of all three kernels."""
