@@ -168,8 +168,9 @@ int slayer_spike_bwd_corr_f32(float *gradIn, const float *gradOut, const float *
  * the backward pass of a Loihi neuron whose spikes leave delaySteps late (slayer_loihi_get_spikes_delayed_f32),
  * w[n][t] = gradOut[n][t + delaySteps] * (scale / tau) * exp(-|u[n][t] - theta| / tau).  Sums on the
  * matrix cores for rows of any length from 16 samples on and any alignment (the chain's values to rounding, 1e-5; delaySteps
- * may be 0).  SLAYER_EUNSUPPORTED, and nothing is done, for rows that the fused kernel does not serve (fewer than 16 samples, filters outside 34 to 129 taps, delays beyond
- * the row): slayer_shift_f32 and slayer_spike_bwd_corr_f32 then.
+ * may be 0).  SLAYER_EUNSUPPORTED, and nothing is done, for rows that the fused kernel does not serve (fewer than 16
+ * samples, filters outside 34 to 129 taps, a delay beyond the row, and delayed rows of at most 304
+ * samples that are whole vectors of an odd number): slayer_shift_f32 and slayer_spike_bwd_corr_f32 then.
  */
 int slayer_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradOut, const float *u, const float *filt,
                                       int64_t nNeurons, int64_t T, int64_t F, int64_t delaySteps, float theta,

@@ -1527,8 +1527,7 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
 // wavefront order, into one workspace row per range.
 constexpr int kWgPix = 4;            // pixels per block (one per wavefront)
 constexpr int kWgRow = 128;          // bytes per patch row: 32 samples
-constexpr int kWgMaxRows = 288;      // patch rows per buffer (9 passes of 32); row kWgMaxRows of a buffer holds zeros
-constexpr int kWgBuf = (kWgMaxRows + 1) * kWgRow;
+constexpr int kWgMaxRows = 288;      // patch rows per buffer: NS = 3, 6 or 9 passes of 32; the row behind them holds zeros
 
 struct WgradLdsArgs {
     const float *gradOut, *in;
@@ -1543,11 +1542,20 @@ struct WgradLdsArgs {
     FastDiv byColGroups, byOGroups, byGroups, byKK, byKW, bySteps, byBlocks, byBlocksPerRow, byPatch, byWX;
 };
 
+constexpr int wg_buffer(int NS) { return (32 * NS + 1) * kWgRow; }
+
+// two patches and their flags, or the four wavefronts' tiles at the end
+constexpr int wg_lds_bytes(int MT, int NT, int NS)
+{
+    return 2 * wg_buffer(NS) + 32 > 4 * MT * NT * 1024 ? 2 * wg_buffer(NS) + 32 : 4 * MT * NT * 1024;
+}
+
 template <int MT, int NT, int NS>
 __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs g)
 {
     extern __shared__ __align__(16) float lds[];
     char *const ldsBytes = reinterpret_cast<char *>(lds);
+    constexpr int ROWS = 32 * NS, BUF = wg_buffer(NS);
     const SynGeom &s = g.s;
     uint32_t rest = xcd_contiguous(blockIdx.x, gridDim.x);
     uint32_t qq = fastdiv(rest, g.byColGroups);
@@ -1585,7 +1593,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
         const int ij = col - static_cast<int>(cl * g.byKK.d);
         const int i = static_cast<int>(fastdiv(static_cast<uint32_t>(ij), g.byKW));
         const int j = ij - i * s.KW;
-        const int row = col < g.CK ? ((static_cast<int>(cl) - c0) * s.KH + i) * g.WX + j * s.dW + wave * s.sW : kWgMaxRows;
+        const int row = col < g.CK ? ((static_cast<int>(cl) - c0) * s.KH + i) * g.WX + j * s.dW + wave * s.sW : ROWS;
         bAddr[0][nt] = row * kWgRow + ((h ^ (row & 7)) << 4);
         bAddr[1][nt] = row * kWgRow + (((4 + h) ^ (row & 7)) << 4);
     }
@@ -1598,7 +1606,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
 
     if (tid < 2 * (kWgRow / 4)) {
         const int b = tid / (kWgRow / 4), e = tid - b * (kWgRow / 4);
-        lds[(b * kWgBuf + kWgMaxRows * kWgRow) / 4 + e] = 0.f;
+        lds[(b * BUF + ROWS * kWgRow) / 4 + e] = 0.f;
     }
 
     const int p0 = slice * g.pairsPerSlice, p1 = min(g.pairs, p0 + g.pairsPerSlice);
@@ -1674,7 +1682,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
         }
     };
     // registers -> patch; a wavefront notes whether any of its samples has more than the upper 16 bits
-    uint32_t *const flags = reinterpret_cast<uint32_t *>(ldsBytes + 2 * kWgBuf);   // [2][4]
+    uint32_t *const flags = reinterpret_cast<uint32_t *>(ldsBytes + 2 * BUF);   // [2][4]
     auto stage = [&](const float4 (&R)[NS], int buf) {
         uint32_t low = 0;
 #pragma unroll
@@ -1738,7 +1746,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
         int block = static_cast<int>(fastdiv(static_cast<uint32_t>(p0), g.bySteps));
         int st = p0 - block * g.steps;
         float4 R[NS], A[2][MT];
-        int buf = kWgBuf;
+        int buf = BUF;
         bool first = true;
 #pragma nounroll
         for (int p = p0 - 1;; ++p) {
@@ -1757,7 +1765,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
             __builtin_amdgcn_sched_barrier(0);
             if (!more) break;
             if ((st << 5) > g.tLast) forget(R, An, (st << 5) - g.tLast);
-            buf = kWgBuf - buf;
+            buf = BUF - buf;
             stage(R, buf);
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf)
@@ -2255,7 +2263,9 @@ static LdsPlan plan_wgrad_lds(const SynGeom &s, const MfmaPlan &m)
     const int64_t base = static_cast<int64_t>(s.groups) * m.oGroups * m.colGroups;
     // two work-groups per compute unit; a few short of the 512 places, which measured faster than all of them
     // (504: 110 us, 512: 123 us on the 2 -> 16 channel 5 x 5 layer)
-    int64_t slices = 504 / base;
+    // small patches and few tiles (25 KB of LDS, 119 registers: the 2 -> 16 channel 5 x 5 layer): three per compute unit
+    // (two, three, four: (12, 300) on 34x34 pixels 112, 101, 103 us; batch of 64 558, 502, 526; spikes, (8, 300) on 32x32 55, 48, 58)
+    int64_t slices = (p.NS == 3 && m.MT * m.NT <= 4 ? 756 : 504) / base;
     if (slices < 1) slices = 1;
     if (slices > pairs) slices = pairs;
     p.pairsPerSlice = static_cast<int>(ceil_div(pairs, slices));
@@ -2266,7 +2276,7 @@ static LdsPlan plan_wgrad_lds(const SynGeom &s, const MfmaPlan &m)
 template <int MT, int NT, int NS>
 static int launch_wgrad_lds_one(const WgradLdsArgs &g, unsigned blocks, hipStream_t st)
 {
-    // two patches of kWgBuf bytes: more than the 64 KB a kernel may use without asking; asked once per device
+    // two patches: more than the 64 KB a kernel may use without asking; asked once per device
     // (a host-side setting of the kernel, no allocation)
     static std::atomic<bool> raised[64];
     int device = 0;
@@ -2274,11 +2284,11 @@ static int launch_wgrad_lds_one(const WgradLdsArgs &g, unsigned blocks, hipStrea
     if (err == hipSuccess && (device < 0 || device >= 64)) err = hipErrorInvalidDevice;
     if (err == hipSuccess && !raised[device].load(std::memory_order_acquire)) {
         err = hipFuncSetAttribute(reinterpret_cast<const void *>(&synapse_wgrad_lds_kernel<MT, NT, NS>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kWgBuf + 32);
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, wg_lds_bytes(MT, NT, NS));
         if (err == hipSuccess) raised[device].store(true, std::memory_order_release);
     }
     if (err != hipSuccess) return note_hip_error(err);
-    hipLaunchKernelGGL((synapse_wgrad_lds_kernel<MT, NT, NS>), dim3(blocks), dim3(256), 2 * kWgBuf + 32, st, g);
+    hipLaunchKernelGGL((synapse_wgrad_lds_kernel<MT, NT, NS>), dim3(blocks), dim3(256), wg_lds_bytes(MT, NT, NS), st, g);
     return launch_status();
 }
 
