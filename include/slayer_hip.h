@@ -540,6 +540,13 @@ int slayer_spike_loss_f32(float *loss, float *error, const float *out, const flo
                           const float *addend, const float *srm, float *workspace, int64_t rows,
                           int64_t T, int64_t F, float Ts, void *stream);
 
+/*
+ * Gradient of that loss with respect to `out`: grad = Ts * corr(error * (gradLoss * Ts), srm), gradLoss one float on the
+ * device, in one launch.  Agrees with slayer_corr_f32 of the scaled error to rounding (1e-5).  Same limits.
+ */
+int slayer_spike_loss_grad_f32(float *grad, const float *error, const float *gradLoss, const float *srm,
+                               int64_t rows, int64_t T, int64_t F, float Ts, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -31,7 +31,7 @@ import torch
 from . import _lib
 
 __all__ = ["getSpikes", "conv", "corr", "shift", "spikeBackward", "spikeBackwardCorr", "spikeBackwardDelayedCorr",
-           "pspSpike", "delayGrad", "getSpikesDelayed", "spikeBackwardDelayed", "spikeLoss", "pspAlpha", "spikeBackwardPspAlpha",
+           "pspSpike", "delayGrad", "getSpikesDelayed", "spikeBackwardDelayed", "spikeLoss", "spikeLossGrad", "pspAlpha", "spikeBackwardPspAlpha",
            "pspSpikeBackwardAlpha"]
 
 
@@ -520,3 +520,27 @@ def spikeLoss(spikeOut, spikeDesired, srmKernel, Ts, addend=None):
         return None
     _lib.check(status, "slayer_spike_loss_f32")
     return loss, error
+
+
+def spikeLossGrad(error, gradLoss, srmKernel, Ts):
+    """``corr(error * (gradLoss * Ts), srmKernel, Ts)``, the gradient of :func:`spikeLoss` with respect to its
+    ``spikeOut`` for the gradient ``gradLoss`` (one element) of the loss, in one launch where a row fits the
+    kernel of :func:`spikeLoss`."""
+    _check_input(error, "error")
+    _check_input(gradLoss, "gradLoss")
+    _check_input(srmKernel, "srmKernel")
+    _check_device(error, gradLoss, "error", "gradLoss")
+    _check_device(error, srmKernel, "error", "srmKernel")
+    if gradLoss.numel() != 1:
+        raise RuntimeError("gradLoss must have one element")
+    Ts = _scalar(Ts, "Ts")
+    lib = _lib.load()
+    rows, T = _rows(error)
+    grad = torch.empty_like(error)
+    with _on_device_of(error) as stream:
+        status = lib.slayer_spike_loss_grad_f32(_ptr(grad), _ptr(error), gradLoss.data_ptr(), _ptr(srmKernel), rows, T,
+                                                srmKernel.numel(), Ts, stream)
+    if status == 2:
+        return corr(error * (gradLoss * Ts), srmKernel, Ts)
+    _lib.check(status, "slayer_spike_loss_grad_f32")
+    return grad

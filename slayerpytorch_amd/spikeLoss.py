@@ -31,7 +31,11 @@ class _spikeLossFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gradLoss):
         error, srmKernel = ctx.saved_tensors
-        grad = slayerCuda.corr(error * (gradLoss * ctx.Ts), srmKernel, ctx.Ts)
+        if gradLoss.is_cuda and gradLoss.dtype == torch.float32:
+            # scaling and correlation in one kernel
+            grad = slayerCuda.spikeLossGrad(error, gradLoss.contiguous(), srmKernel, ctx.Ts)
+        else:
+            grad = slayerCuda.corr(error * (gradLoss * ctx.Ts), srmKernel, ctx.Ts)
         return (grad if ctx.needs_input_grad[0] else None, -grad if ctx.needs_input_grad[1] else None,
                 None, None, None)
 

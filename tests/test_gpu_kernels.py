@@ -1155,3 +1155,36 @@ def test_spike_backward_delayed_equals_shift_then_spike_backward(shape, delay):
     neg = -d if isinstance(d, np.ndarray) else -d
     want = O.spike_bwd(O.shift(g, neg, dTs), u, 10.0, 10.0, 1.0)
     assert rel_err(host(got), want) <= REL_TOL
+
+
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 63, 64, 350, 1023, 1024, 1029, 2000])
+@pytest.mark.parametrize("Fl", [1, 3, 4, 5, 8, 77, 110])
+def test_spike_loss_and_its_gradient(T, Fl):
+    """Rows of any length: the error has the bits of conv (and an infinite sample reaches what it reaches there), the loss is
+    within 1e-5 of the exact sum of its positive terms, the gradient, whose sums are in double precision, within three roundings
+    (scale, sample, output: 2e-7) of the sum of the magnitudes."""
+    rng = np.random.default_rng(100 * T + Fl)
+    s = (rng.random((3, 5, T)) < 0.3).astype(np.float32)
+    d = rng.standard_normal((3, 5, T)).astype(np.float32)
+    add = rng.standard_normal((3, 5, T)).astype(np.float32)
+    f = rng.standard_normal(Fl).astype(np.float32)
+    Ts, up = 0.5, np.float32(1.7)
+    for addend in (None, add):
+        loss, error = slayerCuda.spikeLoss(dev(s), dev(d), dev(f), Ts, None if addend is None else dev(addend))
+        want = O.conv(s - d, f, Ts, fused=True)
+        want = want if addend is None else want + addend
+        assert np.array_equal(bits(host(error)), bits(want))
+        exact = 0.5 * Ts * np.sum(want.astype(np.float64) ** 2)
+        assert abs(float(loss) - exact) <= 1e-5 * exact
+    got = host(slayerCuda.spikeLossGrad(error, torch.tensor(up, device="cuda"), dev(f), Ts)).astype(np.float64).reshape(15, T)
+    exact, mag, _ = sum_bounds(want.reshape(15, T).astype(np.float64) * (float(up) * Ts), f)
+    assert np.all(np.abs(got - Ts * exact) <= 2e-7 * Ts * mag + 1e-37)
+    s[1, 2, T // 2] = np.inf
+    _, error = slayerCuda.spikeLoss(dev(s), dev(d), dev(f), Ts)
+    want = O.conv(s - d, f, Ts, fused=True)
+    assert np.array_equal(host(error), want, equal_nan=True)
+    e = rng.standard_normal((15, T)).astype(np.float32)
+    e[7, T // 3] = np.inf
+    got = host(slayerCuda.spikeLossGrad(dev(e), torch.tensor(np.float32(1.0), device="cuda"), dev(f), 1.0))
+    want = O.corr(e, f, 1.0, fused=True)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want)) and np.array_equal(got[~np.isfinite(want)], want[~np.isfinite(want)], equal_nan=True)
