@@ -50,7 +50,7 @@ def measured_traffic(op):
     except (OSError, ValueError, KeyError):
         return None, None
 KERNEL_OF = {"psp_conv": "slayer::alpha_psp_kernel<true, 4, 0, true> (conv with the alpha kernel as a recursion over time)",
-             "spike": "slayer::spike_tile_kernel<12, 1, 12, 8>",
+             "spike": "slayer::spike_rows_kernel<8, 3, unsigned long>",
              "shift": "slayer::shift_vec_kernel<0>", "shift_bwd": "slayer::shift_vec_kernel<0>",
              "spike_bwd": "slayer::spike_bwd_vec_kernel",
              "psp_corr": "slayer::alpha_psp_kernel<false, 4, 0, true> (corr with the alpha kernel as a recursion over time)"}
@@ -766,7 +766,7 @@ def main():
         psp_fwd = lambda x: slayerCuda.conv(x, srm_t, 1.0)
         psp_bwd = lambda g: slayerCuda.corr(g, srm_t, 1.0)
         KERNEL_OF["psp_conv"] = "slayer::fir_tiled_kernel<true, true, 16, false, 6> (conv as a sum over the taps; spike trains: event-driven path)"
-        KERNEL_OF["psp_corr"] = "slayer::fir_mfma_kernel<6, 20, true, false> (corr as a sum over the taps, matrix cores)"
+        KERNEL_OF["psp_corr"] = "slayer::fir_mfma_split_kernel<3, 4, 20, false> (corr as a sum over the taps, matrix cores)"
     else:
         psp_fwd = lambda x: slayerCuda.pspAlpha(x, srm_t, params["tauSr"], 1.0, 1.0, True)
         psp_bwd = lambda g: slayerCuda.pspAlpha(g, srm_t, params["tauSr"], 1.0, 1.0, False)
