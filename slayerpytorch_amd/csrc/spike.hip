@@ -1009,7 +1009,8 @@ __global__ __launch_bounds__(256) void spike_bwd_scalar_kernel(float *gradIn, co
 
 namespace slayer {
 
-constexpr int kRowsPiecesFrom = 1600;
+constexpr int kRowsPiecesFrom = 700;
+constexpr int64_t kRowsPiecesSamples = 8400000;
 
 // The whole-row kernel for rows whose blocks fit the bit registers; SLAYER_EUNSUPPORTED when they do not (rows beyond
 // 4032 samples).  Lanes per row: 8 for short refractory kernels, 16 for long ones (fewer trips per spike), more while
@@ -1080,9 +1081,11 @@ static int launch_get_spikes(float *s, float *u, const float *nu, int64_t nNeuro
     const bool stream_ok = !generic_forced() && T < (1LL << 30) && groups < (1LL << 31);
     const bool window_ok = stream_ok && T <= kBufferMaxT;
     const bool vec = T % 4 == 0 && aligned16(s) && aligned16(u);
-    // Long rows of whole vectors with a short kernel, and enough of them to fill the GPU, go in pieces: 16384 rows of
-    // 2000 samples take 98 us that way and 107 us whole (of 1500: 79 and 80; 2048 rows of 2000: 41 and 24).
-    const bool pieces = vec && nuSize <= 24 && T > kRowsPiecesFrom && nNeurons >= 8192 && (!dl.on || T <= kSpikeRecordMaxT);
+    // Long rows of whole vectors with a short kernel, and enough samples to fill the GPU, go in pieces.  Smooth potentials,
+    // whole / in pieces: 16000 rows of 600 samples 43 / 45 us, 700: 54 / 50, 1000: 87 / 60, 1400: 132 / 80, 1500: 145 / 87;
+    // of 1000 samples 5000 rows 41 / 47, 8000 49 / 50, 11000 69 / 54; of 1500 3000 rows 43 / 66, 5000 67 / 66, 8000 88 / 71.
+    const bool pieces = vec && nuSize <= 24 && T > kRowsPiecesFrom && nNeurons >= ceil_div(kRowsPiecesSamples, T) &&
+                        (!dl.on || T <= kSpikeRecordMaxT);
     if (window_ok && !pieces) {
         const int status = launch_spike_rows(s, u, nu, nNeurons, T, nuSize, theta, Ts, st, dl);
         if (status != SLAYER_EUNSUPPORTED) return status;

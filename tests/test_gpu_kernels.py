@@ -1188,3 +1188,19 @@ def test_spike_loss_and_its_gradient(T, Fl):
     got = host(slayerCuda.spikeLossGrad(dev(e), torch.tensor(np.float32(1.0), device="cuda"), dev(f), 1.0))
     want = O.corr(e, f, 1.0, fused=True)
     assert np.array_equal(np.isfinite(got), np.isfinite(want)) and np.array_equal(got[~np.isfinite(want)], want[~np.isfinite(want)], equal_nan=True)
+
+
+@pytest.mark.parametrize("T", [700, 704, 1000, 1500, 1604])
+def test_spikes_of_many_long_rows_are_those_of_a_few(T):
+    """Many rows of more than 700 samples (8.4 million samples together) go in pieces, fewer as whole rows: the same bits."""
+    rows = 8400000 // T + 70
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    u = torch.randn((rows, 1, 1, 1, T), device="cuda", generator=gen).cumsum(-1).mul_(0.5).remainder_(24.0).sub_(8.0)
+    nu = dev(np.array([0, -20, -14.7, -8.1, -4.0, -1.8, -0.8, -0.35, -0.15], np.float32))
+    many = u.clone()
+    s = slayerCuda.getSpikes(many, nu, 10.0, 1.0)
+    assert float(s.mean()) > 0.01
+    for a in (0, rows // 2, rows - 50):
+        few = u[a:a + 50].clone()
+        sf = slayerCuda.getSpikes(few, nu, 10.0, 1.0)
+        assert torch.equal(s[a:a + 50], sf) and torch.equal(many[a:a + 50], few)
