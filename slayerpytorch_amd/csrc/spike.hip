@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "spike_rows.h"
 
 namespace slayer {
 
@@ -839,8 +840,12 @@ __global__ __launch_bounds__(64) void spike_rows_kernel(float *__restrict__ s, f
                 for (int i = 0; i < BATCH; ++i) tq[k][i] = tapOf[i * PARTS - k];
             for (int b0 = 0; b0 < NB; b0 += kBlocks) {
                 float w[kBlocks + BATCH - 1];
+                float *at[kBlocks + BATCH - 1];
 #pragma unroll
-                for (int m = 0; m < kBlocks + BATCH - 1; ++m) w[m] = mine[(b0 + m) * PARTS];
+                for (int m = 0; m < kBlocks + BATCH - 1; ++m) {
+                    at[m] = mine + spike_walk_block(b0, m, BATCH, P / PARTS) * PARTS;
+                    w[m] = *at[m];
+                }
                 float hit[2] = {0.0f, 0.0f};   // the spikes as sums of powers of two (one instruction each)
 #pragma unroll
                 for (int k = 0; k < 32; ++k) {
@@ -851,7 +856,7 @@ __global__ __launch_bounds__(64) void spike_rows_kernel(float *__restrict__ s, f
                     for (int i = 0; i < BATCH; ++i) w[k / PARTS + i] = __builtin_fmaf(one, tq[k % PARTS][i], w[k / PARTS + i]);
                 }
 #pragma unroll
-                for (int m = 0; m < kBlocks + BATCH - 1; ++m) mine[(b0 + m) * PARTS] = w[m];
+                for (int m = 0; m < kBlocks + BATCH - 1; ++m) *at[m] = w[m];
                 const uint32_t hits = static_cast<uint32_t>(hit[0]) | static_cast<uint32_t>(hit[1]) << 16;
 #pragma unroll
                 for (int m = 0; m < kBlocks; ++m) fired |= static_cast<Bits>((hits >> (m * PARTS + part)) & 1u) << (b0 + m);
@@ -1012,34 +1017,14 @@ namespace slayer {
 constexpr int kRowsPiecesFrom = 700;
 constexpr int64_t kRowsPiecesSamples = 8400000;
 
-// The whole-row kernel for rows whose blocks fit the bit registers; SLAYER_EUNSUPPORTED when they do not (rows beyond
-// 4032 samples).  Lanes per row: 8 for short refractory kernels, 16 for long ones (fewer trips per spike), more while
-// a tile would take over 11 KB of LDS (fewer than 14 tiles per compute unit: (12,16,34,34,496) takes 228 us with 8
-// lanes and 194 us with 16) or the tensor has too few rows for four wavefronts per compute unit.
+// The whole-row kernel; SLAYER_EUNSUPPORTED for rows that it does not serve (spike_rows_layout).
 static int launch_spike_rows(float *s, float *u, const float *nu, int64_t nNeurons, int64_t T, int64_t nuSize,
                              float theta, float Ts, hipStream_t st, const SpikeDelay &dl)
 {
-    if (T > 4096 || nuSize > 4096) return SLAYER_EUNSUPPORTED;
-    int parts = nuSize <= 24 ? 8 : 16;
-    int rounds, NB, P;
-    size_t lds;
-    for (;; parts *= 2) {
-        rounds = static_cast<int>((nuSize + 2 * parts - 2) / parts);
-        if (rounds < 2) rounds = 2;
-        if (rounds > 3) rounds = (rounds + 3) & ~3;
-        NB = static_cast<int>(ceil_div(T, parts));
-        P = (NB + rounds) * parts;
-        while (P % 64 != parts % 64) P += parts;   // (the rows of a tile start in different banks)
-        const int R = kWave / parts;
-        lds = (static_cast<size_t>(R) * P + 2 * kWave + 3 * R + (rounds + 1) * parts) * sizeof(float);
-        const bool fits = NB <= 63 && rounds <= 60;
-        if (parts == 64) {
-            if (!fits) return SLAYER_EUNSUPPORTED;
-            break;
-        }
-        if (fits && lds <= 11 * 1024 && ceil_div(nNeurons, R) >= 4 * compute_units()) break;
-    }
-    const int R = kWave / parts;
+    const SpikeRowsLayout l = spike_rows_layout(T, nuSize, nNeurons, compute_units());
+    if (!l.served) return SLAYER_EUNSUPPORTED;
+    const int P = l.pitch, NB = l.blocks, rounds = l.rounds, R = kWave / l.parts;
+    const size_t lds = l.ldsBytes;
     const int64_t groups = ceil_div(nNeurons, R);
     if (groups >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
     const FastDiv byNV = make_fastdiv(static_cast<uint32_t>(T >= 4 ? T / 4 : 1));
@@ -1060,7 +1045,7 @@ static int launch_spike_rows(float *s, float *u, const float *nu, int64_t nNeuro
             else SLAYER_SPIKE_ROWS(PV, 0, uint64_t);                                                                    \
         }                                                                                                               \
     } while (0)
-    switch (parts) {
+    switch (l.parts) {
         case 8: SLAYER_SPIKE_ROWS_OF(8); break;
         case 16: SLAYER_SPIKE_ROWS_OF(16); break;
         case 32: SLAYER_SPIKE_ROWS_OF(32); break;

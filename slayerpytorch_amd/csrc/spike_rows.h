@@ -1,0 +1,54 @@
+// Where the whole-row spike kernel (spike.hip) keeps a tile in LDS.  Plain C++: the kernel, its launch and a host test that
+// walks over every shape share it.
+#ifndef SLAYER_SPIKE_ROWS_H
+#define SLAYER_SPIKE_ROWS_H
+
+#include <cstddef>
+#include <cstdint>
+
+namespace slayer {
+
+struct SpikeRowsLayout {
+    bool served;
+    int parts;      // lanes per row
+    int rounds;     // blocks of `parts` samples that a response reaches
+    int blocks;     // blocks of a row
+    int pitch;      // samples from one row of the tile to the next, a multiple of `parts`
+    size_t ldsBytes;
+};
+
+// Rows whose blocks fit the bit registers (not served: rows beyond 4032 samples, refractory kernels beyond 60 blocks).
+// Lanes per row: 8 for short refractory kernels, 16 for long ones (fewer trips per spike), more while a tile would take
+// over 11 KB of LDS (fewer than 14 tiles per compute unit: (12,16,34,34,496) takes 228 us with 8 lanes and 194 us with
+// 16) or the tensor has too few rows for four wavefronts per compute unit.
+constexpr SpikeRowsLayout spike_rows_layout(int64_t T, int64_t nuSize, int64_t nNeurons, int64_t computeUnits)
+{
+    SpikeRowsLayout l{false, nuSize <= 24 ? 8 : 16, 0, 0, 0, 0};
+    if (T > 4096 || nuSize > 4096) return l;
+    for (;; l.parts *= 2) {
+        l.rounds = static_cast<int>((nuSize + 2 * l.parts - 2) / l.parts);
+        if (l.rounds < 2) l.rounds = 2;
+        if (l.rounds > 3) l.rounds = (l.rounds + 3) & ~3;
+        l.blocks = static_cast<int>((T + l.parts - 1) / l.parts);
+        l.pitch = (l.blocks + l.rounds) * l.parts;
+        while (l.pitch % 64 != l.parts % 64) l.pitch += l.parts;   // (the rows of a tile start in different banks)
+        const int R = 64 / l.parts;
+        l.ldsBytes = (static_cast<size_t>(R) * l.pitch + 2 * 64 + 3 * R + (l.rounds + 1) * l.parts) * sizeof(float);
+        l.served = l.blocks <= 63 && l.rounds <= 60;
+        if (l.parts == 64 || (l.served && l.ldsBytes <= 11 * 1024 && (nNeurons + R - 1) / R >= 4 * computeUnits)) return l;
+    }
+}
+
+// The walk over every sample takes the blocks of a row in steps of 32 samples, with the `reach` blocks behind each that a
+// response touches: block m of the step that starts with block b0.  The last step may look past the row's pitch, where the next
+// row (or the spike bits) lies.  All its blocks from the end of the row on are padding, whose samples never change, so what
+// lies beyond the pitch is taken from the last block before it.  (Only blocks beyond the first `reach` + 1 of a step can: at
+// least one of the step's blocks belongs to the row and the pitch holds `rounds` more.)
+constexpr int spike_walk_block(int b0, int m, int rounds, int pitchBlocks)
+{
+    return m <= rounds || b0 + m < pitchBlocks ? b0 + m : pitchBlocks - 1;
+}
+
+}  // namespace slayer
+
+#endif

@@ -655,6 +655,30 @@ def test_spikes_whole_rows_bit_exact(rows, T, nuSize, kind):
     assert same.all()
 
 
+@pytest.mark.parametrize("rows,T,nuSize", [
+    # 8 lanes per row, responses of two and of three blocks, rows of 1 to 38 blocks: every remainder by the four blocks of a step,
+    # one and two words of bits, rows whose last step looks past the row's pitch (5, 29, 30, 37 and 38 blocks)
+    (9000, 7, 11), (9000, 40, 11), (9000, 225, 17), (9000, 236, 11), (9000, 247, 9), (9000, 250, 11), (9000, 262, 5),
+    (9000, 296, 11), (8197, 300, 11), (9000, 303, 10),
+    # 16 lanes per row
+    (4200, 300, 30), (4099, 400, 11), (4100, 510, 33), (4200, 511, 11), (4200, 600, 24)])
+def test_spikes_whole_rows_that_fire_densely_bit_exact(rows, T, nuSize):
+    """Rows above the threshold for most of their samples are walked sample by sample, beside rows that never fire."""
+    rng = np.random.default_rng(rows + T + nuSize)
+    u = rng.standard_normal((rows, T)) * 3
+    u = np.where(rng.random((rows, T)) < 0.85, 10 + np.abs(u), u)
+    u[np.arange(rows) % 3 == 1] -= 30
+    u = u.astype(np.float32).reshape(1, rows, 1, 1, T)
+    nu = (-rng.random(nuSize) * 6 - 0.01).astype(np.float32)
+    nu[0] = -0.0
+    want_s, want_u = O.get_spikes(u, nu, 10.0, 1.0)
+    ud = dev(u)
+    s = slayerCuda.getSpikes(ud, dev(nu), 10.0, 1.0)
+    assert np.array_equal(bits(host(s)), bits(want_s)) and np.array_equal(bits(host(ud)), bits(want_u))
+    # (what the kernel chooses by: one row of a tile above the threshold for more than three fifths of its samples)
+    assert ((u >= 10.0).mean(axis=-1) > 0.62).mean() > 0.6 and want_s.sum() > 0
+
+
 def test_spikes_dense_firing_and_positive_feedback(impl):
     # every sample above threshold, and a refractory kernel that pushes u up (runaway firing)
     rng = np.random.default_rng(3)

@@ -300,3 +300,49 @@ def test_pool_layer_extends_odd_extents_by_zeros():
             assert torch.equal(x.grad, g[:, :, :H, :W])
     finally:
         synapse.synapseConv = keep
+
+
+def test_whole_row_spike_kernel_stays_within_its_rows(tmp_path):
+    """Every block of LDS that the whole-row spike kernel touches lies within its row's pitch, for every row length, number
+    of taps and number of rows that it serves: from spike to spike (block b and the `rounds` from there on, and a finished
+    row's visits to its padding) and sample by sample (spike_walk_block)."""
+    import subprocess
+    source = tmp_path / "walk.cpp"
+    source.write_text("""
+#include "spike_rows.h"
+#include <algorithm>
+#include <cstdio>
+using namespace slayer;
+int main()
+{
+    long shapes = 0, beyond = 0;
+    for (int rows : {1, 1500, 3000, 5000, 1000000})
+        for (int T = 1; T <= 4100; ++T)
+            for (int taps = 0; taps <= 4096; taps += taps < 140 ? 1 : 97) {
+                const SpikeRowsLayout l = spike_rows_layout(T, taps, rows, 256);
+                if (!l.served) continue;
+                ++shapes;
+                const int pitch = l.pitch / l.parts;
+                bool good = l.pitch % l.parts == 0 && l.pitch % 4 == 0 && l.blocks * l.parts >= T && l.blocks + l.rounds <= pitch &&
+                            (l.rounds - 1) * l.parts >= taps - 1 && l.ldsBytes <= 64 * 1024;
+                const int step = std::max(1, 32 / l.parts);
+                for (int b0 = 0; b0 < l.blocks; b0 += step)
+                    for (int m = 0; m < step + l.rounds - 1; ++m) {
+                        const int b = spike_walk_block(b0, m, l.rounds, pitch);
+                        good = good && b >= 0 && b < pitch;
+                        // a block that is not the one asked for is padding, and so is the one taken for it
+                        good = good && (b == b0 + m || (b >= l.blocks && b0 + m >= l.blocks));
+                    }
+                if (!good) {
+                    if (++beyond < 5) std::printf("rows %d T %d taps %d: %d lanes, %d blocks, pitch %d\\n", rows, T, taps, l.parts, l.blocks, pitch);
+                }
+            }
+    std::printf("%ld shapes, %ld beyond\\n", shapes, beyond);
+    return beyond != 0 || shapes < 100000;
+}
+""")
+    program = str(tmp_path / "walk")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "slayerpytorch_amd", "csrc"), str(source), "-o", program],
+                   check=True, timeout=120)
+    r = subprocess.run([program], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout
