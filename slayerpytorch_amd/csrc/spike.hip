@@ -407,10 +407,10 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
                         uint64_t gone = 0u;
 #pragma unroll
                         for (int j = 0; j < kRounds; ++j) {
-                            const bool mineToo = (j + 1) * kParts <= NU || part + j * kParts < NU;
+                            const bool owns = (j + 1) * kParts <= NU || part + j * kParts < NU;
                             const float now = val[j] + myTap[j];
-                            if (mineToo) q[j * kParts] = now;
-                            const uint64_t below = __builtin_amdgcn_ballot_w64(mineToo && now < theta);
+                            if (owns) q[j * kParts] = now;
+                            const uint64_t below = __builtin_amdgcn_ballot_w64(owns && now < theta);
                             gone |= ((below >> (lane - part)) & ((1ull << kParts) - 1ull)) << (j * kParts);
                         }
                         gone <<= k;
@@ -694,28 +694,34 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
 // a row is NaN: never at or above theta.
 // Bound: HBM traffic for short rows; on (12,16,34,34,300) with 11 taps 126-133 us against 143-154 us for the tile
 // kernel (candidate by candidate, every sample written back); not rewriting the blocks of u that no response reached
-// is 15-18 us of that.  Long rows: the chain of LDS round trips from spike to
-// spike, about 0.35 us a spike with one wavefront per SIMD: (4,16,32,32,1450) 262-285 us (tile kernel: 1010 us),
+// is 15-18 us of that.  Long rows: the chain of LDS round trips from spike to spike, about 0.2 us a spike with one
+// wavefront per SIMD, or in the walk over every sample 20-25 ns a sample: (4,16,32,32,1450) 262-285 us (tile kernel: 1010 us),
 // (12,512,1,1,350) 13-17 us (25 us); 110 taps on (12,16,32,32,300) 125-140 us (ring kernel: 2400-3400 us).
-template <int PARTS>
-__device__ __forceinline__ uint32_t row_min(uint32_t x)   // minimum over the PARTS lanes of a row
+template <int PARTS, typename Op>
+__device__ __forceinline__ uint32_t row_reduce(uint32_t x, Op op)   // over the PARTS lanes of a row
 {
-    auto step = [](uint32_t v, auto perm) {
+    auto step = [&](uint32_t v, auto perm) {
         const int o = __builtin_amdgcn_update_dpp(-1, static_cast<int>(v), decltype(perm)::value, 0xf, 0xf, false);
-        return min(v, static_cast<uint32_t>(o));
+        return op(v, static_cast<uint32_t>(o));
     };
     x = step(x, std::integral_constant<int, 0xb1>{});    // quad_perm [1,0,3,2]
     x = step(x, std::integral_constant<int, 0x4e>{});    // quad_perm [2,3,0,1]
     x = step(x, std::integral_constant<int, 0x141>{});   // row_half_mirror
     if constexpr (PARTS >= 16) x = step(x, std::integral_constant<int, 0x140>{});   // row_mirror
     if constexpr (PARTS >= 32) {
-        const uint32_t a = min(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 0)),
-                               static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 16)));
-        const uint32_t b = min(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 32)),
-                               static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 48)));
-        x = PARTS == 64 ? min(a, b) : threadIdx.x < 32 ? a : b;
+        const uint32_t a = op(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 0)),
+                              static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 16)));
+        const uint32_t b = op(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 32)),
+                              static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 48)));
+        x = PARTS == 64 ? op(a, b) : threadIdx.x < 32 ? a : b;
     }
     return x;
+}
+
+template <int PARTS>
+__device__ __forceinline__ uint32_t row_min(uint32_t x)
+{
+    return row_reduce<PARTS>(x, [](uint32_t a, uint32_t b) { return min(a, b); });
 }
 
 // The sample that lane k of each row keeps, in all the row's lanes (8 or 16 lanes per row).
@@ -755,7 +761,11 @@ __global__ __launch_bounds__(64) void spike_rows_kernel(float *__restrict__ s, f
 {
     constexpr int R = kWave / PARTS;
     constexpr int BATCH = ROUNDS ? ROUNDS : 4;
-    constexpr bool kDenseWalk = PARTS <= 16 && ROUNDS != 0;
+    // the walk over every sample: lanes per row (groups of 16 lanes of one row do the same work beside each other) and blocks
+    // of as many samples that a response reaches
+    constexpr SpikeWalk walk = spike_walk(PARTS, ROUNDS);
+    constexpr bool kDenseWalk = ROUNDS != 0 && walk.exists;
+    constexpr int W = walk.lanes, WR = walk.rounds;
     const int rounds = ROUNDS ? ROUNDS : roundsArg;   // blocks that a response reaches, a multiple of BATCH
     extern __shared__ __align__(16) float lds[];
     float *tile = lds;                                                                   // [R][P]
@@ -789,9 +799,17 @@ __global__ __launch_bounds__(64) void spike_rows_kernel(float *__restrict__ s, f
     }
     if (rem && cr < nRows && part < rem) tile[cr * P + 4 * nv + part] = buffer_load(bufU, (cr * T + 4 * nv + part) * 4, 0);
     for (int c = T + part; c < P; c += PARTS) tile[cr * P + c] = __builtin_nanf("");
-    for (int j = lane; j < (rounds + 1) * PARTS; j += kWave) {
-        const int tj = j - (PARTS - 1);
-        taps[j] = (tj >= 0 && tj < nuSize) ? nu[tj] : -0.0f;
+    int quiet = 1;        // samples that a spike keeps below theta, see below
+    bool lowers = true;   // every tap lowers the potential (or is -0.0)
+    for (int j0 = 0; j0 < (rounds + 1) * PARTS; j0 += kWave) {   // (all lanes: they agree on what they count)
+        const int j = j0 + lane, tj = j - (PARTS - 1);
+        const float tap = (tj >= 0 && tj < nuSize) ? nu[tj] : -0.0f;
+        if (j < (rounds + 1) * PARTS) taps[j] = tap;
+        if constexpr (kDenseWalk) {
+            quiet += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tj > 0 && tap < -0.25f * fabsf(theta)));
+            const bool raises = !(tap <= 0.0f && tap > -__builtin_inff() && (__builtin_bit_cast(uint32_t, tap) >> 31) != 0u);
+            lowers = lowers && __builtin_amdgcn_ballot_w64(raises) == 0u;
+        }
     }
     if (dl.on && lane < nRows) {
         const float d = dl.lut ? dl.lut[(row0 + lane) % dl.lutSize] : dl.delay;
@@ -810,56 +828,60 @@ __global__ __launch_bounds__(64) void spike_rows_kernel(float *__restrict__ s, f
     const float *tapOf = taps + (PARTS - 1) + part;
     auto first_of = [](Bits m) { return sizeof(Bits) == 8 ? __builtin_ctzll(m) : __builtin_ctz(static_cast<uint32_t>(m)); };
     const uint32_t none = static_cast<uint32_t>(NB * PARTS);   // a row without further spikes works on its padding
-    // Going from spike to spike takes a tile about 45 instructions per spike of its busiest row; the walk over every sample
-    // about 8 per sample, whatever fires.  The number of spikes is not known, but the samples at or above theta bound
-    // it: tiles with a row that arrives above theta for more than three fifths of its samples take the latter.
-    // (Pooled potentials on (12,16,32,32,300) firing 14, 31 and 62 % of the time, 50, 81 and 96 % above theta: 197, 308
-    // and 491 us from spike to spike, 164 us sample by sample; firing 6 %, 29 % above: 132 and 168 us.)
+    // Going from spike to spike takes a tile about 45 instructions per spike of its busiest row, one after the other; the
+    // walk over every sample 5 to 8 per sample, whatever fires.  The number of spikes is not known.  It is taken for the
+    // samples that arrive at or above theta over the samples that a spike keeps below it, those with a tap beyond a quarter of
+    // theta (five with the taps of tauRef = 1, ten with tauRef = 2; rows above theta throughout fired 22 and 13 % of the time);
+    // tiles with a row above a tenth, by that measure, are walked sample by sample.  From spike to spike / sample by sample /
+    // the tile kernel: 24 rows of 3000 samples that fire 69 % of the time 390 / 76 / 111 us, 12 %: 94 / 76 / 132, 7 %: 44 /
+    // 58 / 94; 40000 rows of 600 samples, four to a tile, 12 %: 108 / 93 / 90, 7 %: 78 / 93 / 94.
     bool dense = false;
     if constexpr (kDenseWalk) {
-        int count = __builtin_popcountll(static_cast<uint64_t>(above));
-#pragma unroll
-        for (int off = PARTS / 2; off > 0; off >>= 1) count += __shfl_xor(count, off, kWave);
-        if (__builtin_amdgcn_ballot_w64(count * 5 > T * 3) != 0u) {
-            bool lowers = true;
-            for (int j = lane; j < (rounds + 1) * PARTS; j += kWave)
-                lowers = lowers && taps[j] <= 0.0f && taps[j] > -__builtin_inff() && (__builtin_bit_cast(uint32_t, taps[j]) >> 31) != 0u;
-            dense = __builtin_amdgcn_ballot_w64(!lowers) == 0u;
-        }
+        const uint32_t count = row_reduce<PARTS>(static_cast<uint32_t>(__builtin_popcountll(static_cast<uint64_t>(above))),
+                                                 [](uint32_t a, uint32_t b) { return a + b; });
+        dense = lowers && nuSize <= (WR - 1) * W + 1 && __builtin_amdgcn_ballot_w64(static_cast<int>(count) * 10 > T * quiet) != 0u;
     }
     if constexpr (kDenseWalk) {
         if (dense) {
             // 32 samples at a time in registers, as they lie in the row's lanes; the sample under test is broadcast to
             // them by lane-permuting moves and the response added as fma(1 or 0, tap, sample) - the addition when the
-            // sample fired, and no change (zeros and their signs included: the taps are negative or -0.0) when not.
-            constexpr int kBlocks = 32 / PARTS;
-            float tq[PARTS][BATCH];   // tq[k][i]: what a spike at lane k's sample adds to this lane's, i blocks on
+            // sample fired, and no change (zeros and their signs included: the taps are negative or -0.0) when not.  What
+            // a spike adds to its own sample is the last addition to it and waits until the step's samples are through:
+            // until then the sample tells whether it fired.
+            constexpr int kBlocks = 32 / W;
+            const int wpart = lane % W;
+            float *const wrow = tile + cr * P + wpart;
+            const float own = taps[PARTS - 1];
+            float tq[W][WR];   // tq[k][i]: what a spike at lane k's sample adds to this lane's, i blocks on
 #pragma unroll
-            for (int k = 0; k < PARTS; ++k)
+            for (int k = 0; k < W; ++k)
 #pragma unroll
-                for (int i = 0; i < BATCH; ++i) tq[k][i] = tapOf[i * PARTS - k];
-            for (int b0 = 0; b0 < NB; b0 += kBlocks) {
-                float w[kBlocks + BATCH - 1];
-                float *at[kBlocks + BATCH - 1];
+                for (int i = 0; i < WR; ++i) tq[k][i] = i == 0 && wpart <= k ? -0.0f : taps[(PARTS - 1) + wpart + i * W - k];
+            const int end = (T + W - 1) / W;
+            for (int b0 = 0; b0 < end; b0 += kBlocks) {
+                float w[kBlocks + WR - 1];
+                float *at[kBlocks + WR - 1];
 #pragma unroll
-                for (int m = 0; m < kBlocks + BATCH - 1; ++m) {
-                    at[m] = mine + spike_walk_block(b0, m, BATCH, P / PARTS) * PARTS;
+                for (int m = 0; m < kBlocks + WR - 1; ++m) {
+                    at[m] = wrow + spike_walk_block(b0, m, WR, P / W) * W;
                     w[m] = *at[m];
                 }
-                float hit[2] = {0.0f, 0.0f};   // the spikes as sums of powers of two (one instruction each)
 #pragma unroll
                 for (int k = 0; k < 32; ++k) {
-                    const bool f = row_sample<PARTS>(w[k / PARTS], k % PARTS) >= theta;
-                    const float one = f ? 1.0f : 0.0f;
-                    hit[k / 16] = __builtin_fmaf(one, static_cast<float>(1u << (k % 16)), hit[k / 16]);
+                    const float one = row_sample<W>(w[k / W], k % W) >= theta ? 1.0f : 0.0f;
 #pragma unroll
-                    for (int i = 0; i < BATCH; ++i) w[k / PARTS + i] = __builtin_fmaf(one, tq[k % PARTS][i], w[k / PARTS + i]);
+                    for (int i = 0; i < WR; ++i) w[k / W + i] = __builtin_fmaf(one, tq[k % W][i], w[k / W + i]);
                 }
 #pragma unroll
-                for (int m = 0; m < kBlocks + BATCH - 1; ++m) *at[m] = w[m];
-                const uint32_t hits = static_cast<uint32_t>(hit[0]) | static_cast<uint32_t>(hit[1]) << 16;
+                for (int m = 0; m < kBlocks; ++m) {
+                    const bool f = w[m] >= theta;
+                    w[m] = f ? w[m] + own : w[m];
+                    // (block b of W samples is part b % (PARTS / W) of block b / (PARTS / W) of PARTS)
+                    const bool owns = PARTS == W || part / W == (b0 + m) % (PARTS / W);
+                    fired |= static_cast<Bits>(f && owns ? 1 : 0) << ((b0 + m) / (PARTS / W));
+                }
 #pragma unroll
-                for (int m = 0; m < kBlocks; ++m) fired |= static_cast<Bits>((hits >> (m * PARTS + part)) & 1u) << (b0 + m);
+                for (int m = 0; m < kBlocks + WR - 1; ++m) *at[m] = w[m];
             }
             dirty = ~static_cast<Bits>(0);
             above = 0;
@@ -1014,14 +1036,10 @@ __global__ __launch_bounds__(256) void spike_bwd_scalar_kernel(float *gradIn, co
 
 namespace slayer {
 
-constexpr int kRowsPiecesFrom = 700;
-constexpr int64_t kRowsPiecesSamples = 8400000;
-
 // The whole-row kernel; SLAYER_EUNSUPPORTED for rows that it does not serve (spike_rows_layout).
-static int launch_spike_rows(float *s, float *u, const float *nu, int64_t nNeurons, int64_t T, int64_t nuSize,
-                             float theta, float Ts, hipStream_t st, const SpikeDelay &dl)
+static int launch_spike_rows(const SpikeRowsLayout &l, float *s, float *u, const float *nu, int64_t nNeurons, int64_t T,
+                             int64_t nuSize, float theta, float Ts, hipStream_t st, const SpikeDelay &dl)
 {
-    const SpikeRowsLayout l = spike_rows_layout(T, nuSize, nNeurons, compute_units());
     if (!l.served) return SLAYER_EUNSUPPORTED;
     const int P = l.pitch, NB = l.blocks, rounds = l.rounds, R = kWave / l.parts;
     const size_t lds = l.ldsBytes;
@@ -1038,10 +1056,12 @@ static int launch_spike_rows(float *s, float *u, const float *nu, int64_t nNeuro
         if (small) {                                                                                                    \
             if (rounds == 2) SLAYER_SPIKE_ROWS(PV, 2, uint32_t);                                                        \
             else if (rounds == 3) SLAYER_SPIKE_ROWS(PV, 3, uint32_t);                                                   \
+            else if (PV == 8 && rounds == 4) SLAYER_SPIKE_ROWS(PV, (PV == 8 ? 4 : 3), uint32_t);                        \
             else SLAYER_SPIKE_ROWS(PV, 0, uint32_t);                                                                    \
         } else {                                                                                                        \
             if (rounds == 2) SLAYER_SPIKE_ROWS(PV, 2, uint64_t);                                                        \
             else if (rounds == 3) SLAYER_SPIKE_ROWS(PV, 3, uint64_t);                                                   \
+            else if (PV == 8 && rounds == 4) SLAYER_SPIKE_ROWS(PV, (PV == 8 ? 4 : 3), uint64_t);                        \
             else SLAYER_SPIKE_ROWS(PV, 0, uint64_t);                                                                    \
         }                                                                                                               \
     } while (0)
@@ -1066,13 +1086,11 @@ static int launch_get_spikes(float *s, float *u, const float *nu, int64_t nNeuro
     const bool stream_ok = !generic_forced() && T < (1LL << 30) && groups < (1LL << 31);
     const bool window_ok = stream_ok && T <= kBufferMaxT;
     const bool vec = T % 4 == 0 && aligned16(s) && aligned16(u);
-    // Long rows of whole vectors with a short kernel, and enough samples to fill the GPU, go in pieces.  Smooth potentials,
-    // whole / in pieces: 16000 rows of 600 samples 43 / 45 us, 700: 54 / 50, 1000: 87 / 60, 1400: 132 / 80, 1500: 145 / 87;
-    // of 1000 samples 5000 rows 41 / 47, 8000 49 / 50, 11000 69 / 54; of 1500 3000 rows 43 / 66, 5000 67 / 66, 8000 88 / 71.
-    const bool pieces = vec && nuSize <= 24 && T > kRowsPiecesFrom && nNeurons >= ceil_div(kRowsPiecesSamples, T) &&
-                        (!dl.on || T <= kSpikeRecordMaxT);
+    const int64_t cus = compute_units();
+    const SpikeRowsLayout whole = spike_rows_layout(T, nuSize, nNeurons, cus);
+    const bool pieces = vec && nuSize <= 24 && (!dl.on || T <= kSpikeRecordMaxT) && spike_rows_better_in_pieces(whole, T, nNeurons, cus);
     if (window_ok && !pieces) {
-        const int status = launch_spike_rows(s, u, nu, nNeurons, T, nuSize, theta, Ts, st, dl);
+        const int status = launch_spike_rows(whole, s, u, nu, nNeurons, T, nuSize, theta, Ts, st, dl);
         if (status != SLAYER_EUNSUPPORTED) return status;
     }
     // a shifted output of rows in pieces: rows of whole vectors whose spike bits fit into LDS
@@ -1080,7 +1098,6 @@ static int launch_get_spikes(float *s, float *u, const float *nu, int64_t nNeuro
     if (window_ok && nuSize <= 24) {
         // 16 rows per tile and pieces of 256 samples unless that would leave wavefront slots of the GPU empty: then 8
         // rows and, for rows of whole vectors, pieces of 512 samples, which doubles the bytes in flight per wavefront
-        const int cus = compute_units();
         int Tc = kTilePiece16, P = 0, MP = 0;
         auto layout = [&]() {
             const int cols = (kTileLag + Tc + 31) & ~31;  // the walk goes in groups of 32 columns
@@ -1091,7 +1108,7 @@ static int launch_get_spikes(float *s, float *u, const float *nu, int64_t nNeuro
             MP = cols / 32 + 1;
         };
         layout();
-        const int64_t slots16 = static_cast<int64_t>(cus) * (160 * 1024 / ((16LL * P + 32 * MP + 16) * 4));
+        const int64_t slots16 = cus * (160 * 1024 / ((16LL * P + 32 * MP + 16) * 4));
         const int rowsPerTile = ceil_div(nNeurons, 16) >= slots16 ? 16 : 8;
         if (rowsPerTile == 8 && vec) {
             Tc = kTilePiece8;
@@ -1112,7 +1129,7 @@ static int launch_get_spikes(float *s, float *u, const float *nu, int64_t nNeuro
         }
         const size_t lds = lds_bytes();
         const int64_t tiles = ceil_div(nNeurons, rowsPerTile);
-        const int64_t resident = static_cast<int64_t>(cus) * (160 * 1024 / static_cast<int64_t>(lds));
+        const int64_t resident = cus * (160 * 1024 / static_cast<int64_t>(lds));
         if (tiles >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
         const dim3 grid(static_cast<unsigned>(tiles < resident ? tiles : resident));
 #define SLAYER_SPIKE_TILE_LAUNCH(NU, VECV, RV)                                                                        \

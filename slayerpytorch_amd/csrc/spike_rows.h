@@ -39,14 +39,34 @@ constexpr SpikeRowsLayout spike_rows_layout(int64_t T, int64_t nuSize, int64_t n
     }
 }
 
-// The walk over every sample takes the blocks of a row in steps of 32 samples, with the `reach` blocks behind each that a
-// response touches: block m of the step that starts with block b0.  The last step may look past the row's pitch, where the next
-// row (or the spike bits) lies.  All its blocks from the end of the row on are padding, whose samples never change, so what
-// lies beyond the pitch is taken from the last block before it.  (Only blocks beyond the first `reach` + 1 of a step can: at
-// least one of the step's blocks belongs to the row and the pitch holds `rounds` more.)
-constexpr int spike_walk_block(int b0, int m, int rounds, int pitchBlocks)
+// The walk over every sample takes a row in blocks of as many samples as lanes serve it, 16 at most, and in steps of 32
+// samples; block m of the step that starts with block b0, of `walkRounds` blocks that a response reaches.  The last step may
+// look past the row's pitch, where the next row (or the spike bits) lies.  All its blocks from the end of the row on are
+// padding, whose samples never change, so what lies beyond the pitch is taken from the last block before it.  (Only blocks
+// beyond the first `walkRounds` + 1 of a step can: one of the step's blocks at least belongs to the row, and the pitch holds
+// as many more.)
+constexpr int spike_walk_block(int b0, int m, int walkRounds, int pitchBlocks)
 {
-    return m <= rounds || b0 + m < pitchBlocks ? b0 + m : pitchBlocks - 1;
+    return m <= walkRounds || b0 + m < pitchBlocks ? b0 + m : pitchBlocks - 1;
+}
+
+// Whether that walk exists for a layout, and its lanes per row and blocks.
+struct SpikeWalk {
+    bool exists;
+    int lanes, rounds;
+};
+
+constexpr SpikeWalk spike_walk(int parts, int rounds)
+{
+    return {parts == 8 ? rounds <= 4 : parts == 16 ? rounds <= 3 : rounds == 2, parts < 16 ? parts : 16, parts <= 16 ? rounds : 3};
+}
+
+// Long rows of whole vectors with a short kernel, and enough samples to fill the GPU, go in pieces.  Smooth potentials,
+// whole / in pieces: 16000 rows of 600 samples 43 / 45 us, 700: 54 / 50, 1000: 87 / 60, 1400: 132 / 80, 1500: 145 / 87;
+// of 1000 samples 5000 rows 41 / 47, 8000 49 / 50, 11000 69 / 54; of 1500 3000 rows 43 / 66, 5000 67 / 66, 8000 88 / 71.
+constexpr bool spike_rows_better_in_pieces(const SpikeRowsLayout &, int64_t T, int64_t nNeurons, int64_t)
+{
+    return T > 700 && nNeurons >= (8400000 + T - 1) / T;
 }
 
 }  // namespace slayer

@@ -661,7 +661,11 @@ def test_spikes_whole_rows_bit_exact(rows, T, nuSize, kind):
     (9000, 7, 11), (9000, 40, 11), (9000, 225, 17), (9000, 236, 11), (9000, 247, 9), (9000, 250, 11), (9000, 262, 5),
     (9000, 296, 11), (8197, 300, 11), (9000, 303, 10),
     # 16 lanes per row
-    (4200, 300, 30), (4099, 400, 11), (4100, 510, 33), (4200, 511, 11), (4200, 600, 24)])
+    (4200, 300, 30), (4099, 400, 11), (4100, 510, 33), (4200, 511, 11), (4200, 600, 24), (4200, 1000, 20),
+    # 8 lanes and four blocks per response; 32 and 64 lanes, whose groups of 16 walk a row together, one and two words of bits,
+    # rows that end within the first half of a block, and with the most taps that this walk takes
+    (9000, 247, 20), (9000, 300, 24), (2500, 300, 11), (2500, 401, 17), (2500, 700, 33), (2051, 1999, 11), (144, 300, 11),
+    (144, 33, 20), (37, 1450, 33), (5, 1984, 24), (3, 2017, 12), (3, 3971, 11), (1, 4032, 20)])
 def test_spikes_whole_rows_that_fire_densely_bit_exact(rows, T, nuSize):
     """Rows above the threshold for most of their samples are walked sample by sample, beside rows that never fire."""
     rng = np.random.default_rng(rows + T + nuSize)
@@ -669,14 +673,13 @@ def test_spikes_whole_rows_that_fire_densely_bit_exact(rows, T, nuSize):
     u = np.where(rng.random((rows, T)) < 0.85, 10 + np.abs(u), u)
     u[np.arange(rows) % 3 == 1] -= 30
     u = u.astype(np.float32).reshape(1, rows, 1, 1, T)
-    nu = (-rng.random(nuSize) * 6 - 0.01).astype(np.float32)
-    nu[0] = -0.0
+    nu = (-rng.random(nuSize) * 2.4 - 0.01).astype(np.float32)     # (no tap beyond a quarter of theta)
+    nu[0] = -0.0 if T % 2 else -1.5
     want_s, want_u = O.get_spikes(u, nu, 10.0, 1.0)
     ud = dev(u)
     s = slayerCuda.getSpikes(ud, dev(nu), 10.0, 1.0)
     assert np.array_equal(bits(host(s)), bits(want_s)) and np.array_equal(bits(host(ud)), bits(want_u))
-    # (what the kernel chooses by: one row of a tile above the threshold for more than three fifths of its samples)
-    assert ((u >= 10.0).mean(axis=-1) > 0.62).mean() > 0.6 and want_s.sum() > 0
+    assert ((u >= 10.0).mean(axis=-1) > 0.5).mean() >= 0.5 and want_s.sum() > 0     # (the kernel chooses by the former)
 
 
 def test_spikes_dense_firing_and_positive_feedback(impl):

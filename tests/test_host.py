@@ -310,8 +310,8 @@ def test_whole_row_spike_kernel_stays_within_its_rows(tmp_path):
     source = tmp_path / "walk.cpp"
     source.write_text("""
 #include "spike_rows.h"
-#include <algorithm>
 #include <cstdio>
+#include <initializer_list>
 using namespace slayer;
 int main()
 {
@@ -325,13 +325,14 @@ int main()
                 const int pitch = l.pitch / l.parts;
                 bool good = l.pitch % l.parts == 0 && l.pitch % 4 == 0 && l.blocks * l.parts >= T && l.blocks + l.rounds <= pitch &&
                             (l.rounds - 1) * l.parts >= taps - 1 && l.ldsBytes <= 64 * 1024;
-                const int step = std::max(1, 32 / l.parts);
-                for (int b0 = 0; b0 < l.blocks; b0 += step)
-                    for (int m = 0; m < step + l.rounds - 1; ++m) {
-                        const int b = spike_walk_block(b0, m, l.rounds, pitch);
-                        good = good && b >= 0 && b < pitch;
-                        // a block that is not the one asked for is padding, and so is the one taken for it
-                        good = good && (b == b0 + m || (b >= l.blocks && b0 + m >= l.blocks));
+                const SpikeWalk walk = spike_walk(l.parts, l.rounds);
+                const int blocks = (T + walk.lanes - 1) / walk.lanes, end = l.pitch / walk.lanes, step = 32 / walk.lanes;
+                good = good && l.pitch % walk.lanes == 0;
+                for (int b0 = 0; walk.exists && b0 < blocks; b0 += step)
+                    for (int m = 0; m < step + walk.rounds - 1; ++m) {
+                        const int b = spike_walk_block(b0, m, walk.rounds, end);
+                        // within the row; a block that is not the one asked for is padding, and so is the one taken for it
+                        good = good && b >= 0 && b < end && (b == b0 + m || (b >= blocks && b0 + m >= blocks));
                     }
                 if (!good) {
                     if (++beyond < 5) std::printf("rows %d T %d taps %d: %d lanes, %d blocks, pitch %d\\n", rows, T, taps, l.parts, l.blocks, pitch);
