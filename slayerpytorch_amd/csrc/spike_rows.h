@@ -18,9 +18,11 @@ struct SpikeRowsLayout {
 };
 
 // Rows whose blocks fit the bit registers (not served: rows beyond 4032 samples, refractory kernels beyond 60 blocks).
-// Lanes per row: 8 for short refractory kernels, 16 for long ones (fewer trips per spike), more while a tile would take
-// over 11 KB of LDS (fewer than 14 tiles per compute unit: (12,16,34,34,496) takes 228 us with 8 lanes and 194 us with
-// 16) or the tensor has too few rows for four wavefronts per compute unit.
+// Lanes per row: 8 for short refractory kernels, 16 for long ones (fewer trips per spike); 16 too where a tile of 8 rows
+// would take over 11 KB of LDS (fewer than 14 tiles per compute unit: (12,16,34,34,496) takes 228 us with 8 lanes and
+// 194 us with 16); more where a tile of 4 or 2 rows would take over 20 KB (8000 rows of 1000 samples: 37 us with 17 KB tiles of
+// 16 lanes per row, 58 us with 32 lanes; tiles of 12 KB the other way cost rows of 640 samples half as much again) or
+// the tensor has too few rows for four wavefronts per compute unit.
 constexpr SpikeRowsLayout spike_rows_layout(int64_t T, int64_t nuSize, int64_t nNeurons, int64_t computeUnits)
 {
     SpikeRowsLayout l{false, nuSize <= 24 ? 8 : 16, 0, 0, 0, 0};
@@ -35,7 +37,7 @@ constexpr SpikeRowsLayout spike_rows_layout(int64_t T, int64_t nuSize, int64_t n
         const int R = 64 / l.parts;
         l.ldsBytes = (static_cast<size_t>(R) * l.pitch + 2 * 64 + 3 * R + (l.rounds + 1) * l.parts) * sizeof(float);
         l.served = l.blocks <= 63 && l.rounds <= 60;
-        if (l.parts == 64 || (l.served && l.ldsBytes <= 11 * 1024 && (nNeurons + R - 1) / R >= 4 * computeUnits)) return l;
+        if (l.parts == 64 || (l.served && l.ldsBytes <= (l.parts == 8 ? 11 : 20) * 1024 && (nNeurons + R - 1) / R >= 4 * computeUnits)) return l;
     }
 }
 
@@ -61,12 +63,23 @@ constexpr SpikeWalk spike_walk(int parts, int rounds)
     return {parts == 8 ? rounds <= 4 : parts == 16 ? rounds <= 3 : rounds == 2, parts < 16 ? parts : 16, parts <= 16 ? rounds : 3};
 }
 
-// Long rows of whole vectors with a short kernel, and enough samples to fill the GPU, go in pieces.  Smooth potentials,
-// whole / in pieces: 16000 rows of 600 samples 43 / 45 us, 700: 54 / 50, 1000: 87 / 60, 1400: 132 / 80, 1500: 145 / 87;
-// of 1000 samples 5000 rows 41 / 47, 8000 49 / 50, 11000 69 / 54; of 1500 3000 rows 43 / 66, 5000 67 / 66, 8000 88 / 71.
-constexpr bool spike_rows_better_in_pieces(const SpikeRowsLayout &, int64_t T, int64_t nNeurons, int64_t)
+// Whether all tiles of a layout are on the GPU at once (160 KB of LDS per compute unit, in granules of 1280 bytes).
+constexpr bool spike_rows_at_once(const SpikeRowsLayout &l, int64_t nNeurons, int64_t computeUnits)
 {
-    return T > 700 && nNeurons >= (8400000 + T - 1) / T;
+    const int64_t perUnit = 160 * 1024 / static_cast<int64_t>((l.ldsBytes + 1279) / 1280 * 1280);
+    return (nNeurons + 64 / l.parts - 1) / (64 / l.parts) <= perUnit * computeUnits;
+}
+
+// Rows of whole vectors of more than 600 samples, with a short kernel, go in pieces where the tiles of the whole-row
+// kernel are more than the GPU holds at once - but for rows of at most 700 samples that would leave the pieces' second
+// round of eight-row tiles about half empty.  Whole / in pieces, potentials that fire 7 % of the time (22 %): 14000 rows of 600
+// samples 34 / 42 us (39 / 42), 40000: 79 / 94 (95 / 88); of 640, 12000 rows 31 / 41 (36 / 40), 14000 41 / 42 (50 / 41),
+// 20000 53 / 68 (63 / 63), 40000 87 / 88 (105 / 78); of 1000, 8000 rows 36 / 49 (42 / 50), 10000 58 / 52 (73 / 55),
+// 16000 78 / 58 (98 / 62); of 1200, 6000 rows 47 / 58 (58 / 54), 8000 68 / 60 (90 / 57).
+constexpr bool spike_rows_better_in_pieces(const SpikeRowsLayout &whole, int64_t T, int64_t nNeurons, int64_t computeUnits)
+{
+    const bool halfRound = T <= 700 && nNeurons > 64 * computeUnits && nNeurons <= 104 * computeUnits;
+    return T > 600 && !(whole.served && (halfRound || spike_rows_at_once(whole, nNeurons, computeUnits)));
 }
 
 }  // namespace slayer

@@ -347,3 +347,28 @@ int main()
                    check=True, timeout=120)
     r = subprocess.run([program], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout
+
+
+def test_whole_rows_or_pieces_where_each_was_measured_faster(tmp_path):
+    """Rows by length that took longer whole than in pieces, and the other way round (256 compute units, 11 taps)."""
+    import subprocess
+    pieces = [(640, 16000), (640, 40000), (700, 12000), (700, 16000), (760, 11000), (760, 16000), (800, 12000), (1000, 10000),
+              (1000, 40000), (1200, 8000), (1500, 8000), (4036, 8000), (8000, 3)]
+    whole = [(300, 200000), (600, 16000), (600, 40000), (640, 8000), (640, 12000), (640, 20000), (700, 11000), (700, 24000),
+             (760, 10000), (800, 8000), (1000, 8000), (1200, 6000), (1500, 4000), (3000, 1000)]
+    source = tmp_path / "rule.cpp"
+    source.write_text("""
+#include "spike_rows.h"
+#include <cstdio>
+int main()
+{
+    long T, rows;
+    while (std::scanf("%ld %ld", &T, &rows) == 2)
+        std::printf("%d\\n", slayer::spike_rows_better_in_pieces(slayer::spike_rows_layout(T, 11, rows, 256), T, rows, 256) ? 1 : 0);
+}
+""")
+    program = str(tmp_path / "rule")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "slayerpytorch_amd", "csrc"), str(source), "-o", program],
+                   check=True, timeout=120)
+    r = subprocess.run([program], input="".join("%d %d\n" % s for s in pieces + whole), capture_output=True, text=True, timeout=60)
+    assert r.stdout.split() == ["1"] * len(pieces) + ["0"] * len(whole)
