@@ -906,23 +906,36 @@ def test_psp_spike_on_matrix_cores_special_cases(kind):
     assert flat_s.sum() > 0
 
 
-def test_spikes_many_long_rows_use_16_row_tiles():
-    # enough long rows to fill the GPU with 16-row tiles (pieces of 256 samples): sampled rows against the oracle
+@pytest.mark.parametrize("T,kind,delay", [(704, "sparse", None), (704, "above", None), (704, "sparse", [3, -5, 0, 1000]),
+                                          (1501, "sparse", None), (4033, "sparse", None), (4033, "above", None)])
+def test_spikes_many_long_rows_use_16_row_tiles(T, kind, delay):
+    """Enough long rows to fill the GPU with 16-row tiles (pieces of 256 samples; rows of 1501 samples go whole beside
+    them): sampled rows against the oracle, potentials below and, for the walk without branches, above the threshold most of the
+    time, spikes that leave late or early."""
+    rows = 34000
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    u = torch.randn((1, rows, 1, 1, T), device="cuda", generator=gen).mul_(6.0)
+    if kind == "above":
+        u.abs_().add_(8.0)
+    nu = np.array(alphaKernel(1.0, 1.0, T, mult=-20.0 if kind == "sparse" else -3.0), dtype=np.float32)
     rng = np.random.default_rng(77)
-    rows, T = 70000, 400
-    u = (rng.standard_normal((1, rows, 1, 1, T)) * 6).astype(np.float32)
-    nu = np.array(alphaKernel(1.0, 1.0, T, mult=-20.0), dtype=np.float32)
-    ud = dev(u)
-    s = host(slayerCuda.getSpikes(ud, dev(nu), 10.0, 1.0)).reshape(rows, T)
-    un = host(ud).reshape(rows, T)
-    pick = np.concatenate([np.arange(40), rng.integers(0, rows, 400), np.arange(rows - 40, rows)])
-    ws, wu = O.get_spikes(u.reshape(rows, T)[pick].reshape(1, len(pick), 1, 1, T), nu, 10.0, 1.0)
-    assert np.array_equal(bits(s[pick]), bits(ws.reshape(len(pick), T)))
-    assert np.array_equal(bits(un[pick]), bits(wu.reshape(len(pick), T)))
+    pick = np.concatenate([np.arange(40), rng.integers(0, rows, 160), np.arange(rows - 40, rows)])
+    index = torch.from_numpy(pick).to(u.device)
+    before = host(u[0, index, 0, 0])
+    if delay is None:
+        s = slayerCuda.getSpikes(u, dev(nu), 10.0, 1.0)
+    else:
+        table = np.resize(np.array(delay, np.float32), rows)
+        s = slayerCuda.getSpikesDelayed(u, dev(nu), 10.0, 1.0, dev(table))
+    s, un = host(s[0, index, 0, 0]), host(u[0, index, 0, 0])
+    ws, wu = O.get_spikes(before.reshape(1, len(pick), 1, 1, T), nu, 10.0, 1.0)
+    if delay is not None:
+        ws = np.stack([O.shift(r.reshape(1, 1, 1, 1, T), float(d), 1.0).reshape(T) for r, d in zip(ws.reshape(len(pick), T), table[pick])])
+    assert np.array_equal(bits(s), bits(ws.reshape(len(pick), T)))
+    assert np.array_equal(bits(un), bits(wu.reshape(len(pick), T)))
     assert ws.sum() > 0
 
 
-# ------------------------------------------------------------------------------------------ delay gradient
 @pytest.mark.parametrize("shape,Ts", [((4, 6, 1, 1, 80), 0.1), ((64, 20, 1, 1, 2000), 1.0), ((3, 2, 5, 7, 33), 0.5),
                                       ((1, 1, 1, 1, 1), 1.0)])
 def test_delay_grad(shape, Ts):
