@@ -696,12 +696,72 @@ struct GatherMfmaArgs {
     // masked.  Other rows: T - 32, so that every vector of every step lies within its row; the samples that the last
     // step shares with the one before are computed and stored twice, with the same values.  (16 -> 32 channels 3x3 on
     // 16x16 pixels, 4 x 1450 samples, against the vector kernel with one sample per access, which such rows took
-    // before: forward 283 -> 155 us, input gradient 334 -> 194 us; like every product on the matrix cores here, a
-    // non-finite sample may give NaN where that kernel gave an infinity.)
+    // before: forward 283 -> 155 us, input gradient 334 -> 194 us.)
     int tLast;
     int band;                                    // pixel blocks per band (whole rows; planes kernel)
     FastDiv byOGroups, byGroups, byKK, byKW, bySteps, byBlocks, byBlocksPerRow, byPatch, byWX;
 };
+
+// A matrix instruction multiplies every operand of its groups, the zeros of taps that are not there among them, and the parts
+// of a split infinity are an infinity and NaN: with a sample or a weight that is not finite, sums come out as NaN that the
+// chain of the vector kernel makes infinite or finite.  So sums that are not finite are made again, as that chain, straight
+// from memory; the others are what they are in any case.  (The check: five instructions per channel tile and half step.)
+template <typename Acc, int OT>
+__device__ __forceinline__ bool gather_not_finite(const Acc (&acc)[2][OT])
+{
+    float z = 0.f;
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot) z = fmaf((acc[hf][ot][0] + acc[hf][ot][1]) + (acc[hf][ot][2] + acc[hf][ot][3]), 0.f, z);
+    return __builtin_amdgcn_ballot_w64(z != 0.f) != 0u;
+}
+
+// n: batch item; pixel: byte offset of the destination pixel in a channel plane; t0: first sample of the step
+template <bool BACKWARD, typename Acc, int OT>
+__device__ __forceinline__ void gather_again(const GatherMfmaArgs &g, Acc (&acc)[2][OT], int n, int grp, int og, int pixel, int t0)
+{
+    const int r = threadIdx.x & 15, h = (threadIdx.x & 63) >> 4;
+    const int64_t srcPlane = static_cast<int64_t>(g.SH) * g.SW * g.T;
+    const BufferRsrc srcB = make_buffer(g.src + (static_cast<int64_t>(n) * g.SC + static_cast<int64_t>(grp) * g.Qg) * srcPlane);
+    const int ab = pixel / (g.T * 4), a = ab / g.DW, b = ab - a * g.DW, KK = g.KH * g.KW;
+    Acc again[2][OT];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot) again[hf][ot] = Acc{0.f, 0.f, 0.f, 0.f};
+#pragma nounroll
+    for (int k = 0; k < g.Qg * KK; ++k) {
+        const int q = k / KK, ij = k - q * KK, i = ij / g.KW, j = ij - i * g.KW;
+        const int y = a * g.mulH + g.offH + i * g.stepH, x = b * g.mulW + g.offW + j * g.stepW;
+        const bool ok = static_cast<unsigned>(y) < static_cast<unsigned>(g.SH) && static_cast<unsigned>(x) < static_cast<unsigned>(g.SW);
+        const int off = q * static_cast<int>(srcPlane) * 4 + ((y * g.SW + x) * g.T + t0 + h * 4) * 4;
+        float4 v[2];
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) v[hf] = buffer_load4<0>(srcB, masked_offset(ok && t0 + hf * 16 + h * 4 < g.T, off + hf * 64), 0);
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot) {
+            const int m = (og * OT + ot) * 16 + r;
+            const float w = m >= g.Mg ? 0.f
+                            : BACKWARD ? g.w[(static_cast<int64_t>(grp * g.Og + q) * g.Cg + m) * KK + ij]
+                                       : g.w[(static_cast<int64_t>(grp * g.Og + m) * g.Cg + q) * KK + ij];
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) {
+                again[hf][ot][0] = fmaf(w, v[hf].x, again[hf][ot][0]);
+                again[hf][ot][1] = fmaf(w, v[hf].y, again[hf][ot][1]);
+                again[hf][ot][2] = fmaf(w, v[hf].z, again[hf][ot][2]);
+                again[hf][ot][3] = fmaf(w, v[hf].w, again[hf][ot][3]);
+            }
+        }
+    }
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                acc[hf][ot][e] = fabsf(acc[hf][ot][e]) < __builtin_inff() ? acc[hf][ot][e] : again[hf][ot][e];
+}
 
 template <int OT, bool BACKWARD>
 __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs g)
@@ -860,9 +920,10 @@ __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs
     // instruction writes 64 bytes of each of 16 channel rows, and a pixel's row is 4 T bytes long: cached stores, so
     // that L2 puts the pieces of a line together (streaming stores of these pieces: 137 us instead of 114 us on
     // the 16 -> 32 channel layer)
-    auto store = [&](int pix, int st) {
+    auto store = [&](int n, int pix, int st) {
         if (pix < 0) return;
         const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
+        if (gather_not_finite(acc)) gather_again<BACKWARD>(g, acc, n, grp, og, pix, t0);
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             const bool live = t0 + hf * 16 + (h << 2) < g.T;
@@ -926,7 +987,7 @@ __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs
                 if (passCur == g.passes - 1) {
                     if (nCur >= 0) {
                         dstB = make_buffer(g.dst + (static_cast<int64_t>(nCur) * g.DC + static_cast<int64_t>(grp) * g.Mg) * dstPlane);
-                        store(pixCur, stCur);
+                        store(nCur, pixCur, stCur);
                     }
                     clear();
                 }
@@ -955,8 +1016,7 @@ __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs
 // A pass has room for 5 groups (160 taps >= the 144 of a pass; taps beyond the pass read the zero row and carry zero
 // weights).  With at most two (pass, channel tile) sets of weights the two patches of the kernel above fit beside
 // them; with up to four there is one patch, written between two barriers after the matrix work.  Numbers below
-// 2^-126 in a part are flushed by the instruction; a non-finite input sample gives NaN where the fp32 sum may
-// give an infinity.
+// 2^-126 in a part are flushed by the instruction.
 constexpr int kGsGroups = 5;
 constexpr int kGsUnitBytes = kGsGroups * 3 * 1024;      // weights of one (pass, channel tile)
 
@@ -1156,9 +1216,10 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    auto store = [&](int pix, int st) {
+    auto store = [&](int n, int pix, int st) {
         if (pix < 0) return;
         const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
+        if (gather_not_finite(acc)) gather_again<BACKWARD>(g, acc, n, grp, og, pix, t0);
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             const bool live = t0 + hf * 16 + (h << 2) < g.T;
@@ -1218,7 +1279,7 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
                 if (passCur == g.passes - 1) {
                     if (nCur >= 0) {
                         dstB = make_buffer(g.dst + (static_cast<int64_t>(nCur) * g.DC + static_cast<int64_t>(grp) * g.Mg) * dstPlane);
-                        store(pixCur, stCur);
+                        store(nCur, pixCur, stCur);
                     }
                     clear();
                 }
@@ -1425,9 +1486,10 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    auto store = [&](int pix, int st) {
+    auto store = [&](int n, int pix, int st) {
         if (pix < 0) return;
         const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
+        if (gather_not_finite(acc)) gather_again<BACKWARD>(g, acc, n, grp, og, pix, t0);
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             const bool live = t0 + hf * 16 + (h << 2) < g.T;
@@ -1493,7 +1555,7 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
                 if (passCur == g.passes - 1) {
                     if (nCur >= 0) {
                         dstB = make_buffer(g.dst + (static_cast<int64_t>(nCur) * g.DC + static_cast<int64_t>(grp) * g.Mg) * dstPlane);
-                        store(pixCur, stCur);
+                        store(nCur, pixCur, stCur);
                     }
                     clear();
                 }
@@ -1806,35 +1868,74 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
 // gradW[q] = sum of the workspace rows: lane (q, part) adds rows part, part+PARTS, ... in order, then
 // the PARTS sums of a weight are added in order (a fixed association for a given geometry).  A group
 // handles 256 / PARTS weights; few weights take more parts so that the launch still fills the GPU.
-template <int PARTS>
+// AGAIN (the rows come from matrix instructions, which make NaN of products with an infinity, see gather_not_finite): sums
+// that are not finite are made again from memory, as chains, by the group together.
+struct WgradAgain {
+    const float *gradOut, *in;
+    SynGeom s;
+};
+
+template <int PARTS, bool AGAIN>
 __global__ __launch_bounds__(256) void synapse_wgrad_sum_kernel(float *__restrict__ gradW,
-                                                                const float *__restrict__ partial, int rows, int nW)
+                                                                const float *__restrict__ partial, int rows, int nW, WgradAgain m)
 {
     constexpr int kWeights = 256 / PARTS;
     __shared__ float part[PARTS][kWeights + 1];
+    __shared__ uint32_t bad;   // a bit per weight
+    __shared__ float waves[4];
     const int ql = threadIdx.x % kWeights, pt = threadIdx.x / kWeights;
     const int q = blockIdx.x * kWeights + ql;
     float acc = 0.f;
     if (q < nW)
         for (int r = pt; r < rows; r += PARTS) acc += partial[static_cast<int64_t>(r) * nW + q];
     part[pt][ql] = acc;
+    if (AGAIN && threadIdx.x == 0) bad = 0u;
     __syncthreads();
     if (threadIdx.x < kWeights && q < nW) {
         float v = part[0][ql];
 #pragma unroll
         for (int k = 1; k < PARTS; ++k) v += part[k][ql];
         gradW[q] = v;
+        if (AGAIN && !(fabsf(v) < __builtin_inff())) atomicOr(&bad, 1u << ql);
+    }
+    if constexpr (AGAIN) {
+        static_assert(kWeights <= 32, "a bit per weight");
+        __syncthreads();
+        const SynGeom &s = m.s;
+        const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+        const int KK = s.KH * s.KW, Cg = s.C / s.groups, Og = s.O / s.groups;
+        for (uint32_t left = bad; left != 0u; left &= left - 1u) {   // (the same in every lane)
+            const int w = blockIdx.x * kWeights + __builtin_ctz(left);
+            const int o = w / (Cg * KK), ck = w - o * Cg * KK, c = o / Og * Cg + ck / KK, ij = ck % KK, i = ij / s.KW, jj = ij - i * s.KW;
+            float sum = 0.f;
+            for (int64_t row = wave; row < static_cast<int64_t>(s.N) * s.OH * s.OW; row += 4) {   // (n, a, b)
+                const int n = static_cast<int>(row / (s.OH * s.OW)), ab = static_cast<int>(row - static_cast<int64_t>(n) * s.OH * s.OW);
+                const int y = ab / s.OW * s.sH - s.pH + i * s.dH, x = ab % s.OW * s.sW - s.pW + jj * s.dW;
+                const bool ok = static_cast<unsigned>(y) < static_cast<unsigned>(s.H) && static_cast<unsigned>(x) < static_cast<unsigned>(s.W);
+                const float *go = m.gradOut + ((static_cast<int64_t>(n) * s.O + o) * s.OH * s.OW + ab) * s.T;
+                const float *in = m.in + (((static_cast<int64_t>(n) * s.C + c) * s.H + (ok ? y : 0)) * s.W + (ok ? x : 0)) * s.T;
+#pragma unroll 4
+                for (int t = lane; t < s.T; t += kWave) sum = fmaf(go[t], ok ? in[t] : 0.f, sum);
+            }
+#pragma unroll
+            for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_down(sum, off, kWave);
+            if (lane == 0) waves[wave] = sum;
+            __syncthreads();
+            if (threadIdx.x == 0) gradW[w] = ((waves[0] + waves[1]) + waves[2]) + waves[3];
+            __syncthreads();
+        }
     }
 }
 
-static void launch_wgrad_sum(float *gradW, const float *workspace, int rows, int nW, hipStream_t st)
+template <bool AGAIN>
+static void launch_wgrad_sum(float *gradW, const float *workspace, int rows, int nW, const WgradAgain &m, hipStream_t st)
 {
     if (nW < 2048)
-        hipLaunchKernelGGL(synapse_wgrad_sum_kernel<64>, dim3(static_cast<unsigned>(ceil_div(nW, 4))), dim3(256), 0, st,
-                           gradW, workspace, rows, nW);
+        hipLaunchKernelGGL((synapse_wgrad_sum_kernel<64, AGAIN>), dim3(static_cast<unsigned>(ceil_div(nW, 4))), dim3(256), 0, st,
+                           gradW, workspace, rows, nW, m);
     else
-        hipLaunchKernelGGL(synapse_wgrad_sum_kernel<16>, dim3(static_cast<unsigned>(ceil_div(nW, 16))), dim3(256), 0, st,
-                           gradW, workspace, rows, nW);
+        hipLaunchKernelGGL((synapse_wgrad_sum_kernel<16, AGAIN>), dim3(static_cast<unsigned>(ceil_div(nW, 16))), dim3(256), 0, st,
+                           gradW, workspace, rows, nW, m);
 }
 
 // ---- host side -------------------------------------------------------------------------------------
@@ -2443,7 +2544,7 @@ extern "C" int slayer_synapse_conv_grad_weight_f32(float *gradW, const float *gr
             rows = l.use ? launch_wgrad_lds(gradOut, in, workspace, s, m, l, nW, st)
                          : launch_wgrad_mfma(gradOut, in, workspace, s, m, nW, st);
             if (rows < 0) return -rows;
-            launch_wgrad_sum(gradW, workspace, rows, nW, st);
+            launch_wgrad_sum<true>(gradW, workspace, rows, nW, WgradAgain{gradOut, in, s}, st);
             return launch_status();
         }
         WgradArgs g{};
@@ -2479,6 +2580,6 @@ extern "C" int slayer_synapse_conv_grad_weight_f32(float *gradW, const float *gr
         if (st1 != SLAYER_OK) return st1;
         rows = s.N * p.slicesPerItem;
     }
-    launch_wgrad_sum(gradW, workspace, rows, nW, st);
+    launch_wgrad_sum<false>(gradW, workspace, rows, nW, WgradAgain{}, st);
     return launch_status();
 }

@@ -760,3 +760,55 @@ def test_dense_layer_sums_over_the_events_of_sparse_input(shape, monkeypatch):
     assert third._inputIsSparse(dev(mid).reshape(3, K, T)) == ((False, True) if many else (False, False))
     with torch.no_grad():                                          # inference takes the events as well
         close(host(fc(dev(x))).reshape(3, O, T), np.einsum("ok,nkt->not", w2, x3), np.einsum("ok,nkt->not", np.abs(w2), np.abs(x3)))
+
+
+@pytest.mark.parametrize("geom", [
+    # planes (3x3, 16 channels), split patch and vector kernel forward; input gradients of both kinds; the weight gradient
+    # from an LDS patch; rows of whole vectors and others
+    (2, 16, 7, 9, 36, 32, (3, 3), 1, 0, 1, 1), (2, 16, 7, 9, 45, 32, (3, 3), 1, 1, 1, 1), (1, 32, 6, 9, 173, 16, (3, 3), 1, 0, 1, 1),
+    (1, 16, 9, 11, 64, 16, (3, 3), 2, 0, 1, 1), (1, 8, 9, 9, 33, 16, (5, 5), 1, 0, 1, 1), (2, 16, 9, 9, 50, 8, (5, 5), 1, 2, 1, 1),
+    (2, 2, 12, 12, 40, 16, (5, 5), 1, 2, 1, 1), (2, 2, 12, 12, 41, 16, (5, 5), 1, 0, 1, 1)])
+@pytest.mark.parametrize("where", ["samples", "weights", "huge"])
+def test_numbers_that_are_not_finite_stay_in_their_sums(geom, where):
+    """An infinity among samples, gradients or weights makes the sums that it enters infinite (NaN where it meets a zero or
+    another sign) and leaves all others as they are, whichever kernel makes them; so do numbers next to the largest."""
+    N, C, H, W, T, O_, K, stride, pad, dil, groups = geom
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((N, C, H, W, T)).astype(np.float32)
+    w = rng.standard_normal((O_, C // groups) + K).astype(np.float32)
+    args = (stride, pad, dil, groups)
+    go = rng.standard_normal(O.synapse_conv(x, w, *args).shape).astype(np.float32)
+    special = [np.inf, -np.inf, np.nan] if where != "huge" else [3.4e38, -3.4e38, 3.39e38]
+    if where == "weights":
+        if pad != 0:
+            pytest.skip("a padding zero times such a weight is NaN, which the oracle leaves out")
+        w[3, 1, 0, 0], w[5, 0, 1, 1] = special[:2]
+    else:
+        for k, v in enumerate(special):
+            x[k % N, k % C, 2 * k, 3, T - 1 - 7 * k] = v
+            go[(k + 1) % N, 2 * k, 2 + k % 2, 2, 11 * k] = v     # (no tap of these pixels reaches the padding)
+        if where == "huge":     # (so that the products stay in range)
+            w *= np.float32(0.01)
+
+    def check(got, f, a, b, part=slice(None)):
+        got, want = got[part], f(a, b)[part]
+        with np.errstate(all="ignore"):
+            fits = np.abs(want) < 1e38
+            fin = np.isfinite(want) & fits
+            same = np.where(np.isnan(want), np.isnan(got), np.where(np.isinf(want), got == want, fin <= np.isfinite(got)))
+        assert same.all(), "%d of %d" % ((~same).sum(), same.size)
+        tame = [np.where(np.isfinite(v), np.abs(v), 0).astype(np.float32) for v in (a, b)]
+        scale = f(*tame)[part]
+        assert (np.abs(got.astype(np.float64) - want)[fin] <= SUM_TOL * scale[fin] + 1e-30).all()
+
+    with np.errstate(all="ignore"):
+        check(host(synapse.conv(dev(x), dev(w), *args)), lambda a, b: O.synapse_conv(a, b, *args), x, w)
+        # (weights: the pixels that every tap reaches; a tap outside, or between strides, multiplies a zero)
+        inner = (Ellipsis, slice(K[0] - 1, H - K[0] + 1), slice(K[1] - 1, W - K[1] + 1), slice(None)) if where == "weights" else slice(None)
+        if where != "weights" or stride == 1:
+            check(host(synapse.convGradInput(dev(go), dev(w), x.shape, *args)),
+                  lambda a, b: O.synapse_conv_grad_input(a, b, x.shape, *args), go, w, inner)
+        if where == "huge":
+            x = rng.standard_normal(x.shape).astype(np.float32) * np.float32(0.01)
+        check(host(synapse.convGradWeight(dev(go), dev(x), w.shape, *args)),
+              lambda a, b: O.synapse_conv_grad_weight(a, b, w.shape, *args), go, x)
