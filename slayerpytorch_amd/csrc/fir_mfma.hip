@@ -41,14 +41,14 @@ struct MfmaFirArgs {
 };
 
 // ---- bf16 instructions on a three-way split of both operands ------------------------------------------------------
-// v_mfma_f32_16x16x32_bf16 multiplies 8 pairs in the time the fp32 instruction takes for one.  An fp32 number is,
-// to 2^-24 of its size, the sum of three bf16 numbers: its upper 16 bits, the upper 16 bits of what is left, and
-// the same again (8 + 8 + 8 significant bits, each cut, not rounded, so that all three have the number's sign and no
-// part overflows).  A product of two split numbers is then the sum of nine bf16 products, each exact in the
-// instruction's fp32 accumulator.  The three smallest (mid x low, low x mid, low x low: each below 2^-23 of the
-// product) are left out; the six others take 6 / 8 of an fp32 instruction's time.  Measured against the exact sum,
-// the result stays within 5e-7 * sum |x| |filt| (the instructions round their accumulator too) on samples and taps
-// of ordinary size.  The instruction reads a bf16 operand below 2^-126 as zero, which drops parts of samples and taps
+// v_mfma_f32_16x16x32_bf16 multiplies 8 pairs in the time the fp32 instruction takes for one.  An fp32 number is the sum of
+// three bf16 numbers: the nearest one, the one nearest to the remainder, and what is left then (8 significant bits each and
+// the signs of the remainders: all 24 bits).  A product of two split numbers is then the sum of nine bf16 products, each
+// exact in the instruction's fp32 accumulator.  The three smallest (mid x low, low x mid, low x low: below 2^-24 of the
+// product together, of either sign) are left out; the six others take 6 / 8 of an fp32 instruction's time.  (Cut instead
+// of rounded parts leave out up to 2^-21, always towards zero: sums of one term were 5.8e-8 off, root mean square, where the
+// chain is 2.5e-8 off.  Rounded: 2.6e-8, and full windows 5.5e-8 instead of 7.6e-8 of their 2-norm, the chain 1.6e-7.)
+// The instruction reads a bf16 operand below 2^-126 as zero, which drops parts of samples and taps
 // below 2^-102 of size: at most 2^-124 * (sum |filt| + sum |x| over an output's window) in absolute terms.
 // A tap that is not finite has no split, so then all tiles take the chains (as a tile with such a sample does).
 //
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(64, 2) void fir_mfma_split_kernel(MfmaFirArgs p)
 // Measured, against the kernels that these rows took before (chains on the vector ALUs for rows that are not whole
 // vectors, fp32 matrix instructions for the others): gated, 110 taps, rows of 1450 samples: 65536 rows 580 -> 340 us, 8192
 // rows 79 -> 40, 44 rows 13.4 -> 9.5; plain, 77 taps: (16384, 2000) 92 -> 46 us, (60000, 512) 84 -> 48, (25, 500) 11.2 ->
-// 7.6.  Error against double precision (2-norm): 2.5e-7 -> 1.1e-7.  Bound by the pieces of many rows that it reads and writes
+// 7.6.  Error against double precision (2-norm): 1.6e-7 -> 5.5e-8, sums of one term 2.5e-8 -> 2.6e-8.  Bound by the pieces of many rows that it reads and writes
 // (3.4 TB/s; 4.1 where rows start on memory lines, 5.6 on tensors in the last-level cache): 77 taps take as long as 110, and
 // a gate with half the instructions changed nothing.
 struct WalkArgs {

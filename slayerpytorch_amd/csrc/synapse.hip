@@ -721,7 +721,9 @@ __device__ __forceinline__ bool gather_not_finite(const Acc (&acc)[2][OT])
 template <bool BACKWARD, typename Acc, int OT>
 __device__ __forceinline__ void gather_again(const GatherMfmaArgs &g, Acc (&acc)[2][OT], int n, int grp, int og, int pixel, int t0)
 {
-    const int r = threadIdx.x & 15, h = (threadIdx.x & 63) >> 4;
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));   // (nothing of this is worked out ahead and kept in registers)
+    const int r = lane & 15, h = lane >> 4;
     const int64_t srcPlane = static_cast<int64_t>(g.SH) * g.SW * g.T;
     const BufferRsrc srcB = make_buffer(g.src + (static_cast<int64_t>(n) * g.SC + static_cast<int64_t>(grp) * g.Qg) * srcPlane);
     const int ab = pixel / (g.T * 4), a = ab / g.DW, b = ab - a * g.DW, KK = g.KH * g.KW;
@@ -1006,16 +1008,18 @@ __global__ __launch_bounds__(512) void synapse_gather_mfma_kernel(GatherMfmaArgs
 // ---- gather on the matrix cores, bf16 instructions over split operands ---------------------------------------
 // The same work-group, patch and loop as above, with v_mfma_f32_16x16x32_bf16 in place of the fp32 instruction: 32
 // taps per instruction in half the time of the fp32 instruction's four.  Every fp32 number is the sum of three bf16
-// numbers (its upper 16 bits, those of the remainder, and those of what is left), so a product of two is the sum
-// of nine partial products, of which the six largest are kept (the error, below 2^-22 of |x| |w| per term, is that
-// of the fp32 sum itself).  The weights are split once per work-group, in LDS in the register layout of the
+// numbers (the nearest one, the one nearest to the remainder, and what is left), so a product of two is the sum of nine
+// partial products, of which the six largest are kept (what is left out is below 2^-24 of |x| |w|).  The leading products
+// have sums of their own, which the small ones join at the end: the instruction cuts off what lies beyond a sum's last bit,
+// once per product that joins it (error against double precision, 2-norm: six products per sum 1.6e-7 on 16 -> 32 channels
+// 3x3, one 6.6e-8, the fp32 chain 2.1e-7; sums of one term 3.5e-8, 2.6e-8 and 2.6e-8).  The weights are split once per work-group, in LDS in the register layout of the
 // instruction's second operand ([pass][channel tile][group of 32 taps][part][lane], 16 bytes each).  The patch
 // stays fp32: lane (r, h) reads its sample r of the 8 taps 32 G + 8 h .. + 7 as eight dwords and splits them in
 // registers - or only packs their upper halves when the patch holds nothing else, which the staging wavefronts
 // note per patch (spike tensors: 0 and 1 / Ts with few significant bits): three products instead of six.
 // A pass has room for 5 groups (160 taps >= the 144 of a pass; taps beyond the pass read the zero row and carry zero
 // weights).  With at most two (pass, channel tile) sets of weights the two patches of the kernel above fit beside
-// them; with up to four there is one patch, written between two barriers after the matrix work.  Numbers below
+// them; with more, or with two channel tiles, there is one patch, written between two barriers after the matrix work.  Numbers below
 // 2^-126 in a part are flushed by the instruction.
 constexpr int kGsGroups = 5;
 constexpr int kGsUnitBytes = kGsGroups * 3 * 1024;      // weights of one (pass, channel tile)
@@ -1064,7 +1068,7 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
                 v[j] = g.w[idx];
             }
         }
-        const SplitPlanes sp = split_bf16(v);
+        const SplitPlanes sp = split_bf16<false>(v);
         uint4_ext *unit = wl + (po * NG + G) * 3 * 64 + l;
         unit[0] = sp.hi;
         unit[64] = sp.mid;
@@ -1148,12 +1152,12 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
         if (lane == 0) flags[buf * 8 + wave] = any ? 1u : 0u;
     };
 
-    f32x4 acc[2][OT];
+    f32x4 acc[2][OT], small[2][OT];
     auto clear = [&]() {
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-            for (int ot = 0; ot < OT; ++ot) acc[hf][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int ot = 0; ot < OT; ++ot) acc[hf][ot] = small[hf][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
     // the matrix work of one pass on the patch in buffer BUF; HALVES = 1 when the second half of the step lies past
     // the end of the row.  The samples of a group of taps are read while the group before is multiplied.
@@ -1186,14 +1190,14 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
             if (allParts) {
 #pragma unroll
                 for (int hf = 0; hf < HALVES; ++hf) {
-                    const SplitPlanes a = split_bf16(av[set][hf]);
+                    const SplitPlanes a = split_bf16<false>(av[set][hf]);
 #pragma unroll
                     for (int ot = 0; ot < OT; ++ot) {
-                        acc[hf][ot] = mfma_bf16(a.hi, wq[ot][2], acc[hf][ot]);
-                        acc[hf][ot] = mfma_bf16(a.lo, wq[ot][0], acc[hf][ot]);
-                        acc[hf][ot] = mfma_bf16(a.mid, wq[ot][1], acc[hf][ot]);
-                        acc[hf][ot] = mfma_bf16(a.hi, wq[ot][1], acc[hf][ot]);
-                        acc[hf][ot] = mfma_bf16(a.mid, wq[ot][0], acc[hf][ot]);
+                        small[hf][ot] = mfma_bf16(a.hi, wq[ot][2], small[hf][ot]);
+                        small[hf][ot] = mfma_bf16(a.lo, wq[ot][0], small[hf][ot]);
+                        small[hf][ot] = mfma_bf16(a.mid, wq[ot][1], small[hf][ot]);
+                        small[hf][ot] = mfma_bf16(a.hi, wq[ot][1], small[hf][ot]);
+                        small[hf][ot] = mfma_bf16(a.mid, wq[ot][0], small[hf][ot]);
                         acc[hf][ot] = mfma_bf16(a.hi, wq[ot][0], acc[hf][ot]);
                     }
                 }
@@ -1207,8 +1211,8 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
                                                       __builtin_bit_cast(uint32_t, av[set][hf][2 * w2]), 0x07060302u);
 #pragma unroll
                     for (int ot = 0; ot < OT; ++ot) {
-                        acc[hf][ot] = mfma_bf16(a, wq[ot][2], acc[hf][ot]);
-                        acc[hf][ot] = mfma_bf16(a, wq[ot][1], acc[hf][ot]);
+                        small[hf][ot] = mfma_bf16(a, wq[ot][2], small[hf][ot]);
+                        small[hf][ot] = mfma_bf16(a, wq[ot][1], small[hf][ot]);
                         acc[hf][ot] = mfma_bf16(a, wq[ot][0], acc[hf][ot]);
                     }
                 }
@@ -1219,6 +1223,10 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
     auto store = [&](int n, int pix, int st) {
         if (pix < 0) return;
         const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int ot = 0; ot < OT; ++ot) acc[hf][ot] += small[hf][ot];
         if (gather_not_finite(acc)) gather_again<BACKWARD>(g, acc, n, grp, og, pix, t0);
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
@@ -1309,7 +1317,7 @@ __global__ __launch_bounds__(512) void synapse_gather_split_kernel(GatherMfmaArg
 // (a wavefront reads 60 KB per trip with two channel tiles) and matrix instructions together, 3840 cycles per trip each.
 // 3x3, (12, 300), split kernel / fp32 instructions before -> now: 16 -> 32 channels on 16x16 pixels forward 101 -> 80 us,
 // input gradient 126 -> 102; 32 -> 64 on 8x8: 85 -> 67, 109 -> 87.  Batch of 64: 643 -> 470, 634 -> 598, 427 -> 336, 529 ->
-// 464.  Error against double precision unchanged (forward 1.7e-7) or smaller (gradient 2.9e-7 -> 2.4e-7).
+// 464.  Error against double precision (2-norm): forward 1.8e-7 -> 6.6e-8, gradient 3.0e-7 -> 9.2e-8.
 constexpr int kGpPos = 30;                        // patch positions (filter rows x patch columns)
 constexpr int kGpPosBytes = 3 * 1024;             // 3 planes x 32 samples x 16 channels; position kGpPos holds zeros
 constexpr int kGpPatch = (kGpPos + 1) * kGpPosBytes;
@@ -1354,7 +1362,7 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
                 v[j] = g.w[idx];
             }
         }
-        const SplitPlanes sp = split_bf16(v);
+        const SplitPlanes sp = split_bf16<false>(v);
         uint4_ext *unit = wl + (po * NG + G) * 3 * 64 + l;
         unit[0] = sp.hi;
         unit[64] = sp.mid;
@@ -1362,17 +1370,16 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
     }
     if (tid < kGpPosBytes / 16) reinterpret_cast<uint4_ext *>(ldsBytes + kGpPos * kGpPosBytes)[tid] = uint4_ext{0u, 0u, 0u, 0u};
 
-    // LDS address of this lane's operand of group G for samples 16 hf + r (plane `hi`; the others lie 1 and 2 KB on)
-    uint32_t aTab[NG][2];
+    // LDS address of this lane's operand of group G for sample r (plane `hi`; the others lie 1 and 2 KB on), and how far
+    // sample 16 + r is from it
+    uint32_t aTab[NG];
+    const int halfStep = (r & 1) != 0 ? -64 : 64;
 #pragma unroll
     for (int G = 0; G < NG; ++G) {
         const int ij = 2 * G + (h >> 1);
         const int i = static_cast<int>(fastdiv(static_cast<uint32_t>(ij), g.byKW)), j = ij - i * g.KW;
         const int pos = ij < KK ? i * g.WX + wave * g.mulW + j * g.stepW + g.xBias : kGpPos;
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf)
-            aTab[G][hf] = ldsBase + static_cast<uint32_t>(pos * kGpPosBytes + (r & 3) * 256 +
-                                                          ((((h & 1) * 8 + (r >> 2) + 4 * hf) ^ (4 * (r & 3))) << 4));
+        aTab[G] = ldsBase + static_cast<uint32_t>(pos * kGpPosBytes + (r & 3) * 256 + ((((h & 1) * 8 + (r >> 2)) ^ (4 * (r & 3))) << 4));
     }
     const uint32_t wAddr = ldsBase + kGpPatch + lane * 16;
 
@@ -1426,7 +1433,7 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
                 v[c] = e == 0 ? R[c].x : e == 1 ? R[c].y : e == 2 ? R[c].z : R[c].w;
                 low |= __builtin_bit_cast(uint32_t, v[c]);
             }
-            const SplitPlanes sp = split_bf16(v);
+            const SplitPlanes sp = split_bf16<false>(v);
             if (stages) {
                 uint4_ext *at = reinterpret_cast<uint4_ext *>(ldsBytes + stageAddr + e * 256 + (((oct * 8 + u) ^ (4 * e)) << 4));
                 at[0] = sp.hi;
@@ -1438,12 +1445,12 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
         if (lane == 0) flags[wave] = any ? 1u : 0u;
     };
 
-    f32x4 acc[2][OT];
+    f32x4 acc[2][OT], small[2][OT];
     auto clear = [&]() {
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-            for (int ot = 0; ot < OT; ++ot) acc[hf][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int ot = 0; ot < OT; ++ot) acc[hf][ot] = small[hf][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
     // the products of one pass; PARTS = 1 when the patch holds bf16 numbers only (three products instead of six);
     // HALVES = 1 when the second half of the step lies past the end of the row.  Operands are read one group ahead.
@@ -1461,7 +1468,7 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
             for (int hf = 0; hf < HALVES; ++hf)
 #pragma unroll
                 for (int part = 0; part < PARTS; ++part)
-                    x[set][hf][part] = *reinterpret_cast<LdsUint4>(static_cast<size_t>(aTab[G][hf] + part * 1024));
+                    x[set][hf][part] = *reinterpret_cast<LdsUint4>(static_cast<size_t>(aTab[G] + (hf ? halfStep : 0) + part * 1024));
         };
         fetch(0, 0);
 #pragma unroll
@@ -1469,19 +1476,19 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
             const int set = G & 1;
             if (G + 1 < NG) fetch(set ^ 1, G + 1);
             __builtin_amdgcn_sched_barrier(0);
-#define SLAYER_PLANES_MUL(XP, WP)                                                                                      \
+#define SLAYER_PLANES_MUL(SUM, XP, WP)                                                                                 \
     _Pragma("unroll") for (int hf = 0; hf < HALVES; ++hf) _Pragma("unroll") for (int ot = 0; ot < OT; ++ot)            \
-        acc[hf][ot] = mfma_bf16(x[set][hf][XP], wq[set][ot][WP], acc[hf][ot]);
-            SLAYER_PLANES_MUL(0, 2)
+        SUM[hf][ot] = mfma_bf16(x[set][hf][XP], wq[set][ot][WP], SUM[hf][ot]);
+            SLAYER_PLANES_MUL(small, 0, 2)
             if constexpr (PARTS == 3) {
-                SLAYER_PLANES_MUL(2, 0)
-                SLAYER_PLANES_MUL(1, 1)
+                SLAYER_PLANES_MUL(small, 2, 0)
+                SLAYER_PLANES_MUL(small, 1, 1)
             }
-            SLAYER_PLANES_MUL(0, 1)
+            SLAYER_PLANES_MUL(small, 0, 1)
             if constexpr (PARTS == 3) {
-                SLAYER_PLANES_MUL(1, 0)
+                SLAYER_PLANES_MUL(small, 1, 0)
             }
-            SLAYER_PLANES_MUL(0, 0)
+            SLAYER_PLANES_MUL(acc, 0, 0)
 #undef SLAYER_PLANES_MUL
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -1489,6 +1496,10 @@ __global__ __launch_bounds__(512) void synapse_gather_planes_kernel(GatherMfmaAr
     auto store = [&](int n, int pix, int st) {
         if (pix < 0) return;
         const int t0 = min(st << 5, g.tLast), uniform = pix + t0 * 4;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int ot = 0; ot < OT; ++ot) acc[hf][ot] += small[hf][ot];
         if (gather_not_finite(acc)) gather_again<BACKWARD>(g, acc, n, grp, og, pix, t0);
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
@@ -1647,7 +1658,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
         const int o = ((og * MT + mt) << 4) + r;
         offA[mt] = masked_offset(o < g.Og, o * static_cast<int>(goPlane) * 4 + h * 16);
     }
-    int bAddr[2][NT];                      // (columns past the filter read the zero row)
+    int bAddr[NT];                      // (columns past the filter read the zero row)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int col = ((cg * NT + nt) << 4) + r;
@@ -1656,8 +1667,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
         const int i = static_cast<int>(fastdiv(static_cast<uint32_t>(ij), g.byKW));
         const int j = ij - i * s.KW;
         const int row = col < g.CK ? ((static_cast<int>(cl) - c0) * s.KH + i) * g.WX + j * s.dW + wave * s.sW : ROWS;
-        bAddr[0][nt] = row * kWgRow + ((h ^ (row & 7)) << 4);
-        bAddr[1][nt] = row * kWgRow + (((4 + h) ^ (row & 7)) << 4);
+        bAddr[nt] = row * kWgRow + ((h ^ (row & 7)) << 4);   // (samples 16 on: the same with bit 6 turned)
     }
 
     floatx4 acc[MT][NT];
@@ -1768,15 +1778,15 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const float v[8] = {A[0][mt].x, A[0][mt].y, A[0][mt].z, A[0][mt].w, A[1][mt].x, A[1][mt].y, A[1][mt].z, A[1][mt].w};
-            a[mt] = split_bf16(v);
+            a[mt] = split_bf16<false>(v);
         }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const float4 b0 = *reinterpret_cast<const float4 *>(ldsBytes + buf + bAddr[0][nt]);
-            const float4 b1 = *reinterpret_cast<const float4 *>(ldsBytes + buf + bAddr[1][nt]);
+            const float4 b0 = *reinterpret_cast<const float4 *>(ldsBytes + buf + bAddr[nt]);
+            const float4 b1 = *reinterpret_cast<const float4 *>(ldsBytes + ((buf + bAddr[nt]) ^ 64));
             const float v[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
             if (allParts) {
-                const SplitPlanes b = split_bf16(v);
+                const SplitPlanes b = split_bf16<false>(v);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     acc[mt][nt] = mfma_bf16(a[mt].lo, b.hi, acc[mt][nt]);
@@ -2082,31 +2092,29 @@ static int launch_gather_mfma(const GatherArgs &a, const SynGeom &s, bool stride
         return launch_status();
     } else {
         const int units = passes * OT;
-        const bool twoPatches = units <= 2;      // (beside the weights of two sets; more leave room for one patch)
+        // two patches beside the weights of two sets of one channel tile each (more sets leave room for one, and two tiles with
+        // their sums of small products for the addresses of one: 12 -> 32 channels 3x3 372 us, 573 with registers spilled)
+        const bool twoPatches = OT == 1 && units <= 2;
         const int ldsBytes = (twoPatches ? 2 * kGmBuf : kGmBuf) + units * kGsUnitBytes + 64;
         // more LDS than a kernel may use without asking; asked once per device (a host-side setting, no allocation)
-        static std::atomic<bool> raised[2][2][64];
+        static std::atomic<bool> raised[3][64];
         int device = 0;
         hipError_t err = hipGetDevice(&device);
         if (err == hipSuccess && (device < 0 || device >= 64)) err = hipErrorInvalidDevice;
-        const void *fn = OT == 2 ? (twoPatches ? reinterpret_cast<const void *>(&synapse_gather_split_kernel<2, BACKWARD, true>)
-                                               : reinterpret_cast<const void *>(&synapse_gather_split_kernel<2, BACKWARD, false>))
-                                 : (twoPatches ? reinterpret_cast<const void *>(&synapse_gather_split_kernel<1, BACKWARD, true>)
-                                               : reinterpret_cast<const void *>(&synapse_gather_split_kernel<1, BACKWARD, false>));
-        if (err == hipSuccess && !raised[OT - 1][twoPatches][device].load(std::memory_order_acquire)) {
+        const void *fn = OT == 2      ? reinterpret_cast<const void *>(&synapse_gather_split_kernel<2, BACKWARD, false>)
+                         : twoPatches ? reinterpret_cast<const void *>(&synapse_gather_split_kernel<1, BACKWARD, true>)
+                                      : reinterpret_cast<const void *>(&synapse_gather_split_kernel<1, BACKWARD, false>);
+        std::atomic<bool> &done = raised[OT == 2 ? 2 : twoPatches ? 1 : 0][device < 0 || device >= 64 ? 0 : device];
+        if (err == hipSuccess && !done.load(std::memory_order_acquire)) {
             err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       (twoPatches ? 2 * kGmBuf + 2 * kGsUnitBytes : kGmBuf + 4 * kGsUnitBytes) + 64);
-            if (err == hipSuccess) raised[OT - 1][twoPatches][device].store(true, std::memory_order_release);
+            if (err == hipSuccess) done.store(true, std::memory_order_release);
         }
         if (err != hipSuccess) return note_hip_error(err);
         const dim3 grid(static_cast<unsigned>(blocks));
-        if (OT == 2) {
-            if (twoPatches) hipLaunchKernelGGL((synapse_gather_split_kernel<2, BACKWARD, true>), grid, dim3(512), ldsBytes, st, g);
-            else hipLaunchKernelGGL((synapse_gather_split_kernel<2, BACKWARD, false>), grid, dim3(512), ldsBytes, st, g);
-        } else {
-            if (twoPatches) hipLaunchKernelGGL((synapse_gather_split_kernel<1, BACKWARD, true>), grid, dim3(512), ldsBytes, st, g);
-            else hipLaunchKernelGGL((synapse_gather_split_kernel<1, BACKWARD, false>), grid, dim3(512), ldsBytes, st, g);
-        }
+        if (OT == 2) hipLaunchKernelGGL((synapse_gather_split_kernel<2, BACKWARD, false>), grid, dim3(512), ldsBytes, st, g);
+        else if (twoPatches) hipLaunchKernelGGL((synapse_gather_split_kernel<1, BACKWARD, true>), grid, dim3(512), ldsBytes, st, g);
+        else hipLaunchKernelGGL((synapse_gather_split_kernel<1, BACKWARD, false>), grid, dim3(512), ldsBytes, st, g);
         return launch_status();
     }
 }
@@ -2328,12 +2336,12 @@ static int launch_wgrad_mfma(const float *gradOut, const float *in, float *works
     return status == SLAYER_OK ? s.N * p.slices : -status;
 }
 
-// Tiling of the LDS-staged matrix-core weight gradient: the tiles of plan_wgrad_mfma, blocks of kWgPix
+// Tiling of the LDS-staged matrix-core weight gradient: blocks of kWgPix
 // pixels, and ranges of (block, step) pairs so that one wave of work-groups (two per compute unit of the
 // 256) covers the tensor.
 struct LdsPlan {
     bool use;
-    int NS, WX, rows, blocksPerRow, steps, pairs, slices, pairsPerSlice;
+    int NT, colGroups, NS, WX, rows, blocksPerRow, steps, pairs, slices, pairsPerSlice;
 };
 
 static LdsPlan plan_wgrad_lds(const SynGeom &s, const MfmaPlan &m)
@@ -2342,9 +2350,11 @@ static LdsPlan plan_wgrad_lds(const SynGeom &s, const MfmaPlan &m)
     if (!m.use) return p;
     const int Cg = s.C / s.groups, KK = s.KH * s.KW, CK = Cg * KK;
     const int64_t WX = static_cast<int64_t>(kWgPix - 1) * s.sW + static_cast<int64_t>(s.KW - 1) * s.dW + 1;
+    p.NT = m.NT;
+    p.colGroups = m.colGroups;
     int channels = 0;  // most channels that one column group's columns belong to
-    for (int cg = 0; cg < m.colGroups; ++cg) {
-        const int col0 = cg * m.NT * 16, col1 = (CK < col0 + m.NT * 16 ? CK : col0 + m.NT * 16) - 1;
+    for (int cg = 0; cg < p.colGroups; ++cg) {
+        const int col0 = cg * p.NT * 16, col1 = (CK < col0 + p.NT * 16 ? CK : col0 + p.NT * 16) - 1;
         if (col1 >= col0 && col1 / KK - col0 / KK + 1 > channels) channels = col1 / KK - col0 / KK + 1;
     }
     const int64_t rows = channels * s.KH * WX;
@@ -2361,12 +2371,12 @@ static LdsPlan plan_wgrad_lds(const SynGeom &s, const MfmaPlan &m)
         return p;
     }
     p.pairs = static_cast<int>(pairs);
-    const int64_t base = static_cast<int64_t>(s.groups) * m.oGroups * m.colGroups;
+    const int64_t base = static_cast<int64_t>(s.groups) * m.oGroups * p.colGroups;
     // two work-groups per compute unit; a few short of the 512 places, which measured faster than all of them
     // (504: 110 us, 512: 123 us on the 2 -> 16 channel 5 x 5 layer)
     // small patches and few tiles (25 KB of LDS, 119 registers: the 2 -> 16 channel 5 x 5 layer): three per compute unit
     // (two, three, four: (12, 300) on 34x34 pixels 112, 101, 103 us; batch of 64 558, 502, 526; spikes, (8, 300) on 32x32 55, 48, 58)
-    int64_t slices = (p.NS == 3 && m.MT * m.NT <= 4 ? 756 : 504) / base;
+    int64_t slices = (p.NS == 3 && m.MT * p.NT <= 4 ? 756 : 504) / base;
     if (slices < 1) slices = 1;
     if (slices > pairs) slices = pairs;
     p.pairsPerSlice = static_cast<int>(ceil_div(pairs, slices));
@@ -2412,11 +2422,11 @@ static int launch_wgrad_lds(const float *gradOut, const float *in, float *worksp
     WgradLdsArgs g{};
     g.gradOut = gradOut; g.in = in; g.partial = workspace; g.s = s;
     g.Cg = s.C / s.groups; g.Og = s.O / s.groups; g.CK = g.Cg * s.KH * s.KW;
-    g.oGroups = m.oGroups; g.colGroups = m.colGroups;
+    g.oGroups = m.oGroups; g.colGroups = p.colGroups;
     g.WX = p.WX; g.rows = p.rows; g.blocksPerRow = p.blocksPerRow; g.steps = p.steps;
     g.pairs = p.pairs; g.slices = p.slices; g.pairsPerSlice = p.pairsPerSlice; g.nW = nW;
     g.tLast = s.T % 4 == 0 ? (p.steps - 1) * 32 : s.T - 32;
-    g.byColGroups = make_fastdiv(static_cast<uint32_t>(m.colGroups));
+    g.byColGroups = make_fastdiv(static_cast<uint32_t>(p.colGroups));
     g.byOGroups = make_fastdiv(static_cast<uint32_t>(m.oGroups));
     g.byGroups = make_fastdiv(static_cast<uint32_t>(s.groups));
     g.byKK = make_fastdiv(static_cast<uint32_t>(s.KH * s.KW));
@@ -2426,16 +2436,16 @@ static int launch_wgrad_lds(const float *gradOut, const float *in, float *worksp
     g.byBlocksPerRow = make_fastdiv(static_cast<uint32_t>(p.blocksPerRow));
     g.byPatch = make_fastdiv(static_cast<uint32_t>(s.KH * p.WX));
     g.byWX = make_fastdiv(static_cast<uint32_t>(p.WX));
-    const int64_t blocks = static_cast<int64_t>(s.groups) * m.oGroups * m.colGroups * p.slices;
+    const int64_t blocks = static_cast<int64_t>(s.groups) * m.oGroups * p.colGroups * p.slices;
     if (blocks >= (1LL << 31)) return -SLAYER_EUNSUPPORTED;
     const unsigned nb = static_cast<unsigned>(blocks);
     int status;
     if (m.MT == 2) {
-        status = p.NS == 9 ? launch_wgrad_lds_nt<2, 9>(g, m.NT, nb, st)
-               : p.NS == 6 ? launch_wgrad_lds_nt<2, 6>(g, m.NT, nb, st) : launch_wgrad_lds_nt<2, 3>(g, m.NT, nb, st);
+        status = p.NS == 9 ? launch_wgrad_lds_nt<2, 9>(g, p.NT, nb, st)
+               : p.NS == 6 ? launch_wgrad_lds_nt<2, 6>(g, p.NT, nb, st) : launch_wgrad_lds_nt<2, 3>(g, p.NT, nb, st);
     } else {
-        status = p.NS == 9 ? launch_wgrad_lds_nt<1, 9>(g, m.NT, nb, st)
-               : p.NS == 6 ? launch_wgrad_lds_nt<1, 6>(g, m.NT, nb, st) : launch_wgrad_lds_nt<1, 3>(g, m.NT, nb, st);
+        status = p.NS == 9 ? launch_wgrad_lds_nt<1, 9>(g, p.NT, nb, st)
+               : p.NS == 6 ? launch_wgrad_lds_nt<1, 6>(g, p.NT, nb, st) : launch_wgrad_lds_nt<1, 3>(g, p.NT, nb, st);
     }
     return status == SLAYER_OK ? p.slices : -status;
 }

@@ -189,10 +189,9 @@ def sum_bounds(x, f):
 
 @pytest.mark.parametrize("Fl", [40, 60, 77, 90, 110, 129])
 def test_corr_from_split_operands_is_as_close_as_the_chain(Fl):
-    # Whole rows with T / 4 odd run on bf16 matrix instructions over a three-way split of samples and taps.  The split
-    # leaves out products below 2^-23 of a term and every instruction rounds its accumulator: the result stays within
-    # 1e-6 of the sum of the terms' magnitudes (a tenth of the tolerance; measured: up to 4.4e-7 where one term
-    # dominates a sum, 2.8e-7 on samples of one size), for samples and taps of every size and mixed signs ...
+    # Whole rows run on bf16 matrix instructions over a three-way split of samples and taps.  The split leaves out products
+    # below 2^-24 of a term and every instruction rounds its accumulator: the result stays within 1e-6 of the sum of the
+    # terms' magnitudes (a tenth of the tolerance), for samples and taps of every size and mixed signs ...
     rng = np.random.default_rng(Fl)
     T = 300
     f = (rng.standard_normal(Fl) * np.exp2(rng.integers(-20, 20, Fl))).astype(np.float32)
@@ -210,6 +209,32 @@ def test_corr_from_split_operands_is_as_close_as_the_chain(Fl):
             exact, mag, win = sum_bounds(xx, ff)
             floor = 2.0 ** -124 * (np.sum(np.abs(ff.astype(np.float64))) + win)
             assert np.all(np.abs(got - exact) <= 1e-6 * mag + floor), scale
+
+
+@pytest.mark.parametrize("T,Fl,delay", [(300, 77, None), (300, 110, None), (512, 40, None), (512, 77, None), (1448, 129, None),
+                                        (300, 110, 0), (173, 110, 3), (1450, 110, 1)])
+def test_split_products_of_one_term_are_as_close_as_the_chain(T, Fl, delay):
+    """Sums of one product: the rounding of an fp32 product is 2^-24 of it, what the split leaves out as much again at most
+    (root mean square: 2.5e-8 and 0.6e-8).  Numbers next to the largest have a split, too."""
+    rng = np.random.default_rng(T + Fl)
+    f = rng.standard_normal(Fl).astype(np.float32)
+    x = np.zeros((400, T), np.float32)
+    x[np.arange(400), rng.integers(0, T, 400)] = rng.standard_normal(400)
+    u = np.full(x.shape, 10.0, np.float32)      # (a gate of exactly 1 / 4)
+    if delay is None:
+        got, shift = host(slayerCuda.corr(dev(x), dev(f), 1.0)), 0
+    else:
+        got, shift = host(slayerCuda.spikeBackwardDelayedCorr(dev(x), dev(u), dev(f), delay, 10.0, 4.0, 1.0, 1.0)), delay
+    moved = np.concatenate([x[:, shift:], np.zeros((400, shift), np.float32)], axis=1) * np.float32(1.0 if delay is None else 0.25)
+    exact, mag, _ = sum_bounds(moved, f)
+    err = (np.abs(got - exact)[mag > 0] / mag[mag > 0])
+    assert err.size > 2000 and err.max() <= 2.0 ** -23 * 1.01 and np.sqrt((err ** 2).mean()) <= 3e-8
+    if delay is None:
+        x[5, 7], x[6, T - 1], x[7, T // 2] = 3.4028234e38, -3.4e38, 3.3896e38
+        f = (f * 0.01).astype(np.float32)
+        got = host(slayerCuda.corr(dev(x), dev(f), 1.0))
+        exact, mag, _ = sum_bounds(x, f)
+        assert np.all(np.abs(got - exact) <= 1e-6 * mag)
 
 
 def test_corr_from_split_operands_with_a_tap_that_is_not_finite():

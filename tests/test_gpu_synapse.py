@@ -812,3 +812,37 @@ def test_numbers_that_are_not_finite_stay_in_their_sums(geom, where):
             x = rng.standard_normal(x.shape).astype(np.float32) * np.float32(0.01)
         check(host(synapse.convGradWeight(dev(go), dev(x), w.shape, *args)),
               lambda a, b: O.synapse_conv_grad_weight(a, b, w.shape, *args), go, x)
+
+
+@pytest.mark.parametrize("C,O_,K,pad,T", [(16, 32, 3, 1, 300), (16, 32, 3, 0, 173), (32, 16, 3, 1, 45), (16, 16, (2, 3), 0, 64),   # planes
+                                          (4, 32, 5, 2, 60), (4, 16, 5, 2, 61), (12, 32, 3, 1, 45), (12, 16, 3, 1, 44),     # split patches
+                                          (48, 20, 3, 1, 33), (2, 16, 5, 2, 70)])
+def test_sums_of_one_term_are_as_close_as_the_fp32_product(C, O_, K, pad, T):
+    """One non-zero sample (gradient) per batch item and time: every output is one product, within its fp32 rounding, 2^-24,
+    and as much again for what split operands leave out (root mean square: 2.5e-8 and 0.6e-8)."""
+    rng = np.random.default_rng(C + T)
+    N, H, W = 3, 9, 11
+    KH, KW = (K, K) if isinstance(K, int) else K
+    w = rng.standard_normal((O_, C, KH, KW)).astype(np.float32)
+
+    def alone(channels, h, wd):
+        a = np.zeros((N, channels, h, wd, T), np.float32)
+        n, t = np.meshgrid(np.arange(N), np.arange(T), indexing="ij")
+        a[n, rng.integers(0, channels, n.shape), rng.integers(0, h, n.shape), rng.integers(0, wd, n.shape), t] = rng.standard_normal(n.shape)
+        return a
+
+    def check(got, exact):
+        some = exact != 0
+        err = np.abs(got.astype(np.float64) - exact)[some] / np.abs(exact[some])
+        assert err.size > 1000 and err.max() <= 2.0 ** -23 * 1.01 and np.sqrt((err ** 2).mean()) <= 3e-8
+        assert not got[~some].any()
+
+    def conv(a, b, transposed):
+        f = torch.nn.functional.conv_transpose3d if transposed else torch.nn.functional.conv3d
+        return f(torch.from_numpy(a).double(), torch.from_numpy(b).double()[..., None], padding=(pad, pad, 0)).numpy()
+
+    x = alone(C, H, W)
+    y = host(synapse.conv(dev(x), dev(w), 1, pad))
+    check(y, conv(x, w, False))
+    go = alone(O_, y.shape[2], y.shape[3])
+    check(host(synapse.convGradInput(dev(go), dev(w), x.shape, 1, pad)), conv(go, w, True))
