@@ -1772,6 +1772,12 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
     // parts per number (fir_core.h); the patch rows are, too - or, when the patch holds nothing beyond the upper 16
     // bits of its numbers (spikes), only packed: three products per tile instead of six.  Samples past the end of
     // a row were loaded as zeros.
+    // The instruction cuts what it adds to a sum to the sum's last bit, which over the hundreds of steps of a large batch
+    // comes to 5e-6 of the gradient (2-norm; 16 -> 32 channels 3x3, (64, 300)), 2e-5 on the 2 -> 16 channel 5x5 layer.  So
+    // the products of a step start from zero, the leading ones apart from the small ones, and are added to the sums by
+    // the vector ALU, which rounds: 7e-8 in either case.  This takes 8 registers more, which two by nine tiles of sums have not
+    // got: plan_wgrad_lds.  ((12, 300): 16 -> 32 channels 91 -> 103 us, spikes (8, 300) 65 -> 53 us; 5x5 91 -> 97 us.)
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     auto multiply = [&](const float4 (&A)[2][MT], int buf) {
         const bool allParts = __builtin_amdgcn_ballot_w64(lane < 4 && flags[(buf != 0 ? 4 : 0) + (lane & 3)] != 0u) != 0;
         SplitPlanes a[MT];
@@ -1789,12 +1795,12 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
                 const SplitPlanes b = split_bf16<false>(v);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    acc[mt][nt] = mfma_bf16(a[mt].lo, b.hi, acc[mt][nt]);
-                    acc[mt][nt] = mfma_bf16(a[mt].hi, b.lo, acc[mt][nt]);
-                    acc[mt][nt] = mfma_bf16(a[mt].mid, b.mid, acc[mt][nt]);
-                    acc[mt][nt] = mfma_bf16(a[mt].mid, b.hi, acc[mt][nt]);
-                    acc[mt][nt] = mfma_bf16(a[mt].hi, b.mid, acc[mt][nt]);
-                    acc[mt][nt] = mfma_bf16(a[mt].hi, b.hi, acc[mt][nt]);
+                    f32x4 t = mfma_bf16(a[mt].lo, b.hi, zero);
+                    t = mfma_bf16(a[mt].hi, b.lo, t);
+                    t = mfma_bf16(a[mt].mid, b.mid, t);
+                    t = mfma_bf16(a[mt].mid, b.hi, t);
+                    t = mfma_bf16(a[mt].hi, b.mid, t);
+                    acc[mt][nt] += mfma_bf16(a[mt].hi, b.hi, zero) + t;
                 }
             } else {
                 uint4_ext bh;
@@ -1803,9 +1809,7 @@ __global__ __launch_bounds__(256, 2) void synapse_wgrad_lds_kernel(WgradLdsArgs 
                     bh[w2] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, v[2 * w2 + 1]), __builtin_bit_cast(uint32_t, v[2 * w2]), 0x07060302u);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    acc[mt][nt] = mfma_bf16(a[mt].lo, bh, acc[mt][nt]);
-                    acc[mt][nt] = mfma_bf16(a[mt].mid, bh, acc[mt][nt]);
-                    acc[mt][nt] = mfma_bf16(a[mt].hi, bh, acc[mt][nt]);
+                    acc[mt][nt] += mfma_bf16(a[mt].hi, bh, zero) + mfma_bf16(a[mt].mid, bh, mfma_bf16(a[mt].lo, bh, zero));
                 }
             }
         }
@@ -1890,21 +1894,22 @@ __global__ __launch_bounds__(256) void synapse_wgrad_sum_kernel(float *__restric
                                                                 const float *__restrict__ partial, int rows, int nW, WgradAgain m)
 {
     constexpr int kWeights = 256 / PARTS;
-    __shared__ float part[PARTS][kWeights + 1];
+    __shared__ double part[PARTS][kWeights + 1];
     __shared__ uint32_t bad;   // a bit per weight
     __shared__ float waves[4];
     const int ql = threadIdx.x % kWeights, pt = threadIdx.x / kWeights;
     const int q = blockIdx.x * kWeights + ql;
-    float acc = 0.f;
+    double acc = 0.0;
     if (q < nW)
         for (int r = pt; r < rows; r += PARTS) acc += partial[static_cast<int64_t>(r) * nW + q];
     part[pt][ql] = acc;
     if (AGAIN && threadIdx.x == 0) bad = 0u;
     __syncthreads();
     if (threadIdx.x < kWeights && q < nW) {
-        float v = part[0][ql];
+        double total = part[0][ql];
 #pragma unroll
-        for (int k = 1; k < PARTS; ++k) v += part[k][ql];
+        for (int k = 1; k < PARTS; ++k) total += part[k][ql];
+        const float v = static_cast<float>(total);
         gradW[q] = v;
         if (AGAIN && !(fabsf(v) < __builtin_inff())) atomicOr(&bad, 1u << ql);
     }
@@ -2350,8 +2355,12 @@ static LdsPlan plan_wgrad_lds(const SynGeom &s, const MfmaPlan &m)
     if (!m.use) return p;
     const int Cg = s.C / s.groups, KK = s.KH * s.KW, CK = Cg * KK;
     const int64_t WX = static_cast<int64_t>(kWgPix - 1) * s.sW + static_cast<int64_t>(s.KW - 1) * s.dW + 1;
-    p.NT = m.NT;
-    p.colGroups = m.colGroups;
+    // tiles of columns per work-group: at most six beside two tiles of output channels, nine beside one (registers), in
+    // groups as even as the kernel's instances allow
+    const int cTiles = static_cast<int>(ceil_div(CK, 16)), most = m.MT == 2 ? 6 : 9;
+    const int even = static_cast<int>(ceil_div(cTiles, ceil_div(cTiles, most)));
+    p.NT = even <= 2 ? even : even <= 4 ? 4 : even <= 6 ? even : 9;
+    p.colGroups = static_cast<int>(ceil_div(cTiles, p.NT));
     int channels = 0;  // most channels that one column group's columns belong to
     for (int cg = 0; cg < p.colGroups; ++cg) {
         const int col0 = cg * p.NT * 16, col1 = (CK < col0 + p.NT * 16 ? CK : col0 + p.NT * 16) - 1;
@@ -2407,8 +2416,9 @@ template <int MT, int NS>
 static int launch_wgrad_lds_nt(const WgradLdsArgs &g, int NT, unsigned blocks, hipStream_t st)
 {
     switch (NT) {
-        case 9: return launch_wgrad_lds_one<MT, 9, NS>(g, blocks, st);
+        case 9: return launch_wgrad_lds_one<MT, (MT == 1 ? 9 : 6), NS>(g, blocks, st);   // (one tile of output channels only)
         case 6: return launch_wgrad_lds_one<MT, 6, NS>(g, blocks, st);
+        case 5: return launch_wgrad_lds_one<MT, 5, NS>(g, blocks, st);
         case 4: return launch_wgrad_lds_one<MT, 4, NS>(g, blocks, st);
         case 2: return launch_wgrad_lds_one<MT, 2, NS>(g, blocks, st);
         default: return launch_wgrad_lds_one<MT, 1, NS>(g, blocks, st);

@@ -773,6 +773,8 @@ def test_numbers_that_are_not_finite_stay_in_their_sums(geom, where):
     """An infinity among samples, gradients or weights makes the sums that it enters infinite (NaN where it meets a zero or
     another sign) and leaves all others as they are, whichever kernel makes them; so do numbers next to the largest."""
     N, C, H, W, T, O_, K, stride, pad, dil, groups = geom
+    if where == "weights":
+        pad = 0     # (a padding zero times such a weight is NaN, which the oracle leaves out)
     rng = np.random.default_rng(T)
     x = rng.standard_normal((N, C, H, W, T)).astype(np.float32)
     w = rng.standard_normal((O_, C // groups) + K).astype(np.float32)
@@ -780,8 +782,6 @@ def test_numbers_that_are_not_finite_stay_in_their_sums(geom, where):
     go = rng.standard_normal(O.synapse_conv(x, w, *args).shape).astype(np.float32)
     special = [np.inf, -np.inf, np.nan] if where != "huge" else [3.4e38, -3.4e38, 3.39e38]
     if where == "weights":
-        if pad != 0:
-            pytest.skip("a padding zero times such a weight is NaN, which the oracle leaves out")
         w[3, 1, 0, 0], w[5, 0, 1, 1] = special[:2]
     else:
         for k, v in enumerate(special):
@@ -846,3 +846,35 @@ def test_sums_of_one_term_are_as_close_as_the_fp32_product(C, O_, K, pad, T):
     check(y, conv(x, w, False))
     go = alone(O_, y.shape[2], y.shape[3])
     check(host(synapse.convGradInput(dev(go), dev(w), x.shape, 1, pad)), conv(go, w, True))
+
+
+@pytest.mark.parametrize("N,C,O_,H,K,pad,T", [(12, 16, 32, 12, 3, 1, 173), (6, 16, 32, 12, 3, 1, 300), (3, 32, 64, 8, 3, 1, 333),
+                                              (12, 2, 16, 20, 5, 2, 173), (6, 2, 16, 20, 5, 1, 300), (4, 16, 20, 9, 3, 1, 45)])
+@pytest.mark.parametrize("kind", ["signed", "positive", "spikes", "one term"])
+def test_weight_gradient_sums_are_rounded_and_not_cut(N, C, O_, H, K, pad, T, kind):
+    """Error of the weight gradient against double precision, 2-norm: every sum of 32 products is rounded (2^-24 at most)
+    and joins its sum with a rounding (2^-25 root mean square of what the sum is by then): of n such additions, signs
+    independent, sqrt(n / 2) * 2^-25, and 2^-25 * sqrt(n) / 2 where all terms are positive; 2e-7 for the n here (under 200
+    per sum, partial sums added in double precision).  Sums of one term: as close as an fp32 product."""
+    rng = np.random.default_rng(H + T)
+    x = rng.standard_normal((N, C, H, H, T)).astype(np.float32)
+    OH = H + 2 * pad - K + 1
+    go = rng.standard_normal((N, O_, OH, OH, T)).astype(np.float32)
+    if kind == "positive":
+        x, go = np.abs(x), np.abs(go)
+    elif kind == "spikes":
+        x = (rng.random(x.shape) < 0.05).astype(np.float32)
+    elif kind == "one term":
+        at = go[1, :, OH // 2, OH // 2 - 2, T - 3].copy()
+        go[:] = 0
+        go[1, :, OH // 2, OH // 2 - 2, T - 3] = at
+    got = host(synapse.convGradWeight(dev(go), dev(x), (O_, C, K, K), 1, pad)).astype(np.float64)
+    xp = torch.nn.functional.pad(dev(x), (0, 0, pad, pad, pad, pad)).double().transpose(0, 1)
+    g = dev(go).double().transpose(0, 1).reshape(O_, -1)
+    exact = torch.stack([torch.stack([g @ xp[:, :, i:i + OH, j:j + OH].reshape(C, -1).t().contiguous() for j in range(K)], -1)
+                         for i in range(K)], -2).cpu().numpy()
+    if kind == "one term":
+        err = np.abs(got - exact) / np.abs(exact)
+        assert err.max() <= 2.0 ** -23 * 1.01 and np.sqrt((err ** 2).mean()) <= 3e-8
+    else:
+        assert np.linalg.norm(got - exact) <= 2e-7 * np.linalg.norm(exact)
