@@ -120,6 +120,13 @@ __global__ __launch_bounds__(256) void spike_loss_grad_kernel(float *__restrict_
         };
         for (int k = 0; k + 4 <= F; k += 4) block(k, 4);
         if ((F & 3) != 0) block(F & ~3, F & 3);
+        if (((acc[0] + acc[1]) + (acc[2] + acc[3])) * 0.0 != 0.0) {   // a tap that is not finite has met the zeros behind the row
+            for (int j = 0; j < 4; ++j) {
+                double sum = 0.0;
+                for (int k = 0; k < min(T - t - j, F); ++k) sum = fma(static_cast<double>(x.row[t + j + k]), static_cast<double>(x.filt[k]), sum);
+                acc[j] = sum;
+            }
+        }
         const float y[4] = {static_cast<float>(acc[0]) * Ts, static_cast<float>(acc[1]) * Ts, static_cast<float>(acc[2]) * Ts,
                             static_cast<float>(acc[3]) * Ts};
         store4(grad + base, t, T, y, vec);

@@ -1255,10 +1255,23 @@ def test_spike_loss_and_its_gradient(T, Fl):
     assert np.array_equal(np.isfinite(got), np.isfinite(want)) and np.array_equal(got[~np.isfinite(want)], want[~np.isfinite(want)], equal_nan=True)
 
 
-@pytest.mark.parametrize("T", [700, 704, 1000, 1500, 1604])
-def test_spikes_of_many_long_rows_are_those_of_a_few(T):
-    """Many rows of more than 700 samples (8.4 million samples together) go in pieces, fewer as whole rows: the same bits."""
-    rows = 8400000 // T + 70
+@pytest.mark.parametrize("T,Fl", [(5, 3), (350, 8), (1029, 77)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_spike_loss_gradient_with_a_tap_that_is_not_finite(T, Fl, bad):
+    rng = np.random.default_rng(T)
+    f = rng.standard_normal(Fl).astype(np.float32)
+    f[Fl - 2] = bad
+    e = rng.standard_normal((7, T)).astype(np.float32)
+    got = host(slayerCuda.spikeLossGrad(dev(e), torch.tensor(np.float32(0.5), device="cuda"), dev(f), 2.0))
+    want = O.corr(e, f, 2.0, fused=True)        # (0.5 * 2 = 1)
+    fin = np.isfinite(want)
+    assert fin.any() and not fin.all() and np.array_equal(got[~fin], want[~fin], equal_nan=True)
+    assert np.isfinite(got[fin]).all() and np.max(np.abs(got[fin] - want[fin])) <= 1e-5 * np.max(np.abs(want[fin]))
+
+
+@pytest.mark.parametrize("rows,T", [(12100, 700), (12100, 704), (12070, 1000), (8070, 1500), (8070, 1604)])
+def test_spikes_of_many_long_rows_are_those_of_a_few(rows, T):
+    """Rows of more than 600 samples go in pieces when they are more than the GPU holds whole at once, else whole: the same bits."""
     gen = torch.Generator(device="cuda").manual_seed(T)
     u = torch.randn((rows, 1, 1, 1, T), device="cuda", generator=gen).cumsum(-1).mul_(0.5).remainder_(24.0).sub_(8.0)
     nu = dev(np.array([0, -20, -14.7, -8.1, -4.0, -1.8, -0.8, -0.35, -0.15], np.float32))
