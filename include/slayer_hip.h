@@ -98,13 +98,12 @@ int slayer_conv_f32(float *out, const float *in, const float *filt, int64_t nNeu
  *
  * out[n][t] = Ts * sum_{i=0..F-1, t+i<T} in[n][t+i] * filt[i].
  *
- * Rows of whole 16-byte vectors with 34 to 129 taps are computed on the matrix cores, which add the
- * terms in another order than the sequential loop - whole rows of up to 316 samples whose T / 4 is odd
- * (T = 300) with bf16 instructions over a three-way split of samples and taps, the others with fp32
- * instructions: those results agree with the loop to rounding (every output within 1e-6 of the sum of the
- * magnitudes of its own terms; parts of samples and taps below 2^-126 are read as zero, at most
- * 2^-124 * (sum |filt| + sum |in| over an output's window) in absolute terms), all others bit for bit
- * with the fused-multiply-add loop.
+ * Rows of whole 16-byte vectors of at least 16 samples, with 34 to 129 taps, are computed on the matrix cores
+ * (bf16 instructions over a three-way split of samples and taps), which add the terms in another order than the
+ * sequential loop: those results agree with the loop to rounding (every output within 1e-6 of the sum of the
+ * magnitudes of its own terms, a sum of one term within 2^-23 of it; parts of samples and taps below 2^-126 are
+ * read as zero, at most 2^-124 * (sum |filt| + sum |in| over an output's window) in absolute terms), all others
+ * bit for bit with the fused-multiply-add loop.
  */
 int slayer_corr_f32(float *out, const float *in, const float *filt, int64_t nNeurons, int64_t T,
                     int64_t F, float Ts, void *stream);
@@ -167,8 +166,7 @@ int slayer_spike_bwd_corr_f32(float *gradIn, const float *gradOut, const float *
  * slayer_spike_bwd_corr_f32 of a gradient that first moves back in time by delaySteps samples (zeros move in at the end):
  * the backward pass of a Loihi neuron whose spikes leave delaySteps late (slayer_loihi_get_spikes_delayed_f32),
  * w[n][t] = gradOut[n][t + delaySteps] * (scale / tau) * exp(-|u[n][t] - theta| / tau).  Sums on the
- * matrix cores for rows of any length from 16 samples on and any alignment (the chain's values to rounding, 1e-5; delaySteps
- * may be 0).  SLAYER_EUNSUPPORTED, and nothing is done, for rows that the fused kernel does not serve (fewer than 16
+ * matrix cores, as by slayer_corr_f32, for rows of any length from 16 samples on and any alignment (delaySteps may be 0).  SLAYER_EUNSUPPORTED, and nothing is done, for rows that the fused kernel does not serve (fewer than 16
  * samples, filters outside 34 to 129 taps, a delay beyond the row, and delayed rows of at most 304
  * samples that are whole vectors of an odd number): slayer_shift_f32 and slayer_spike_bwd_corr_f32 then.
  */
@@ -253,8 +251,8 @@ int slayer_psp_spike_bwd_alpha_f32(float *gradIn, const float *gradPsp, const fl
  * s[t] = spike[t - k] with k = (int)(d / delayTs) (0 where t - k is outside the row); d is
  * delayLut[neuron % lutSize] when delayLut is given (one delay per neuron of a batch item, nNeurons a
  * multiple of lutSize) and `delay` otherwise, of any size and sign.  `u` is updated in place and NOT shifted,
- * exactly as by slayer_get_spikes_f32.  Fused shapes: rows of at most 4032 samples (refractory kernels of up to about
- * 900 taps, up to 3600 on the longest rows), and with nuSize <= 24 longer rows of whole 16-byte vectors up to 16384
+ * exactly as by slayer_get_spikes_f32.  Fused shapes: rows of at most 4032 samples (refractory kernels of up to 3777
+ * taps), and with nuSize <= 24 longer rows of whole 16-byte vectors up to 16384
  * samples (those travel in pieces: the kernel keeps the spike bits of the whole row and stores the shifted spikes
  * behind the row's last piece).  Other shapes return
  * SLAYER_EUNSUPPORTED with nothing launched - call the two functions then.

@@ -227,7 +227,7 @@ __device__ __forceinline__ void fir_sparse_tile(const BufferRsrc &bufOut, const 
 // VEC: rows are whole 16-byte vectors (T % 4 == 0, pointers 16-byte aligned)
 // GATED: the staged samples are in * pdf(gate.u), computed once per staged sample
 // DM: 0 = dense tiles run the register-window chains; 4..9 = dense tiles run on the matrix cores with a window
-//     of DM blocks of 16 samples (VEC, U = 16, R = 16 rows, LD >= tile + 16 (DM - 1))
+//     of DM blocks of 16 samples (the convolution; VEC, U = 16, R = 16 rows, LD >= tile + 16 (DM - 1))
 template <bool CAUSAL, bool VEC, int U, bool GATED, int DM>
 __global__ __launch_bounds__(256, DM > 0 ? 2 : 1) void fir_tiled_kernel(float *__restrict__ out,
                                                         const float *__restrict__ in,
@@ -235,6 +235,7 @@ __global__ __launch_bounds__(256, DM > 0 ? 2 : 1) void fir_tiled_kernel(float *_
                                                         int64_t rows, int T, int F, int TT, int LD, int R,
                                                         float Ts, FirGate gate)
 {
+    static_assert(DM == 0 || (CAUSAL && VEC && U == 16 && !GATED), "dense tiles on the matrix cores: the convolution's");
     extern __shared__ __align__(16) float X[];
     // filter copy for the sparse path: taps -63 .. 191, zeros outside [0, F)
     float *fL = X + R * LD + (kWave - 1);
@@ -414,12 +415,10 @@ __global__ __launch_bounds__(256, DM > 0 ? 2 : 1) void fir_tiled_kernel(float *_
                 }
                 acc = f32x4{y[0], y[1], y[2], y[3]};
             }
-            // times t0 + m0 .. (correlation) or tHi - m0 - 3 .. tHi - m0 (convolution); both are multiples of 4 and so
-            // is the tile's end, so the vector is all in or all out
-            const int tl = CAUSAL ? (tHi - m0 - 3) : (t0 + m0);
+            // times tHi - m0 - 3 .. tHi - m0, a multiple of 4, as is the tile's end, so the vector is all in or all out
+            const int tl = tHi - m0 - 3;
             const bool valid = on && tl >= t0 && tl + 3 < t0 + tt;
-            const float4 y = CAUSAL ? make_float4(acc.w * Ts, acc.z * Ts, acc.y * Ts, acc.x * Ts)
-                                    : make_float4(acc.x * Ts, acc.y * Ts, acc.z * Ts, acc.w * Ts);
+            const float4 y = make_float4(acc.w * Ts, acc.z * Ts, acc.y * Ts, acc.x * Ts);
             // the columns of a wavefront are consecutive in memory: neighbouring stores complete each other's lines
             buffer_store4<0>(bufOut, masked_offset(valid, (r * T + tl) * 4), 0, y);
         }

@@ -779,8 +779,8 @@ def test_spike_bwd_corr_is_the_two_ops_in_one(impl, shape, Fl):
 @pytest.mark.parametrize("rows", [1, 19, 32])
 def test_spike_bwd_delayed_corr(T, Fl, rows):
     """Rows of any length (whole chunks of 32 samples, a last chunk of 1 to 31, one chunk, segments of a long row), inputs that
-    start anywhere, delays up to the whole row: every element within 2e-6 of the sum of its terms' magnitudes of the exact sum
-    (the 1e-6 that split operands are held to elsewhere, and 1e-6 for the gate's rounding);
+    start anywhere, delays up to the whole row: every element within 1e-6 of the sum of its terms' magnitudes of the exact sum
+    over the gated samples (those of spikeBackward), as split operands are held to elsewhere;
     an infinite gradient or potential reaches what it reaches in shift, spikeBackward and corr."""
     rng = np.random.default_rng(T + Fl + rows)
     theta, tau, scale, Ts = 10.0, 5.0, 1.5, 0.5
@@ -794,9 +794,8 @@ def test_spike_bwd_delayed_corr(T, Fl, rows):
         gd.copy_(torch.from_numpy(g))
         got = host(slayerCuda.spikeBackwardDelayedCorr(gd, vd, dev(f), delay, theta, tau, scale, Ts)).astype(np.float64)
         moved = np.concatenate([g[:, delay:], np.zeros((rows, delay), np.float32)], axis=1)
-        w = moved.astype(np.float64) * (scale / tau) * np.exp(-np.abs(v.astype(np.float64) - theta) / tau)
-        exact, mag, _ = sum_bounds(w, f)
-        assert np.all(np.abs(got - Ts * exact) <= 2e-6 * Ts * mag + 1e-37), (delay, np.max(np.abs(got - Ts * exact) / (Ts * mag + 1e-37)))
+        exact, mag, _ = sum_bounds(host(slayerCuda.spikeBackward(dev(moved), vd, theta, tau, scale)), f)
+        assert np.all(np.abs(got - Ts * exact) <= 1e-6 * Ts * mag + 1e-37), (delay, np.max(np.abs(got - Ts * exact) / (Ts * mag + 1e-37)))
         if rows > 1:
             g[rows // 2, T // 2], v[0, T // 3] = -np.inf, np.inf
             got = host(slayerCuda.spikeBackwardDelayedCorr(dev(g), dev(v), dev(f), delay, theta, tau, scale, Ts))
