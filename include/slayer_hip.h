@@ -166,9 +166,10 @@ int slayer_spike_bwd_corr_f32(float *gradIn, const float *gradOut, const float *
  * slayer_spike_bwd_corr_f32 of a gradient that first moves back in time by delaySteps samples (zeros move in at the end):
  * the backward pass of a Loihi neuron whose spikes leave delaySteps late (slayer_loihi_get_spikes_delayed_f32),
  * w[n][t] = gradOut[n][t + delaySteps] * (scale / tau) * exp(-|u[n][t] - theta| / tau).  Sums on the
- * matrix cores, as by slayer_corr_f32, for rows of any length from 16 samples on and any alignment (delaySteps may be 0).  SLAYER_EUNSUPPORTED, and nothing is done, for rows that the fused kernel does not serve (fewer than 16
- * samples, filters outside 34 to 129 taps, a delay beyond the row, and delayed rows of at most 304
- * samples that are whole vectors of an odd number): slayer_shift_f32 and slayer_spike_bwd_corr_f32 then.
+ * matrix cores, as by slayer_corr_f32, for rows of any length from 16 samples on and any alignment (delaySteps may
+ * be 0).  SLAYER_EUNSUPPORTED, and nothing is done, for rows that the fused kernel does not serve (fewer than 16 samples,
+ * filters outside 34 to 129 taps, a delay beyond the row, and delayed rows of at most 304 samples that are whole vectors
+ * of an odd number): slayer_shift_f32 and slayer_spike_bwd_corr_f32 then.
  */
 int slayer_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradOut, const float *u, const float *filt,
                                       int64_t nNeurons, int64_t T, int64_t F, int64_t delaySteps, float theta,
@@ -359,11 +360,13 @@ int slayer_loihi_get_spikes_delayed_f32(float *s, float *v, float *u, const floa
  *
  * Arithmetic: fp32 sums; the order of the additions depends on the geometry, not on the launch (no
  * atomics).  The forward pass of layers with at least 16 output channels and about 100 or more taps
- * per output, and the weight gradient of layers large enough for the matrix cores, multiply on bf16
- * matrix instructions over operands split into three bf16 parts each (six of the nine partial
+ * per output, the input gradient of such layers with passes of 16 output channels and at most ten taps
+ * per channel (3x3 filters), and the weight gradient of layers large enough for the matrix cores multiply
+ * on bf16 matrix instructions over operands split into three bf16 parts each (six of the nine partial
  * products; three when the input holds nothing below the upper 16 bits of its numbers, as spike
- * tensors do): every result within 1e-6 of the sum of its terms' magnitudes.  Parts below 2^-126 are
- * flushed to zero, and a non-finite input sample gives NaN where an fp32 sum may give an infinity.
+ * tensors do): every result within 1e-6 of the sum of its terms' magnitudes, a sum of one term within
+ * 2^-23 of it.  Parts below 2^-126 are flushed to zero.  Infinities and NaNs reach the sums that they
+ * enter and no others, as in a chain of fp32 multiply-adds.
  */
 typedef struct slayer_synapse_geom {
     int32_t N, C, H, W, T;

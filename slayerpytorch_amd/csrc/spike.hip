@@ -363,9 +363,10 @@ __global__ __launch_bounds__(64) void spike_tile_kernel(float *__restrict__ s, f
             // Going from candidate to candidate costs a round trip through LDS per visit, and the wavefront stays as long
             // as its busiest row.  Visits are spikes plus the candidates that no response has removed (below), so the
             // count of candidates on arrival only bounds them: a smooth potential that fires 4 % of the time arrives with
-            // 19 % candidates (137 us this way, 156 us sample by sample, on (12,16,32,32,300)), one that fires 12 % of
-            // the time with 45 % (198 us against 170 us).  Tiles with a row above the threshold half of the time or more
-            // take the walk over every sample (a third: 145 us on the first of the two tensors).
+            // 19 % candidates (137 us this way, 156 us sample by sample, on (12,16,32,32,300) in tiles of whole rows, which
+            // this kernel took then), one that fires 12 % of the time with 45 % (198 us against 170 us).  Tiles with a row
+            // above the threshold half of the time or more take the walk over every sample (a third: 145 us on the first
+            // of the two tensors).
             hop = __builtin_amdgcn_ballot_w64(mine * 2 > W) == 0;
         }
         const bool steady = monotone && signedTaps && !hop;

@@ -960,6 +960,7 @@ def test_spikes_many_long_rows_use_16_row_tiles(T, kind, delay):
     assert ws.sum() > 0
 
 
+# ------------------------------------------------------------------------------------------ delay gradient
 @pytest.mark.parametrize("shape,Ts", [((4, 6, 1, 1, 80), 0.1), ((64, 20, 1, 1, 2000), 1.0), ((3, 2, 5, 7, 33), 0.5),
                                       ((1, 1, 1, 1, 1), 1.0)])
 def test_delay_grad(shape, Ts):
