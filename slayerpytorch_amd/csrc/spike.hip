@@ -1045,7 +1045,7 @@ static int launch_spike_rows(const SpikeRowsLayout &l, float *s, float *u, const
     const int P = l.pitch, NB = l.blocks, rounds = l.rounds, R = kWave / l.parts;
     const size_t lds = l.ldsBytes;
     const int64_t groups = ceil_div(nNeurons, R);
-    if (groups >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
+    if (groups * kWave >= (1LL << 32)) return SLAYER_EUNSUPPORTED;   // (what lies beyond, a launch leaves out without an error)
     const FastDiv byNV = make_fastdiv(static_cast<uint32_t>(T >= 4 ? T / 4 : 1));
     const dim3 grid(static_cast<unsigned>(groups));
     const bool small = NB <= 31 && rounds <= 31;

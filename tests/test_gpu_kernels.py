@@ -960,6 +960,18 @@ def test_spikes_many_long_rows_use_16_row_tiles(T, kind, delay):
     assert ws.sum() > 0
 
 
+@pytest.mark.parametrize("nuSize,rows", [(3, 2 ** 29 + 9), (30, 2 ** 28 + 5)])
+def test_spikes_of_more_rows_than_a_launch_has_lanes_for(nuSize, rows):
+    """Tiles of 8 (4) rows per wavefront would be more than the 2^32 lanes that one launch can have.  Rows of one sample: a
+    spike where the potential is at or above theta, which then takes the response's first tap."""
+    u = torch.arange(rows, device="cuda", dtype=torch.int32).remainder_(37).float().view(1, rows, 1, 1, 1)
+    want = (u >= 10.0).float()
+    after = torch.addcmul(u, want, torch.full((), -4.0, device="cuda"))
+    nu = torch.full((nuSize,), -4.0, device="cuda")
+    s = slayerCuda.getSpikes(u, nu, 10.0, 1.0)
+    assert torch.equal(s, want) and torch.equal(u, after)
+
+
 # ------------------------------------------------------------------------------------------ delay gradient
 @pytest.mark.parametrize("shape,Ts", [((4, 6, 1, 1, 80), 0.1), ((64, 20, 1, 1, 2000), 1.0), ((3, 2, 5, 7, 33), 0.5),
                                       ((1, 1, 1, 1, 1), 1.0)])
