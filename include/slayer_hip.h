@@ -534,7 +534,7 @@ int slayer_bin_events_f32(float *tensor, const float *base, const int32_t *x, co
  * error inside the target region).  out, desired, error and the optional addend are [rows][T]; psp
  * is the causal filter of slayer_conv_f32 with the same arithmetic; `loss` is one float.  The sum
  * has a fixed association (deterministic).  `workspace` holds slayer_spike_loss_workspace_bytes(rows)
- * bytes.  Rows whose T + 2 F floats exceed 60 KB return SLAYER_EUNSUPPORTED (nothing launched).
+ * bytes.  Rows whose T + 2 F floats exceed 60 KB, and 2^24 rows or more, return SLAYER_EUNSUPPORTED (nothing launched).
  */
 int64_t slayer_spike_loss_workspace_bytes(int64_t rows);
 int slayer_spike_loss_f32(float *loss, float *error, const float *out, const float *desired,

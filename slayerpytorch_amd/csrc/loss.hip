@@ -147,8 +147,12 @@ __global__ __launch_bounds__(256) void spike_loss_sum_kernel(float *__restrict__
     if (threadIdx.x == 0) loss[0] = (((wsum[0] + wsum[1]) + wsum[2]) + wsum[3]) * scale;
 }
 
-// A row and the filter must fit the LDS of one work-group (60 KB without what rounds them up).
-static bool row_fits(int64_t T, int64_t F) { return (2 * F + T) * static_cast<int64_t>(sizeof(float)) <= 60 * 1024; }
+// A row and the filter must fit the LDS of one work-group (60 KB without what rounds them up), and the work-groups, one per
+// row, a launch (lanes beyond the 2^32 of a launch would be left out without an error).
+static bool rows_fit(int64_t rows, int64_t T, int64_t F)
+{
+    return (2 * F + T) * static_cast<int64_t>(sizeof(float)) <= 60 * 1024 && rows < (1LL << 24);
+}
 static int64_t row_lds_bytes(int64_t T, int64_t F) { return (2 * ((F + 3) & ~3LL) + ((T + 3) & ~3LL) + 8) * static_cast<int64_t>(sizeof(float)); }
 
 }  // namespace slayer
@@ -169,8 +173,7 @@ extern "C" int slayer_spike_loss_f32(float *loss, float *error, const float *out
     const int64_t live = (rows > 0 && T > 0) ? rows : 0;
     if (live > 0) {
         if (!error || !out || !desired || !workspace || (F > 0 && !srm)) return SLAYER_EINVAL;
-        // a row and the filter must fit the LDS of one work-group
-        if (!row_fits(T, F) || live >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
+        if (!rows_fit(live, T, F)) return SLAYER_EUNSUPPORTED;
         const int64_t ldsBytes = row_lds_bytes(T, F);
         hipLaunchKernelGGL(spike_loss_rows_kernel, dim3(static_cast<unsigned>(live)), dim3(256),
                            static_cast<size_t>(ldsBytes), st, error, workspace, out, desired, addend, srm,
@@ -189,7 +192,7 @@ extern "C" int slayer_spike_loss_grad_f32(float *grad, const float *error, const
     if (rows < 0 || T < 0 || F < 0) return SLAYER_EINVAL;
     if (rows == 0 || T == 0) return SLAYER_OK;
     if (!grad || !error || !gradLoss || (F > 0 && !srm)) return SLAYER_EINVAL;
-    if (!row_fits(T, F) || rows >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
+    if (!rows_fit(rows, T, F)) return SLAYER_EUNSUPPORTED;
     hipLaunchKernelGGL(spike_loss_grad_kernel, dim3(static_cast<unsigned>(rows)), dim3(256),
                        static_cast<size_t>(row_lds_bytes(T, F)), static_cast<hipStream_t>(stream), grad, error, gradLoss, srm,
                        static_cast<int>(T), static_cast<int>(F), Ts, T % 4 == 0 && aligned16(grad));

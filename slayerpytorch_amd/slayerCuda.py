@@ -493,7 +493,7 @@ def delayGradStatic(output, gradOutput, Ts, out=None):
 def spikeLoss(spikeOut, spikeDesired, srmKernel, Ts, addend=None):
     """``error = conv(spikeOut - spikeDesired, srmKernel, Ts) [+ addend]`` and
     ``loss = 1/2 * sum(error**2) * Ts`` in two launches.  Returns ``(loss, error)`` (``loss`` is a
-    0-dim tensor), or ``None`` when a row does not fit the kernel (nothing was launched)."""
+    0-dim tensor), or ``None`` when the rows do not fit the kernel (nothing was launched)."""
     _check_input(spikeOut, "spikeOut")
     _check_input(spikeDesired, "spikeDesired")
     _check_input(srmKernel, "srmKernel")
@@ -524,7 +524,7 @@ def spikeLoss(spikeOut, spikeDesired, srmKernel, Ts, addend=None):
 
 def spikeLossGrad(error, gradLoss, srmKernel, Ts):
     """``corr(error * (gradLoss * Ts), srmKernel, Ts)``, the gradient of :func:`spikeLoss` with respect to its
-    ``spikeOut`` for the gradient ``gradLoss`` (one element) of the loss, in one launch where a row fits the
+    ``spikeOut`` for the gradient ``gradLoss`` (one element) of the loss, in one launch where the rows fit the
     kernel of :func:`spikeLoss`."""
     _check_input(error, "error")
     _check_input(gradLoss, "gradLoss")

@@ -1,8 +1,8 @@
 """Spike-train losses on top of the PSP kernel (src/spikeLoss.py:7-104), computed on the device.
 
 ``spikeTime``: half the squared van Rossum distance between output and desired spike trains, from the
-fused error + squared-sum kernels of ``slayerCuda.spikeLoss`` (rows too long for them take the tensor
-expression of the reference).
+fused error + squared-sum kernels of ``slayerCuda.spikeLoss`` (rows too long or too many for them take the
+tensor expression of the reference).
 ``numSpikes``: spike count inside a target region against a desired count, spike-time loss
 outside it.  The reference builds the target region, the desired counts and the count error on
 the host (numpy round trips, src/spikeLoss.py:91-102); here every step is a tensor operation on
@@ -41,8 +41,10 @@ class _spikeLossFunction(torch.autograd.Function):
 
 
 def _fits(spike, srmKernel):
-    # the fused loss keeps one row and the filter in the LDS of a work-group
-    return spike.is_cuda and spike.dtype == torch.float32 and (spike.shape[-1] + 2 * srmKernel.numel()) * 4 <= 60 * 1024
+    # the fused loss keeps one row and the filter in the LDS of a work-group, of which a launch has less than 2^24
+    T = spike.shape[-1]
+    return (spike.is_cuda and spike.dtype == torch.float32 and (T + 2 * srmKernel.numel()) * 4 <= 60 * 1024
+            and spike.numel() < max(T, 1) * 2 ** 24)
 
 
 class spikeLoss(torch.nn.Module):

@@ -12,6 +12,7 @@ import torch
 from oracle import oracle as O
 from slayerpytorch_amd import _lib, slayerCuda, slayerLoihiCuda
 from slayerpytorch_amd.slayer import alphaKernel
+from slayerpytorch_amd.spikeLoss import spikeLoss
 
 from _util import rel_err
 
@@ -1279,6 +1280,30 @@ def test_spike_loss_gradient_with_a_tap_that_is_not_finite(T, Fl, bad):
     fin = np.isfinite(want)
     assert fin.any() and not fin.all() and np.array_equal(got[~fin], want[~fin], equal_nan=True)
     assert np.isfinite(got[fin]).all() and np.max(np.abs(got[fin] - want[fin])) <= 1e-5 * np.max(np.abs(want[fin]))
+
+
+def test_spike_loss_of_more_rows_than_a_launch_has_work_groups_for():
+    """One work-group per row would be more than the 2^32 lanes of a launch: the gradient is the correlation's, the loss the
+    tensor expression's."""
+    rows, T = 2 ** 24 + 5, 2
+    e = torch.arange(rows * T, device="cuda", dtype=torch.int32).remainder_(23).sub_(11).float().view(rows, 1, 1, 1, T)
+    f = torch.tensor([2.0, 0.5, -1.0], device="cuda")
+    want = e * 4.0      # (gradLoss 0.5, Ts 2: x = e, times Ts and the first tap)
+    want[..., 0] += e[..., 1]
+    assert torch.equal(slayerCuda.spikeLossGrad(e, torch.tensor(0.5, device="cuda"), f, 2.0), want)
+    assert slayerCuda.spikeLoss(e, torch.zeros_like(e), f, 2.0) is None
+    net = {"neuron": {"type": "SRMALPHA", "theta": 10, "tauSr": 1.0, "tauRef": 1.0, "scaleRef": 2, "tauRho": 1, "scaleRho": 1},
+           "simulation": {"Ts": 1.0, "tSample": T}, "training": {"error": {"type": "SpikeTime"}}}
+    loss = spikeLoss(net).cuda()
+    x = e.clone().requires_grad_(True)
+    value = loss.spikeTime(x, torch.zeros_like(e))
+    value.backward()
+    part = e[:1000].clone().requires_grad_(True)
+    loss.spikeTime(part, torch.zeros_like(part)).backward()
+    tail = e[-1000:].clone().requires_grad_(True)
+    loss.spikeTime(tail, torch.zeros_like(tail)).backward()
+    for got, ref in ((x.grad[:1000], part.grad), (x.grad[-1000:], tail.grad)):
+        assert torch.allclose(got, ref, rtol=1e-5, atol=1e-5)
 
 
 @pytest.mark.parametrize("rows,T", [(12100, 700), (12100, 704), (12070, 1000), (8070, 1500), (8070, 1604)])
