@@ -484,8 +484,8 @@ bool launch_fir_corr_walk(float *out, const float *in, const float *filt, int64_
     const int nCh = static_cast<int>(ceil_div(T, 32));
     const int nce = static_cast<int>((15 + F + 31) / 32), nc = static_cast<int>((31 + F + 31) / 32);
     const int64_t rowGroups = ceil_div(rows, 16), resident = static_cast<int64_t>(compute_units()) * 8;
-    if (rowGroups >= (1LL << 24)) return false;
-    int segs = walk_segments(rowGroups, nCh, nc, resident);
+    if (rowGroups >= (1LL << 31)) return false;
+    int segs = rowGroups < (1LL << 24) ? walk_segments(rowGroups, nCh, nc, resident) : 1;   // (items are counted in 32 bits)
     const int segChunks = static_cast<int>(ceil_div(nCh, segs));
     segs = static_cast<int>(ceil_div(nCh, segChunks));
     const int64_t items = rowGroups * segs;

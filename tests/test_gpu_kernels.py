@@ -238,6 +238,18 @@ def test_split_products_of_one_term_are_as_close_as_the_chain(T, Fl, delay):
         assert np.all(np.abs(got - exact) <= 1e-6 * mag)
 
 
+def test_corr_of_very_many_rows_is_that_of_a_few():
+    """2^28 rows and more (17 GB) are walked on the matrix cores like fewer ones: the same bits."""
+    rows, T = 2 ** 28 + 21, 16
+    x = torch.randn((rows, 1, 1, 1, T), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    f = dev(np.random.default_rng(3).standard_normal(40).astype(np.float32))
+    y = slayerCuda.corr(x, f, 1.0)
+    for part in (slice(0, 4096), slice(2 ** 27 + 16, 2 ** 27 + 4112), slice(rows - 4101, rows)):
+        assert torch.equal(y[part], slayerCuda.corr(x[part].contiguous(), f, 1.0))
+    del x, y
+    torch.cuda.empty_cache()
+
+
 def test_corr_from_split_operands_with_a_tap_that_is_not_finite():
     # such a tap has no split: every tile takes the chains, whose bits are the oracle's
     rng = np.random.default_rng(77)
