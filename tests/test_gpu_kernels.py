@@ -106,7 +106,7 @@ def on_matrix_cores(op, T, Fl, generic=0):
 
 def close_to_chain(got, x, f, Ts, op):
     """Element-wise bound for a sum that was added up in another order: |got - exact| <= 1e-5 * Ts * sum_i |x||f|
-    (the north star's 1e-5 relative, taken against the sum of the magnitudes of each output's own terms, so a small
+    (1e-5 relative, which this path is held to, taken against the sum of the magnitudes of each output's own terms, so a small
     output next to large ones is held as tightly as a large one).  Exact sum and bound in double precision."""
     x64, f64 = np.asarray(x, np.float64), np.asarray(f, np.float64)
     flat = x64.reshape(-1, x64.shape[-1])

@@ -537,7 +537,7 @@ DENSE_ROWS_CASES = [
 @pytest.mark.parametrize("transposed", [False, True])
 def test_dense_rows_product(case, transposed):
     # the dense layer's product and (transposed) input gradient on bf16 matrix instructions over split operands: every
-    # output within 1e-6 of the sum of its terms' magnitudes (the bound the header states; the north star asks for
+    # output within 1e-6 of the sum of its terms' magnitudes (the bound the header states; the path is held to
     # 1e-5), on spikes and on dense inputs of mixed magnitude
     N, K, O, T, spikes = case
     rng = np.random.default_rng(N + K + O + T)
