@@ -396,6 +396,25 @@ int slayer_synapse_conv_f32(float *out, const float *in, const float *weight,
 int slayer_synapse_conv_grad_input_f32(float *gradIn, const float *gradOut, const float *weight,
                                        const slayer_synapse_geom *geom, void *stream);
 
+/*
+ * Sum pooling of every channel of in [N][C][H][W][T] over windows of KH x KW pixels that do not overlap, with one
+ * weight per position of the window (weight [KH][KW]): slayer_synapse_conv_f32 with strides KH and KW on the channels
+ * as images of one channel each.  An extent that is no multiple of the window counts as extended by extent % window
+ * rows or columns of zeros: OH = (H + H % KH) / KH, OW likewise (src/slayer.py:565-575).  out [N][C][OH][OW][T].
+ */
+int slayer_pool_f32(float *out, const float *in, const float *weight, int64_t N, int64_t C, int64_t H, int64_t W, int64_t T,
+                    int64_t KH, int64_t KW, void *stream);
+
+/*
+ * Gradient of slayer_pool_f32 with respect to `in`.  With a membrane potential u (same shape as gradIn; may be NULL)
+ * every result is multiplied by the surrogate gradient of slayer_spike_bwd_f32 at u (theta, tau, scale as there): with
+ * gradOut filtered by slayer_psp_alpha_f32 (causal = 0) or slayer_corr_f32 first, that is what pool(psp(spike(u))) sends
+ * back to u, since pooling and a filter along time commute.
+ */
+int slayer_pool_grad_input_f32(float *gradIn, const float *gradOut, const float *weight, const float *u, float theta,
+                               float tau, float scale, int64_t N, int64_t C, int64_t H, int64_t W, int64_t T, int64_t KH,
+                               int64_t KW, void *stream);
+
 /* Bytes of caller-provided device workspace for slayer_synapse_conv_grad_weight_f32 (may be 0). */
 int64_t slayer_synapse_conv_grad_weight_workspace_bytes(const slayer_synapse_geom *geom);
 

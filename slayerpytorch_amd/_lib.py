@@ -74,6 +74,9 @@ SIGNATURES = {
     "slayer_synapse_out_shape": (ctypes.c_int, [_geomp, _i32p, _i32p]),
     "slayer_synapse_conv_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _geomp, _stream]),
     "slayer_synapse_conv_grad_input_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _geomp, _stream]),
+    "slayer_pool_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _stream]),
+    "slayer_pool_grad_input_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _f32, _f32, _f32, _i64, _i64, _i64, _i64, _i64,
+                                                  _i64, _i64, _stream]),
     "slayer_synapse_conv_grad_weight_workspace_bytes": (_i64, [_geomp]),
     "slayer_synapse_conv_grad_weight_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _geomp, _stream]),
     "slayer_quantize_f32": (ctypes.c_int, [_f32p, _f32p, _i64, ctypes.c_double, _stream]),

@@ -25,7 +25,7 @@ import numpy as np
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.utils.weak import WeakTensorKeyDictionary
+from torch.utils.weak import TensorWeakRef, WeakTensorKeyDictionary
 
 from . import slayerCuda
 from . import synapse
@@ -88,7 +88,11 @@ class spikeLayer(nn.Module):
         alpha = self._srmKernelIsAlpha()
         origin = _fresh_spikes(spike) if alpha is not None and _recursion_serves(spike) else None
         if origin is not None:
-            return _pspOfSpikeFunction.apply(spike, origin[0], self.srmKernel, self.simulation["Ts"], alpha, *origin[1:])
+            psp = _pspOfSpikeFunction.apply(spike, origin[0], self.srmKernel, self.simulation["Ts"], alpha, *origin[1:])
+            # for a pooling layer: which potential's spikes these are the filtered ones of (see _spikeNotes)
+            _pspOfSpikeNotes[psp] = (weakref.ref(origin[0]), self.srmKernel, float(self.simulation["Ts"]), alpha, *origin[1:],
+                                     psp._version, origin[0]._version)
+            return psp
         psp = _pspFunction.apply(spike, self.srmKernel, self.simulation["Ts"], alpha)
         if PAIR_SPIKE_PSP and alpha is not None and psp.requires_grad and _recursion_serves(spike):
             # for spike(): what this signal was filtered from, and that it has not been touched since
@@ -377,13 +381,28 @@ class _poolLayer(nn.Conv3d):
 
     def forward(self, input):
         kH, kW = self.weight.shape[2], self.weight.shape[3]
-        if input.shape[2] % kH != 0 or input.shape[3] % kW != 0:
+        weight = self.weight if self.preHookFx is None else self.preHookFx(self.weight)
+        ragged = input.shape[2] % kH != 0 or input.shape[3] % kW != 0
+        if self._windows(input, weight):
+            origin = _fresh_psp_of_spikes(input, kH, kW)
+            if origin is not None:
+                return _poolOfPspFunction.apply(input, origin[0], weight.contiguous(), *origin[1:])
+            if ragged:
+                return synapse.synapsePool(input, weight)
+        if ragged:
             input = F.pad(input, (0, 0, 0, input.shape[3] % kW, 0, input.shape[2] % kH))
         N, C, H, W, T = input.shape
-        weight = self.weight if self.preHookFx is None else self.preHookFx(self.weight)
         result = synapse.synapseConv(input.reshape(N, 1, C * H, W, T), weight, self.stride[:2], self.padding[:2],
                                      self.dilation[:2], 1)
         return result.reshape(result.shape[0], C, -1, result.shape[3], result.shape[4])
+
+    def _windows(self, input, weight):
+        """Whether this is ``synapse.pool``: windows side by side, constant weights, a tensor its kernels take.  (A ragged
+        tensor needs no copy that is extended by zeros then, and no gradient that is cut back.)"""
+        return tuple(self.stride) == tuple(self.kernel_size) and not any(self.padding) and tuple(self.dilation) == (1, 1, 1) \
+            and input.dim() == 5 and input.is_cuda and input.dtype == torch.float32 and input.numel() > 0 \
+            and weight.device == input.device and weight.dtype == torch.float32 and not weight.requires_grad \
+            and tuple(weight.shape) == (1, 1) + tuple(self.kernel_size) and synapse.poolSupported(input.shape, weight.shape)
 
 
 class _convTransposeLayer(nn.ConvTranspose3d):
@@ -512,10 +531,30 @@ def _fresh_spikes(spike):
     return membranePotential, origin[1], origin[2], origin[3]
 
 
+def _fresh_psp_of_spikes(psp, kH, kW):
+    """(membranePotential, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale) when ``psp`` is what ``spikeLayer.psp`` has
+    just returned for the fresh spikes of that potential and the recursion serves the tensor pooled by kH x kW, else None."""
+    origin = _pspOfSpikeNotes.get(psp) if PAIR_SPIKE_PSP else None
+    if origin is None or not torch.is_grad_enabled() or not psp.requires_grad or psp._version != origin[7] \
+            or not isinstance(psp.grad_fn, _pspOfSpikeFunction._backward_cls) or not _unobserved(psp) or not psp.is_contiguous():
+        return None
+    membranePotential = origin[0]()
+    if membranePotential is None or membranePotential.shape != psp.shape or not membranePotential.is_contiguous() \
+            or membranePotential._version != origin[8]:
+        return None
+    N, C, H, W, T = psp.shape
+    pooled = N * C * ((H + H % kH) // kH) * ((W + W % kW) // kW) * T
+    if pooled == 0 or (pooled % 4 if T <= 512 else T % 4):
+        return None
+    return (membranePotential,) + origin[1:7]
+
+
 # The pairing notes live beside the tensors, not on them: a tensor with Python attributes is pickled with them
 # (torch.save of a layer's output would carry the note, or fail on it), and an entry goes when its tensor does.
 _pspNotes = WeakTensorKeyDictionary()     # psp() output -> (its input, kernel, (tau, mult), version)
 _spikeNotes = WeakTensorKeyDictionary()   # spike() output -> (weak potential, theta, pdf tau, pdf scale, versions)
+
+_pspOfSpikeNotes = WeakTensorKeyDictionary()   # psp(spike()) output -> (weak potential, kernel, Ts, (tau, mult), theta, ...)
 
 
 def _unobserved(tensor):
@@ -638,18 +677,47 @@ class _pspOfSpikeFunction(torch.autograd.Function):
     def forward(ctx, spike, membranePotential, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale):
         psp = slayerCuda.pspAlpha(spike.contiguous(), filter, alpha[0], alpha[1], Ts, causal=True)
         ctx.save_for_backward(membranePotential, filter)
+        ctx.set_materialize_grads(False)   # a pooling layer's gradient goes past this node (_poolOfPspFunction)
         ctx.Ts, ctx.alpha = float(Ts), alpha
         ctx.theta, ctx.pdfTimeConstant, ctx.pdfScale = theta, pdfTimeConstant, pdfScale
         return psp
 
     @staticmethod
     def backward(ctx, gradOutput):
-        membranePotential, filter = ctx.saved_tensors
         grad = None
-        if ctx.needs_input_grad[1]:
+        if gradOutput is not None and ctx.needs_input_grad[1]:
+            membranePotential, filter = ctx.saved_tensors
             grad = slayerCuda.pspSpikeBackwardAlpha(gradOutput.contiguous(), None, membranePotential, filter, ctx.alpha[0],
                                                     ctx.alpha[1], ctx.theta, ctx.pdfTimeConstant, ctx.pdfScale, ctx.Ts)
         return None, grad, None, None, None, None, None, None
+
+
+class _poolOfPspFunction(torch.autograd.Function):
+    """The pooling layer (src/slayer.py:565-575) of a signal that ``_pspOfSpikeFunction`` has just made from the spikes of
+    ``membranePotential``.  Forward: the pooling.  Backward: pooling and the filter along time commute, so the gradient
+    is correlated with the filter while it is still pooled - a KH KW-th of the samples - and goes to
+    ``membranePotential`` directly, spread over the windows and multiplied by the spike function's surrogate gradient in
+    one kernel.  Where ``psp`` is still held by someone when the backward pass runs, who may ask for its gradient, it gets
+    it, and its own node does the rest."""
+
+    @staticmethod
+    def forward(ctx, psp, membranePotential, weight, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale):
+        ctx.save_for_backward(membranePotential, weight, filter)
+        ctx.Ts, ctx.alpha = Ts, alpha
+        ctx.theta, ctx.pdfTimeConstant, ctx.pdfScale = theta, pdfTimeConstant, pdfScale
+        ctx.psp = TensorWeakRef(psp)
+        return synapse.pool(psp, weight)
+
+    @staticmethod
+    def backward(ctx, gradOutput):
+        membranePotential, weight, filter = ctx.saved_tensors
+        gradOutput = gradOutput.contiguous()
+        if ctx.psp() is not None:
+            return (synapse.poolGradInput(gradOutput, weight, membranePotential.shape),) + (None,) * 8
+        filtered = slayerCuda.pspAlpha(gradOutput, filter, ctx.alpha[0], ctx.alpha[1], ctx.Ts, causal=False)
+        grad = synapse.poolGradInput(filtered, weight, membranePotential.shape, membranePotential, ctx.theta,
+                                     ctx.pdfTimeConstant, ctx.pdfScale)
+        return (None, grad) + (None,) * 7
 
 
 class _spikePspFunction(torch.autograd.Function):

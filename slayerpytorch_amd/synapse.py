@@ -18,7 +18,7 @@ from .slayerCuda import _check_device, _check_input, _on_device_of, _ptr
 __all__ = ["conv", "convGradInput", "convGradWeight", "outShape", "supported", "synapseConv", "synapseConvTranspose",
            "denseEvents", "denseEventsGradWeight", "denseEventsSupported", "synapseDenseEvents", "denseRows",
            "denseRowsSupported", "denseRowsPays", "synapseDenseRows", "denseRowsGradWeight",
-           "denseRowsGradWeightSupported"]
+           "denseRowsGradWeightSupported", "pool", "poolGradInput", "synapsePool"]
 
 
 def _pair(v, name):
@@ -237,6 +237,93 @@ def synapseConvTranspose(input, weight, stride=1, padding=0, dilation=1, groups=
         return torch.nn.functional.conv_transpose3d(input, w5, None, _triple(stride, 1), _triple(padding, 0), 0, groups,
                                                     _triple(dilation, 1))
     return _synapseConvTransposeFunction.apply(input, weight, stride, padding, dilation, groups)
+
+
+def _windows(inShape, wShape):
+    """Extents of the pooled image: an extent that is no multiple of the window counts as extended by
+    ``extent % window`` (src/slayer.py:565-575)."""
+    H, W, KH, KW = int(inShape[2]), int(inShape[3]), int(wShape[2]), int(wShape[3])
+    return (H + H % KH) // KH, (W + W % KW) // KW
+
+
+def _check_window(weight):
+    _check_input(weight, "weight")
+    if weight.dim() not in (4, 5) or weight.numel() != weight.shape[2] * weight.shape[3]:
+        raise RuntimeError("pooling takes a weight of shape (1, 1, KH, KW[, 1]), got %r" % (tuple(weight.shape),))
+
+
+def pool(input, weight):
+    """Sums over windows of ``weight``'s extent that do not overlap, channel by channel: ``conv`` with the window as
+    stride on every channel by itself, ``input`` (N, C, H, W, T), ``weight`` (1, 1, KH, KW[, 1]).  ``None`` for sizes
+    that the kernel does not index."""
+    _check_input(input, "input")
+    _check_window(weight)
+    _check_device(input, weight, "input", "weight")
+    if input.dim() != 5:
+        raise RuntimeError("expected a 5 dimensional (N,C,H,W,T) tensor, got %d dimensions" % input.dim())
+    N, C, H, W, T = input.shape
+    lib = _lib.load()
+    out = torch.empty((N, C) + _windows(input.shape, weight.shape) + (T,), dtype=input.dtype, device=input.device)
+    with _on_device_of(input) as stream:
+        status = lib.slayer_pool_f32(_ptr(out), _ptr(input), _ptr(weight), N, C, H, W, T, weight.shape[2], weight.shape[3],
+                                     stream)
+    if status == 2:
+        return None
+    _lib.check(status, "slayer_pool_f32")
+    return out
+
+
+def poolGradInput(gradOutput, weight, inShape, membranePotential=None, theta=0.0, tau=1.0, scale=1.0):
+    """Gradient of :func:`pool` with respect to its input of shape ``inShape``; with a ``membranePotential`` of that shape
+    times the surrogate gradient of ``slayerCuda.spikeBackward`` at it."""
+    _check_input(gradOutput, "gradOutput")
+    _check_window(weight)
+    _check_device(gradOutput, weight, "gradOutput", "weight")
+    N, C, H, W, T = (int(v) for v in inShape)
+    if tuple(gradOutput.shape) != (N, C) + _windows(inShape, weight.shape) + (T,):
+        raise RuntimeError("gradOutput has shape %r, expected %r"
+                           % (tuple(gradOutput.shape), (N, C) + _windows(inShape, weight.shape) + (T,)))
+    if membranePotential is not None:
+        _check_input(membranePotential, "membranePotential")
+        _check_device(gradOutput, membranePotential, "gradOutput", "membranePotential")
+        if tuple(membranePotential.shape) != (N, C, H, W, T):
+            raise RuntimeError("membranePotential has shape %r, expected %r" % (tuple(membranePotential.shape), (N, C, H, W, T)))
+    lib = _lib.load()
+    gradIn = torch.empty((N, C, H, W, T), dtype=gradOutput.dtype, device=gradOutput.device)
+    with _on_device_of(gradOutput) as stream:
+        _lib.check(lib.slayer_pool_grad_input_f32(_ptr(gradIn), _ptr(gradOutput), _ptr(weight),
+                                                  None if membranePotential is None else _ptr(membranePotential), theta, tau,
+                                                  scale, N, C, H, W, T, weight.shape[2], weight.shape[3], stream),
+                   "slayer_pool_grad_input_f32")
+    return gradIn
+
+
+class _synapsePoolFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, input, weight):
+        ctx.save_for_backward(weight)
+        ctx.inShape = tuple(input.shape)
+        return pool(input, weight)
+
+    @staticmethod
+    def backward(ctx, gradOutput):
+        (weight,) = ctx.saved_tensors
+        return poolGradInput(gradOutput.contiguous(), weight, ctx.inShape), None
+
+
+def poolSupported(inShape, wShape):
+    """Whether the pooling kernels index these sizes: one channel's image, and the image of a batch item's channels below one
+    another where the window divides the height, as in :func:`supported`."""
+    N, C, H, W, T = (int(v) for v in inShape)
+    KH, KW = int(wShape[2]), int(wShape[3])
+    limit = ((1 << 31) - (1 << 24)) // 4
+    return (KH < 1024 and KW < 1024 and max(H, W) < (1 << 24) - 1024 and (H + KH) * (W + KW) * T < limit and N * C < (1 << 31)
+            and (KH * W + KW) * T * 4 < (1 << 24) and N * C * ((H * W * ((T + 3) // 4)) // 256 + 1) < (1 << 31))
+
+
+def synapsePool(input, weight):
+    """Differentiable :func:`pool` for a weight that gets no gradient and sizes that :func:`poolSupported` takes."""
+    return _synapsePoolFunction.apply(input.contiguous(), weight.contiguous())
 
 
 def denseEventsSupported(N, K, O, T):

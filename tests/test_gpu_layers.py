@@ -276,6 +276,47 @@ def test_spike_of_a_fresh_psp_signal_sends_its_gradient_past_the_filter(monkeypa
         assert all(torch.equal(a, b) for a, b in zip(apart[:3], other[:3]))
 
 
+@pytest.mark.parametrize("C,H,W,T,window", [(3, 8, 8, 300, 2), (4, 7, 9, 173, 2), (2, 5, 6, 173, 2), (4, 10, 7, 520, 3),
+                                            (2, 6, 8, 9, (2, 4)), (4, 5, 5, 3, 2), (1, 2, 2, 20, 2)])
+def test_pool_of_fresh_psp_sends_its_gradient_past_filter_and_spike_function(C, H, W, T, window, monkeypatch):
+    """pool(psp(spike(u))): the pooling layer correlates its gradient while it is still pooled and sends it to u in one
+    kernel.  Same values as with the Functions apart and as torch's own pooling of the extended tensor; the gradient to
+    rounding (weight and filter change places: two roundings per term, REL_TOL).  A psp tensor that is still held gets its
+    own gradient."""
+    from slayerpytorch_amd import slayer as slayer_module
+    layer = snn.layer(neuron(), {"Ts": 1.0, "tSample": max(T, 100)}).to(DEV)
+    pool = layer.pool(window).to(DEV)
+    with torch.no_grad():
+        pool.weight.mul_(torch.rand(pool.weight.shape, device=DEV) + 0.5)     # a weight per position of the window
+    torch.manual_seed(7)
+    u0 = torch.randn((4, C, H, W, T), device=DEV) * 6 + 5
+    KH, KW = pool.kernel_size[0], pool.kernel_size[1]
+    g = torch.randn((4, C, (H + H % KH) // KH, (W + W % KW) // KW, T), device=DEV)
+
+    def run(pair, hold):
+        monkeypatch.setattr(slayer_module, "PAIR_SPIKE_PSP", pair)
+        u = u0.clone().requires_grad_(True)
+        a = layer.psp(layer.spike(u * 1.0))
+        values = a.detach()
+        y = pool(a)
+        name = type(y.grad_fn).__name__
+        wanted = [u, a] if hold else [u]
+        del a
+        return y.detach(), values, name, torch.autograd.grad(y, wanted, g)
+
+    y0, a0, _, (ref,) = run(False, False)
+    y1, _, name, (got,) = run(True, False)
+    assert torch.equal(y0, y1) and float(ref.abs().sum()) > 0
+    if y1.numel() % 4 == 0 if T <= 512 else T % 4 == 0:
+        assert name == "_poolOfPspFunctionBackward"
+    assert rel_err(host(got), host(ref)) <= REL_TOL
+    (ref_u, ref_a), (got_u, got_a) = run(False, True)[3], run(True, True)[3]
+    assert torch.equal(ref_u, got_u) and torch.equal(ref_a, got_a)
+    padded = F.pad(a0.double().cpu(), (0, 0, 0, W % KW, 0, H % KH))
+    want = F.conv3d(padded.reshape(4 * C, 1, *padded.shape[2:]), pool.weight.detach().double().cpu(), None, (KH, KW, 1))
+    assert rel_err(host(y1), want.reshape(y1.shape).numpy()) <= REL_TOL
+
+
 @pytest.mark.parametrize("learnable", [True, False])
 def test_delay_of_fresh_spikes_sends_its_gradient_past_the_spike_function(learnable, monkeypatch):
     """Reference-style delay(spike(u)) / delayShift(spike(u), d): the delay recognises a tensor that spike() has just
