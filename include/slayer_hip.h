@@ -561,6 +561,15 @@ int slayer_spike_loss_f32(float *loss, float *error, const float *out, const flo
                           int64_t T, int64_t F, float Ts, void *stream);
 
 /*
+ * The spike-count loss (src/spikeLoss.py:60-104) in two launches: error = psp(out outside [start, stop)) plus, inside,
+ * (Ts * sum of out[start..stop) - count) / length * scale, count = countTrue where wanted[row] is not zero, else
+ * countFalse, in double precision and rounded to fp32 at the end.  0 <= start, stop <= T; everything else as above.
+ */
+int slayer_count_loss_f32(float *loss, float *error, const float *out, const uint8_t *wanted, const float *srm,
+                          float *workspace, int64_t rows, int64_t T, int64_t F, float Ts, int64_t start, int64_t stop,
+                          double countTrue, double countFalse, double length, double scale, void *stream);
+
+/*
  * Gradient of that loss with respect to `out`: grad = Ts * corr(error * (gradLoss * Ts), srm), gradLoss one float on the
  * device, in one launch.  Agrees with slayer_corr_f32 of the scaled error to rounding (1e-5).  Same limits.
  */

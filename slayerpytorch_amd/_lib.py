@@ -70,6 +70,8 @@ SIGNATURES = {
     "slayer_spike_loss_workspace_bytes": (_i64, [_i64]),
     "slayer_spike_loss_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _f32,
                                              _stream]),
+    "slayer_count_loss_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _f32, _i64, _i64,
+                                             ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, _stream]),
     "slayer_spike_loss_grad_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _f32, _stream]),
     "slayer_synapse_out_shape": (ctypes.c_int, [_geomp, _i32p, _i32p]),
     "slayer_synapse_conv_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _geomp, _stream]),

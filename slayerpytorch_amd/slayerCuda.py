@@ -31,7 +31,7 @@ import torch
 from . import _lib
 
 __all__ = ["getSpikes", "conv", "corr", "shift", "spikeBackward", "spikeBackwardCorr", "spikeBackwardDelayedCorr",
-           "pspSpike", "delayGrad", "getSpikesDelayed", "spikeBackwardDelayed", "spikeLoss", "spikeLossGrad", "pspAlpha", "spikeBackwardPspAlpha",
+           "pspSpike", "delayGrad", "getSpikesDelayed", "spikeBackwardDelayed", "spikeLoss", "countLoss", "spikeLossGrad", "pspAlpha", "spikeBackwardPspAlpha",
            "pspSpikeBackwardAlpha"]
 
 
@@ -519,6 +519,33 @@ def spikeLoss(spikeOut, spikeDesired, srmKernel, Ts, addend=None):
     if status == 2:
         return None
     _lib.check(status, "slayer_spike_loss_f32")
+    return loss, error
+
+
+def countLoss(spikeOut, wanted, srmKernel, Ts, start, stop, countTrue, countFalse, length, scale):
+    """The spike-count loss of ``spikeOut`` (..., T): ``error`` = ``conv`` of the spikes outside samples ``start`` to
+    ``stop`` plus, inside, ``(spikes in there - count) / length * scale`` with ``count`` = ``countTrue`` or ``countFalse`` by
+    ``wanted`` (one truth value per row), and ``loss = 1/2 * sum(error**2) * Ts``, in two launches.  Returns
+    ``(loss, error)``, or ``None`` when the rows do not fit the kernel."""
+    _check_input(spikeOut, "spikeOut")
+    _check_input(srmKernel, "srmKernel")
+    _check_device(spikeOut, srmKernel, "spikeOut", "srmKernel")
+    rows, T = _rows(spikeOut)
+    if not wanted.is_cuda or not wanted.is_contiguous() or wanted.dtype != torch.bool or wanted.numel() != rows:
+        raise RuntimeError("wanted must be a contiguous CUDA tensor of %d truth values" % rows)
+    _check_device(spikeOut, wanted, "spikeOut", "wanted")
+    Ts = _scalar(Ts, "Ts")
+    lib = _lib.load()
+    loss = torch.empty((), dtype=spikeOut.dtype, device=spikeOut.device)
+    error = torch.empty_like(spikeOut)
+    workspace = torch.empty((max(rows, 1),), dtype=torch.float32, device=spikeOut.device)
+    with _on_device_of(spikeOut) as stream:
+        status = lib.slayer_count_loss_f32(loss.data_ptr(), _ptr(error), _ptr(spikeOut), _ptr(wanted), _ptr(srmKernel),
+                                           workspace.data_ptr(), rows, T, srmKernel.numel(), Ts, start, stop, countTrue,
+                                           countFalse, length, scale, stream)
+    if status == 2:
+        return None
+    _lib.check(status, "slayer_count_loss_f32")
     return loss, error
 
 

@@ -4,7 +4,7 @@
 fused error + squared-sum kernels of ``slayerCuda.spikeLoss`` (rows too long or too many for them take the
 tensor expression of the reference).
 ``numSpikes``: spike count inside a target region against a desired count, spike-time loss
-outside it.  The reference builds the target region, the desired counts and the count error on
+outside it, from ``slayerCuda.countLoss`` (other rows and shapes: tensor expressions).  The reference builds the target region, the desired counts and the count error on
 the host (numpy round trips, src/spikeLoss.py:91-102); here every step is a tensor operation on
 the device of ``spikeOut``, so the loss never synchronises with the host.
 """
@@ -38,6 +38,20 @@ class _spikeLossFunction(torch.autograd.Function):
             grad = slayerCuda.corr(error * (gradLoss * ctx.Ts), srmKernel, ctx.Ts)
         return (grad if ctx.needs_input_grad[0] else None, -grad if ctx.needs_input_grad[1] else None,
                 None, None, None)
+
+
+class _countLossFunction(torch.autograd.Function):
+    """The spike-count loss over ``slayerCuda.countLoss``; the count error is a constant (src/spikeLoss.py:87-104), so the
+    backward pass is that of ``_spikeLossFunction``."""
+
+    @staticmethod
+    def forward(ctx, spikeOut, wanted, srmKernel, Ts, target):
+        loss, error = slayerCuda.countLoss(spikeOut.contiguous(), wanted, srmKernel, Ts, *target)
+        ctx.save_for_backward(error, srmKernel)
+        ctx.Ts = float(Ts)
+        return loss
+
+    backward = _spikeLossFunction.backward
 
 
 def _fits(spike, srmKernel):
@@ -79,6 +93,15 @@ class spikeLoss(torch.nn.Module):
         count = self.errorDescriptor["tgtSpikeCount"]
         startID = int(round(region["start"] / Ts))      # round half to even, like numpy.rint
         stopID = int(round(region["stop"] / Ts))
+        if _fits(spikeOut, self.slayer.srmKernel) and spikeOut.dim() == 5 and spikeOut.numel() > 0 \
+                and type(numSpikesScale) in (int, float) and stopID != startID \
+                and tuple(desiredClass.shape) == tuple(spikeOut.shape[:4]) + (1,):
+            wanted = desiredClass.to(spikeOut.device)
+            wanted = (wanted if wanted.dtype == torch.bool else wanted == True).contiguous()       # noqa: E712
+            start, stop, _ = slice(startID, stopID).indices(spikeOut.shape[-1])
+            return _countLossFunction.apply(spikeOut, wanted, self.slayer.srmKernel, Ts,
+                                            (start, stop, float(count[True]), float(count[False]), float(stopID - startID),
+                                             float(numSpikesScale)))
         with torch.no_grad():
             out = spikeOut.detach()
             inRegion = torch.zeros(out.shape[-1], dtype=out.dtype, device=out.device)

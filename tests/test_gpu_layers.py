@@ -875,6 +875,38 @@ def test_spike_time_loss_kernel_matches_tensor_expression(Ts, T, shape):
     assert abs(float(loss) - 0.5 * float((eo.astype(np.float64) ** 2).sum()) * Ts) <= 1e-5 * abs(float(ref))
 
 
+@pytest.mark.parametrize("Ts,T,region,shape", [(1.0, 300, (0, 150), (4, 10, 1, 1)), (0.5, 129, (10, 1000), (2, 3, 1, 2)),
+                                               (1.0, 65, (-20, -3), (1, 1, 1, 1)), (1.0, 4, (3, 1), (3, 2, 1, 1))])
+def test_count_loss_kernel_matches_the_tensor_expressions(Ts, T, region, shape, monkeypatch):
+    """The spike-count loss in two launches against the tensor expressions that stand for rows that do not fit it: loss and
+    gradient to rounding (1e-5), for regions inside, across the end, counted from the end and empty, and classes given as
+    truth values or numbers."""
+    from slayerpytorch_amd import spikeLoss as module
+    params = neuron(tauSr=5.0)
+    error = snn.loss({"neuron": params, "simulation": {"Ts": Ts, "tSample": int(T * Ts) + 50}, "training": {"error": {
+        "type": "NumSpikes", "tgtSpikeRegion": {"start": region[0] * Ts, "stop": region[1] * Ts},
+        "tgtSpikeCount": {True: 20, False: 3}}}}).to(DEV)
+    torch.manual_seed(3)
+    out = ((torch.rand(shape + (T,)) < 0.2).float() / Ts).to(DEV)
+    cls = (torch.rand(shape + (1,)) < 0.5).to(DEV)
+
+    def run(wanted, scale=1):
+        x = out.clone().requires_grad_(True)
+        loss = error.numSpikes(x, wanted, scale)
+        loss.backward()
+        return type(loss.grad_fn).__name__, float(loss.detach()), host(x.grad)
+
+    got = run(cls)
+    assert got[0] == "_countLossFunctionBackward"
+    assert all(a == b for a, b in zip(got[:2], run(cls.float())[:2]))
+    scaled = run(cls, 2.5)
+    monkeypatch.setattr(module, "_fits", lambda *a: False)
+    for mine, scale in ((got, 1), (scaled, 2.5)):
+        want = run(cls, scale)
+        assert want[0] != mine[0] and abs(mine[1] - want[1]) <= 1e-5 * abs(want[1]) and want[1] > 0
+        assert rel_err(mine[2], want[2]) <= REL_TOL
+
+
 @pytest.mark.parametrize("scale", [100.0, 0.5])
 def test_cpu_plumbing_configuration(scale):
     """The reference's CPU-runnable case: Bernoulli(0.02) spikes (4, 2, 34, 34, 300), dense 2312 -> 512 as a
