@@ -502,6 +502,20 @@ int slayer_dense_rows_grad_weight_f32(float *gradW, const float *gradOut, const 
                                       int64_t K, int64_t O, int64_t T, void *stream);
 
 /*
+ * The same product and its two gradients for few outputs (O <= 32) and any other extents whose 16-byte vectors number
+ * below 2^30: fp32 multiply-adds from tensors of any 4-byte alignment, sums of fixed order.  `workspace` of the product and
+ * of the weight gradient holds slayer_dense_thin_workspace_bytes bytes (gradWeight = 0 / 1; may be 0: NULL).
+ */
+int slayer_dense_thin_supported(int64_t N, int64_t K, int64_t O, int64_t T);
+int64_t slayer_dense_thin_workspace_bytes(int64_t N, int64_t K, int64_t O, int64_t T, int32_t gradWeight);
+int slayer_dense_thin_f32(float *out, const float *weight, const float *x, float *workspace, int64_t N, int64_t K, int64_t O,
+                          int64_t T, void *stream);
+int slayer_dense_thin_grad_input_f32(float *gradIn, const float *weight, const float *gradOut, int64_t N, int64_t K, int64_t O,
+                                     int64_t T, void *stream);
+int slayer_dense_thin_grad_weight_f32(float *gradW, const float *gradOut, const float *x, float *workspace, int64_t N, int64_t K,
+                                      int64_t O, int64_t T, void *stream);
+
+/*
  * ---- Weight quantisation of the Loihi layers ---------------------------------------------------
  * out[i] = round(in[i] / step) * step the way torch evaluates the expression on the GPU for a Python number
  * `step`: in[i] times the fp32 rounding of the double-precision reciprocal of step, to the nearest integer with

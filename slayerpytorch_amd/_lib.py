@@ -91,6 +91,11 @@ SIGNATURES = {
     "slayer_dense_rows_grad_weight_supported": (ctypes.c_int, [_i64, _i64, _i64, _i64]),
     "slayer_dense_rows_grad_weight_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),
     "slayer_dense_rows_grad_weight_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _stream]),
+    "slayer_dense_thin_supported": (ctypes.c_int, [_i64, _i64, _i64, _i64]),
+    "slayer_dense_thin_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i32]),
+    "slayer_dense_thin_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _stream]),
+    "slayer_dense_thin_grad_input_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _stream]),
+    "slayer_dense_thin_grad_weight_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _stream]),
     "slayer_dense_rows_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _i64, _i64, _stream]),
 }
 

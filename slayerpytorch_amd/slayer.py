@@ -249,6 +249,9 @@ DENSE_EVENTS_CHECK_EVERY = 4
 # False keeps the library products.
 DENSE_ROWS = True
 
+# The dense layer's product and gradients from synapse.denseThin where its outputs are few.  False keeps the library products.
+DENSE_THIN = True
+
 
 class _denseLayer(nn.Conv3d):
     """Fully connected synapse: an (outFeatures, C, H, W, 1) weight applied at every time step
@@ -327,6 +330,11 @@ class _denseLayer(nn.Conv3d):
             if DENSE_ROWS and input.is_cuda and input.dtype == torch.float32 and weight.dtype == torch.float32 \
                     and synapse.denseRowsPays(N, K, O, T):
                 return synapse.synapseDenseRows(input.reshape(N, K, T), weight.reshape(O, K)).reshape(N, O, 1, 1, T)
+            # layers with few outputs, an output layer above all: streams of their input, and of its gradient
+            if DENSE_THIN and input.is_cuda and weight.device == input.device and input.dtype == torch.float32 \
+                    and weight.dtype == torch.float32 and synapse.denseThinPays(N, K, O, T) \
+                    and synapse.plainTensors(input, weight):
+                return synapse.synapseDenseThin(input.reshape(N, K, T), weight.reshape(O, K)).reshape(N, O, 1, 1, T)
             # batched product with the weight matrix repeated by a zero stride: torch.matmul of a
             # 2-D by a 3-D tensor would first copy the input into a (K, N*T) layout
             return torch.bmm(weight.reshape(1, O, K).expand(N, O, K), input.reshape(N, K, T)).reshape(N, O, 1, 1, T)

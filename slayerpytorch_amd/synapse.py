@@ -18,7 +18,8 @@ from .slayerCuda import _check_device, _check_input, _on_device_of, _ptr
 __all__ = ["conv", "convGradInput", "convGradWeight", "outShape", "supported", "synapseConv", "synapseConvTranspose",
            "denseEvents", "denseEventsGradWeight", "denseEventsSupported", "synapseDenseEvents", "denseRows",
            "denseRowsSupported", "denseRowsPays", "synapseDenseRows", "denseRowsGradWeight",
-           "denseRowsGradWeightSupported", "pool", "poolGradInput", "synapsePool"]
+           "denseRowsGradWeightSupported", "pool", "poolGradInput", "synapsePool",
+           "denseThin", "denseThinGradInput", "denseThinGradWeight", "synapseDenseThin"]
 
 
 def _pair(v, name):
@@ -500,6 +501,147 @@ class _synapseDenseRowsFunction(torch.autograd.Function):
             else:
                 gradWeight = torch.bmm(gradOutput, input.transpose(1, 2)).sum(0)
         return gradInput, gradWeight
+
+
+def _thin_extents(x, weight, channels):
+    if x.dim() != 3 or weight.dim() != 2 or weight.shape[channels] != x.shape[1]:
+        raise RuntimeError("the dense layer takes tensors (N, channels, T) and a weight (O, K); got %r and %r"
+                           % (tuple(x.shape), tuple(weight.shape)))
+    return x.shape[0], weight.shape[1], weight.shape[0], x.shape[2]
+
+
+def _workspace(nbytes, like):
+    return torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=like.device) if nbytes else None
+
+
+def denseThin(input, weight):
+    """``weight @ input[n]`` for every batch item, ``input`` (N, K, T), ``weight`` (O, K), for few outputs
+    (``slayer_dense_thin_f32``)."""
+    _check_input(input, "input")
+    _check_input(weight, "weight")
+    _check_device(input, weight, "input", "weight")
+    N, K, O, T = _thin_extents(input, weight, 1)
+    lib = _lib.load()
+    out = torch.empty((N, O, T), dtype=input.dtype, device=input.device)
+    workspace = _workspace(lib.slayer_dense_thin_workspace_bytes(N, K, O, T, 0), input)
+    with _on_device_of(input) as stream:
+        _lib.check(lib.slayer_dense_thin_f32(_ptr(out), _ptr(weight), _ptr(input), None if workspace is None else _ptr(workspace),
+                                             N, K, O, T, stream), "slayer_dense_thin_f32")
+    return out
+
+
+def denseThinGradInput(gradOutput, weight):
+    """``weight.T @ gradOutput[n]`` for every batch item, ``gradOutput`` (N, O, T), ``weight`` (O, K)."""
+    _check_input(gradOutput, "gradOutput")
+    _check_input(weight, "weight")
+    _check_device(gradOutput, weight, "gradOutput", "weight")
+    N, K, O, T = _thin_extents(gradOutput, weight, 0)
+    lib = _lib.load()
+    gradIn = torch.empty((N, K, T), dtype=gradOutput.dtype, device=gradOutput.device)
+    with _on_device_of(gradOutput) as stream:
+        _lib.check(lib.slayer_dense_thin_grad_input_f32(_ptr(gradIn), _ptr(weight), _ptr(gradOutput), N, K, O, T, stream),
+                   "slayer_dense_thin_grad_input_f32")
+    return gradIn
+
+
+def denseThinGradWeight(gradOutput, input):
+    """``sum_n gradOutput[n] @ input[n].T`` as (O, K), ``gradOutput`` (N, O, T), ``input`` (N, K, T)."""
+    _check_input(gradOutput, "gradOutput")
+    _check_input(input, "input")
+    _check_device(gradOutput, input, "gradOutput", "input")
+    if input.dim() != 3 or gradOutput.dim() != 3 or gradOutput.shape[0] != input.shape[0] \
+            or gradOutput.shape[2] != input.shape[2]:
+        raise RuntimeError("denseThinGradWeight takes gradOutput (N, O, T) and input (N, K, T); got %r and %r"
+                           % (tuple(gradOutput.shape), tuple(input.shape)))
+    N, K, T = input.shape
+    O = gradOutput.shape[1]
+    lib = _lib.load()
+    gradW = torch.empty((O, K), dtype=input.dtype, device=input.device)
+    workspace = _workspace(lib.slayer_dense_thin_workspace_bytes(N, K, O, T, 1), input)
+    with _on_device_of(input) as stream:
+        _lib.check(lib.slayer_dense_thin_grad_weight_f32(_ptr(gradW), _ptr(gradOutput), _ptr(input),
+                                                         None if workspace is None else _ptr(workspace), N, K, O, T, stream),
+                   "slayer_dense_thin_grad_weight_f32")
+    return gradW
+
+
+DENSE_THIN_MAX_OUTPUTS = 16
+
+
+def _thin_product(N, K, O, T):
+    # (us, ours / library: 4096 -> 10 at (1, 300) 8 / 14, (12, 300) 23 / 24, (64, 300) 76 / 84; 5760 -> 10 at (5, 173) 15 / 22;
+    # 512 -> 4 at (1, 100) 6 / 12; but 512 -> 10 at (12, 350) 11 / 8, 400 -> 25 at (32, 500) 24 / 9)
+    return (K > 512 and O <= 16) or O <= 4
+
+
+def _thin_grad_input(N, K, O, T):
+    # (4096 -> 10 at (12, 300) 14 / 33, (64, 300) 66 / 134; 512 -> 10 at (12, 350) 5 / 12; 512 -> 11 at (4, 1450) 6 / 9;
+    # 256 -> 8 at (64, 2000) 23 / 58; 250 -> 25 at (1, 500) 7.4 / 4.5, 4096 -> 32 at (16, 300) 38 / 37)
+    return O <= 16
+
+
+def _thin_grad_weight(N, K, O, T):
+    # (4096 -> 10 at (12, 300) 18 / 27, (64, 300) 65 / 94; 512 -> 10 at (1, 350) 6 / 8, (12, 350) 10 / 12; 250 -> 25 at
+    # (1, 500) 10 / 25; 400 -> 25 at (32, 500) 21 / 20, 4096 -> 32 at (16, 300) 47 / 24)
+    return O <= 16 or N == 1
+
+
+def denseThinPays(N, K, O, T):
+    """Whether the product (N, K, T) -> (N, O, T) or one of its gradients is taken by the kernels for few outputs.  (Below
+    3 * 2^20 inputs the few microseconds that they save are less than what a Function of our own takes on the host: training
+    the 250-25-1 network 379 -> 432 us, 2312-512-10 on (12, 350) 491 -> 487; 4032 -> 10 on (5, 173) gains 40 us.)"""
+    return O <= DENSE_THIN_MAX_OUTPUTS and N * K * T >= 3 << 20 and bool(_lib.load().slayer_dense_thin_supported(N, K, O, T))
+
+
+def plainTensors(*tensors):
+    """Whether nothing but autograd looks at operations on these tensors: no transform, no forward-mode derivative, no
+    tracing or compiling, no autocast, no mode and no subclass that an autograd Function would hide the operation from."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and not torch.is_autocast_enabled("cuda") and torch._C._get_tracing_state() is None
+            and not torch.compiler.is_compiling())
+
+
+class _synapseDenseThinFunction(torch.autograd.Function):
+    """The product and its gradients for few outputs, each from the kernel of this library or torch's batched product,
+    whichever is the faster one at its size.  A backward pass that is itself recorded (``create_graph``) is torch's."""
+
+    @staticmethod
+    def forward(ctx, input, weight):
+        ctx.save_for_backward(input, weight)
+        N, K, T = input.shape
+        O = weight.shape[0]
+        if _thin_product(N, K, O, T):
+            return denseThin(input, weight.contiguous())
+        return torch.bmm(weight.unsqueeze(0).expand(N, O, K), input)
+
+    @staticmethod
+    def backward(ctx, gradOutput):
+        input, weight = ctx.saved_tensors
+        gradInput = gradWeight = None
+        N, K, T = input.shape
+        O = weight.shape[0]
+        own = not torch.is_grad_enabled() and gradOutput.dtype == torch.float32
+        if own:
+            gradOutput = gradOutput.contiguous()
+        if ctx.needs_input_grad[0]:
+            if own and _thin_grad_input(N, K, O, T):
+                gradInput = denseThinGradInput(gradOutput, weight.contiguous())
+            else:
+                gradInput = torch.bmm(weight.t().unsqueeze(0).expand(N, K, O), gradOutput)
+        if ctx.needs_input_grad[1]:
+            if own and _thin_grad_weight(N, K, O, T):
+                gradWeight = denseThinGradWeight(gradOutput, input)
+            else:
+                gradWeight = torch.bmm(gradOutput, input.transpose(1, 2)).sum(0)
+        return gradInput, gradWeight
+
+
+def synapseDenseThin(input, weight):
+    """``weight @ input[n]`` for every batch item (``input`` (N, K, T), ``weight`` (O, K)) with its gradients, for layers with
+    few outputs (:func:`denseThinPays`)."""
+    return _synapseDenseThinFunction.apply(input.contiguous(), weight)
 
 
 def synapseDenseRows(input, weight):

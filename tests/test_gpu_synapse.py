@@ -878,3 +878,74 @@ def test_weight_gradient_sums_are_rounded_and_not_cut(N, C, O_, H, K, pad, T, ki
         assert err.max() <= 2.0 ** -23 * 1.01 and np.sqrt((err ** 2).mean()) <= 3e-8
     else:
         assert np.linalg.norm(got - exact) <= 2e-7 * np.linalg.norm(exact)
+
+
+@pytest.mark.parametrize("N,K,O,T", [(1, 1, 1, 1), (2, 3, 2, 3), (1, 25, 1, 500), (1, 250, 25, 501), (3, 65, 4, 4), (2, 513, 5, 37),
+                                     (5, 129, 8, 130), (12, 512, 10, 350), (3, 1500, 12, 173), (1, 2100, 13, 300), (2, 700, 16, 2053),
+                                     (1, 100, 17, 9), (2, 600, 31, 66), (1, 520, 32, 1450)])
+def test_dense_layers_with_few_outputs(N, K, O, T):
+    """Product and gradients for few outputs against sums in double precision: every element within 1e-6 of the sum of its
+    terms' magnitudes (chains of at most 16384 additions, split over wavefronts: each partial sum has at most 8 + 128
+    roundings of 2^-24 in a row, then a tree).  Tensors start 4 bytes behind a 16-byte boundary; an infinity reaches the sums
+    it enters and no others."""
+    from slayerpytorch_amd import synapse as S
+    gen = torch.Generator(device="cuda").manual_seed(N + K + O + T)
+
+    def tensor(*shape):
+        n = int(np.prod(shape))
+        return torch.randn(n + 1, generator=gen, device="cuda")[1:].view(*shape)
+
+    x, w, g = tensor(N, K, T), tensor(O, K), tensor(N, O, T)
+    xd, wd, gd = x.cpu().double(), w.cpu().double(), g.cpu().double()
+
+    def check(got, f):
+        want, bound = f(xd, wd, gd), f(xd.abs(), wd.abs(), gd.abs())
+        assert got.shape == want.shape and bool(((got.cpu().double() - want).abs() <= 1e-6 * bound).all())
+
+    def grad_weight(a, b, c):
+        return torch.stack([c[n] @ a[n].t() for n in range(N)]).sum(0)
+
+    check(S.denseThin(x, w), lambda a, b, c: b @ a)
+    check(S.denseThinGradInput(g, w), lambda a, b, c: b.t() @ c)
+    check(S.denseThinGradWeight(g, x), grad_weight)
+    x[N - 1, K // 2, T // 2] = float("inf")
+    y, gw = S.denseThin(x, w), S.denseThinGradWeight(g, x)
+    assert not torch.isfinite(y[N - 1, :, T // 2]).any() and int((~torch.isfinite(y)).sum()) == O
+    assert not torch.isfinite(gw[:, K // 2]).any() and int((~torch.isfinite(gw)).sum()) == O
+    g[0, O - 1, T - 1] = float("inf")
+    gi = S.denseThinGradInput(g, w)
+    assert not torch.isfinite(gi[0, :, T - 1]).any() and int((~torch.isfinite(gi)).sum()) == K
+    assert torch.equal(S.denseThinGradWeight(g, x).nan_to_num(), S.denseThinGradWeight(g, x).nan_to_num())
+
+
+@pytest.mark.parametrize("O,T", [(10, 1800), (3, 1801)])
+def test_dense_layer_with_few_outputs_keeps_what_torch_does_with_a_product(O, T):
+    """Through the layer: the kernels' Function where nothing looks at the operations, gradients of gradients by torch, and
+    torch's product under forward-mode derivatives, vmap and autocast."""
+    layer = snn.layer(NEURON, SIM).cuda()
+    fc = layer.dense(600, O).cuda()
+    x = torch.randn((4, 600, 1, 1, T), device="cuda", requires_grad=True)
+    y = fc(x)
+    seen, node = [], y.grad_fn
+    while node is not None:
+        seen.append(type(node).__name__)
+        node = node.next_functions[0][0] if node.next_functions else None
+    assert "_synapseDenseThinFunctionBackward" in seen
+    ref = torch.einsum("ok,nkt->not", fc.weight.double().reshape(O, 600), x.double().reshape(4, 600, T)).reshape(y.shape)
+    assert float((y.double() - ref).norm() / ref.norm()) < 1e-6
+    (gx,) = torch.autograd.grad(y.square().sum(), x, create_graph=True)
+    (again,) = torch.autograd.grad(gx.square().sum(), fc.weight)
+    w = fc.weight.detach().double().requires_grad_(True)
+    yd = torch.einsum("ok,nkt->not", w.reshape(O, 600), x.detach().double().reshape(4, 600, T))
+    gd = 2 * torch.einsum("ok,not->nkt", w.reshape(O, 600), yd)
+    (want,) = torch.autograd.grad(gd.square().sum(), w)
+    assert float((again.double() - want).norm() / want.norm()) < 1e-5
+    import torch.autograd.forward_ad as fwAD
+    with fwAD.dual_level(), torch.no_grad():
+        out = fwAD.unpack_dual(fc(fwAD.make_dual(x.detach(), torch.ones_like(x))))
+        assert out.tangent is not None and torch.allclose(out.tangent, fc(torch.ones_like(x)), rtol=1e-4, atol=1e-3)
+    with torch.no_grad():
+        many = torch.func.vmap(lambda v: fc(v))(torch.stack([x.detach(), 2 * x.detach()]))
+        assert torch.allclose(many[1], 2 * many[0], rtol=1e-4, atol=1e-3)
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert fc(x).dtype == torch.float16
