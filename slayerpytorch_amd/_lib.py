@@ -4,10 +4,13 @@ There is no CPU or PyTorch fallback: if the library is missing, the import error
 build it, and every call raises on a non-zero status.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libslayer_hip.so")
+HOST_PATH = os.path.join(_HERE, "lib", "_slayer_host.so")
 
 _f32p = ctypes.c_void_p          # device pointers travel as integers (tensor.data_ptr())
 _i64 = ctypes.c_int64
@@ -128,6 +131,26 @@ def load():
         raise ImportError("libslayer_hip.so has ABI version %d, expected %d" % (got, ABI_VERSION))
     _lib = lib
     return lib
+
+
+class _Host:
+    """The extension module of ``csrc/host.cpp``, loaded at the first use of one of its functions: the plain case of the
+    calls that a layer makes on every pass, in one step each.  A function answers ``None`` for anything else, with
+    nothing launched."""
+
+    def __getattr__(self, name):
+        if not os.path.exists(HOST_PATH):
+            raise ImportError("_slayer_host.so is not built (%s). Build it with `make -C %s`; there is no fallback "
+                              "implementation." % (HOST_PATH, os.path.join(_HERE, "csrc")))
+        load()
+        loader = importlib.machinery.ExtensionFileLoader("_slayer_host", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_slayer_host", loader))
+        loader.exec_module(module)
+        self.__dict__.update((k, v) for k, v in vars(module).items() if not k.startswith("__"))
+        return self.__dict__[name]
+
+
+host = _Host()
 
 
 def check(status, what):

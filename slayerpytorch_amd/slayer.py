@@ -29,6 +29,7 @@ from torch.utils.weak import TensorWeakRef, WeakTensorKeyDictionary
 
 from . import slayerCuda
 from . import synapse
+from ._function import Function
 
 
 # spikeLayer.psp filters with the alpha kernel as a recursion over time when the kernel has more taps than this
@@ -88,11 +89,7 @@ class spikeLayer(nn.Module):
         alpha = self._srmKernelIsAlpha()
         origin = _fresh_spikes(spike) if alpha is not None and _recursion_serves(spike) else None
         if origin is not None:
-            psp = _pspOfSpikeFunction.apply(spike, origin[0], self.srmKernel, self.simulation["Ts"], alpha, *origin[1:])
-            # for a pooling layer: which potential's spikes these are the filtered ones of (see _spikeNotes)
-            _pspOfSpikeNotes[psp] = (weakref.ref(origin[0]), self.srmKernel, float(self.simulation["Ts"]), alpha, *origin[1:],
-                                     psp._version, origin[0]._version)
-            return psp
+            return _pspOfSpikeFunction.apply(spike, origin[0], self.srmKernel, self.simulation["Ts"], alpha, *origin[1:])
         psp = _pspFunction.apply(spike, self.srmKernel, self.simulation["Ts"], alpha)
         if PAIR_SPIKE_PSP and alpha is not None and psp.requires_grad and _recursion_serves(spike):
             # for spike(): what this signal was filtered from, and that it has not been touched since
@@ -299,13 +296,13 @@ class _denseLayer(nn.Conv3d):
     def _inputIsSparse(self, x):
         """(product, weight gradient): which of the two are summed over the events in this call (see DENSE_EVENTS)."""
         N, K, T = x.shape
-        if DENSE_EVENTS is False or not x.is_cuda or x.dtype != torch.float32 or x.numel() == 0 \
+        if DENSE_EVENTS is False or (K < DENSE_EVENTS_MIN_CHANNELS and DENSE_EVENTS is not True):
+            return False, False
+        if not x.is_cuda or x.dtype != torch.float32 or x.numel() == 0 \
                 or not synapse.denseEventsSupported(N, K, self.weight.shape[0], T):
             return False, False
         if DENSE_EVENTS is True:
             return True, True
-        if K < DENSE_EVENTS_MIN_CHANNELS:
-            return False, False
         if not torch.cuda.is_current_stream_capturing():
             self._measureDensity(x)
         if self._eventDensity is None:
@@ -459,7 +456,7 @@ class _dropoutLayer(nn.Dropout3d):
                            self.inplace).reshape(shape)
 
 
-class _spikeFunction(torch.autograd.Function):
+class _spikeFunction(Function):
     """Forward: ``slayerCuda.getSpikes``; backward: spike-function surrogate gradient
     ``gradOutput * scaleRho/(tauRho*theta) * exp(-|u - theta| / (tauRho*theta))``
     (src/slayer.py:817-865)."""
@@ -488,7 +485,7 @@ class _spikeFunction(torch.autograd.Function):
         return gradInput, None, None, None
 
 
-class _spikeDelayedFunction(torch.autograd.Function):
+class _spikeDelayedFunction(Function):
     """``_spikeFunction`` followed by ``_delayFunction`` / ``_delayFunctionNoGradient``
     (src/slayer.py:817-865, 930-979) as one Function over ``slayerCuda.getSpikesDelayed`` and
     ``slayerCuda.spikeBackwardDelayed``.  ``delay`` is a number or a tensor; a tensor that requires
@@ -530,39 +527,43 @@ def _fresh_spikes(spike):
     if origin is None or not torch.is_grad_enabled() or not spike.requires_grad or spike._version != origin[4] \
             or not isinstance(spike.grad_fn, _spikeFunction._backward_cls) or not _unobserved(spike):
         return None
-    membranePotential = origin[0]()
-    # (a potential changed in place after spike() must reach the spike function's own backward pass, whose saved
-    # tensor then raises; the paired kernel would silently use the changed values)
-    if membranePotential is None or membranePotential.shape != spike.shape or not membranePotential.is_contiguous() \
-            or membranePotential._version != origin[5]:
+    membranePotential = _untouched(origin[0], origin[5], spike)
+    return None if membranePotential is None else (membranePotential, origin[1], origin[2], origin[3])
+
+
+def _untouched(potential, version, result):
+    """The membrane potential behind the weak reference ``potential`` that led to ``result``, if it is as it was.  (A potential
+    changed in place after spike() must reach the spike function's own backward pass, whose saved tensor then raises; the
+    paired kernels would silently use the changed values.)"""
+    membranePotential = potential()
+    if membranePotential is None or membranePotential.shape != result.shape or not membranePotential.is_contiguous() \
+            or membranePotential._version != version:
         return None
-    return membranePotential, origin[1], origin[2], origin[3]
+    return membranePotential
 
 
 def _fresh_psp_of_spikes(psp, kH, kW):
     """(membranePotential, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale) when ``psp`` is what ``spikeLayer.psp`` has
     just returned for the fresh spikes of that potential and the recursion serves the tensor pooled by kH x kW, else None."""
-    origin = _pspOfSpikeNotes.get(psp) if PAIR_SPIKE_PSP else None
-    if origin is None or not torch.is_grad_enabled() or not psp.requires_grad or psp._version != origin[7] \
-            or not isinstance(psp.grad_fn, _pspOfSpikeFunction._backward_cls) or not _unobserved(psp) or not psp.is_contiguous():
+    node = psp.grad_fn if PAIR_SPIKE_PSP else None
+    if type(node) is not _pspOfSpikeFunction._backward_cls or not torch.is_grad_enabled() or psp._version != 0 \
+            or not _unobserved(psp) or not psp.is_contiguous():
         return None
-    membranePotential = origin[0]()
-    if membranePotential is None or membranePotential.shape != psp.shape or not membranePotential.is_contiguous() \
-            or membranePotential._version != origin[8]:
+    membranePotential = _untouched(node.potential, node.potentialVersion, psp)
+    if membranePotential is None:
         return None
     N, C, H, W, T = psp.shape
     pooled = N * C * ((H + H % kH) // kH) * ((W + W % kW) // kW) * T
     if pooled == 0 or (pooled % 4 if T <= 512 else T % 4):
         return None
-    return (membranePotential,) + origin[1:7]
+    return membranePotential, node.filter, node.Ts, node.alpha, node.theta, node.pdfTimeConstant, node.pdfScale
 
 
 # The pairing notes live beside the tensors, not on them: a tensor with Python attributes is pickled with them
-# (torch.save of a layer's output would carry the note, or fail on it), and an entry goes when its tensor does.
+# (torch.save of a layer's output would carry the note, or fail on it), and an entry goes when its tensor does.  (What the
+# pooling layer goes by keeps nothing alive and lives on the node behind the psp signal.)
 _pspNotes = WeakTensorKeyDictionary()     # psp() output -> (its input, kernel, (tau, mult), version)
 _spikeNotes = WeakTensorKeyDictionary()   # spike() output -> (weak potential, theta, pdf tau, pdf scale, versions)
-
-_pspOfSpikeNotes = WeakTensorKeyDictionary()   # psp(spike()) output -> (weak potential, kernel, Ts, (tau, mult), theta, ...)
 
 
 def _unobserved(tensor):
@@ -578,7 +579,7 @@ def _recursion_serves(x):
     return x.numel() % 4 == 0 if T <= 512 else T % 4 == 0
 
 
-class _pspSpikeFunction(torch.autograd.Function):
+class _pspSpikeFunction(Function):
     """``_pspFunction`` followed by ``_spikeFunction`` (src/slayer.py:817-899) as one Function:
     forward is ``slayerCuda.pspSpike``; backward is the spike function's surrogate gradient
     followed by the correlation with the SRM kernel, also in one kernel."""
@@ -614,7 +615,7 @@ class _pspSpikeFunction(torch.autograd.Function):
         return gradInput, None, None, None, None, None
 
 
-class _pspFunction(torch.autograd.Function):
+class _pspFunction(Function):
     """Forward: causal conv with the SRM kernel; backward: correlation with the same kernel;
     the kernel itself gets no gradient (src/slayer.py:875-899).  ``alpha`` = (tau, mult) when the
     kernel is known to be that alpha kernel: both then run as recursions over time."""
@@ -646,7 +647,7 @@ class _pspFunction(torch.autograd.Function):
         return gradInput, None, None, None
 
 
-class _spikeOfPspFunction(torch.autograd.Function):
+class _spikeOfPspFunction(Function):
     """``_spikeFunction`` (src/slayer.py:817-865) for a membrane potential that ``_pspFunction`` has just produced
     from ``pspInput`` with the alpha kernel as a recursion.  Forward: the spike function.  Backward: the gradient
     goes to ``pspInput`` directly - surrogate gradient, then the correlation of ``_pspFunction.backward``
@@ -674,7 +675,7 @@ class _spikeOfPspFunction(torch.autograd.Function):
         return None, grad, None, None, None, None, None
 
 
-class _pspOfSpikeFunction(torch.autograd.Function):
+class _pspOfSpikeFunction(Function):
     """``_pspFunction`` (src/slayer.py:875-899) for a spike tensor that ``_spikeFunction`` has just produced from
     ``membranePotential``, with the alpha kernel as a recursion.  Forward: the PSP filter.  Backward: the
     gradient goes to ``membranePotential`` directly - correlation, then the spike function's surrogate
@@ -688,6 +689,8 @@ class _pspOfSpikeFunction(torch.autograd.Function):
         ctx.set_materialize_grads(False)   # a pooling layer's gradient goes past this node (_poolOfPspFunction)
         ctx.Ts, ctx.alpha = float(Ts), alpha
         ctx.theta, ctx.pdfTimeConstant, ctx.pdfScale = theta, pdfTimeConstant, pdfScale
+        # for _fresh_psp_of_spikes (the filter is a buffer of the layer's)
+        ctx.potential, ctx.potentialVersion, ctx.filter = weakref.ref(membranePotential), membranePotential._version, filter
         return psp
 
     @staticmethod
@@ -700,7 +703,7 @@ class _pspOfSpikeFunction(torch.autograd.Function):
         return None, grad, None, None, None, None, None, None
 
 
-class _poolOfPspFunction(torch.autograd.Function):
+class _poolOfPspFunction(Function):
     """The pooling layer (src/slayer.py:565-575) of a signal that ``_pspOfSpikeFunction`` has just made from the spikes of
     ``membranePotential``.  Forward: the pooling.  Backward: pooling and the filter along time commute, so the gradient
     is correlated with the filter while it is still pooled - a KH KW-th of the samples - and goes to
@@ -728,7 +731,7 @@ class _poolOfPspFunction(torch.autograd.Function):
         return (None, grad) + (None,) * 7
 
 
-class _spikePspFunction(torch.autograd.Function):
+class _spikePspFunction(Function):
     """``_spikeFunction`` followed by ``_pspFunction`` (src/slayer.py:817-899) with both results as outputs.
     Forward: ``slayerCuda.getSpikes``, then the PSP filter; backward: correlation of the PSP gradient, plus the
     gradient that reaches the spikes directly, times the surrogate gradient - one kernel when the PSP kernel
@@ -797,7 +800,7 @@ class _delayLayer(nn.Module):
         return _delayFunction.apply(input, table, self.Ts)
 
 
-class _delayFunction(torch.autograd.Function):
+class _delayFunction(Function):
     """Shift by a per-neuron delay table with gradients for both the input (shift by the
     negated delay) and the delays (src/slayer.py:930-957)."""
 
@@ -817,7 +820,7 @@ class _delayFunction(torch.autograd.Function):
         return gradInput, gradDelay, None
 
 
-class _delayOfSpikeFunction(torch.autograd.Function):
+class _delayOfSpikeFunction(Function):
     """``_delayFunction`` / ``_delayFunctionNoGradient`` (src/slayer.py:930-979) for a spike tensor that
     ``_spikeFunction`` has just produced from ``membranePotential``.  Forward: the shift.  Backward: the gradient
     goes to ``membranePotential`` directly - shifted back and multiplied by the spike function's surrogate gradient
@@ -849,7 +852,7 @@ class _delayOfSpikeFunction(torch.autograd.Function):
         return None, grad, gradDelay, None, None, None, None, None
 
 
-class _delayFunctionNoGradient(torch.autograd.Function):
+class _delayFunctionNoGradient(Function):
     """Shift by a fixed delay (number or tensor); backward shifts the gradient by the negated
     delay (src/slayer.py:959-979)."""
 

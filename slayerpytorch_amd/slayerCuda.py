@@ -29,6 +29,7 @@ import numbers
 import torch
 
 from . import _lib
+from ._lib import host
 
 __all__ = ["getSpikes", "conv", "corr", "shift", "spikeBackward", "spikeBackwardCorr", "spikeBackwardDelayedCorr",
            "pspSpike", "delayGrad", "getSpikesDelayed", "spikeBackwardDelayed", "spikeLoss", "countLoss", "spikeLossGrad", "pspAlpha", "spikeBackwardPspAlpha",
@@ -108,6 +109,9 @@ def getSpikes(d_u, d_nu, theta, Ts):
     """Spikes of the membrane potential ``d_u`` (N,C,H,W,T); ``d_u`` is updated IN PLACE with
     the refractory response ``d_nu`` of every spike.  Returns the spike tensor (``1/Ts`` at
     spikes)."""
+    out = host.getSpikes(d_u, d_nu, theta, Ts)
+    if out is not None:
+        return out
     _check_input(d_u, "d_u")
     _check_input(d_nu, "d_nu")
     _check_device(d_u, d_nu, "d_u", "d_nu")
@@ -145,11 +149,17 @@ def _fir(entry, name, input, filter, Ts):
 
 def conv(input, filter, Ts):
     """Causal convolution in time (last axis) of every neuron row with ``filter``, times ``Ts``."""
+    out = host.conv(input, filter, Ts)
+    if out is not None:
+        return out
     return _fir("slayer_conv_f32", "conv", input, filter, Ts)
 
 
 def corr(input, filter, Ts):
     """Anti-causal correlation in time (adjoint of :func:`conv`), times ``Ts``."""
+    out = host.corr(input, filter, Ts)
+    if out is not None:
+        return out
     return _fir("slayer_corr_f32", "corr", input, filter, Ts)
 
 
@@ -159,6 +169,9 @@ def pspAlpha(input, filter, tau, mult, Ts, causal=True):
     ``spikeLayer.calculateSrmKernel`` builds), computed as a recursion over time instead of a sum over
     the taps.  Agrees with ``conv`` / ``corr`` to rounding; see ``slayer_psp_alpha_f32`` in the header
     for the bound.  The caller vouches for ``filter`` being that kernel."""
+    out = host.pspAlpha(input, filter, tau, mult, Ts, causal)
+    if out is not None:
+        return out
     _check_input(input, "input")
     _check_input(filter, "filter")
     _check_device(input, filter, "input", "filter")
@@ -178,6 +191,9 @@ def spikeBackwardPspAlpha(gradOutput, membranePotential, filter, tauSr, mult, th
     """:func:`spikeBackwardCorr` for a ``filter`` that holds the alpha kernel of :func:`pspAlpha`
     (``tauSr``, ``mult``): the surrogate gradient (``theta``, ``tau``, ``scale`` as in
     :func:`spikeBackward`) and the correlation as a recursion over time, in one kernel."""
+    out = host.spikeBackwardPspAlpha(gradOutput, membranePotential, filter, tauSr, mult, theta, tau, scale, Ts)
+    if out is not None:
+        return out
     _check_input(gradOutput, "gradOutput")
     _check_input(membranePotential, "membranePotential")
     _check_input(filter, "filter")
@@ -204,6 +220,9 @@ def pspSpikeBackwardAlpha(gradPsp, gradSpike, membranePotential, filter, tauSr, 
     (``tauSr``, ``mult``): ``spikeBackward(corr(gradPsp, filter, Ts) + gradSpike, u, theta, tau, scale)`` in one
     kernel; ``gradSpike`` (the gradient that reaches the spikes directly) may be ``None``.  Shapes the
     recursion does not serve take those three calls."""
+    out = host.pspSpikeBackwardAlpha(gradPsp, gradSpike, membranePotential, filter, tauSr, mult, theta, tau, scale, Ts)
+    if out is not None:
+        return out
     _check_input(gradPsp, "gradPsp")
     _check_input(membranePotential, "membranePotential")
     _check_input(filter, "filter")
@@ -244,6 +263,9 @@ def shift(input, shiftLUT, Ts=1.0, sign=1.0):
     device) or a tensor with one delay per neuron of a batch item (``numel == C*H*W``).
     ``sign`` (+1/-1, extension) multiplies the delays, for the backward shift.
     """
+    out = host.shift(input, shiftLUT, Ts, sign)
+    if out is not None:
+        return out
     _check_input(input, "input")
     sign = float(sign)
     if isinstance(shiftLUT, torch.Tensor):
@@ -318,6 +340,9 @@ def getSpikesDelayed(d_u, d_nu, theta, Ts, delay, delayTs=1.0):
 def spikeBackwardDelayed(gradOutput, membranePotential, theta, tau, scale, delay, delayTs=1.0):
     """``spikeBackward(shift(gradOutput, delay, delayTs, sign=-1), membranePotential, ...)`` in one
     pass: the backward of :func:`getSpikesDelayed` with respect to the membrane potential."""
+    out = host.spikeBackwardDelayed(gradOutput, membranePotential, theta, tau, scale, delay, delayTs)
+    if out is not None:
+        return out
     _check_input(gradOutput, "gradOutput")
     _check_input(membranePotential, "membranePotential")
     _check_device(gradOutput, membranePotential, "gradOutput", "membranePotential")
@@ -339,6 +364,9 @@ def spikeBackwardDelayed(gradOutput, membranePotential, theta, tau, scale, delay
 def spikeBackward(gradOutput, membranePotential, theta, tau, scale):
     """``gradOutput * scale/tau * exp(-|membranePotential - theta| / tau)`` in one pass
     (``tau`` is the scaled time constant ``tauRho * theta``)."""
+    out = host.spikeBackward(gradOutput, membranePotential, theta, tau, scale)
+    if out is not None:
+        return out
     _check_input(gradOutput, "gradOutput")
     _check_input(membranePotential, "membranePotential")
     _check_device(gradOutput, membranePotential, "gradOutput", "membranePotential")
@@ -408,6 +436,9 @@ def spikeBackwardDelayedCorr(gradOutput, membranePotential, filter, delaySteps, 
     """:func:`spikeBackwardCorr` of ``shift(gradOutput, delaySteps, 1.0, sign=-1.0)``: the backward pass of a
     Loihi neuron whose spikes leave ``delaySteps >= 0`` samples late.  One kernel, on the matrix cores, for
     rows of any length from 16 samples on and 34 to 129 taps; the two calls elsewhere."""
+    out = host.spikeBackwardDelayedCorr(gradOutput, membranePotential, filter, delaySteps, theta, tau, scale, Ts)
+    if out is not None:
+        return out
     _check_corr(gradOutput, membranePotential, filter)
     theta, tau, scale, Ts = _scalar(theta, "theta"), _scalar(tau, "tau"), _scalar(scale, "scale"), _scalar(Ts, "Ts")
     lib = _lib.load()
@@ -428,6 +459,9 @@ def spikeBackwardDelayedCorr(gradOutput, membranePotential, filter, delaySteps, 
 def delayGrad(output, gradOutput, Ts):
     """Gradient of ``shift`` with respect to its per-neuron delays: ``Ts * sum over batch and
     time of gradOutput * (output[t-1] - output[t]) / Ts``; shape ``output.shape[1:-1]``."""
+    out = host.delayGrad(output, gradOutput, Ts)
+    if out is not None:
+        return out
     _check_input(output, "output")
     _check_input(gradOutput, "gradOutput")
     _check_device(output, gradOutput, "output", "gradOutput")
@@ -494,6 +528,9 @@ def spikeLoss(spikeOut, spikeDesired, srmKernel, Ts, addend=None):
     """``error = conv(spikeOut - spikeDesired, srmKernel, Ts) [+ addend]`` and
     ``loss = 1/2 * sum(error**2) * Ts`` in two launches.  Returns ``(loss, error)`` (``loss`` is a
     0-dim tensor), or ``None`` when the rows do not fit the kernel (nothing was launched)."""
+    out = host.spikeLoss(spikeOut, spikeDesired, srmKernel, Ts, addend)
+    if out is not None:
+        return out
     _check_input(spikeOut, "spikeOut")
     _check_input(spikeDesired, "spikeDesired")
     _check_input(srmKernel, "srmKernel")
@@ -553,6 +590,9 @@ def spikeLossGrad(error, gradLoss, srmKernel, Ts):
     """``corr(error * (gradLoss * Ts), srmKernel, Ts)``, the gradient of :func:`spikeLoss` with respect to its
     ``spikeOut`` for the gradient ``gradLoss`` (one element) of the loss, in one launch where the rows fit the
     kernel of :func:`spikeLoss`."""
+    out = host.spikeLossGrad(error, gradLoss, srmKernel, Ts)
+    if out is not None:
+        return out
     _check_input(error, "error")
     _check_input(gradLoss, "gradLoss")
     _check_input(srmKernel, "srmKernel")

@@ -10,9 +10,10 @@ import numpy as np
 import torch
 
 from . import slayer, slayerCuda, slayerLoihiCuda
+from ._function import Function
 
 
-class quantizeWeights(torch.autograd.Function):
+class quantizeWeights(Function):
     """``round(w / step) * step`` with a straight-through gradient (src/quantizeParams.py:3-31)."""
 
     @staticmethod
@@ -125,7 +126,7 @@ class spikeLayer(slayer.spikeLayer):
         return slayer._unpoolLayer(self._poolWeight(), kernelSize, stride, padding, dilation, preHookFx)
 
 
-class _spike(torch.autograd.Function):
+class _spike(Function):
     @staticmethod
     def _scaled(weightedSpikes, Ts):
         # the reference multiplies by Ts unconditionally; by 1 that is a copy of the tensor

@@ -10,6 +10,7 @@ import operator
 import torch
 
 from . import _lib
+from ._lib import host
 from .slayerCuda import _check_input, _on_device_of, _ptr, _rows
 
 __all__ = ["getSpikes", "getSpikesDelayed", "quantize", "MAX_FUSED_DELAY"]
@@ -72,6 +73,10 @@ def getSpikesDelayed(weightedSpikes, wgtExp, theta, iDecay, vDecay, refDelay, de
     followed by ``shift(spike, delaySteps)``, in one kernel; ``0 <= delaySteps <= MAX_FUSED_DELAY``.
     Voltage and current are not shifted; with ``voltage=False`` / ``current=False`` they are not
     computed into memory at all and ``None`` is returned in their place."""
+    if current is False:
+        out = host.loihiSpikesDelayed(weightedSpikes, wgtExp, theta, iDecay, vDecay, refDelay, delaySteps, voltage)
+        if out is not None:
+            return out
     _check_input(weightedSpikes, "weightedSpikes")
     wgtExp, theta, iDecay, vDecay, refDelay = _neuron_args(wgtExp, theta, iDecay, vDecay, refDelay)
     delaySteps = _unsigned(delaySteps, "delaySteps")
@@ -93,6 +98,9 @@ def getSpikesDelayed(weightedSpikes, wgtExp, theta, iDecay, vDecay, refDelay, de
 def quantize(weights, step):
     """``torch.round(weights / step) * step`` (src/quantizeParams.py:17-23) from one kernel, the same values
     bit for bit.  Has no counterpart in the reference extension."""
+    out = host.quantize(weights, step)
+    if out is not None:
+        return out
     _check_input(weights, "weights")
     step = float(step)
     if step == 0.0 or step != step:

@@ -11,10 +11,11 @@ the device of ``spikeOut``, so the loss never synchronises with the host.
 import torch
 
 from . import slayerCuda
+from ._function import Function
 from .slayer import spikeLayer
 
 
-class _spikeLossFunction(torch.autograd.Function):
+class _spikeLossFunction(Function):
     """``1/2 * sum((psp(out - desired) + addend)**2) * Ts`` over ``slayerCuda.spikeLoss``; the backward
     pass is the correlation of the saved error signal, as autograd derives it for the reference's
     expression (src/spikeLoss.py:56-58)."""
@@ -40,7 +41,7 @@ class _spikeLossFunction(torch.autograd.Function):
                 None, None, None)
 
 
-class _countLossFunction(torch.autograd.Function):
+class _countLossFunction(Function):
     """The spike-count loss over ``slayerCuda.countLoss``; the count error is a constant (src/spikeLoss.py:87-104), so the
     backward pass is that of ``_spikeLossFunction``."""
 

@@ -13,6 +13,8 @@ import functools
 import torch
 
 from . import _lib
+from ._function import Function
+from ._lib import host
 from .slayerCuda import _check_device, _check_input, _on_device_of, _ptr
 
 __all__ = ["conv", "convGradInput", "convGradWeight", "outShape", "supported", "synapseConv", "synapseConvTranspose",
@@ -109,6 +111,9 @@ def _triple(v, last):
 def conv(input, weight, stride=1, padding=0, dilation=1, groups=1):
     """``F.conv3d(input, weight, None, (sH,sW,1), (pH,pW,0), (dH,dW,1), groups)`` for a weight of
     time extent 1."""
+    out = host.conv2d(input, weight, stride, padding, dilation, groups)
+    if out is not None:
+        return out
     _check_input(input, "input")
     _check_input(weight, "weight")
     _check_device(input, weight, "input", "weight")
@@ -160,7 +165,7 @@ def convGradWeight(gradOutput, input, wShape, stride=1, padding=0, dilation=1, g
     return gradW
 
 
-class _synapseConvFunction(torch.autograd.Function):
+class _synapseConvFunction(Function):
     @staticmethod
     def forward(ctx, input, weight, stride, padding, dilation, groups):
         input = input.contiguous()
@@ -175,13 +180,17 @@ class _synapseConvFunction(torch.autograd.Function):
         gradOutput = gradOutput.contiguous()
         gradInput = gradWeight = None
         if ctx.needs_input_grad[0]:
-            gradInput = convGradInput(gradOutput, weight, input.shape, *ctx.args)
+            gradInput = host.conv2dGradInput(gradOutput, weight, input, *ctx.args)
+            if gradInput is None:
+                gradInput = convGradInput(gradOutput, weight, input.shape, *ctx.args)
         if ctx.needs_input_grad[1]:
-            gradWeight = convGradWeight(gradOutput, input, weight.shape, *ctx.args)
+            gradWeight = host.conv2dGradWeight(gradOutput, input, weight, *ctx.args)
+            if gradWeight is None:
+                gradWeight = convGradWeight(gradOutput, input, weight.shape, *ctx.args)
         return gradInput, gradWeight, None, None, None, None
 
 
-class _synapseConvTransposeFunction(torch.autograd.Function):
+class _synapseConvTransposeFunction(Function):
     """The transposed synapse: its forward pass is the input gradient of the convolution whose
     weight tensor it shares, its input gradient is that convolution."""
 
@@ -257,6 +266,9 @@ def pool(input, weight):
     """Sums over windows of ``weight``'s extent that do not overlap, channel by channel: ``conv`` with the window as
     stride on every channel by itself, ``input`` (N, C, H, W, T), ``weight`` (1, 1, KH, KW[, 1]).  ``None`` for sizes
     that the kernel does not index."""
+    out = host.pool(input, weight)
+    if out is not None:
+        return out
     _check_input(input, "input")
     _check_window(weight)
     _check_device(input, weight, "input", "weight")
@@ -277,6 +289,10 @@ def pool(input, weight):
 def poolGradInput(gradOutput, weight, inShape, membranePotential=None, theta=0.0, tau=1.0, scale=1.0):
     """Gradient of :func:`pool` with respect to its input of shape ``inShape``; with a ``membranePotential`` of that shape
     times the surrogate gradient of ``slayerCuda.spikeBackward`` at it."""
+    if membranePotential is not None and inShape == membranePotential.shape:
+        out = host.poolSpikeBackward(gradOutput, weight, membranePotential, theta, tau, scale)
+        if out is not None:
+            return out
     _check_input(gradOutput, "gradOutput")
     _check_window(weight)
     _check_device(gradOutput, weight, "gradOutput", "weight")
@@ -299,7 +315,7 @@ def poolGradInput(gradOutput, weight, inShape, membranePotential=None, theta=0.0
     return gradIn
 
 
-class _synapsePoolFunction(torch.autograd.Function):
+class _synapsePoolFunction(Function):
     @staticmethod
     def forward(ctx, input, weight):
         ctx.save_for_backward(weight)
@@ -338,6 +354,9 @@ def denseEvents(input, weight):
     """``weight @ input[n]`` for every batch item, ``input`` (N, K, T), ``weight`` (O, K), summed over the
     non-zero inputs only (ascending k): the dense layer's product for spike tensors.  The work grows with
     the number of non-zero inputs."""
+    out = host.denseEvents(input, weight)
+    if out is not None:
+        return out
     _check_input(input, "input")
     _check_input(weight, "weight")
     _check_device(input, weight, "input", "weight")
@@ -360,6 +379,9 @@ def denseEventsGradWeight(gradOutput, input):
     """Weight gradient of the dense layer's product ``out[n] = weight @ input[n]``, ``input`` (N, K, T),
     ``gradOutput`` (N, O, T): ``sum_n gradOutput[n] @ input[n].T`` as (O, K), summed over the non-zero
     inputs only, in a fixed order.  The work grows with the number of non-zero inputs."""
+    out = host.denseEventsGradWeight(gradOutput, input)
+    if out is not None:
+        return out
     _check_input(gradOutput, "gradOutput")
     _check_input(input, "input")
     _check_device(gradOutput, input, "gradOutput", "input")
@@ -408,7 +430,7 @@ def denseRows(input, weight, transposed=False):
     return out
 
 
-class _synapseDenseEventsFunction(torch.autograd.Function):
+class _synapseDenseEventsFunction(Function):
     @staticmethod
     def forward(ctx, input, weight, product, gradient):
         ctx.save_for_backward(input, weight)
@@ -477,7 +499,7 @@ def _aligned(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-class _synapseDenseRowsFunction(torch.autograd.Function):
+class _synapseDenseRowsFunction(Function):
     @staticmethod
     def forward(ctx, input, weight):
         ctx.save_for_backward(input, weight)
@@ -517,6 +539,9 @@ def _workspace(nbytes, like):
 def denseThin(input, weight):
     """``weight @ input[n]`` for every batch item, ``input`` (N, K, T), ``weight`` (O, K), for few outputs
     (``slayer_dense_thin_f32``)."""
+    out = host.denseThin(input, weight)
+    if out is not None:
+        return out
     _check_input(input, "input")
     _check_input(weight, "weight")
     _check_device(input, weight, "input", "weight")
@@ -532,6 +557,9 @@ def denseThin(input, weight):
 
 def denseThinGradInput(gradOutput, weight):
     """``weight.T @ gradOutput[n]`` for every batch item, ``gradOutput`` (N, O, T), ``weight`` (O, K)."""
+    out = host.denseThinGradInput(gradOutput, weight)
+    if out is not None:
+        return out
     _check_input(gradOutput, "gradOutput")
     _check_input(weight, "weight")
     _check_device(gradOutput, weight, "gradOutput", "weight")
@@ -546,6 +574,9 @@ def denseThinGradInput(gradOutput, weight):
 
 def denseThinGradWeight(gradOutput, input):
     """``sum_n gradOutput[n] @ input[n].T`` as (O, K), ``gradOutput`` (N, O, T), ``input`` (N, K, T)."""
+    out = host.denseThinGradWeight(gradOutput, input)
+    if out is not None:
+        return out
     _check_input(gradOutput, "gradOutput")
     _check_input(input, "input")
     _check_device(gradOutput, input, "gradOutput", "input")
@@ -603,7 +634,7 @@ def plainTensors(*tensors):
             and not torch.compiler.is_compiling())
 
 
-class _synapseDenseThinFunction(torch.autograd.Function):
+class _synapseDenseThinFunction(Function):
     """The product and its gradients for few outputs, each from the kernel of this library or torch's batched product,
     whichever is the faster one at its size.  A backward pass that is itself recorded (``create_graph``) is torch's."""
 

@@ -1331,3 +1331,66 @@ def test_spikes_of_many_long_rows_are_those_of_a_few(rows, T):
         few = u[a:a + 50].clone()
         sf = slayerCuda.getSpikes(few, nu, 10.0, 1.0)
         assert torch.equal(s[a:a + 50], sf) and torch.equal(many[a:a + 50], few)
+
+
+def test_the_plain_case_of_a_call_equals_the_general_path(monkeypatch):
+    """The functions of the host module against the checks and ctypes calls that they stand for: the same bits, and no
+    answer (so that the general path raises or converts) for anything that is not an exact, contiguous fp32 tensor of one
+    GPU and Python numbers."""
+    from slayerpytorch_amd import _lib, slayerCuda, slayerLoihiCuda, synapse
+    gen = torch.Generator(device="cuda").manual_seed(4)
+
+    def t(*shape):
+        return torch.randn(shape, generator=gen, device="cuda")
+
+    x, u, f, nu = t(2, 3, 4, 5, 40), t(2, 3, 4, 5, 40), t(9), -t(6).abs()
+    w, pw, d2, wide = t(4, 3, 3, 3, 1), t(1, 1, 2, 2, 1), t(3, 4, 5), t(5, 12)
+    rows, grad = t(2, 12, 40), t(2, 5, 40)
+    weighted = (x * 40).round() * 2
+    calls = [
+        (slayerCuda.conv, (x, f, 1.0)), (slayerCuda.corr, (x, f, 0.5)), (slayerCuda.pspAlpha, (x, f.abs(), 2.0, 1.0, 1.0)),
+        (slayerCuda.pspAlpha, (x, f.abs(), 2.0, 1.0, 1.0, False)), (slayerCuda.spikeBackward, (x, u, 10.0, 9.0, 2)),
+        (slayerCuda.spikeBackwardPspAlpha, (x, u, f, 2.0, 1.0, 1.0, 3.0, 1.0, 1.0)),
+        (slayerCuda.pspSpikeBackwardAlpha, (x, None, u, f, 2.0, 1.0, 1.0, 3.0, 1.0, 1.0)),
+        (slayerCuda.pspSpikeBackwardAlpha, (x, u, u, f, 2.0, 1.0, 1.0, 3.0, 1.0, 1.0)),
+        (slayerCuda.shift, (x, 3)), (slayerCuda.shift, (x, 2.5, 0.5, -1.0)), (slayerCuda.shift, (x, d2 * 5, 1.0)),
+        (slayerCuda.shift, (x, d2[:1, :1, 0].contiguous(), 1.0)),
+        (slayerCuda.spikeBackwardDelayed, (x, u, 1.0, 3.0, 1.0, 2.0)), (slayerCuda.spikeBackwardDelayed, (x, u, 1.0, 3.0, 1.0, d2 * 4, 0.5)),
+        (slayerCuda.delayGrad, (x, u, 1.0)), (slayerCuda.spikeBackwardDelayedCorr, (x, u, t(40), 1, 1.0, 3.0, 1.0, 1.0)),
+        (slayerCuda.spikeBackwardDelayedCorr, (x, u, f, 1, 1.0, 3.0, 1.0, 1.0)),
+        (slayerCuda.spikeLoss, (x, u, f, 1.0)), (slayerCuda.spikeLoss, (x, u, f, 1.0, u)), (slayerCuda.spikeLossGrad, (x, t(1), f, 1.0)),
+        (slayerLoihiCuda.quantize, (x, 2)),
+        (slayerLoihiCuda.getSpikesDelayed, (weighted, 0, 5120, 1024, 128, 1, 1, True, False)),
+        (slayerLoihiCuda.getSpikesDelayed, (weighted, 0, 5120, 1024, 128, 2, 0, False, False)),
+        (synapse.conv, (x, w, 1, (1, 1))), (synapse.conv, (x, w, (2, 1), 0, (1, 1), 1)), (synapse.pool, (x, pw)),
+        (synapse.poolGradInput, (t(2, 3, 2, 3, 40), pw, x.shape, u, 1.0, 3.0, 1.0)),
+        (synapse.denseEvents, (rows, wide)), (synapse.denseEventsGradWeight, (grad, rows)),
+        (synapse.denseThin, (rows, wide)), (synapse.denseThinGradInput, (grad, wide)), (synapse.denseThinGradWeight, (grad, rows)),
+    ]
+
+    class Nobody:
+        def __getattr__(self, name):
+            return lambda *args: None
+
+    def flat(r):
+        return [v for v in r if v is not None] if isinstance(r, (list, tuple)) else [r]
+
+    for fn, args in calls:
+        got = flat(fn(*args))
+        with monkeypatch.context() as m:
+            for module in (slayerCuda, slayerLoihiCuda, synapse):
+                m.setattr(module, "host", Nobody())
+            want = flat(fn(*args))
+        assert len(got) == len(want) and all(a.shape == b.shape and torch.equal(a, b) for a, b in zip(got, want)), (fn.__name__, len(args))
+    uA, uB = u.clone(), u.clone()
+    sA = slayerCuda.getSpikes(uA, nu, 0.5, 1.0)
+    monkeypatch.setattr(slayerCuda, "host", Nobody())
+    assert torch.equal(sA, slayerCuda.getSpikes(uB, nu, 0.5, 1.0)) and torch.equal(uA, uB)
+    host = _lib.host
+    assert host.conv(x, f, 1.0) is not None
+    for bad in (x.double(), x.cpu(), x.transpose(0, 1), torch.nn.Parameter(x.half()), [1.0], None):
+        assert host.conv(bad, f, 1.0) is None
+    assert host.conv(x, f, t(1)) is None and host.conv(x, f, True) is None and host.conv(x, f) is None
+    assert host.spikeBackward(x, u[:1].contiguous(), 1.0, 1.0, 1.0) is None
+    assert host.conv2d(x, w, -1, 0, 1, 1) is None and host.conv2d(x, w, 1, 0, 1, 2) is None
+    assert host.unwrapped(x, 3, None) and not host.unwrapped(torch.ones(2).as_subclass(type("Sub", (torch.Tensor,), {})))
