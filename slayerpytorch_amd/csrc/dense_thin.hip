@@ -10,6 +10,7 @@
 // Rows that are not whole vectors: the last vector of a row starts at sample T - 4 and overlaps the one before; product and
 // input gradient store the shared samples twice with the same values, the weight gradient counts them once.
 #include "common.h"
+#include "fir_core.h"   // f32x4
 
 namespace slayer {
 
@@ -47,111 +48,121 @@ template <int VEC>
 __device__ __forceinline__ int thin_start(int tv, int T) { return VEC == 4 ? min(tv * 4, T - 4) : tv; }
 
 // ---- product -----------------------------------------------------------------------------------------
-// A work-group owns 64 vectors (of any items) and a range of inputs, whose weights it lays into LDS as [k][o] first.  Its
-// wavefronts take eight inputs each in turn: a lane keeps its vector's OB sums, loads the next eight rows' vectors while it
-// multiplies these, and reads the weights as broadcasts, without a barrier.  The wavefronts' sums meet in LDS in three steps.
-constexpr int thin_rows(int VEC) { return VEC == 4 ? 8 : 16; }   // rows of x in each of a wavefront's two sets of registers
-constexpr int kDtChunk = kDtWaves * 16;                // a work-group's range is a multiple of this
-constexpr int kDtWeights = 16384;                      // floats of weights in LDS, at most
+// On fp32 matrix instructions, v_mfma_f32_16x16x4_f32, straight from memory: lane (r, h) holds four weights W[r][k + 4 h ..]
+// with one 16-byte load, and the vector r of rows k + 4 h .. + 3 with four, which is 4 VEC instructions' worth of operands (a
+// vector's four samples are columns of four products).  Neither needs LDS, and two steps of loads are in flight while a
+// wavefront multiplies (four times as many: no faster, (64, 256, 2000) -> 8 27 -> 40 us).  A work-group owns 16 vectors (of any items) and a range of inputs, 16 at a time per
+// wavefront; the wavefronts' sums meet in LDS in three steps.  Vector instructions with the weights as broadcasts from LDS
+// or the scalar cache: 512 -> 11 on (8, 300) 10.2 us, 4096 -> 10 on (64, 300) 76.
+constexpr int kDtSteps = 1;                            // steps of 16 inputs in each of a wavefront's two sets of registers
+constexpr int kDtChunk = kDtWaves * kDtSteps * 16;     // inputs of a work-group's trip
 
-constexpr int thin_sums(int OB, int VEC) { return 4 * (OB < 16 ? OB : 16) * VEC * 64; }   // floats of the sums of four wavefronts
-
-template <int OB, int VEC>
+template <int OT, int VEC>
 __global__ __launch_bounds__(64 * kDtWaves) void dense_thin_kernel(ThinArgs p)
 {
     typedef typename ThinVec<VEC>::V V;
-    constexpr int RB = OB < 16 ? OB : 16;              // outputs per round of the final sum
-    constexpr int ROWS = thin_rows(VEC), TRIP = kDtWaves * ROWS;
-    extern __shared__ __align__(16) float lds[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ __align__(16) f32x4 lds[kDtWaves / 2 * OT * VEC * 64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, h = lane >> 4;
     const int split = static_cast<int>(fastdiv(blockIdx.x, p.byVecBlocks));
-    const int v = (static_cast<int>(blockIdx.x) - split * static_cast<int>(p.byVecBlocks.d)) * 64 + lane;
+    const int v = (static_cast<int>(blockIdx.x) - split * static_cast<int>(p.byVecBlocks.d)) * 16 + r;
     const bool live = v < p.vectors;
     const int n = static_cast<int>(fastdiv(static_cast<uint32_t>(live ? v : 0), p.byTV));
     const int t = thin_start<VEC>((live ? v : 0) - n * p.TV, p.T);
     const int k0 = split * p.perSplit, k1 = min(p.K, k0 + p.perSplit);
     const float *x = p.x + static_cast<int64_t>(n) * p.K * p.T + t;
+    // (outputs that are not there: the last one again, into sums that nobody stores)
+    const float *w[OT];
+#pragma unroll
+    for (int ot = 0; ot < OT; ++ot) w[ot] = p.w + static_cast<int64_t>(min(ot * 16 + r, p.O - 1)) * p.K;
 
-    V acc[OB];
+    f32x4 acc[OT][VEC];
 #pragma unroll
-    for (int o = 0; o < OB; ++o) acc[o] = V(0.0f);
-    V a[ROWS], b[ROWS];
-    auto fetch = [&](V (&r)[ROWS], int k) {         // (rows behind the range: the last one again)
+    for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
-        for (int i = 0; i < ROWS; ++i) r[i] = ThinVec<VEC>::load(x + static_cast<int64_t>(min(k + i, k1 - 1)) * p.T);
-    };
-    auto multiply = [&](V (&r)[ROWS], int k) {
-        if (k + ROWS <= k1) {
+        for (int e = 0; e < VEC; ++e) acc[ot][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Set {
+        V x[kDtSteps][4];
+        float4_ext w[kDtSteps][OT];
+    } a, b;
+    // inputs k .. k + 16 kDtSteps; those behind the range as zeros, both factors (nothing may meet an infinity)
+    auto fetch = [&](Set &s, int k) {
 #pragma unroll
-            for (int i = 0; i < ROWS; ++i) {
-                const float *w = lds + (k - k0 + i) * OB;
+        for (int i = 0; i < kDtSteps; ++i) {
+            const int kk = k + i * 16 + 4 * h;
+            if (k + i * 16 + 16 <= k1) {
 #pragma unroll
-                for (int o = 0; o < OB; ++o) acc[o] = __builtin_elementwise_fma(V(w[o]), r[i], acc[o]);
-            }
-        } else {
+                for (int ot = 0; ot < OT; ++ot) s.w[i][ot] = ThinVec<4>::load(w[ot] + kk);
 #pragma unroll
-            for (int i = 0; i < ROWS; ++i)
-                if (k + i < k1) {
-                    const float *w = lds + (k - k0 + i) * OB;
+                for (int j = 0; j < 4; ++j) s.x[i][j] = ThinVec<VEC>::load(x + static_cast<int64_t>(kk + j) * p.T);
+            } else {
 #pragma unroll
-                    for (int o = 0; o < OB; ++o) acc[o] = __builtin_elementwise_fma(V(w[o]), r[i], acc[o]);
+                for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                    for (int ot = 0; ot < OT; ++ot) s.w[i][ot][j] = kk + j < k1 ? w[ot][kk + j] : 0.f;
+                    s.x[i][j] = kk + j < k1 ? ThinVec<VEC>::load(x + static_cast<int64_t>(kk + j) * p.T) : V(0.f);
                 }
+            }
         }
     };
-    int k = k0 + wave * ROWS;
-    fetch(a, k);
-    fetch(b, k + TRIP);
-    {   // lanes along k: contiguous loads, four of them in flight
-        const int inputs = k1 - k0, cells = inputs * OB;
-        const float inverse = 1.0f / static_cast<float>(inputs);
-        for (int e0 = threadIdx.x; e0 < cells; e0 += 4 * 64 * kDtWaves) {
-            float w[4];
-            int at[4];
+    auto multiply = [&](const Set &s) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int e = e0 + j * 64 * kDtWaves;
-                int o, i;
-                divmod_small(e, inputs, inverse, o, i);
-                at[j] = e < cells ? i * OB + o : -1;
-                w[j] = (e < cells && o < p.O) ? p.w[static_cast<int64_t>(o) * p.K + k0 + i] : 0.0f;
-            }
+        for (int i = 0; i < kDtSteps; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (at[j] >= 0) lds[at[j]] = w[j];
-        }
-    }
-    __syncthreads();
-    for (; k < k1; k += 2 * TRIP) {
-        multiply(a, k);
-        fetch(a, k + 2 * TRIP);
-        if (k + TRIP < k1) multiply(b, k + TRIP);
-        fetch(b, k + 3 * TRIP);
+#pragma unroll
+                for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        float xe;
+                        if constexpr (VEC == 4) xe = s.x[i][j][e];
+                        else xe = s.x[i][j];
+                        acc[ot][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(s.w[i][ot][j], xe, acc[ot][e], 0, 0, 0);
+                    }
+    };
+    int k = k0 + wave * kDtSteps * 16;
+    fetch(a, k);
+    for (;;) {
+        if (k >= k1) break;
+        if (k + kDtChunk < k1) fetch(b, k + kDtChunk);
+        multiply(a);
+        k += kDtChunk;
+        if (k >= k1) break;
+        if (k + kDtChunk < k1) fetch(a, k + kDtChunk);
+        multiply(b);
+        k += kDtChunk;
     }
 
-    float *out = p.out + static_cast<int64_t>(split) * p.N * p.O * p.T;
+    auto meet = [&](int half) {                        // wavefronts half .. 2 half - 1 to 0 .. half - 1
+        __syncthreads();
+        if (wave >= half && wave < 2 * half) {
 #pragma unroll
-    for (int o0 = 0; o0 < OB; o0 += RB) {
-        auto meet = [&](int half) {                    // wavefronts half .. 2 half - 1 to 0 .. half - 1
-            __syncthreads();
-            if (wave >= half && wave < 2 * half) {
+            for (int c = 0; c < OT * VEC; ++c) lds[((wave - half) * OT * VEC + c) * 64 + lane] = acc[c / VEC][c % VEC];
+        }
+        __syncthreads();
+        if (wave < half) {
 #pragma unroll
-                for (int o = 0; o < RB; ++o) reinterpret_cast<V *>(lds)[((wave - half) * RB + o) * 64 + lane] = acc[o0 + o];
-            }
-            __syncthreads();
-            if (wave < half) {
-#pragma unroll
-                for (int o = 0; o < RB; ++o) acc[o0 + o] += reinterpret_cast<const V *>(lds)[(wave * RB + o) * 64 + lane];
-            }
-        };
-        static_assert(kDtWaves == 8, "three steps");
-        meet(4);
-        meet(2);
-        meet(1);
-    }
+            for (int c = 0; c < OT * VEC; ++c) acc[c / VEC][c % VEC] += lds[(wave * OT * VEC + c) * 64 + lane];
+        }
+    };
+    static_assert(kDtWaves == 8, "three steps");
+    meet(4);
+    meet(2);
+    meet(1);
+    // element q of a sum is output 4 h + q of its tile, for vector r
     if (wave == 0 && live) {
+        float *out = p.out + static_cast<int64_t>(split) * p.N * p.O * p.T + static_cast<int64_t>(n) * p.O * p.T + t;
 #pragma unroll
-        for (int o = 0; o < OB; ++o)
-            if (o < p.O) ThinVec<VEC>::store(out + (static_cast<int64_t>(n) * p.O + o) * p.T + t, acc[o]);
+        for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int o = ot * 16 + 4 * h + q;
+                if (o >= p.O) continue;
+                if constexpr (VEC == 4)
+                    ThinVec<4>::store(out + static_cast<int64_t>(o) * p.T,
+                                      float4_ext{acc[ot][0][q], acc[ot][1][q], acc[ot][2][q], acc[ot][3][q]});
+                else
+                    ThinVec<1>::store(out + static_cast<int64_t>(o) * p.T, acc[ot][0][q]);
+            }
     }
 }
 
@@ -330,9 +341,7 @@ struct ThinPlan {
 };
 
 constexpr int kDtKB = 4;
-constexpr int kDtOneLaunch = 512;
-
-static int thin_outputs(int64_t O) { return O <= 2 ? static_cast<int>(O) : O <= 4 ? 4 : O <= 8 ? 8 : O <= 12 ? 12 : O <= 16 ? 16 : 32; }
+constexpr int kDtOneLaunch = 1024, kDtBlocks = 2048;
 
 static bool thin_plan(int64_t N, int64_t K, int64_t O, int64_t T, ThinPlan &p)
 {
@@ -343,17 +352,16 @@ static bool thin_plan(int64_t N, int64_t K, int64_t O, int64_t T, ThinPlan &p)
     p.TV = static_cast<int>(TV);
     p.vectors = static_cast<int>(N * TV);
     p.vecBlocks = (p.vectors + 63) / 64;
-    // The product: vectors of four samples unless there are so few that most compute units would stand by.  One work-group of
-    // eight wavefronts per 64 vectors while the inputs are few (a second launch costs more than a longer one), then as many
-    // ranges of inputs as give two work-groups per compute unit; their weights fit LDS.
-    p.fwdVec = VEC == 4 && p.vecBlocks >= 64 ? 4 : 1;
+    // The product: vectors of four samples unless there are so few that most compute units would stand by (one / four samples:
+    // 512 -> 11 on (8, 300), 600 vectors, 4.0 / 6.2 us; 512 -> 10 on (12, 350), 1056, 5.6 / 6.2; 4096 -> 10 on (12, 300), 900,
+    // 29 / 20; 512 -> 16 on (32, 350) 12.7 / 7.6).  One work-group of eight wavefronts per 16 vectors while the inputs are few
+    // (a second launch costs more than a longer one), then as many ranges of inputs as give eight work-groups per compute unit.
+    p.fwdVec = VEC == 4 && p.vectors >= 800 ? 4 : 1;
     p.fwdTV = p.fwdVec == 4 ? p.TV : static_cast<int>(T);
-    p.fwdBlocks = static_cast<int>(ceil_div(N * p.fwdTV, 64));
-    const int64_t mostPer = kDtWeights / thin_outputs(O) / kDtChunk * kDtChunk;
-    int64_t splits = K <= kDtOneLaunch ? 1 : 512 / p.fwdBlocks;
+    p.fwdBlocks = static_cast<int>(ceil_div(N * p.fwdTV, 16));
+    int64_t splits = K <= kDtOneLaunch ? 1 : kDtBlocks / p.fwdBlocks;
     if (splits < 1) splits = 1;
-    int64_t per = ceil_div(ceil_div(K, splits), kDtChunk) * kDtChunk;
-    if (per > mostPer) per = mostPer;
+    const int64_t per = ceil_div(ceil_div(K, splits), kDtChunk) * kDtChunk;
     p.perSplit = static_cast<int>(per);
     p.splits = static_cast<int>(ceil_div(K, per));
     // The weight gradient: 32 inputs per work-group; as many ranges of vectors as give about 1024 work-groups, at least
@@ -384,7 +392,7 @@ static int thin_sum(float *out, const float *part, int64_t n, int splits, hipStr
 
 }  // namespace slayer
 
-// outputs per lane: as thin_outputs()
+// outputs per lane
 #define SLAYER_THIN(KERNEL, GRID, BLOCK, ...)                                                                                  \
     do {                                                                                                                       \
         if (O <= 1) { if (vec) KERNEL(1, 4, GRID, BLOCK, __VA_ARGS__); else KERNEL(1, 1, GRID, BLOCK, __VA_ARGS__); }            \
@@ -426,13 +434,10 @@ extern "C" int slayer_dense_thin_f32(float *out, const float *weight, const floa
     a.byTV = make_fastdiv(static_cast<uint32_t>(p.fwdTV));
     a.byVecBlocks = make_fastdiv(static_cast<uint32_t>(p.fwdBlocks));
     const dim3 grid(static_cast<unsigned>(p.fwdBlocks * p.splits)), block(64 * kDtWaves);
-    const bool vec = p.fwdVec == 4;
-    const int weights = p.perSplit < a.K ? p.perSplit : a.K;
-#define SLAYER_THIN_FWD(OB, VEC, G, B, A)                                                                                     \
-    hipLaunchKernelGGL((dense_thin_kernel<OB, VEC>), G, B,                                                                     \
-                       4 * (thin_sums(OB, VEC) > weights * OB ? thin_sums(OB, VEC) : weights * OB), st, A)
-    SLAYER_THIN(SLAYER_THIN_FWD, grid, block, a);
-#undef SLAYER_THIN_FWD
+    if (O <= 16 && p.fwdVec == 4) hipLaunchKernelGGL((dense_thin_kernel<1, 4>), grid, block, 0, st, a);
+    else if (O <= 16) hipLaunchKernelGGL((dense_thin_kernel<1, 1>), grid, block, 0, st, a);
+    else if (p.fwdVec == 4) hipLaunchKernelGGL((dense_thin_kernel<2, 4>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((dense_thin_kernel<2, 1>), grid, block, 0, st, a);
     const int status = launch_status();
     if (status != SLAYER_OK || p.splits == 1) return status;
     return thin_sum(out, workspace, N * O * T, p.splits, st);

@@ -596,32 +596,17 @@ def denseThinGradWeight(gradOutput, input):
     return gradW
 
 
-DENSE_THIN_MAX_OUTPUTS = 16
-
-
-def _thin_product(N, K, O, T):
-    # (us, ours / library: 4096 -> 10 at (1, 300) 8 / 14, (12, 300) 23 / 24, (64, 300) 76 / 84; 5760 -> 10 at (5, 173) 15 / 22;
-    # 512 -> 4 at (1, 100) 6 / 12; but 512 -> 10 at (12, 350) 11 / 8, 400 -> 25 at (32, 500) 24 / 9)
-    return (K > 512 and O <= 16) or O <= 4
-
-
-def _thin_grad_input(N, K, O, T):
-    # (4096 -> 10 at (12, 300) 14 / 33, (64, 300) 66 / 134; 512 -> 10 at (12, 350) 5 / 12; 512 -> 11 at (4, 1450) 6 / 9;
-    # 256 -> 8 at (64, 2000) 23 / 58; 250 -> 25 at (1, 500) 7.4 / 4.5, 4096 -> 32 at (16, 300) 38 / 37)
-    return O <= 16
-
-
-def _thin_grad_weight(N, K, O, T):
-    # (4096 -> 10 at (12, 300) 18 / 27, (64, 300) 65 / 94; 512 -> 10 at (1, 350) 6 / 8, (12, 350) 10 / 12; 250 -> 25 at
-    # (1, 500) 10 / 25; 400 -> 25 at (32, 500) 21 / 20, 4096 -> 32 at (16, 300) 47 / 24)
-    return O <= 16 or N == 1
-
-
 def denseThinPays(N, K, O, T):
-    """Whether the product (N, K, T) -> (N, O, T) or one of its gradients is taken by the kernels for few outputs.  (Below
-    3 * 2^20 inputs the few microseconds that they save are less than what a Function of our own takes on the host: training
-    the 250-25-1 network 379 -> 432 us, 2312-512-10 on (12, 350) 491 -> 487; 4032 -> 10 on (5, 173) gains 40 us.)"""
-    return O <= DENSE_THIN_MAX_OUTPUTS and N * K * T >= 3 << 20 and bool(_lib.load().slayer_dense_thin_supported(N, K, O, T))
+    """Whether the layer's product (N, K, T) -> (N, O, T) is taken by the kernels for few outputs: up to 16, or up to 32 where
+    the layer is so small that its launches count more than its work."""
+    # (us, ours / library: 4096 -> 10 at (1, 300) 6 / 14, (12, 300) 20 / 24, (64, 300) 75 / 82; 5760 -> 10 at (5, 173) 15 / 22;
+    # 512 -> 10 at (1, 350) 4.1 / 5.7, (12, 350) 6 / 8; 250 -> 25 at (1, 500) 4.3 / 5.9; 400 -> 25 at (32, 500) 18 / 9.
+    # Input gradient: 4096 -> 10 at (12, 300) 14 / 33, (64, 300) 66 / 134; 512 -> 10 at (12, 350) 5 / 12; 512 -> 11 at
+    # (4, 1450) 6 / 9; 256 -> 8 at (64, 2000) 23 / 58; 250 -> 25 at (1, 500) 7 / 5; 4096 -> 32 at (16, 300) 38 / 37.  Weight
+    # gradient: 4096 -> 10 at (12, 300) 18 / 27, (64, 300) 65 / 94; 512 -> 10 at (1, 350) 6 / 8, (12, 350) 8 / 12; 250 -> 25 at
+    # (1, 500) 10 / 25; 400 -> 25 at (32, 500) 24 / 20.  On the host a product of the library's and its gradients take 90 us,
+    # these 30.)
+    return (O <= 16 or (O <= 32 and N * K * T <= 1 << 20)) and bool(_lib.load().slayer_dense_thin_supported(N, K, O, T))
 
 
 def plainTensors(*tensors):
@@ -635,17 +620,14 @@ def plainTensors(*tensors):
 
 
 class _synapseDenseThinFunction(Function):
-    """The product and its gradients for few outputs, each from the kernel of this library or torch's batched product,
-    whichever is the faster one at its size.  A backward pass that is itself recorded (``create_graph``) is torch's."""
+    """The product and its gradients for few outputs.  A backward pass that is itself recorded (``create_graph``) is torch's."""
 
     @staticmethod
     def forward(ctx, input, weight):
         ctx.save_for_backward(input, weight)
         N, K, T = input.shape
         O = weight.shape[0]
-        if _thin_product(N, K, O, T):
-            return denseThin(input, weight.contiguous())
-        return torch.bmm(weight.unsqueeze(0).expand(N, O, K), input)
+        return denseThin(input, weight.contiguous())
 
     @staticmethod
     def backward(ctx, gradOutput):
@@ -657,12 +639,12 @@ class _synapseDenseThinFunction(Function):
         if own:
             gradOutput = gradOutput.contiguous()
         if ctx.needs_input_grad[0]:
-            if own and _thin_grad_input(N, K, O, T):
+            if own:
                 gradInput = denseThinGradInput(gradOutput, weight.contiguous())
             else:
                 gradInput = torch.bmm(weight.t().unsqueeze(0).expand(N, K, O), gradOutput)
         if ctx.needs_input_grad[1]:
-            if own and _thin_grad_weight(N, K, O, T):
+            if own:
                 gradWeight = denseThinGradWeight(gradOutput, input)
             else:
                 gradWeight = torch.bmm(gradOutput, input.transpose(1, 2)).sum(0)

@@ -918,7 +918,7 @@ def test_dense_layers_with_few_outputs(N, K, O, T):
     assert torch.equal(S.denseThinGradWeight(g, x).nan_to_num(), S.denseThinGradWeight(g, x).nan_to_num())
 
 
-@pytest.mark.parametrize("O,T", [(10, 1800), (3, 1801)])
+@pytest.mark.parametrize("O,T", [(10, 1800), (3, 33), (20, 40)])
 def test_dense_layer_with_few_outputs_keeps_what_torch_does_with_a_product(O, T):
     """Through the layer: the kernels' Function where nothing looks at the operations, gradients of gradients by torch, and
     torch's product under forward-mode derivatives, vmap and autocast."""
