@@ -21,6 +21,7 @@
 
 #include "common.h"
 #include "fir_core.h"   // split_bf16, mfma_bf16
+#include "synapse_ring.h"
 
 namespace slayer {
 
@@ -2024,6 +2025,13 @@ static int launch_gather_mfma(const GatherArgs &a, const SynGeom &s, bool stride
 {
     if (strided || a.Mg < 16 || (a.T % 4 != 0 && a.T < 32)) return SLAYER_EUNSUPPORTED;
     const int KK = a.KH * a.KW;
+    constexpr int kStep = BACKWARD ? -1 : 1;
+    if (a.KH == 3 && a.KW == 3 && a.mulH == 1 && a.mulW == 1 && a.stepH == kStep && a.stepW == kStep) {
+        const RingGeom r{a.src, a.w, a.dst, s.N, a.SC, a.SH, a.SW, a.DC, a.DH, a.DW, a.T, a.groups, a.Qg, a.Mg, a.Cg, a.Og,
+                         s.pH, s.pW};
+        const int status = launch_gather_ring<BACKWARD>(r, st);
+        if (status != SLAYER_EUNSUPPORTED) return status;
+    }
     if (KK > 4 * kGmSteps) return SLAYER_EUNSUPPORTED;
     int chans = 4 * kGmSteps / KK;
     if (chans > a.Qg) chans = a.Qg;

@@ -1,0 +1,418 @@
+// The 3x3, stride-1 gather (forward pass and input gradient of a convolution synapse) with the source rows in a ring.
+//
+// As in synapse_gather_planes_kernel the taps and 16 source channels are the reduction axis of v_mfma_f32_16x16x32_bf16 over
+// operands split into three bf16 parts, and every sample is split once, when it is staged, into three planes in LDS.  There a
+// work-group reloads and resplits the three rows under every row of destination pixels, between two barriers, which is more
+// than half of its time.  Here it walks a strip of columns (eight pixels wide, four where there are two passes of 16 source
+// channels) down the image, one step of 32 samples at a time: LDS holds four source rows of the strip as a ring, three that
+// are read and the one below that is staged meanwhile, so that a sample is loaded 1.25 (1.5) times instead of 3.75 and a row
+// costs one barrier.  The weights sit in registers, 60 per pass and tile of 16 channels: that makes the room in LDS and
+// halves its reads.  Four wavefronts stage and four multiply, one of each on a SIMD, so that splitting runs beside the matrix
+// instructions (all eight doing both, in phase or in opposite phases: 425 to 475 us where this takes 370).
+//
+// Measured, planes kernel -> this: 16 -> 32 channels on 16x16 pixels, (64, 300): forward 484 -> 370 us, input gradient 609 ->
+// 345; (12, 300): 87 -> 76, 109 -> 74; (4, 1450): 150 -> 111, 187 -> 98; 32 -> 64 on 8x8, (64, 300), forward: 336 -> 280.
+// Bound, in the forward pass of 16 -> 32 channels on large tensors, by its stores (rows of 300 samples start 16 bytes into a
+// memory line and on: 286 us without the products, 179 with rows of 288 samples) and by the products (190 us without the
+// stores, 130 of them matrix instructions), which overlap in part: a multiplying wavefront waits where its stores do.
+#include <atomic>
+#include <type_traits>
+
+#include "fir_core.h"
+#include "synapse_ring.h"
+
+namespace slayer {
+
+constexpr int kRgPos = 3 * 1024;     // bytes of a patch position: 3 planes x 32 samples x 16 channels
+constexpr int kRgGroups = 5;         // groups of two taps (the tenth tap is not there: zeros)
+constexpr int kRgSlots = 4;
+constexpr int kRgMul = 4, kRgStage = 4;   // multiplying and staging wavefronts: one of each per SIMD
+
+constexpr int ring_pixels(int P) { return P == 1 ? 8 : 4; }
+constexpr int ring_slot(int P) { return (ring_pixels(P) + 2) * P * kRgPos; }
+constexpr int ring_lds(int P) { return kRgSlots * ring_slot(P) + kRgPos + 128; }
+
+struct RingArgs {
+    RingGeom s;
+    int oGroups, workers, units, steps, tLast, strips, segs, segRows;
+    FastDiv byOGroups, byGroups, bySteps, byStrips, bySegs;
+};
+
+// Sums that are not finite, made again as chains from memory (a matrix instruction multiplies the parts of an infinity with
+// the zeros of taps that are not there): lane (r, h) has channel m, samples t .. t + 3 of pixel (a, b).
+template <bool BACKWARD>
+__device__ __forceinline__ f32x4 ring_again(const RingGeom &s, f32x4 acc, int n, int grp, int m, int a, int b, int t, bool live)
+{
+    asm volatile("" : "+v"(t));   // (nothing of this is worked out ahead and kept in registers)
+    const int64_t plane = static_cast<int64_t>(s.SH) * s.SW * s.T;
+    const BufferRsrc src = make_buffer(s.src + (static_cast<int64_t>(n) * s.SC + static_cast<int64_t>(grp) * s.Qg) * plane);
+    f32x4 again = {0.f, 0.f, 0.f, 0.f};
+#pragma nounroll
+    for (int k = 0; k < s.Qg * 9; ++k) {
+        const int q = k / 9, ij = k - q * 9, i = ij / 3, j = ij - i * 3;
+        const int y = BACKWARD ? a + s.padH - i : a - s.padH + i, x = BACKWARD ? b + s.padW - j : b - s.padW + j;
+        const bool ok = live && static_cast<unsigned>(y) < static_cast<unsigned>(s.SH) && static_cast<unsigned>(x) < static_cast<unsigned>(s.SW);
+        const float4 v = buffer_load4<0>(src, masked_offset(ok, q * static_cast<int>(plane) * 4 + ((y * s.SW + x) * s.T + t) * 4), 0);
+        const float w = m >= s.Mg ? 0.f
+                        : BACKWARD ? s.w[(static_cast<int64_t>(grp * s.Og + q) * s.Cg + m) * 9 + ij]
+                                   : s.w[(static_cast<int64_t>(grp * s.Og + m) * s.Cg + q) * 9 + ij];
+        again[0] = fmaf(w, v.x, again[0]);
+        again[1] = fmaf(w, v.y, again[1]);
+        again[2] = fmaf(w, v.z, again[2]);
+        again[3] = fmaf(w, v.w, again[3]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = fabsf(acc[e]) < __builtin_inff() ? acc[e] : again[e];
+    return acc;
+}
+
+// P: passes of 16 source channels.  TW: tiles of 16 destination channels of a wavefront.  NT: groups of TW tiles of the
+// work-group; the multiplying wavefronts of a group share out the strip's pixels.
+template <int P, int TW, int NT, bool BACKWARD>
+__global__ __launch_bounds__(512) void synapse_gather_ring_kernel(RingArgs g)
+{
+    constexpr int PX = ring_pixels(P), WX = PX + 2, SLOT = ring_slot(P), NG = kRgGroups;
+    constexpr int PIXELS = PX * NT / kRgMul;           // pixels of a multiplying wavefront
+    constexpr int CELLS = WX * P, TASKS = (CELLS + kRgStage - 1) / kRgStage;   // positions of a row, and those of a staging wavefront
+    static_assert(PIXELS >= 1, "every multiplying wavefront has products to make");
+    extern __shared__ __align__(16) float lds[];
+    char *const ldsBytes = reinterpret_cast<char *>(lds);
+    typedef const uint4_ext __attribute__((address_space(3))) *LdsUint4;
+    const uint32_t ldsBase = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char *)ldsBytes));
+    const RingGeom &s = g.s;
+
+    uint32_t rest = xcd_contiguous(blockIdx.x, gridDim.x), qq = fastdiv(rest, g.byOGroups);
+    const int og = static_cast<int>(rest - qq * g.byOGroups.d);
+    rest = qq; qq = fastdiv(rest, g.byGroups);
+    const int grp = static_cast<int>(rest - qq * g.byGroups.d), worker = static_cast<int>(qq);
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, h = lane >> 4;
+    const int64_t srcPlane = static_cast<int64_t>(s.SH) * s.SW * s.T, dstPlane = static_cast<int64_t>(s.DH) * s.DW * s.T;
+    const int planeBytes = static_cast<int>(srcPlane) * 4, rowBytes = s.SW * s.T * 4, pixBytes = s.T * 4;
+
+    if (tid < kRgPos / 16) reinterpret_cast<uint4_ext *>(ldsBytes + kRgSlots * SLOT)[tid] = uint4_ext{0u, 0u, 0u, 0u};
+    uint32_t *const flags = reinterpret_cast<uint32_t *>(ldsBytes + kRgSlots * SLOT + kRgPos);   // [slot][staging wavefront]
+
+    // ---- the walk: unit after unit, the rows of a unit (two more than it has destination rows) one after the other
+    struct Place {
+        int unit, row, n, t0, x0, a0, rows;            // rows: source rows of the unit; row: which of them
+    };
+    auto decode = [&](Place &p) {
+        const uint32_t v = static_cast<uint32_t>(min(p.unit, g.units - 1));
+        const uint32_t q = fastdiv(v, g.bySteps), q2 = fastdiv(q, g.byStrips), q3 = fastdiv(q2, g.bySegs);
+        p.t0 = min(static_cast<int>(v - q * g.bySteps.d) << 5, g.tLast);
+        p.x0 = static_cast<int>(q - q2 * g.byStrips.d) * PX;
+        p.a0 = static_cast<int>(q2 - q3 * g.bySegs.d) * g.segRows;
+        p.n = static_cast<int>(q3);
+        p.rows = min(g.segRows, s.DH - p.a0) + 2;
+    };
+    auto advance = [&](Place &p) {
+        if (++p.row == p.rows) {
+            p.row = 0;
+            p.unit += g.workers;
+            decode(p);
+        }
+    };
+    Place at{worker, 0, 0, 0, 0, 0, 0};
+    decode(at);
+    int trips = 0;                                     // rows of all units of this worker
+    for (Place p = at; p.unit < g.units;) {
+        trips += p.rows;
+        p.unit += g.workers;
+        decode(p);
+    }
+
+    if (wave >= kRgMul) {
+        // ---- staging wavefronts: a row from memory, two rows ahead in two sets of registers, into the planes of the slot that
+        // nobody reads.  Wavefront w takes positions w, w + kRgStage .. of the row (pass by pass), a lane sample `sample` of
+        // channels 8 oct .. + 7.  No branches: the compiler then counts the loads in flight exactly.
+        const int stager = wave - kRgMul, sample = lane & 31, oct = lane >> 5;
+        const int stageAddr = (sample & 3) * 256 + (((oct * 8 + (sample >> 2)) ^ (4 * (sample & 3))) << 4);
+        int cell[TASKS], cellX[TASKS], cellBytes[TASKS];
+#pragma unroll
+        for (int i = 0; i < TASKS; ++i) {
+            cell[i] = stager + kRgStage * i < CELLS ? stager + kRgStage * i : stager;   // (those that are not there: the first one again)
+            const int pass = cell[i] / WX;
+            cellX[i] = cell[i] - pass * WX;
+            cellBytes[i] = (pass * 16 + oct * 8) * planeBytes + sample * 4;
+        }
+        typedef float Row[TASKS][8];
+        auto issue = [&](Row &R, const Place &p) {     // the place's row into registers (behind the last unit: nothing)
+            const BufferRsrc src = make_buffer(s.src + (static_cast<int64_t>(p.n) * s.SC + static_cast<int64_t>(grp) * s.Qg) * srcPlane);
+            const int y = p.a0 + p.row + (BACKWARD ? s.padH - 2 : -s.padH), x = p.x0 + (BACKWARD ? s.padW - 2 : -s.padW);
+            const bool row = p.unit < g.units && static_cast<unsigned>(y) < static_cast<unsigned>(s.SH) && p.t0 + sample < s.T;
+#pragma unroll
+            for (int i = 0; i < TASKS; ++i) {
+                const bool ok = row && static_cast<unsigned>(x + cellX[i]) < static_cast<unsigned>(s.SW);
+                const int from = masked_offset(ok, cellBytes[i] + y * rowBytes + (x + cellX[i]) * pixBytes + p.t0 * 4);
+#pragma unroll
+                for (int c = 0; c < 8; ++c) R[i][c] = buffer_load<0>(src, from, c * planeBytes);
+            }
+        };
+        int slot = 0;
+        auto stage = [&](const Row &R) {               // registers to the planes of the slot
+            uint32_t low = 0;
+#pragma unroll
+            for (int i = 0; i < TASKS; ++i) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) low |= __builtin_bit_cast(uint32_t, R[i][c]);
+                const SplitPlanes sp = split_bf16<false>(R[i]);
+                uint4_ext *to = reinterpret_cast<uint4_ext *>(ldsBytes + slot * SLOT + cell[i] * kRgPos + stageAddr);
+                to[0] = sp.hi;
+                to[64] = sp.mid;
+                to[128] = sp.lo;
+            }
+            const bool any = __builtin_amdgcn_ballot_w64((low & 0xffffu) != 0u) != 0;
+            if (lane == 0) flags[slot * kRgStage + stager] = any ? 1u : 0u;
+            slot = (slot + 1) & (kRgSlots - 1);
+        };
+        Row RA, RB;
+        issue(RB, at);
+        advance(at);
+        issue(RA, at);
+        stage(RB);                                     // the first row
+        advance(at);
+        issue(RB, at);
+        __syncthreads();
+#pragma nounroll
+        for (int k = 0; k < trips; k += 2) {           // (behind the last row: zeros that nobody reads)
+            stage(RA);
+            advance(at);
+            issue(RA, at);
+            __syncthreads();
+            stage(RB);
+            advance(at);
+            issue(RB, at);
+            __syncthreads();
+        }
+        return;
+    }
+
+    // ---- multiplying wavefronts
+    const int tileGroup = wave % NT, share = wave / NT;
+    // weights of this wavefront's tiles: lane (r, h): channels 8 (h % 2) .. + 7 of the pass at tap 2 G + h / 2, for
+    // destination channel 16 tile + r
+    int mFirst[TW], oOff[TW];                          // first channel that this lane stores
+    uint4_ext wr[P][NG][TW][3];
+#pragma unroll
+    for (int ot = 0; ot < TW; ++ot) {
+        const int m = ((og * NT + tileGroup) * TW + ot) * 16 + r;
+        mFirst[ot] = m - (r & 8);
+        oOff[ot] = mFirst[ot] * static_cast<int>(dstPlane) * 4;
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int G = 0; G < NG; ++G) {
+                const int ij = 2 * G + (h >> 1), q0 = p * 16 + (h & 1) * 8;
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    v[j] = 0.f;
+                    if (ij < 9 && m < s.Mg)
+                        v[j] = s.w[BACKWARD ? (static_cast<int64_t>(grp * s.Og + q0 + j) * s.Cg + m) * 9 + ij
+                                            : (static_cast<int64_t>(grp * s.Og + m) * s.Cg + q0 + j) * 9 + ij];
+                }
+                const SplitPlanes sp = split_bf16<false>(v);
+                wr[p][G][ot][0] = sp.hi;
+                wr[p][G][ot][1] = sp.mid;
+                wr[p][G][ot][2] = sp.lo;
+            }
+    }
+    // Operand of group G for sample r of pixel 0: offset in its slot (the zeros': from the first slot), by the lane's tap.  A
+    // half step 16 samples on lies 64 bytes off, before or behind.
+    const int halfStep = (r & 1) != 0 ? -64 : 64;
+    uint32_t off[NG];
+#pragma unroll
+    for (int G = 0; G < NG; ++G) {
+        const int ij = 2 * G + (h >> 1), j = ij % 3;
+        const uint32_t cell = (r & 3) * 256 + ((((h & 1) * 8 + (r >> 2)) ^ (4 * (r & 3))) << 4);
+        off[G] = ldsBase + cell + (ij < 9 ? static_cast<uint32_t>((BACKWARD ? 2 - j : j) * kRgPos) : static_cast<uint32_t>(kRgSlots * SLOT));
+    }
+    __syncthreads();
+    int slot = 0;                                      // of the row `at`
+#pragma nounroll
+    for (int k = 0; k < ((trips + 1) & ~1); ++k) {
+        const int a = at.a0 + at.row - 2;
+        const bool row = at.row >= 2 && at.unit < g.units;   // a destination row has its window
+        const int s0 = ((slot + 2) & (kRgSlots - 1)) * SLOT, s1 = ((slot + 3) & (kRgSlots - 1)) * SLOT, s2 = slot * SLOT;
+        // slot of filter row i: the oldest of the three is source row 0 of the window
+        const int i0 = BACKWARD ? s2 : s0, i1 = s1, i2 = BACKWARD ? s0 : s2;
+        const uint32_t base[NG] = {static_cast<uint32_t>(i0), static_cast<uint32_t>(h < 2 ? i0 : i1), static_cast<uint32_t>(i1),
+                                   static_cast<uint32_t>(i2), static_cast<uint32_t>(h < 2 ? i2 : 0)};
+        const bool all = __builtin_amdgcn_ballot_w64(lane < kRgSlots * kRgStage && lane / kRgStage != ((slot + 1) & (kRgSlots - 1)) &&
+                                                     flags[lane & (kRgSlots * kRgStage - 1)] != 0u) != 0;
+        const BufferRsrc dst = make_buffer(s.dst + (static_cast<int64_t>(at.n) * s.DC + static_cast<int64_t>(grp) * s.Mg) * dstPlane);
+        if (row) {
+#pragma nounroll
+            for (int c = 0; c < PIXELS; ++c) {
+                const int pixel = share * PIXELS + c, b = at.x0 + pixel;
+                if (b >= s.DW) break;
+                f32x4 sums[2][TW];
+                auto multiply = [&](auto partsTag, int half) {
+                    constexpr int PARTS = decltype(partsTag)::value;
+                    const int shift = pixel * kRgPos + (half ? halfStep : 0);
+                    f32x4 (&acc)[TW] = sums[half];
+                    f32x4 small[TW];
+#pragma unroll
+                    for (int ot = 0; ot < TW; ++ot) acc[ot] = small[ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    constexpr int AHEAD = 1;           // groups whose operands are on their way (two: no faster)
+                    uint4_ext x[AHEAD + 1][PARTS];
+                    auto fetch = [&](int set, int p, int G) {
+                        // (the zeros lie at one place whatever the pixel and the pass)
+                        const uint32_t from = off[G] + base[G] + (G == NG - 1 && h >= 2 ? 0 : shift + p * WX * kRgPos);
+#pragma unroll
+                        for (int part = 0; part < PARTS; ++part)
+                            x[set][part] = *reinterpret_cast<LdsUint4>(static_cast<size_t>(from + part * 1024));
+                    };
+#pragma unroll
+                    for (int pg = 0; pg < AHEAD; ++pg) fetch(pg, pg / NG, pg % NG);
+#pragma unroll
+                    for (int pg = 0; pg < P * NG; ++pg) {
+                        const int set = pg % (AHEAD + 1), p = pg / NG, G = pg % NG;
+                        if (pg + AHEAD < P * NG) fetch((pg + AHEAD) % (AHEAD + 1), (pg + AHEAD) / NG, (pg + AHEAD) % NG);
+                        __builtin_amdgcn_sched_barrier(0);
+#define SLAYER_RING_MUL(SUM, XP, WP) \
+    _Pragma("unroll") for (int ot = 0; ot < TW; ++ot) SUM[ot] = mfma_bf16(x[set][XP], wr[p][G][ot][WP], SUM[ot]);
+                        SLAYER_RING_MUL(small, 0, 2)
+                        if constexpr (PARTS == 3) {
+                            SLAYER_RING_MUL(small, 2, 0)
+                            SLAYER_RING_MUL(small, 1, 1)
+                        }
+                        SLAYER_RING_MUL(small, 0, 1)
+                        if constexpr (PARTS == 3) {
+                            SLAYER_RING_MUL(small, 1, 0)
+                        }
+                        SLAYER_RING_MUL(acc, 0, 0)
+#undef SLAYER_RING_MUL
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int ot = 0; ot < TW; ++ot) acc[ot] += small[ot];
+                };
+                // (a step's second half beyond the row's end: nothing to do)
+                const bool two = at.t0 + 16 < s.T;
+                if (all) {
+                    multiply(std::integral_constant<int, 3>{}, 0);
+                    if (two) multiply(std::integral_constant<int, 3>{}, 1);
+                } else {
+                    multiply(std::integral_constant<int, 1>{}, 0);
+                    if (two) multiply(std::integral_constant<int, 1>{}, 1);
+                }
+                if (!two) {
+#pragma unroll
+                    for (int ot = 0; ot < TW; ++ot) sums[1][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                float z = 0.f;
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+                    for (int ot = 0; ot < TW; ++ot)
+                        z = fmaf((sums[hf][ot][0] + sums[hf][ot][1]) + (sums[hf][ot][2] + sums[hf][ot][3]), 0.f, z);
+                if (__builtin_amdgcn_ballot_w64(z != 0.f) != 0u) {
+#pragma unroll
+                    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+                        for (int ot = 0; ot < TW; ++ot) {
+                            const int t = at.t0 + hf * 16 + h * 4;
+                            sums[hf][ot] = ring_again<BACKWARD>(s, sums[hf][ot], at.n, grp, ((og * NT + tileGroup) * TW + ot) * 16 + r, a, b,
+                                                                t, t < s.T);
+                        }
+                }
+                // lanes r and r + 8 exchange a half step, so that a store writes 128 bytes in a row of eight channels instead of
+                // 64 of sixteen
+                const int t = at.t0 + (r >> 3) * 16 + h * 4, to = (a * s.DW + b) * pixBytes + t * 4;
+#pragma unroll
+                for (int ot = 0; ot < TW; ++ot) {
+                    float first[4], second[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float give = r < 8 ? sums[1][ot][e] : sums[0][ot][e];
+                        const float got = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), 0x128, 0xf, 0xf, false));
+                        first[e] = r < 8 ? sums[0][ot][e] : got;
+                        second[e] = r < 8 ? got : sums[1][ot][e];
+                    }
+                    buffer_store4<0>(dst, masked_offset(t < s.T && mFirst[ot] < s.Mg, oOff[ot] + to), 0,
+                                     make_float4(first[0], first[1], first[2], first[3]));
+                    buffer_store4<0>(dst, masked_offset(t < s.T && mFirst[ot] + 8 < s.Mg, oOff[ot] + 8 * static_cast<int>(dstPlane) * 4 + to), 0,
+                                     make_float4(second[0], second[1], second[2], second[3]));
+                }
+            }
+        }
+        advance(at);
+        slot = (slot + 1) & (kRgSlots - 1);
+        __syncthreads();                               // the next row is staged, and everyone is through with the oldest
+    }
+}
+
+template <int P, int TW, int NT, bool BACKWARD>
+static int launch_ring_one(const RingArgs &g, unsigned blocks, hipStream_t st)
+{
+    // more LDS than a kernel may use without asking; asked once per device (a host-side setting, no allocation)
+    static std::atomic<bool> raised[64];
+    int device = 0;
+    hipError_t err = hipGetDevice(&device);
+    if (err == hipSuccess && (device < 0 || device >= 64)) err = hipErrorInvalidDevice;
+    if (err == hipSuccess && !raised[device].load(std::memory_order_acquire)) {
+        err = hipFuncSetAttribute(reinterpret_cast<const void *>(&synapse_gather_ring_kernel<P, TW, NT, BACKWARD>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, ring_lds(P));
+        if (err == hipSuccess) raised[device].store(true, std::memory_order_release);
+    }
+    if (err != hipSuccess) return note_hip_error(err);
+    hipLaunchKernelGGL((synapse_gather_ring_kernel<P, TW, NT, BACKWARD>), dim3(blocks), dim3(512), ring_lds(P), st, g);
+    return launch_status();
+}
+
+template <bool BACKWARD>
+int launch_gather_ring(const RingGeom &s, hipStream_t st)
+{
+    if ((s.Qg != 16 && s.Qg != 32) || s.Mg < 16 || (s.T % 4 != 0 && s.T < 32)) return SLAYER_EUNSUPPORTED;
+    const int P = s.Qg / 16, PX = ring_pixels(P);
+    const int TW = P == 1 && s.Mg > 16 ? 2 : 1;
+    const int NT = P == 1 ? 1 : s.Mg <= 16 ? 1 : s.Mg <= 32 ? 2 : 4;
+    RingArgs g{};
+    g.s = s;
+    g.oGroups = static_cast<int>(ceil_div(s.Mg, 16 * TW * NT));
+    g.steps = (s.T + 31) / 32;
+    g.tLast = s.T % 4 == 0 ? (g.steps - 1) * 32 : s.T - 32;
+    g.strips = static_cast<int>(ceil_div(s.DW, PX));
+    const int64_t base = static_cast<int64_t>(s.groups) * g.oGroups;
+    const int64_t columns = static_cast<int64_t>(s.N) * g.steps * g.strips;
+    // Few columns of the wide strips mean short segments, whose first rows are staged for nothing: the planes kernel then wins
+    // the forward pass, whose rows are long to multiply (columns: planes / this: (5, 14x18, 173), 90: 29 / 38 us; (8, 16x16,
+    // 300), 160: 55 / 58; (12, 16x16, 300), 240: 87 / 76), but not the input gradient (90: 34 / 30).
+    if (!BACKWARD && P == 1 && columns < 200) return SLAYER_EUNSUPPORTED;
+    int64_t workers = compute_units() / base;
+    if (workers < 1) workers = 1;
+    // The units are columns of the image, cut into the number of segments with the fewest rows to walk for the work-group with
+    // most of them: a segment's two first rows are only staged, which counts as one.
+    int64_t best = 0, segs = 1;
+    for (int64_t k = 1; k <= s.DH && k <= 16; ++k) {
+        const int64_t rows = ceil_div(s.DH, k), used = ceil_div(s.DH, rows);
+        const int64_t cost = ceil_div(columns * used, workers) * (rows + 1);
+        if (best == 0 || cost < best) { best = cost; segs = k; }
+    }
+    g.segRows = static_cast<int>(ceil_div(s.DH, segs));
+    g.segs = static_cast<int>(ceil_div(s.DH, g.segRows));
+    const int64_t units = columns * g.segs;
+    if (units < 1 || units >= (1LL << 30)) return SLAYER_EUNSUPPORTED;
+    g.units = static_cast<int>(units);
+    if (workers > units) workers = units;
+    g.workers = static_cast<int>(workers);
+    const int64_t blocks = base * workers;
+    if (blocks >= (1LL << 22)) return SLAYER_EUNSUPPORTED;
+    g.byOGroups = make_fastdiv(static_cast<uint32_t>(g.oGroups));
+    g.byGroups = make_fastdiv(static_cast<uint32_t>(s.groups));
+    g.bySteps = make_fastdiv(static_cast<uint32_t>(g.steps));
+    g.byStrips = make_fastdiv(static_cast<uint32_t>(g.strips));
+    g.bySegs = make_fastdiv(static_cast<uint32_t>(g.segs));
+    const unsigned nb = static_cast<unsigned>(blocks);
+    if (P == 1) return TW == 2 ? launch_ring_one<1, 2, 1, BACKWARD>(g, nb, st) : launch_ring_one<1, 1, 1, BACKWARD>(g, nb, st);
+    if (NT == 1) return launch_ring_one<2, 1, 1, BACKWARD>(g, nb, st);
+    if (NT == 2) return launch_ring_one<2, 1, 2, BACKWARD>(g, nb, st);
+    return launch_ring_one<2, 1, 4, BACKWARD>(g, nb, st);
+}
+
+template int launch_gather_ring<false>(const RingGeom &, hipStream_t);
+template int launch_gather_ring<true>(const RingGeom &, hipStream_t);
+
+}  // namespace slayer

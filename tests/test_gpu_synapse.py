@@ -949,3 +949,38 @@ def test_dense_layer_with_few_outputs_keeps_what_torch_does_with_a_product(O, T)
         assert torch.allclose(many[1], 2 * many[0], rtol=1e-4, atol=1e-3)
         with torch.autocast("cuda", dtype=torch.float16):
             assert fc(x).dtype == torch.float16
+
+
+@pytest.mark.parametrize("N,C,O,groups,H,W,T,pad,spikes", [
+    (70, 16, 32, 1, 3, 9, 40, 1, False), (70, 16, 32, 1, 3, 9, 40, 1, True), (100, 16, 16, 1, 2, 3, 33, 1, False),
+    (35, 32, 96, 2, 4, 17, 65, 2, False), (2, 32, 16, 1, 1, 4, 32, 1, False), (3, 32, 32, 1, 5, 7, 100, 0, False),
+    (2, 32, 80, 1, 6, 5, 173, 3, True), (1, 64, 32, 2, 19, 6, 300, 1, False), (40, 16, 48, 1, 7, 8, 173, 1, False)])
+def test_gathers_with_the_source_rows_in_a_ring(N, C, O, groups, H, W, T, pad, spikes):
+    """3x3 filters with 16 or 32 source channels per group: strips that end within the image and beyond it, one row, segments
+    of a column, one unit per work-group and several, rows that are no whole vectors, paddings up to the filter's extent,
+    tiles of channels that are partly there.  Forward pass and input gradient within SUM_TOL of the sum of their terms'
+    magnitudes, the latter also of a tensor with an infinity, which reaches what it reaches in a sum."""
+    import torch.nn.functional as F
+    from slayerpytorch_amd import synapse as S
+    gen = torch.Generator().manual_seed(N + C + O + H + W + T)
+    x = (torch.rand((N, C, H, W, T), generator=gen) < 0.1).float() if spikes else torch.randn((N, C, H, W, T), generator=gen)
+    w = torch.randn((O, C // groups, 3, 3), generator=gen)
+    pads = (pad, pad, 0)
+    xd, wd = x.double().requires_grad_(True), w.double()[..., None]
+    want, scale = F.conv3d(xd, wd, None, 1, pads, 1, groups), F.conv3d(x.double().abs(), wd.abs(), None, 1, pads, 1, groups)
+    got = S.conv(x.cuda(), w.cuda(), 1, pad, 1, groups).cpu().double()
+    assert bool(((got - want.detach()).abs() <= SUM_TOL * scale + 1e-30).all())
+    g = torch.randn(want.shape, generator=gen)
+    (wantG,) = torch.autograd.grad(want, xd, g.double())
+    xs = x.double().requires_grad_(True)
+    (scaleG,) = torch.autograd.grad(F.conv3d(xs, wd.abs(), None, 1, pads, 1, groups), xs, g.double().abs())
+    gotG = S.convGradInput(g.cuda(), w.cuda(), x.shape, 1, pad, 1, groups).cpu().double()
+    assert bool(((gotG - wantG).abs() <= SUM_TOL * scaleG + 1e-30).all())
+    n, o, a, b, t = N - 1, O - 1, want.shape[2] // 2, want.shape[3] - 1, T - 1
+    g[n, o, a, b, t] = float("inf")
+    gotG = S.convGradInput(g.cuda(), w.cuda(), x.shape, 1, pad, 1, groups).cpu()
+    reached = torch.zeros(x.shape, dtype=torch.bool)
+    first = (groups - 1) * (C // groups)
+    reached[n, first:, max(0, a - pad):a - pad + 3, max(0, b - pad):b - pad + 3, t] = True
+    assert torch.equal(~torch.isfinite(gotG), reached)
+    assert bool(((gotG.double() - wantG).abs() <= SUM_TOL * scaleG + 1e-30)[~reached].all())
