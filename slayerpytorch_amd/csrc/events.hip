@@ -56,7 +56,9 @@ __device__ __forceinline__ void bin_event(float *tensor, const float *base, int 
 
 // One work-group per (sample, slice of its events).  The polarity of a sample's events is shifted so
 // that its minimum over the WHOLE sample is 0 (event.__init__, src/spikeFileIO.py:33), so every
-// work-group first scans the polarity field of all events of its sample.
+// work-group first scans the polarity field of all events of its sample - until it has seen a 0, below which there is
+// nothing, mostly among the first 256.  One event per lane: the events of a batch are few, and a launch is as long as one
+// work-group's chain of loads.  (12 samples of 5000 events on (2, 34, 34, 300): scanning all and eight events a lane 15.4 us.)
 // table[s] = {first byte of the sample in `bytes`, number of events, time shift in bins}.
 template <int FORMAT>
 __global__ __launch_bounds__(256) void bin_packed_events_kernel(float *tensor, const float *base,
@@ -73,9 +75,10 @@ __global__ __launch_bounds__(256) void bin_packed_events_kernel(float *tensor, c
     if (first < 0 || nEvents < 0 || nEvents > (nBytes - first) / kBytes || first > nBytes) return;
 
     int pmin = 255;
-    for (int64_t e = threadIdx.x; e < nEvents; e += 256) {
-        const int p = FORMAT == 3 ? ev[e * kBytes + 3] : (ev[e * kBytes + 2] >> 7);
-        pmin = min(pmin, p);
+    for (int64_t e0 = 0; e0 < nEvents; e0 += 256) {
+        const int64_t e = e0 + threadIdx.x;
+        if (e < nEvents) pmin = min(pmin, static_cast<int>(FORMAT == 3 ? ev[e * kBytes + 3] : (ev[e * kBytes + 2] >> 7)));
+        if (__syncthreads_or(pmin == 0)) break;
     }
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) pmin = min(pmin, __shfl_xor(pmin, off, kWave));
@@ -129,9 +132,10 @@ extern "C" int slayer_bin_packed_events_f32(float *tensor, const float *base, co
     if (!tensor || !bytes || !sampleTable) return SLAYER_EINVAL;
     if (mode == 1 && (!base || base == tensor)) return SLAYER_EINVAL;
     if (!base) base = tensor;
-    // slices per sample: about 2048 events per work-group
-    int64_t slices = ceil_div(maxEvents, 2048);
-    if (slices > 1024) slices = 1024;
+    // slices per sample: one event per lane up to 4096 work-groups
+    int64_t slices = ceil_div(maxEvents, 256);
+    const int64_t most = ceil_div(4096, nSamples);
+    if (slices > most) slices = most;
     if (nSamples * slices >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
     const dim3 grid(static_cast<unsigned>(nSamples * slices));
     hipStream_t st = static_cast<hipStream_t>(stream);
