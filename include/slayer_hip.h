@@ -176,6 +176,17 @@ int slayer_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradOut, const
                                       float tau, float scale, float Ts, void *stream);
 
 /*
+ * The same where the gradient is that of a pooling layer (slayer_pool_grad_input_f32 of gradPooled [planes][OH][OW][T] with
+ * weight [KH][KW], planes = N * C) which the neuron's spikes, u, gradIn [planes][H][W][T], went to: spread over the windows
+ * on the way in.  Also SLAYER_EUNSUPPORTED where slayer_corr_f32 would take the rows as whole tiles (at most 304 samples, whole
+ * vectors of an odd number), and for extents of 2^15 or more: the two calls then.
+ */
+int slayer_pool_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradPooled, const float *weight, const float *u,
+                                           const float *filt, int64_t planes, int64_t H, int64_t W, int64_t T, int64_t KH,
+                                           int64_t KW, int64_t F, int64_t delaySteps, float theta, float tau, float scale,
+                                           float Ts, void *stream);
+
+/*
  * PSP filter followed by the spike function in one kernel, for layers that apply them back to
  * back: spike(psp(x)), the ordering of the reference's MLP example
  * (example/02_NMNIST_MLP/nmnistMLP.py:59-60).  Replaces the call pair slayerCuda.conv

@@ -54,6 +54,8 @@ SIGNATURES = {
                                                  _stream]),
     "slayer_spike_bwd_delayed_corr_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _f32, _f32,
                                                          _f32, _f32, _stream]),
+    "slayer_pool_spike_bwd_delayed_corr_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _f32p, _i64, _i64, _i64, _i64, _i64,
+                                                              _i64, _i64, _i64, _f32, _f32, _f32, _f32, _stream]),
     "slayer_get_spikes_delayed_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _f32, _f32, _i64, _i64, _i64,
                                                      _f32, _f32, _stream]),
     "slayer_spike_bwd_delayed_f32": (ctypes.c_int, [_f32p, _f32p, _f32p, _f32p, _i64, _f32, _f32, _i64, _i64, _f32,

@@ -670,3 +670,24 @@ extern "C" int slayer_spike_bwd_delayed_corr_f32(float *gradIn, const float *gra
         return SLAYER_EUNSUPPORTED;
     return slayer::launch_status();
 }
+
+extern "C" int slayer_pool_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradPooled, const float *weight, const float *u,
+                                                      const float *filt, int64_t planes, int64_t H, int64_t W, int64_t T,
+                                                      int64_t KH, int64_t KW, int64_t F, int64_t delaySteps, float theta,
+                                                      float tau, float scale, float Ts, void *stream)
+{
+    if (tau == 0.0f || planes < 0 || H < 0 || W < 0 || T < 0 || KH < 1 || KW < 1 || F < 0 || delaySteps < 0) return SLAYER_EINVAL;
+    if (planes == 0 || H == 0 || W == 0 || T == 0) return SLAYER_OK;
+    if (H >= (1 << 15) || W >= (1 << 15) || KH > H + 1 || KW > W + 1 || planes >= (1LL << 31) / (H * W)) return SLAYER_EUNSUPPORTED;
+    const int64_t OH = (H + H % KH) / KH, OW = (W + W % KW) / KW;
+    if (OH < 1 || OW < 1) return SLAYER_EUNSUPPORTED;
+    if (!gradIn || !gradPooled || !weight || !u || (F > 0 && !filt)) return SLAYER_EINVAL;
+    if (slayer::generic_forced()) return SLAYER_EUNSUPPORTED;
+    const slayer::FirGate gate{u, theta, tau, scale / tau};
+    const slayer::FirPool pool{weight, static_cast<int>(H), static_cast<int>(W), static_cast<int>(OH), static_cast<int>(OW),
+                               static_cast<int>(KH), static_cast<int>(KW)};
+    if (!slayer::launch_fir_corr_walk(gradIn, gradPooled, filt, planes * H * W, T, F, delaySteps, Ts, gate,
+                                      static_cast<hipStream_t>(stream), pool))
+        return SLAYER_EUNSUPPORTED;
+    return slayer::launch_status();
+}

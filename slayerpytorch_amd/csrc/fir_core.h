@@ -14,6 +14,13 @@ struct FirGate {
     float theta, tau, gain;
 };
 
+// The input rows are those of a pooled tensor (w == nullptr: they are not): row (plane, y, x) of planes of H x W rows takes its
+// samples, times w[y % KH][x % KW], from row (plane, y / KH, x / KW) of planes of OH x OW rows.
+struct FirPool {
+    const float *w;
+    int H, W, OH, OW, KH, KW;
+};
+
 // Matrix-core correlation (fir_mfma.hip).  Returns false, launching nothing, for shapes it does not serve; with
 // chainBits, rows that are not whole aligned vectors are among those.
 bool launch_fir_corr_mfma(float *out, const float *in, const float *filt, int64_t rows, int64_t T, int64_t F, float Ts,
@@ -21,7 +28,7 @@ bool launch_fir_corr_mfma(float *out, const float *in, const float *filt, int64_
 
 // ... and its kernel for rows of any length and alignment, whose samples are in[t + shift] (zero from T on).
 bool launch_fir_corr_walk(float *out, const float *in, const float *filt, int64_t rows, int64_t T, int64_t F, int64_t shift,
-                          float Ts, const FirGate &gate, hipStream_t stream);
+                          float Ts, const FirGate &gate, hipStream_t stream, const FirPool &pool = FirPool{});
 
 // Filter lengths that the matrix-core paths serve (the correlation kernel of fir_mfma.hip and the dense tiles of
 // the tiled kernel of fir.hip).

@@ -392,6 +392,9 @@ class _poolLayer(nn.Conv3d):
             origin = _fresh_psp_of_spikes(input, kH, kW)
             if origin is not None:
                 return _poolOfPspFunction.apply(input, origin[0], weight.contiguous(), *origin[1:])
+            node = _takes_pooled_gradients(input)
+            if node is not None:
+                return _poolOfSpikesFunction.apply(input, weight.contiguous(), node)
             if ragged:
                 return synapse.synapsePool(input, weight)
         if ragged:
@@ -729,6 +732,58 @@ class _poolOfPspFunction(Function):
         grad = synapse.poolGradInput(filtered, weight, membranePotential.shape, membranePotential, ctx.theta,
                                      ctx.pdfTimeConstant, ctx.pdfScale)
         return (None, grad) + (None,) * 7
+
+
+def _takes_pooled_gradients(spikes):
+    """The node behind ``spikes`` when it is a neuron whose backward pass takes the gradient of a pooling layer as it is, still
+    pooled (``PooledGradients``), and these are its own output, untouched, with the graph being recorded - else None."""
+    node = spikes.grad_fn if PAIR_SPIKE_PSP else None
+    if not isinstance(getattr(node, "pooled", None), PooledGradients) or not torch.is_grad_enabled() or spikes._version != 0 \
+            or not _unobserved(spikes) or not spikes.is_contiguous():
+        return None
+    return node
+
+
+class PooledGradients:
+    """Gradients that pooling layers leave for the node of the neuron whose spikes they took, which runs after them in the
+    same backward pass (it is what their own edges lead to)."""
+
+    def __init__(self):
+        self._left = {}     # by backward pass: a pass that was broken off leaves nothing for another one
+
+    def leave(self, gradOutput, weight, shape):
+        stream = torch.cuda.current_stream(gradOutput.device)
+        self._left.setdefault(torch._C._current_graph_task_id(), []).append((gradOutput, weight, shape, stream))
+
+    def take(self):
+        """[(gradOutput, weight, shape of the spikes), ...], fit for use on the current stream."""
+        left = self._left.pop(torch._C._current_graph_task_id(), [])
+        for gradOutput, weight, shape, stream in left:
+            current = torch.cuda.current_stream(gradOutput.device)
+            if current != stream:
+                current.wait_stream(stream)
+                gradOutput.record_stream(current)
+        return [entry[:3] for entry in left]
+
+
+class _poolOfSpikesFunction(Function):
+    """The pooling layer of spikes whose neuron takes pooled gradients.  Where the spikes are still held by someone when the
+    backward pass runs, who may ask for their gradient, they get it."""
+
+    @staticmethod
+    def forward(ctx, spikes, weight, node):
+        ctx.save_for_backward(weight)
+        ctx.spikes, ctx.shape, ctx.node = TensorWeakRef(spikes), tuple(spikes.shape), node
+        return synapse.pool(spikes, weight)
+
+    @staticmethod
+    def backward(ctx, gradOutput):
+        (weight,) = ctx.saved_tensors
+        gradOutput = gradOutput.contiguous()
+        if ctx.spikes() is not None:
+            return synapse.poolGradInput(gradOutput, weight, ctx.shape), None, None
+        ctx.node.pooled.leave(gradOutput, weight, ctx.shape)
+        return None, None, None
 
 
 class _spikePspFunction(Function):

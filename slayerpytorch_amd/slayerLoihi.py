@@ -9,7 +9,7 @@ src/quantizeParams.py).
 import numpy as np
 import torch
 
-from . import slayer, slayerCuda, slayerLoihiCuda
+from . import slayer, slayerCuda, slayerLoihiCuda, synapse
 from ._function import Function
 
 
@@ -154,6 +154,8 @@ class _spike(Function):
             spike = spike / scale
         if needVoltage:
             ctx.save_for_backward(voltage, srmKernel.clone().detach())
+            ctx.pooled = slayer.PooledGradients()
+        ctx.set_materialize_grads(False)   # a pooling layer's gradient comes by another way
         ctx.theta = float(neuron["theta"])
         ctx.pdfTimeConstant = float(neuron["tauRho"] * neuron["theta"])
         ctx.pdfScale = float(neuron["scaleRho"])
@@ -163,7 +165,19 @@ class _spike(Function):
 
     @staticmethod
     def backward(ctx, gradOutput):
+        pooled = ctx.pooled.take()
+        if gradOutput is None and not pooled:
+            return None, None, None, None, None
         voltage, srmKernel = ctx.saved_tensors
+        if gradOutput is None and len(pooled) == 1:
+            # the gradient of one pooling layer alone: spread over its windows by the kernel below, as well
+            grad = synapse.poolSpikeBackwardDelayedCorr(pooled[0][0], pooled[0][1], voltage, srmKernel, ctx.delaySteps, ctx.theta,
+                                                        ctx.pdfTimeConstant, ctx.pdfScale, ctx.Ts)
+            if grad is not None:
+                return grad, None, None, None, None
+        for gradPooled, weight, shape in pooled:
+            spread = synapse.poolGradInput(gradPooled, weight, shape)
+            gradOutput = spread if gradOutput is None else gradOutput + spread
         # surrogate gradient and correlation with the PSP kernel in one kernel, which also moves the gradient back by
         # as many samples as the spikes left late
         return slayerCuda.spikeBackwardDelayedCorr(gradOutput.contiguous(), voltage, srmKernel, ctx.delaySteps, ctx.theta,

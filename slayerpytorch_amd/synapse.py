@@ -315,6 +315,29 @@ def poolGradInput(gradOutput, weight, inShape, membranePotential=None, theta=0.0
     return gradIn
 
 
+def poolSpikeBackwardDelayedCorr(gradOutput, weight, membranePotential, filter, delaySteps, theta, tau, scale, Ts):
+    """``slayerCuda.spikeBackwardDelayedCorr(poolGradInput(gradOutput, weight, membranePotential.shape), membranePotential,
+    filter, delaySteps, ...)`` in one kernel, or ``None`` for rows and extents that it does not serve (nothing was launched)."""
+    for x, name in ((gradOutput, "gradOutput"), (membranePotential, "membranePotential"), (filter, "filter")):
+        _check_input(x, name)
+        _check_device(gradOutput, x, "gradOutput", name)
+    _check_window(weight)
+    _check_device(gradOutput, weight, "gradOutput", "weight")
+    N, C, H, W, T = membranePotential.shape
+    if tuple(gradOutput.shape) != (N, C) + _windows(membranePotential.shape, weight.shape) + (T,):
+        raise RuntimeError("gradOutput has shape %r, which is not that of the pooled %r" % (tuple(gradOutput.shape), (N, C, H, W, T)))
+    lib = _lib.load()
+    gradIn = torch.empty_like(membranePotential)
+    with _on_device_of(gradOutput) as stream:
+        status = lib.slayer_pool_spike_bwd_delayed_corr_f32(
+            _ptr(gradIn), _ptr(gradOutput), _ptr(weight), _ptr(membranePotential), _ptr(filter), N * C, H, W, T, weight.shape[2],
+            weight.shape[3], filter.numel(), int(delaySteps), theta, tau, scale, Ts, stream)
+    if status == 2:
+        return None
+    _lib.check(status, "slayer_pool_spike_bwd_delayed_corr_f32")
+    return gradIn
+
+
 class _synapsePoolFunction(Function):
     @staticmethod
     def forward(ctx, input, weight):

@@ -661,6 +661,59 @@ def test_loihi_fused_delay_uses_the_shift_kernels_quotient(delay, delayTs):
     assert float(plain.sum()) > 0
 
 
+@pytest.mark.parametrize("C,H,W,T,window,delay", [(3, 8, 8, 310, 2, 1), (2, 7, 9, 173, 2, 1), (1, 5, 6, 64, (2, 3), 0), (4, 3, 2, 33, 2, 5),
+                                                  (2, 10, 7, 40, 3, 2), (2, 4, 4, 300, 2, 1), (2, 4, 4, 12, 2, 1)])
+def test_loihi_neuron_takes_the_gradient_of_a_pooling_layer_as_it_is(C, H, W, T, window, delay, monkeypatch):
+    """pool(spikeLoihi(x)): the neuron's backward kernel spreads the pooled gradient over the windows on the way in.  The same
+    bits as through the pooling layer's own gradient where the kernel sums over rows as they come; also with a second user of
+    the spikes, a backward pass that is run twice, one that runs on another stream, spikes that are still held, and an infinity."""
+    from slayerpytorch_amd import slayer as slayer_module
+    layer = snn.loihi(loihi_neuron(), {"Ts": 1, "tSample": T}).to(DEV)
+    pool = layer.pool(window).to(DEV)
+    with torch.no_grad():
+        pool.weight.mul_(torch.arange(1, 1 + pool.weight.numel(), device=DEV).reshape(pool.weight.shape) / 2.0)
+    rng = np.random.default_rng(C + H + W + T)
+    x0 = dev((2 * rng.integers(-128, 128, (2, C, H, W, T)) * (rng.random((2, C, H, W, T)) < 0.3)).astype(np.float32))
+    KH, KW = pool.kernel_size[0], pool.kernel_size[1]
+    g = dev(rng.standard_normal((2, C, (H + H % KH) // KH, (W + W % KW) // KW, T)).astype(np.float32))
+    more = dev(rng.standard_normal(x0.shape).astype(np.float32))
+
+    def run(pair, how, g=g):
+        monkeypatch.setattr(slayer_module, "PAIR_SPIKE_PSP", pair)
+        x = x0.clone().requires_grad_(True)
+        s = layer.spikeLoihi(x * 1.0, delay=delay)
+        y = pool(s)
+        name = type(y.grad_fn).__name__
+        wanted = [x, s] if how == "held" else [x]
+        out = (y * g).sum() + ((s * more).sum() if how == "both" else 0.0)
+        del s
+        if how == "twice":
+            torch.autograd.grad(out, wanted, retain_graph=True)
+        return name, y.detach(), torch.autograd.grad(out, wanted)
+
+    for how in ("once", "both", "twice", "held"):
+        (_, y0, ref), (name, y1, got) = run(False, how), run(True, how)
+        assert name == "_poolOfSpikesFunctionBackward" and torch.equal(y0, y1)
+        assert len(ref) == len(got) and all(torch.equal(a, b) for a, b in zip(ref, got)), how
+    bad = g.clone()
+    bad[1, C - 1, 0, 0, T // 2] = float("inf")
+    ref, got = run(False, "once", bad)[2][0], run(True, "once", bad)[2][0]
+    assert torch.equal(torch.isfinite(ref), torch.isfinite(got)) and rel_err(host(got.nan_to_num(0, 0, 0)), host(ref.nan_to_num(0, 0, 0))) <= REL_TOL
+    monkeypatch.setattr(slayer_module, "PAIR_SPIKE_PSP", True)
+    x = x0.clone().requires_grad_(True)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    s = layer.spikeLoihi(x * 1.0, delay=delay)
+    with torch.cuda.stream(side):
+        side.wait_stream(torch.cuda.default_stream())
+        y = pool(s)
+        del s
+        gs = g * 1.0
+    torch.cuda.current_stream().wait_stream(side)
+    (got,) = torch.autograd.grad(y, x, gs)
+    assert torch.equal(got, run(False, "once")[2][0])
+
+
 def test_loihi_delay_per_neuron_or_tensor_takes_the_separate_shift():
     layer = snn.loihi(loihi_neuron(scaleRho=2.0), {"Ts": 1.0, "tSample": 120}).to(DEV)
     rng = np.random.default_rng(14)
