@@ -2519,6 +2519,15 @@ static void launch_wgrad_taps(const WgradArgs &g, const WgradPlan &p, unsigned b
     }
 }
 
+// Whether the weight gradient goes by the walk with the source rows in a ring, and its geometry.
+static bool wgrad_takes_ring(const SynGeom &s, const float *gradOut, const float *in, RingGeom &ring)
+{
+    if (s.KH != 3 || s.KW != 3 || s.sH != 1 || s.sW != 1 || s.dH != 1 || s.dW != 1 || s.T < 1) return false;
+    ring = RingGeom{in, nullptr, const_cast<float *>(gradOut), s.N, s.C, s.H, s.W, s.O, s.OH, s.OW, s.T, s.groups, s.C / s.groups,
+                    s.O / s.groups, s.C / s.groups, s.O / s.groups, s.pH, s.pW};
+    return ring_wgrad_rows(ring) > 0;
+}
+
 // ---- pooling -----------------------------------------------------------------------------------------
 // Geometry of a pooling layer as a one-channel synapse: the channels of a batch item as rows of one image where windows do
 // not straddle them, else one image per channel, whose last windows reach past it (KH and KW rows and columns of zeros
@@ -2597,6 +2606,8 @@ extern "C" int64_t slayer_synapse_conv_grad_weight_workspace_bytes(const slayer_
     if (m.use && m.slices > most) most = m.slices;
     int64_t rows = static_cast<int64_t>(s.N) * most;
     if (l.use && l.slices > rows) rows = l.slices;
+    RingGeom ring;
+    if (wgrad_takes_ring(s, nullptr, nullptr, ring) && ring_wgrad_rows(ring) > rows) rows = ring_wgrad_rows(ring);
     return rows * nW * static_cast<int64_t>(sizeof(float));
 }
 
@@ -2624,6 +2635,13 @@ extern "C" int slayer_synapse_conv_grad_weight_f32(float *gradW, const float *gr
         const bool vec = vecT && aligned16(gradOut) && aligned16(in);
         const MfmaPlan m = plan_wgrad_mfma(s);
         const LdsPlan l = plan_wgrad_lds(s, m);
+        RingGeom ring;
+        if (wgrad_takes_ring(s, gradOut, in, ring) && !generic_forced()) {
+            const int launched = launch_wgrad_ring(ring, workspace, st);
+            if (launched != SLAYER_OK) return launched;
+            launch_wgrad_sum<true>(gradW, workspace, ring_wgrad_rows(ring), nW, WgradAgain{gradOut, in, s}, st);
+            return launch_status();
+        }
         if ((l.use || (m.use && vec)) && !generic_forced()) {
             rows = l.use ? launch_wgrad_lds(gradOut, in, workspace, s, m, l, nW, st)
                          : launch_wgrad_mfma(gradOut, in, workspace, s, m, nW, st);

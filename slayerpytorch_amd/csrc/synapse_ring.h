@@ -18,6 +18,11 @@ struct RingGeom {
 // 16 destination channels per group, rows of whole vectors or at least 32 samples.
 template <bool BACKWARD> int launch_gather_ring(const RingGeom &s, hipStream_t st);
 
+// The weight gradient of the same geometry, src the input [N][SC][SH][SW][T], dst (read) the output gradient: rows of partial
+// sums [Og groups][Cg][9] in `workspace`, ring_wgrad_rows() of them (0: not a geometry for it), to be added up.
+int ring_wgrad_rows(const RingGeom &s);
+int launch_wgrad_ring(const RingGeom &s, float *workspace, hipStream_t st);
+
 }  // namespace slayer
 
 #endif

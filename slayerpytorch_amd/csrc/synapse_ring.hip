@@ -412,6 +412,345 @@ int launch_gather_ring(const RingGeom &s, hipStream_t st)
     return launch_ring_one<2, 1, 4, BACKWARD>(g, nb, st);
 }
 
+// ---- weight gradient ---------------------------------------------------------------------------------
+// gradW[o][c][i][j] = sum over n, a, b, t of gradOut[n][o][a][b][t] in[n][c][a - padH + i][b - padW + j][t]: the same walk with
+// time as the reduction axis.  A position in LDS is three planes of 16 channels x 32 samples, time innermost: an operand of tap
+// (i, j) is the position that the tap reads under a pixel, 16 channels at once, one 16-byte read per plane and lane.  A
+// multiplying wavefront has 16 source channels and two pixels of the strip; it takes a pixel's gradients straight from memory,
+// a row ahead, splits them once and multiplies them with the nine positions.  The wavefronts' sums meet in LDS at the end.
+// The kernel with the patch of four pixels in LDS splits a sample once per tap and tile of columns, and loads it up to nine
+// times.  Full samples, spikes: 16 -> 32 channels of 16 x 16, (64, 300): 592, 442 -> 368, 256 us, (12, 300): 118, 81 -> 74, 60;
+// 32 -> 64 channels of 8 x 8, (64, 300): 432, 289 -> 318, 240; 16 -> 16 of 16 x 16, (32, 300): 168, 125 -> 110, 88.  Spikes are
+// near the memory (4 TB/s); full samples are held by the products (148 us at 2.1 GHz) and, in the same wavefronts, the splits
+// of the gradients.  Splitting beside the products of the pixel before needs 24 registers more than there are: 634 us.
+template <int P, int OT>
+__global__ __launch_bounds__(512) void synapse_wgrad_ring_kernel(RingArgs g, float *__restrict__ partial, int nW)
+{
+    constexpr int PX = ring_pixels(P), WX = PX + 2, SLOT = ring_slot(P);
+    constexpr int PIXELS = PX * P / kRgMul;            // of a multiplying wavefront
+    constexpr int CELLS = WX * P, TASKS = (CELLS + kRgStage - 1) / kRgStage;
+    extern __shared__ __align__(16) float lds[];
+    char *const ldsBytes = reinterpret_cast<char *>(lds);
+    typedef const uint4_ext __attribute__((address_space(3))) *LdsUint4;
+    const uint32_t ldsBase = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char *)ldsBytes));
+    const RingGeom &s = g.s;
+
+    uint32_t rest = xcd_contiguous(blockIdx.x, gridDim.x), qq = fastdiv(rest, g.byOGroups);
+    const int og = static_cast<int>(rest - qq * g.byOGroups.d);
+    rest = qq; qq = fastdiv(rest, g.byGroups);
+    const int grp = static_cast<int>(rest - qq * g.byGroups.d), worker = static_cast<int>(qq);
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, h = lane >> 4;
+    const int64_t srcPlane = static_cast<int64_t>(s.SH) * s.SW * s.T, dstPlane = static_cast<int64_t>(s.DH) * s.DW * s.T;
+    const int planeBytes = static_cast<int>(srcPlane) * 4, rowBytes = s.SW * s.T * 4, pixBytes = s.T * 4;
+    uint32_t *const flags = reinterpret_cast<uint32_t *>(ldsBytes + kRgSlots * SLOT);   // [slot][staging wavefront]
+
+    struct Place {
+        int unit, row, n, t0, skip, x0, a0, rows;      // skip: samples of the step that the one before has, too
+    };
+    auto decode = [&](Place &p) {
+        const uint32_t v = static_cast<uint32_t>(min(p.unit, g.units - 1));
+        const uint32_t q = fastdiv(v, g.bySteps), q2 = fastdiv(q, g.byStrips), q3 = fastdiv(q2, g.bySegs);
+        const int t = static_cast<int>(v - q * g.bySteps.d) << 5;
+        p.t0 = min(t, g.tLast);
+        p.skip = t - p.t0;
+        p.x0 = static_cast<int>(q - q2 * g.byStrips.d) * PX;
+        p.a0 = static_cast<int>(q2 - q3 * g.bySegs.d) * g.segRows;
+        p.n = static_cast<int>(q3);
+        p.rows = min(g.segRows, s.DH - p.a0) + 2;
+    };
+    auto advance = [&](Place &p) {
+        if (++p.row == p.rows) {
+            p.row = 0;
+            p.unit += g.workers;
+            decode(p);
+        }
+    };
+    Place at{worker, 0, 0, 0, 0, 0, 0, 0};
+    decode(at);
+    int trips = 0;
+    for (Place p = at; p.unit < g.units;) {
+        trips += p.rows;
+        p.unit += g.workers;
+        decode(p);
+    }
+
+    f32x4 acc[OT][9];
+#pragma unroll
+    for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+        for (int ij = 0; ij < 9; ++ij) acc[ot][ij] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int pass = wave % P, pixel0 = (wave % kRgMul) / P * PIXELS;   // of a multiplying wavefront
+
+    if (wave >= kRgMul) {
+        // ---- staging, as in the gather; a lane samples 8 oct .. + 7 of channel `channel`
+        const int stager = wave - kRgMul, channel = lane >> 2, oct = lane & 3;
+        int cell[TASKS], cellX[TASKS], cellBytes[TASKS];
+#pragma unroll
+        for (int i = 0; i < TASKS; ++i) {
+            cell[i] = stager + kRgStage * i < CELLS ? stager + kRgStage * i : stager;
+            const int of = cell[i] / WX;
+            cellX[i] = cell[i] - of * WX;
+            cellBytes[i] = (of * 16 + channel) * planeBytes + oct * 32;
+        }
+        typedef float4 Row[TASKS][2];
+        auto issue = [&](Row &R, const Place &p) {
+            const BufferRsrc src = make_buffer(s.src + (static_cast<int64_t>(p.n) * s.SC + static_cast<int64_t>(grp) * s.Qg) * srcPlane);
+            const int y = p.a0 + p.row - s.padH, x = p.x0 - s.padW;
+            const bool row = p.unit < g.units && static_cast<unsigned>(y) < static_cast<unsigned>(s.SH);
+#pragma unroll
+            for (int i = 0; i < TASKS; ++i) {
+                const bool ok = row && static_cast<unsigned>(x + cellX[i]) < static_cast<unsigned>(s.SW);
+                const int from = cellBytes[i] + y * rowBytes + (x + cellX[i]) * pixBytes + p.t0 * 4;
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    R[i][q] = buffer_load4<0>(src, masked_offset(ok && p.t0 + oct * 8 + q * 4 < s.T, from + q * 16), 0);
+            }
+        };
+        int slot = 0;
+        auto stage = [&](const Row &R) {
+            uint32_t low = 0;
+#pragma unroll
+            for (int i = 0; i < TASKS; ++i) {
+                const float v[8] = {R[i][0].x, R[i][0].y, R[i][0].z, R[i][0].w, R[i][1].x, R[i][1].y, R[i][1].z, R[i][1].w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) low |= __builtin_bit_cast(uint32_t, v[e]);
+                const SplitPlanes sp = split_bf16<false>(v);
+                uint4_ext *to = reinterpret_cast<uint4_ext *>(ldsBytes + slot * SLOT + cell[i] * kRgPos) + lane;
+                to[0] = sp.hi;
+                to[64] = sp.mid;
+                to[128] = sp.lo;
+            }
+            const bool any = __builtin_amdgcn_ballot_w64((low & 0xffffu) != 0u) != 0;
+            if (lane == 0) flags[slot * kRgStage + stager] = any ? 1u : 0u;
+            slot = (slot + 1) & (kRgSlots - 1);
+        };
+        Row RA, RB;
+        issue(RB, at);
+        advance(at);
+        issue(RA, at);
+        stage(RB);
+        advance(at);
+        issue(RB, at);
+        __syncthreads();
+#pragma nounroll
+        for (int k = 0; k < trips; k += 2) {
+            stage(RA);
+            advance(at);
+            issue(RA, at);
+            __syncthreads();
+            stage(RB);
+            advance(at);
+            issue(RB, at);
+            __syncthreads();
+        }
+    } else {
+        // ---- multiplying: lane (r, h) has channel r of a position and output channel r of a tile, samples 8 h .. + 7
+        int oOff[OT];
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot) {
+            const int o = (og * OT + ot) * 16 + r;
+            oOff[ot] = masked_offset(o < s.Mg, o * static_cast<int>(dstPlane) * 4 + h * 32);
+        }
+        float4 G[PIXELS][OT][2];
+        auto issue = [&](float4 (&to)[OT][2], int c, const Place &p) {   // the gradients under the place's window
+            const BufferRsrc src = make_buffer(s.dst + (static_cast<int64_t>(p.n) * s.DC + static_cast<int64_t>(grp) * s.Mg) * dstPlane);
+            const int a = p.a0 + p.row - 2, b = p.x0 + pixel0 + c, from = (a * s.DW + b) * pixBytes + p.t0 * 4;
+            const bool row = p.row >= 2 && p.unit < g.units && b < s.DW;
+#pragma unroll
+            for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const bool ok = row && oOff[ot] != kOutOfRange && p.t0 + h * 8 + q * 4 < s.T;
+                    int off = ok ? oOff[ot] + from + q * 16 : kOutOfRange;
+                    asm volatile("" : "+v"(off));      // (no branch around a load)
+                    to[ot][q] = buffer_load4<0>(src, off, 0);
+                }
+        };
+        const uint32_t base = ldsBase + r * 64 + h * 16 + (pass * WX + pixel0) * kRgPos;
+        int slot = 0;
+        // the nine taps of one pixel.  The products of a step start from zero, the leading ones apart from the small ones, and
+        // the vector ALU, which rounds, adds them to the sums - those of the tap before, beside the products of this one.
+        auto multiply = [&](const SplitPlanes (&gp)[OT], const uint32_t (&from)[3], auto partsTag) {
+            constexpr int PARTS = decltype(partsTag)::value;
+            uint4_ext x[2][PARTS];
+            f32x4 lead[2][OT], rest[2][OT];
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            auto fetch = [&](int set, int k) {
+#pragma unroll
+                for (int part = 0; part < PARTS; ++part)
+                    x[set][part] = *reinterpret_cast<LdsUint4>(static_cast<size_t>(from[k / 3] + k % 3 * kRgPos + part * 1024));
+            };
+            fetch(0, 0);
+#pragma unroll
+            for (int k = 0; k <= 9; ++k) {
+                const int set = k & 1;
+                if (k + 1 < 9) fetch(set ^ 1, k + 1);
+                if (k < 9) {
+#define SLAYER_RING_MUL(TO, GP, XP, FROM) \
+    _Pragma("unroll") for (int ot = 0; ot < OT; ++ot) TO[set][ot] = mfma_bf16(gp[ot].GP, x[set][XP], FROM);
+                    SLAYER_RING_MUL(rest, lo, 0, zero)
+                    SLAYER_RING_MUL(lead, hi, 0, zero)
+                    if constexpr (PARTS == 3) {
+                        SLAYER_RING_MUL(rest, hi, 2, rest[set][ot])
+                        SLAYER_RING_MUL(rest, mid, 1, rest[set][ot])
+                    }
+                    SLAYER_RING_MUL(rest, mid, 0, rest[set][ot])
+                    if constexpr (PARTS == 3) {
+                        SLAYER_RING_MUL(rest, hi, 1, rest[set][ot])
+                    }
+#undef SLAYER_RING_MUL
+                }
+                if (k > 0) {
+#pragma unroll
+                    for (int ot = 0; ot < OT; ++ot) acc[ot][k - 1] += lead[set ^ 1][ot] + rest[set ^ 1][ot];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        Place ahead = at;
+#pragma unroll
+        for (int c = 0; c < PIXELS; ++c) issue(G[c], c, ahead);
+        advance(ahead);
+        __syncthreads();
+#pragma nounroll
+        for (int k = 0; k < ((trips + 1) & ~1); ++k) {   // (the staging wavefronts take two at a time)
+            const uint32_t from[3] = {base + ((slot + 2) & (kRgSlots - 1)) * SLOT, base + ((slot + 3) & (kRgSlots - 1)) * SLOT, base + slot * SLOT};
+            const bool all = __builtin_amdgcn_ballot_w64(lane < kRgSlots * kRgStage && lane / kRgStage != ((slot + 1) & (kRgSlots - 1)) &&
+                                                         flags[lane & (kRgSlots * kRgStage - 1)] != 0u) != 0;
+            const bool work = at.row >= 2 && at.unit < g.units;
+#pragma unroll
+            for (int c = 0; c < PIXELS; ++c) {
+                SplitPlanes gp[OT];
+#pragma unroll
+                for (int ot = 0; ot < OT; ++ot) {
+                    float v[8] = {G[c][ot][0].x, G[c][ot][0].y, G[c][ot][0].z, G[c][ot][0].w,
+                                  G[c][ot][1].x, G[c][ot][1].y, G[c][ot][1].z, G[c][ot][1].w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = h * 8 + e >= at.skip ? v[e] : 0.f;
+                    gp[ot] = split_bf16<false>(v);
+                    // (here, before the registers are loaded again, and not in the branch)
+                    asm volatile("" : "+v"(gp[ot].hi), "+v"(gp[ot].mid), "+v"(gp[ot].lo));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                issue(G[c], c, ahead);
+                __builtin_amdgcn_sched_barrier(0);
+                if (work && at.x0 + pixel0 + c < s.DW) {
+                    const uint32_t under[3] = {from[0] + c * kRgPos, from[1] + c * kRgPos, from[2] + c * kRgPos};
+                    if (all) multiply(gp, under, std::integral_constant<int, 3>{});
+                    else multiply(gp, under, std::integral_constant<int, 1>{});
+                }
+            }
+            advance(ahead);
+            advance(at);
+            slot = (slot + 1) & (kRgSlots - 1);
+            __syncthreads();
+        }
+    }
+
+    // ---- the wavefronts' sums, in order; element q of a tile is output channel 4 h + q, input channel r
+    __syncthreads();
+    f32x4 *const red = reinterpret_cast<f32x4 *>(lds);
+    constexpr int TILES = OT * 9;
+    if (wave >= P && wave < kRgMul) {
+#pragma unroll
+        for (int k = 0; k < TILES; ++k) red[((wave - P) * TILES + k) * 64 + lane] = acc[k / 9][k % 9];
+    }
+    __syncthreads();
+    if (wave < P) {
+        float *row = partial + static_cast<int64_t>(worker) * nW;
+#pragma unroll
+        for (int k = 0; k < TILES; ++k) {
+            f32x4 v = acc[k / 9][k % 9];
+#pragma unroll
+            for (int w = 1; w < kRgMul / P; ++w) v += red[((w * P + wave - P) * TILES + k) * 64 + lane];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int o = (og * OT + k / 9) * 16 + 4 * h + q, c = pass * 16 + r;
+                if (o < s.Mg) row[static_cast<int64_t>(grp * s.Mg + o) * (s.Qg * 9) + c * 9 + k % 9] = v[q];
+            }
+        }
+    }
+}
+
+// Tiles and walk of the weight gradient; false where the kernel does not take the geometry.
+static bool plan_wgrad_ring(const RingGeom &s, RingArgs &g, int &P, int &OT)
+{
+    if ((s.Qg != 16 && s.Qg != 32) || s.Mg < 16 || (s.T % 4 != 0 && s.T < 32) || s.T < 1) return false;
+    P = s.Qg / 16;
+    OT = s.Mg <= 16 ? 1 : 2;
+    g = RingArgs{};
+    g.s = s;
+    g.oGroups = static_cast<int>(ceil_div(s.Mg, 16 * OT));
+    g.steps = (s.T + 31) / 32;
+    g.tLast = s.T % 4 == 0 ? (g.steps - 1) * 32 : s.T - 32;
+    g.strips = static_cast<int>(ceil_div(s.DW, ring_pixels(P)));
+    const int64_t base = static_cast<int64_t>(s.groups) * g.oGroups, columns = static_cast<int64_t>(s.N) * g.steps * g.strips;
+    int64_t workers = 256 / base;                      // (one work-group per compute unit; a number that sizes alone determine)
+    if (workers < 1) workers = 1;
+    int64_t best = 0, segs = 1;                        // as in the gather
+    for (int64_t k = 1; k <= s.DH && k <= 16; ++k) {
+        const int64_t rows = ceil_div(s.DH, k), used = ceil_div(s.DH, rows);
+        const int64_t cost = ceil_div(columns * used, workers) * (rows + 1);
+        if (best == 0 || cost < best) { best = cost; segs = k; }
+    }
+    if (s.DH < 1 || s.DW < 1 || columns < 1) return false;
+    g.segRows = static_cast<int>(ceil_div(s.DH, segs));
+    g.segs = static_cast<int>(ceil_div(s.DH, g.segRows));
+    const int64_t units = columns * g.segs;
+    if (units < 1 || units >= (1LL << 30) || base >= (1LL << 20)) return false;
+    // Work for the ring to pay: 60 steps of a pixel per compute unit.  Full samples, spikes, the kernel with the patch against
+    // this: 72 steps, 16 -> 32 channels of 17 x 17, (32, 64), 75, 72 against 66, 53 us; 96, 32 -> 96 of 16 x 16, (8, 100), 139, 97
+    // against 124, 95; 47, 16 -> 32 of 14 x 18, (8, 173), 53, 40 against 50, 42; 15, 32 -> 64 of 7 x 9, (5, 173), 38, 29
+    // against 38, 33.
+    if (static_cast<int64_t>(s.N) * g.steps * s.DH * s.DW * base < 60 * 256) return false;
+    g.units = static_cast<int>(units);
+    if (workers > units) workers = units;
+    g.workers = static_cast<int>(workers);
+    g.byOGroups = make_fastdiv(static_cast<uint32_t>(g.oGroups));
+    g.byGroups = make_fastdiv(static_cast<uint32_t>(s.groups));
+    g.bySteps = make_fastdiv(static_cast<uint32_t>(g.steps));
+    g.byStrips = make_fastdiv(static_cast<uint32_t>(g.strips));
+    g.bySegs = make_fastdiv(static_cast<uint32_t>(g.segs));
+    return true;
+}
+
+int ring_wgrad_rows(const RingGeom &s)
+{
+    RingArgs g;
+    int P, OT;
+    return plan_wgrad_ring(s, g, P, OT) ? g.workers : 0;
+}
+
+template <int P, int OT>
+static int launch_wgrad_ring_one(const RingArgs &g, float *workspace, hipStream_t st)
+{
+    static_assert(kRgSlots * ring_slot(P) >= (kRgMul - P) * OT * 9 * 1024, "the sums of three wavefronts fit the ring");
+    static std::atomic<bool> raised[64];
+    int device = 0;
+    hipError_t err = hipGetDevice(&device);
+    if (err == hipSuccess && (device < 0 || device >= 64)) err = hipErrorInvalidDevice;
+    if (err == hipSuccess && !raised[device].load(std::memory_order_acquire)) {
+        err = hipFuncSetAttribute(reinterpret_cast<const void *>(&synapse_wgrad_ring_kernel<P, OT>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, ring_lds(P));
+        if (err == hipSuccess) raised[device].store(true, std::memory_order_release);
+    }
+    if (err != hipSuccess) return note_hip_error(err);
+    const unsigned blocks = static_cast<unsigned>(g.s.groups) * g.oGroups * g.workers;
+    hipLaunchKernelGGL((synapse_wgrad_ring_kernel<P, OT>), dim3(blocks), dim3(512), ring_lds(P), st, g, workspace,
+                       g.s.groups * g.s.Mg * g.s.Qg * 9);
+    return launch_status();
+}
+
+int launch_wgrad_ring(const RingGeom &s, float *workspace, hipStream_t st)
+{
+    RingArgs g;
+    int P, OT;
+    if (!plan_wgrad_ring(s, g, P, OT)) return SLAYER_EUNSUPPORTED;
+    if (P == 1) return OT == 1 ? launch_wgrad_ring_one<1, 1>(g, workspace, st) : launch_wgrad_ring_one<1, 2>(g, workspace, st);
+    return OT == 1 ? launch_wgrad_ring_one<2, 1>(g, workspace, st) : launch_wgrad_ring_one<2, 2>(g, workspace, st);
+}
+
 template int launch_gather_ring<false>(const RingGeom &, hipStream_t);
 template int launch_gather_ring<true>(const RingGeom &, hipStream_t);
 

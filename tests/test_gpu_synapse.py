@@ -984,3 +984,34 @@ def test_gathers_with_the_source_rows_in_a_ring(N, C, O, groups, H, W, T, pad, s
     reached[n, first:, max(0, a - pad):a - pad + 3, max(0, b - pad):b - pad + 3, t] = True
     assert torch.equal(~torch.isfinite(gotG), reached)
     assert bool(((gotG.double() - wantG).abs() <= SUM_TOL * scaleG + 1e-30)[~reached].all())
+
+
+@pytest.mark.parametrize("N,C,O_,groups,H,W,T,pad", [
+    (64, 16, 16, 1, 9, 14, 33, 1), (40, 16, 48, 1, 17, 9, 64, 0), (9, 32, 80, 1, 12, 13, 173, 2), (30, 32, 32, 2, 8, 17, 65, 1),
+    (16, 32, 16, 1, 20, 5, 300, 3), (12, 64, 96, 2, 6, 9, 173, 1), (64, 16, 24, 1, 3, 41, 36, 1)])
+@pytest.mark.parametrize("kind", ["signed", "spikes"])
+def test_weight_gradient_with_the_source_rows_in_a_ring(N, C, O_, groups, H, W, T, pad, kind):
+    """3x3 filters with 16 or 32 input channels per group and work for the ring: strips that end beyond the image, segments of
+    a column, rows that are no whole vectors or no whole steps, tiles of output channels that are partly there, groups.  Error
+    as in test_weight_gradient_sums_are_rounded_and_not_cut (under 200 additions per sum).  An infinity in the gradient reaches
+    the weights of its channel and no others."""
+    rng = np.random.default_rng(H + T)
+    Cg, Og = C // groups, O_ // groups
+    x = rng.standard_normal((N, C, H, W, T)).astype(np.float32)
+    if kind == "spikes":
+        x = (np.abs(x) > 2).astype(np.float32)
+    OH, OW = H + 2 * pad - 2, W + 2 * pad - 2
+    go = rng.standard_normal((N, O_, OH, OW, T)).astype(np.float32)
+    shape = (O_, Cg, 3, 3)
+    got = host(synapse.convGradWeight(dev(go), dev(x), shape, 1, pad, 1, groups)).astype(np.float64)
+    xp = torch.nn.functional.pad(dev(x), (0, 0, pad, pad, pad, pad)).double().transpose(0, 1)
+    g = dev(go).double().transpose(0, 1).reshape(O_, -1)
+    exact = torch.cat([torch.stack([torch.stack([
+        g[k * Og:(k + 1) * Og] @ xp[k * Cg:(k + 1) * Cg, :, i:i + OH, j:j + OW].reshape(Cg, -1).t().contiguous()
+        for j in range(3)], -1) for i in range(3)], -2) for k in range(groups)]).cpu().numpy()
+    assert np.linalg.norm(got - exact) <= 2e-7 * np.linalg.norm(exact)
+    at = (N - 1, O_ - 1, OH // 2, OW // 2, T - 1)
+    assert 1 <= at[2] + 1 - pad < H - 1 and 1 <= at[3] + 1 - pad < W - 1
+    go[at] = np.inf
+    again = host(synapse.convGradWeight(dev(go), dev(x), shape, 1, pad, 1, groups)).astype(np.float64)
+    assert not np.isfinite(again[-1]).any() and np.array_equal(again[:-1], got[:-1])
