@@ -172,18 +172,31 @@ __global__ __launch_bounds__(256) void spike_loss_grad_kernel(float *__restrict_
     }
 }
 
-// loss = scale * sum of the row sums: lane l adds rows l, l+256, ... in order, then a fixed tree.
-__global__ __launch_bounds__(256) void spike_loss_sum_kernel(float *__restrict__ loss, const float *__restrict__ partial,
-                                                             int64_t rows, float scale)
+// loss = scale * sum of the row sums, in an order that the number of rows alone determines.
+__global__ __launch_bounds__(1024) void spike_loss_sum_kernel(float *__restrict__ loss, const float *__restrict__ partial,
+                                                              int64_t rows, float scale)
 {
-    __shared__ float wsum[4];
-    float acc = 0.0f;
-    for (int64_t r = threadIdx.x; r < rows; r += 256) acc += partial[r];
+    // one work-group: 1024 lanes with four sums each, so that the loads of a trip do not wait for one another (12800 rows:
+    // 256 lanes with one sum 14.2 us, this 4.7)
+    __shared__ float wsum[16];
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
+    int64_t r = threadIdx.x;
+    for (; r + 3 * 1024 < rows; r += 4 * 1024) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) part[k] += partial[r + k * 1024];
+    }
+    for (; r < rows; r += 1024) part[0] += partial[r];
+    float acc = (part[0] + part[1]) + (part[2] + part[3]);
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) acc += __shfl_down(acc, off, kWave);
     if ((threadIdx.x & (kWave - 1)) == 0) wsum[threadIdx.x / kWave] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) loss[0] = (((wsum[0] + wsum[1]) + wsum[2]) + wsum[3]) * scale;
+    if (threadIdx.x < kWave) {
+        acc = threadIdx.x < 16 ? wsum[threadIdx.x] : 0.f;
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) acc += __shfl_down(acc, off, kWave);
+        if (threadIdx.x == 0) loss[0] = acc * scale;
+    }
 }
 
 // A row and the filter must fit the LDS of one work-group (60 KB without what rounds them up), and the work-groups, one per
@@ -227,7 +240,7 @@ static int launch_loss(float *loss, float *error, const float *out, const float 
         const int status = launch_status();
         if (status != SLAYER_OK) return status;
     }
-    hipLaunchKernelGGL(spike_loss_sum_kernel, dim3(1), dim3(256), 0, st, loss, workspace, live, 0.5f * Ts);
+    hipLaunchKernelGGL(spike_loss_sum_kernel, dim3(1), dim3(1024), 0, st, loss, workspace, live, 0.5f * Ts);
     return launch_status();
 }
 

@@ -1280,6 +1280,15 @@ def test_spike_loss_and_its_gradient(T, Fl):
     assert np.array_equal(np.isfinite(got), np.isfinite(want)) and np.array_equal(got[~np.isfinite(want)], want[~np.isfinite(want)], equal_nan=True)
 
 
+@pytest.mark.parametrize("rows", [1, 63, 1023, 1024, 1025, 3072, 3073, 4096, 4097, 8193, 12800])
+def test_spike_loss_sum_over_rows(rows):
+    """The sum of the rows' losses at the edges of its trips: every row once.  The rows' numbers are whole and the largest sum
+    below 2^24, so that any order of additions is exact."""
+    d = torch.arange(rows, device="cuda").remainder(37).float().reshape(1, rows, 1, 1, 1)
+    loss, error = slayerCuda.spikeLoss(torch.zeros_like(d), d, torch.ones(1, device="cuda"), 1.0)
+    assert torch.equal(error, -d) and float(loss) == 0.5 * float(d.double().square().sum())
+
+
 @pytest.mark.parametrize("T,Fl", [(5, 3), (350, 8), (1029, 77)])
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
 def test_spike_loss_gradient_with_a_tap_that_is_not_finite(T, Fl, bad):
