@@ -58,7 +58,8 @@ __device__ __forceinline__ void bin_event(float *tensor, const float *base, int 
 // that its minimum over the WHOLE sample is 0 (event.__init__, src/spikeFileIO.py:33), so every
 // work-group first scans the polarity field of all events of its sample - until it has seen a 0, below which there is
 // nothing, mostly among the first 256.  One event per lane: the events of a batch are few, and a launch is as long as one
-// work-group's chain of loads.  (12 samples of 5000 events on (2, 34, 34, 300): scanning all and eight events a lane 15.4 us.)
+// work-group's chain of loads.  (12 samples of 5000 events on (2, 34, 34, 300): scanning all and eight events a lane 15.4 us,
+// this 6.5.)
 // table[s] = {first byte of the sample in `bytes`, number of events, time shift in bins}.
 template <int FORMAT>
 __global__ __launch_bounds__(256) void bin_packed_events_kernel(float *tensor, const float *base,
