@@ -177,8 +177,8 @@ int slayer_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradOut, const
 
 /*
  * The same where the gradient is that of a pooling layer (slayer_pool_grad_input_f32 of gradPooled [planes][OH][OW][T] with
- * weight [KH][KW], planes = N * C) which the neuron's spikes, u, gradIn [planes][H][W][T], went to: spread over the windows
- * on the way in.  Also SLAYER_EUNSUPPORTED where slayer_corr_f32 would take the rows as whole tiles (at most 304 samples, whole
+ * weight [KH][KW], planes = N * C, each pooled by itself) which the neuron's spikes, u, gradIn [planes][H][W][T], went to:
+ * spread over the windows on the way in.  Also SLAYER_EUNSUPPORTED where slayer_corr_f32 would take the rows as whole tiles (at most 304 samples, whole
  * vectors of an odd number), and for extents of 2^15 or more: the two calls then.
  */
 int slayer_pool_spike_bwd_delayed_corr_f32(float *gradIn, const float *gradPooled, const float *weight, const float *u,
@@ -411,7 +411,10 @@ int slayer_synapse_conv_grad_input_f32(float *gradIn, const float *gradOut, cons
  * Sum pooling of every channel of in [N][C][H][W][T] over windows of KH x KW pixels that do not overlap, with one
  * weight per position of the window (weight [KH][KW]): slayer_synapse_conv_f32 with strides KH and KW on the channels
  * as images of one channel each.  An extent that is no multiple of the window counts as extended by extent % window
- * rows or columns of zeros: OH = (H + H % KH) / KH, OW likewise (src/slayer.py:565-575).  out [N][C][OH][OW][T].
+ * rows or columns of zeros: OH = (H + H % KH) / KH, OW likewise.  out [N][C][OH][OW][T].  That is the pooling layer of
+ * src/slayer.py:565-575, which convolves a batch item's extended channels below one another as one image, where no window
+ * of that image runs from one channel into the next: C = 1, or KH divides H + H % KH.  SLAYER_EUNSUPPORTED elsewhere
+ * (slayer_synapse_conv_f32 on that image), and for an image that is smaller than the window.
  */
 int slayer_pool_f32(float *out, const float *in, const float *weight, int64_t N, int64_t C, int64_t H, int64_t W, int64_t T,
                     int64_t KH, int64_t KW, void *stream);
@@ -420,7 +423,7 @@ int slayer_pool_f32(float *out, const float *in, const float *weight, int64_t N,
  * Gradient of slayer_pool_f32 with respect to `in`.  With a membrane potential u (same shape as gradIn; may be NULL)
  * every result is multiplied by the surrogate gradient of slayer_spike_bwd_f32 at u (theta, tau, scale as there): with
  * gradOut filtered by slayer_psp_alpha_f32 (causal = 0) or slayer_corr_f32 first, that is what pool(psp(spike(u))) sends
- * back to u, since pooling and a filter along time commute.
+ * back to u, since pooling and a filter along time commute.  Same sizes as slayer_pool_f32.
  */
 int slayer_pool_grad_input_f32(float *gradIn, const float *gradOut, const float *weight, const float *u, float theta,
                                float tau, float scale, int64_t N, int64_t C, int64_t H, int64_t W, int64_t T, int64_t KH,

@@ -2529,9 +2529,12 @@ static bool wgrad_takes_ring(const SynGeom &s, const float *gradOut, const float
 }
 
 // ---- pooling -----------------------------------------------------------------------------------------
-// Geometry of a pooling layer as a one-channel synapse: the channels of a batch item as rows of one image where windows do
-// not straddle them, else one image per channel, whose last windows reach past it (KH and KW rows and columns of zeros
-// that nobody stores: extending the tensor by them was a copy of it and, in the backward pass, two more).
+// Geometry of a pooling layer as a one-channel synapse: the channels of a batch item as rows of one image where the window
+// divides the height, else one image per channel, whose last windows reach past it (KH and KW rows and columns of zeros
+// that nobody stores: extending the tensor by them was a copy of it and, in the backward pass, two more).  The layer is the
+// convolution of a batch item's extended channels below one another: where the window does not divide the extended height
+// either, windows run from one channel into the next, which only a synapse on that image gives (not taken here, and neither
+// is an image that is smaller than the window).
 static int pool_geom(int64_t N, int64_t C, int64_t H, int64_t W, int64_t T, int64_t KH, int64_t KW, SynGeom &s)
 {
     if (N < 0 || C < 0 || H < 0 || W < 0 || T < 0 || KH < 1 || KW < 1) return SLAYER_EINVAL;
@@ -2545,6 +2548,7 @@ static int pool_geom(int64_t N, int64_t C, int64_t H, int64_t W, int64_t T, int6
                 static_cast<int>(KH), static_cast<int>(KW), static_cast<int>(KH), static_cast<int>(KW), 0, 0, 1, 1, 1, 0, 0};
     s.OH = static_cast<int>((s.H + s.H % KH) / KH);
     s.OW = static_cast<int>((W + W % KW) / KW);
+    if (N * C * H * W * T > 0 && (s.OH < 1 || s.OW < 1 || (C > 1 && (H + H % KH) % KH != 0))) return SLAYER_EUNSUPPORTED;
     if (static_cast<int64_t>(s.OH) * s.OW * T >= lim / 4) return SLAYER_EUNSUPPORTED;
     // the taps' span in bytes, by which the gather's buffer may be moved
     if (KH * W * T * 4 + KW * T * 4 >= (1LL << 24)) return SLAYER_EUNSUPPORTED;
@@ -2707,6 +2711,6 @@ extern "C" int slayer_pool_grad_input_f32(float *gradIn, const float *gradOut, c
     const int status = pool_geom(N, C, H, W, T, KH, KW, s);
     if (status != SLAYER_OK) return status;
     if (static_cast<int64_t>(s.N) * s.H * s.W * s.T == 0) return SLAYER_OK;
-    if (!gradIn || !weight || (!gradOut && s.OH > 0 && s.OW > 0)) return SLAYER_EINVAL;
+    if (!gradIn || !weight || !gradOut) return SLAYER_EINVAL;
     return launch_window(gradIn, gradOut, weight, s, u, theta, tau, scale / tau, static_cast<hipStream_t>(stream));
 }

@@ -375,7 +375,8 @@ def _poolWeight(theta, shape):
 class _poolLayer(nn.Conv3d):
     """Sum pooling as a 1 -> 1 channel synapse with constant weights ``1.1 * theta`` on the tensor
     viewed as (N, 1, C*H, W, T) (src/slayer.py:509-577).  Like the reference, an extent that is not
-    a multiple of the window is extended by ``extent % window`` rows of zeros."""
+    a multiple of the window is extended by ``extent % window`` rows of zeros; where the window does not
+    divide the extended height either, windows run from one channel into the next."""
 
     def __init__(self, theta, kernelSize, stride=None, padding=0, dilation=1, preHookFx=None):
         kernel = _hw(kernelSize, "kernelSize")

@@ -265,7 +265,7 @@ def _check_window(weight):
 def pool(input, weight):
     """Sums over windows of ``weight``'s extent that do not overlap, channel by channel: ``conv`` with the window as
     stride on every channel by itself, ``input`` (N, C, H, W, T), ``weight`` (1, 1, KH, KW[, 1]).  ``None`` for sizes
-    that the kernel does not index."""
+    that the kernel does not take (:func:`poolSupported`)."""
     out = host.pool(input, weight)
     if out is not None:
         return out
@@ -317,7 +317,8 @@ def poolGradInput(gradOutput, weight, inShape, membranePotential=None, theta=0.0
 
 def poolSpikeBackwardDelayedCorr(gradOutput, weight, membranePotential, filter, delaySteps, theta, tau, scale, Ts):
     """``slayerCuda.spikeBackwardDelayedCorr(poolGradInput(gradOutput, weight, membranePotential.shape), membranePotential,
-    filter, delaySteps, ...)`` in one kernel, or ``None`` for rows and extents that it does not serve (nothing was launched)."""
+    filter, delaySteps, ...)`` in one kernel, or ``None`` for rows and extents that it does not serve (nothing was launched);
+    for shapes that :func:`poolSupported` takes."""
     for x, name in ((gradOutput, "gradOutput"), (membranePotential, "membranePotential"), (filter, "filter")):
         _check_input(x, name)
         _check_device(gradOutput, x, "gradOutput", name)
@@ -352,10 +353,14 @@ class _synapsePoolFunction(Function):
 
 
 def poolSupported(inShape, wShape):
-    """Whether the pooling kernels index these sizes: one channel's image, and the image of a batch item's channels below one
-    another where the window divides the height, as in :func:`supported`."""
+    """Whether the pooling kernels take these sizes: windows that lie in one channel each, on the image of a batch item's
+    channels below one another (one channel, or an extended height that the window divides), at least one of them, and what
+    the kernels index - one channel's image, and the image of all channels where the window divides the height, as in
+    :func:`supported`."""
     N, C, H, W, T = (int(v) for v in inShape)
     KH, KW = int(wShape[2]), int(wShape[3])
+    if min(_windows(inShape, wShape)) < 1 or (C > 1 and (H + H % KH) % KH != 0):
+        return False
     limit = ((1 << 31) - (1 << 24)) // 4
     return (KH < 1024 and KW < 1024 and max(H, W) < (1 << 24) - 1024 and (H + KH) * (W + KW) * T < limit and N * C < (1 << 31)
             and (KH * W + KW) * T * 4 < (1 << 24) and N * C * ((H * W * ((T + 3) // 4)) // 256 + 1) < (1 << 31))

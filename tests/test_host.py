@@ -372,3 +372,23 @@ int main()
                    check=True, timeout=120)
     r = subprocess.run([program], input="".join("%d %d\n" % s for s in pieces + whole), capture_output=True, text=True, timeout=60)
     assert r.stdout.split() == ["1"] * len(pieces) + ["0"] * len(whole)
+
+
+def test_pooling_kernels_take_windows_that_lie_in_one_channel():
+    """poolSupported and the entry points agree: sizes where the pooling layer, a convolution of the channels below one another,
+    has no window in two channels and at least one window (EINVAL for the null pointers), and no others (EUNSUPPORTED)."""
+    from slayerpytorch_amd import _lib, synapse
+    lib = _lib.load()
+    for KH in range(1, 6):
+        for KW in (1, 2, 3):
+            for C in range(1, 5):
+                for H in range(1, 14):
+                    for W in (1, 4, 7):
+                        rows = C * (H + H % KH)
+                        channels = [{row // (H + H % KH) for row in range(y, y + KH)} for y in range(0, rows - KH + 1, KH)]
+                        takes = H + H % KH >= KH and W + W % KW >= KW and all(len(c) == 1 for c in channels) \
+                            and len(channels) == C * ((H + H % KH) // KH)
+                        sizes = (2, C, H, W, 8)
+                        assert synapse.poolSupported(sizes, (1, 1, KH, KW)) == takes, (sizes, KH, KW)
+                        assert lib.slayer_pool_f32(None, None, None, *sizes, KH, KW, None) == (1 if takes else 2)
+                        assert lib.slayer_pool_grad_input_f32(None, None, None, None, 0.0, 1.0, 0.0, *sizes, KH, KW, None) == (1 if takes else 2)
