@@ -6,7 +6,8 @@
 // Every function takes the positional arguments of its namesake there and answers None for anything but the plain case
 // (exact torch.Tensor objects, contiguous fp32 on one GPU, Python numbers, sizes that the entry point takes): the caller
 // then goes through its own checks, which raise what they always raised, and its general path.  Nothing has been launched
-// where None is returned.  No state is kept.
+// where None is returned: a launch that reports an error - it may be one that another HIP call left, the kernel running all
+// the same - raises here.  No state is kept.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -15,6 +16,9 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
+
+#include <string>
 
 #include "../../include/slayer_hip.h"
 
@@ -32,13 +36,14 @@ bool plain(const at::Tensor &t)
 
 // The arguments of a call; ok goes false with the first one that is not plain.
 struct Args {
+    const char *name;    // of the function
     PyObject *const *a;
     Py_ssize_t n;
     bool ok;
     c10::Device device;
 
-    Args(PyObject *const *args, Py_ssize_t count, Py_ssize_t expected)
-        : a(args), n(count), ok(count == expected), device(c10::DeviceType::CUDA, -1) {}
+    Args(const char *function, PyObject *const *args, Py_ssize_t count, Py_ssize_t expected)
+        : name(function), a(args), n(count), ok(count == expected), device(c10::DeviceType::CUDA, -1) {}
 
     const at::Tensor *tensor(Py_ssize_t i)
     {
@@ -128,16 +133,27 @@ at::Tensor floats(at::IntArrayRef shape, const c10::Device &device)
     return at::empty(shape, at::TensorOptions().dtype(at::kFloat).device(device));
 }
 
-// Runs the entry point on the tensors' device and PyTorch's current stream there, without the interpreter's lock (as a
-// ctypes call does).  True: launched.
-template <typename Call> bool launch(const c10::Device &device, Call call)
+// The package's error for a launch that reported one, as _lib.check raises it.
+[[noreturn]] void raise_launch_error(const char *name)
 {
-    const c10::DeviceGuard guard(device);
-    void *stream = c10::hip::getCurrentHIPStream(device.index()).stream();
+    const std::string text = std::string(name) + " failed: " + slayer_status_string(SLAYER_ELAUNCH) + " (" + slayer_last_hip_error() + ")";
+    THPObjectPtr module(PyImport_ImportModule("slayerpytorch_amd._lib"));
+    THPObjectPtr error(module ? PyObject_GetAttrString(module.get(), "SlayerHipError") : nullptr);
+    if (error) PyErr_SetString(error.get(), text.c_str());
+    throw python_error();
+}
+
+// Runs the entry point on the tensors' device and PyTorch's current stream there, without the interpreter's lock (as a
+// ctypes call does).  True: launched.  False: refused, nothing was launched.
+template <typename Call> bool launch(const Args &a, Call call)
+{
+    const c10::DeviceGuard guard(a.device);
+    void *stream = c10::hip::getCurrentHIPStream(a.device.index()).stream();
     int status;
     Py_BEGIN_ALLOW_THREADS
     status = call(stream);
     Py_END_ALLOW_THREADS
+    if (status == SLAYER_ELAUNCH) raise_launch_error(a.name);
     return status == SLAYER_OK;
 }
 
@@ -145,7 +161,7 @@ PyObject *none() { Py_RETURN_NONE; }
 PyObject *wrapped(bool launched, const at::Tensor &t) { return launched ? THPVariable_Wrap(t) : none(); }
 
 #define SLAYER_HOST(NAME) PyObject *NAME(PyObject *, PyObject *const *args, Py_ssize_t nargs)
-#define SLAYER_ARGS(COUNT) Args a(args, nargs, COUNT)
+#define SLAYER_ARGS(COUNT) Args a(__func__, args, nargs, COUNT)
 #define SLAYER_PLAIN \
     if (!a.ok) return none()
 
@@ -164,7 +180,7 @@ SLAYER_HOST(getSpikes)   // (d_u, d_nu, theta, Ts)
     int64_t n, T;
     rows(*u, n, T);
     const int64_t taps = nu->dim() ? nu->size(-1) : 1;
-    return wrapped(launch(a.device, [&](void *st) { return slayer_get_spikes_f32(ptr(s), ptr(u), ptr(nu), n, T, taps, theta, Ts, st); }), s);
+    return wrapped(launch(a, [&](void *st) { return slayer_get_spikes_f32(ptr(s), ptr(u), ptr(nu), n, T, taps, theta, Ts, st); }), s);
     END_HANDLE_TH_ERRORS
 }
 
@@ -179,7 +195,7 @@ SLAYER_HOST(fir)         // (input, filter, Ts)
     const at::Tensor y = at::empty_like(*x);
     int64_t n, T;
     rows(*x, n, T);
-    return wrapped(launch(a.device, [&](void *st) { return ENTRY(ptr(y), ptr(x), ptr(f), n, T, f->numel(), Ts, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return ENTRY(ptr(y), ptr(x), ptr(f), n, T, f->numel(), Ts, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -195,7 +211,7 @@ SLAYER_HOST(pspAlpha)    // (input, filter, tau, mult, Ts, causal)
     const at::Tensor y = at::empty_like(*x);
     int64_t n, T;
     rows(*x, n, T);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_psp_alpha_f32(ptr(y), ptr(x), ptr(f), n, T, f->numel(), tau, mult, Ts, causal ? 1 : 0, st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -209,7 +225,7 @@ SLAYER_HOST(spikeBackward)   // (gradOutput, membranePotential, theta, tau, scal
     SLAYER_PLAIN;
     if (!same(g, u)) return none();
     const at::Tensor y = at::empty_like(*g);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_spike_bwd_f32(ptr(y), ptr(g), ptr(u), theta, tau, scale, g->numel(), st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_spike_bwd_f32(ptr(y), ptr(g), ptr(u), theta, tau, scale, g->numel(), st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -225,7 +241,7 @@ SLAYER_HOST(spikeBackwardPspAlpha)   // (gradOutput, membranePotential, filter, 
     const at::Tensor y = at::empty_like(*g);
     int64_t n, T;
     rows(*g, n, T);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_spike_bwd_psp_alpha_f32(ptr(y), ptr(g), ptr(u), ptr(f), n, T, f->numel(), v[0], v[1], v[2], v[3], v[4], v[5], st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -242,7 +258,7 @@ SLAYER_HOST(pspSpikeBackwardAlpha)   // (gradPsp, gradSpike or None, membranePot
     const at::Tensor y = at::empty_like(*g);
     int64_t n, T;
     rows(*g, n, T);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_psp_spike_bwd_alpha_f32(ptr(y), ptr(g), ptr(more), ptr(u), ptr(f), n, T, f->numel(), v[0], v[1], v[2], v[3], v[4], v[5], st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -277,11 +293,11 @@ SLAYER_HOST(shift)       // (input, number or table, Ts, sign)
     if (!delay.fits(*x, n)) return none();
     const at::Tensor y = at::empty_like(*x);
     if (!delay.table)
-        return wrapped(launch(a.device, [&](void *st) {
+        return wrapped(launch(a, [&](void *st) {
             return slayer_shift_f32(ptr(y), ptr(x), static_cast<float>(delay.value * sign), n, T, Ts, st); }), y);
     const bool one = delay.table->numel() == 1;
     const int64_t nBatch = one ? 1 : x->size(0), perBatch = one ? n : n / nBatch;
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_shift_lut_f32(ptr(y), ptr(x), ptr(delay.table), delay.table->numel(), nBatch, perBatch, T, Ts, static_cast<float>(sign), st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -299,7 +315,7 @@ SLAYER_HOST(spikeBackwardDelayed)   // (gradOutput, membranePotential, theta, ta
     rows(*g, n, T);
     if (!same(g, u) || !delay.fits(*g, n)) return none();
     const at::Tensor y = at::empty_like(*g);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_spike_bwd_delayed_f32(ptr(y), ptr(g), ptr(u), ptr(delay.table), delay.table ? delay.table->numel() : 0,
                                             static_cast<float>(delay.value),
                                             delayTs, n, T, theta, tau, scale, st); }), y);
@@ -321,7 +337,7 @@ SLAYER_HOST(delayGrad)   // (output, gradOutput, Ts)
     const at::Tensor out = floats(shape, a.device);
     const int64_t bytes = slayer_delay_grad_workspace_bytes(nBatch, perBatch, T);
     const at::Tensor work = floats({(bytes < 4 ? 4 : bytes) / 4}, a.device);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_delay_grad_f32(ptr(out), ptr(y), ptr(g), work.data_ptr<float>(), nBatch, perBatch, T, Ts, st); }), out);
     END_HANDLE_TH_ERRORS
 }
@@ -338,7 +354,7 @@ SLAYER_HOST(spikeBackwardDelayedCorr)   // (gradOutput, membranePotential, filte
     const at::Tensor y = at::empty_like(*g);
     int64_t n, T;
     rows(*g, n, T);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_spike_bwd_delayed_corr_f32(ptr(y), ptr(g), ptr(u), ptr(f), n, T, f->numel(), steps, theta, tau, scale, Ts, st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -358,7 +374,7 @@ SLAYER_HOST(loihiSpikesDelayed)   // (weightedSpikes, wgtExp, theta, iDecay, vDe
     if (voltage) v = at::empty_like(*x);
     int64_t n, T;
     rows(*x, n, T);
-    const bool launched = launch(a.device, [&](void *st) {
+    const bool launched = launch(a, [&](void *st) {
         return slayer_loihi_get_spikes_delayed_f32(ptr(s), voltage ? ptr(v) : nullptr, nullptr, ptr(x), n, T, static_cast<uint32_t>(wgtExp),
                                                    static_cast<int32_t>(theta), static_cast<uint32_t>(iDecay), static_cast<uint32_t>(vDecay),
                                                    static_cast<uint32_t>(refDelay), static_cast<int32_t>(delay), st); });
@@ -381,7 +397,7 @@ SLAYER_HOST(quantize)    // (weights, step)
     SLAYER_PLAIN;
     if (step == 0.0 || step != step) return none();
     const at::Tensor y = at::empty_like(*w);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_quantize_f32(ptr(y), ptr(w), w->numel(), step, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_quantize_f32(ptr(y), ptr(w), w->numel(), step, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -408,7 +424,7 @@ SLAYER_HOST(spikeLoss)   // (spikeOut, spikeDesired, srmKernel, Ts, addend or No
     int64_t n, T;
     rows(*out, n, T);
     const at::Tensor loss = floats({}, a.device), error = at::empty_like(*out), work = floats({n > 0 ? n : 1}, a.device);
-    return lossAndError(launch(a.device, [&](void *st) {
+    return lossAndError(launch(a, [&](void *st) {
         return slayer_spike_loss_f32(loss.data_ptr<float>(), ptr(error), ptr(out), ptr(desired), ptr(addend), ptr(srm), work.data_ptr<float>(),
                                      n, T, srm->numel(), Ts, st); }), loss, error);
     END_HANDLE_TH_ERRORS
@@ -425,7 +441,7 @@ SLAYER_HOST(spikeLossGrad)   // (error, gradLoss, srmKernel, Ts)
     int64_t n, T;
     rows(*error, n, T);
     const at::Tensor y = at::empty_like(*error);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_spike_loss_grad_f32(ptr(y), ptr(error), ptr(g), ptr(srm), n, T, srm->numel(), Ts, st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -460,7 +476,7 @@ SLAYER_HOST(conv2d)      // (input, weight, stride, padding, dilation, groups)
     int32_t OH, OW;
     if (!geometry(a, x->sizes(), w->sizes(), 2, g, OH, OW)) return none();
     const at::Tensor y = floats({g.N, g.O, OH, OW, g.T}, a.device);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_synapse_conv_f32(ptr(y), ptr(x), ptr(w), &g, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_synapse_conv_f32(ptr(y), ptr(x), ptr(w), &g, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -479,7 +495,7 @@ SLAYER_HOST(conv2dGradInput)   // (gradOutput, weight, input, stride, padding, d
     int32_t OH, OW;
     if (!geometry(a, x->sizes(), w->sizes(), 3, g, OH, OW) || !output_of(*go, g, OH, OW)) return none();
     const at::Tensor y = floats(x->sizes(), a.device);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_synapse_conv_grad_input_f32(ptr(y), ptr(go), ptr(w), &g, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_synapse_conv_grad_input_f32(ptr(y), ptr(go), ptr(w), &g, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -495,7 +511,7 @@ SLAYER_HOST(conv2dGradWeight)  // (gradOutput, input, weight, stride, padding, d
     const at::Tensor y = floats(w->sizes(), a.device);
     const int64_t bytes = slayer_synapse_conv_grad_weight_workspace_bytes(&g);
     const at::Tensor work = floats({(bytes + 3) / 4}, a.device);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_synapse_conv_grad_weight_f32(ptr(y), ptr(go), ptr(x), ptr(work), &g, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_synapse_conv_grad_weight_f32(ptr(y), ptr(go), ptr(x), ptr(work), &g, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -510,7 +526,7 @@ SLAYER_HOST(pool)        // (input, weight)
     if (x->dim() != 5 || !window(*w)) return none();
     const int64_t H = x->size(2), W = x->size(3), KH = w->size(2), KW = w->size(3);
     const at::Tensor y = floats({x->size(0), x->size(1), (H + H % KH) / KH, (W + W % KW) / KW, x->size(4)}, a.device);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_pool_f32(ptr(y), ptr(x), ptr(w), x->size(0), x->size(1), H, W, x->size(4), KH, KW, st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -526,7 +542,7 @@ SLAYER_HOST(poolSpikeBackward)   // (gradOutput, weight, membranePotential, thet
     const int64_t H = u->size(2), W = u->size(3), KH = w->size(2), KW = w->size(3);
     if (g->sizes() != at::IntArrayRef({u->size(0), u->size(1), (H + H % KH) / KH, (W + W % KW) / KW, u->size(4)})) return none();
     const at::Tensor y = at::empty_like(*u);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_pool_grad_input_f32(ptr(y), ptr(g), ptr(w), ptr(u), theta, tau, scale, u->size(0), u->size(1), H, W, u->size(4), KH, KW, st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -541,7 +557,7 @@ SLAYER_HOST(denseEvents)   // (input, weight)
     if (x->dim() != 3 || w->dim() != 2 || w->size(1) != x->size(1)) return none();
     const int64_t N = x->size(0), K = x->size(1), T = x->size(2), O = w->size(0);
     const at::Tensor y = floats({N, O, T}, a.device), work = floats({(slayer_dense_events_workspace_bytes(N, K, O, T) + 3) / 4}, a.device);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_dense_events_f32(ptr(y), ptr(x), ptr(w), ptr(work), N, K, O, T, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_dense_events_f32(ptr(y), ptr(x), ptr(w), ptr(work), N, K, O, T, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -555,7 +571,7 @@ SLAYER_HOST(denseEventsGradWeight)   // (gradOutput, input)
     const int64_t N = x->size(0), K = x->size(1), T = x->size(2), O = g->size(1);
     const at::Tensor y = floats({O, K}, a.device),
                      work = floats({(slayer_dense_events_grad_weight_workspace_bytes(N, K, O, T) + 3) / 4}, a.device);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_dense_events_grad_weight_f32(ptr(y), ptr(g), ptr(x), ptr(work), N, K, O, T, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_dense_events_grad_weight_f32(ptr(y), ptr(g), ptr(x), ptr(work), N, K, O, T, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -571,7 +587,7 @@ SLAYER_HOST(denseThin)   // (input, weight)
     const at::Tensor y = floats({N, O, T}, a.device);
     at::Tensor work;
     if (bytes) work = floats({bytes / 4}, a.device);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_dense_thin_f32(ptr(y), ptr(w), ptr(x), bytes ? ptr(work) : nullptr, N, K, O, T, st); }), y);
     END_HANDLE_TH_ERRORS
 }
@@ -585,7 +601,7 @@ SLAYER_HOST(denseThinGradInput)   // (gradOutput, weight)
     if (g->dim() != 3 || w->dim() != 2 || w->size(0) != g->size(1)) return none();
     const int64_t N = g->size(0), K = w->size(1), T = g->size(2), O = g->size(1);
     const at::Tensor y = floats({N, K, T}, a.device);
-    return wrapped(launch(a.device, [&](void *st) { return slayer_dense_thin_grad_input_f32(ptr(y), ptr(w), ptr(g), N, K, O, T, st); }), y);
+    return wrapped(launch(a, [&](void *st) { return slayer_dense_thin_grad_input_f32(ptr(y), ptr(w), ptr(g), N, K, O, T, st); }), y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -601,7 +617,7 @@ SLAYER_HOST(denseThinGradWeight)   // (gradOutput, input)
     const at::Tensor y = floats({O, K}, a.device);
     at::Tensor work;
     if (bytes) work = floats({bytes / 4}, a.device);
-    return wrapped(launch(a.device, [&](void *st) {
+    return wrapped(launch(a, [&](void *st) {
         return slayer_dense_thin_grad_weight_f32(ptr(y), ptr(g), ptr(x), bytes ? ptr(work) : nullptr, N, K, O, T, st); }), y);
     END_HANDLE_TH_ERRORS
 }

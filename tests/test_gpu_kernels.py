@@ -1403,3 +1403,28 @@ def test_the_plain_case_of_a_call_equals_the_general_path(monkeypatch):
     assert host.spikeBackward(x, u[:1].contiguous(), 1.0, 1.0, 1.0) is None
     assert host.conv2d(x, w, -1, 0, 1, 1) is None and host.conv2d(x, w, 1, 0, 1, 2) is None
     assert host.unwrapped(x, 3, None) and not host.unwrapped(torch.ones(2).as_subclass(type("Sub", (torch.Tensor,), {})))
+
+
+def test_an_error_that_another_call_left_is_raised_once_and_nothing_is_launched_twice():
+    """A HIP call of somebody else's that failed leaves its error to the next launch, which reports it.  The call is not made
+    again (the spike function would add its refractory response a second time)."""
+    import ctypes
+    from slayerpytorch_amd import _lib, slayerCuda
+    lib = _lib.load()
+    lib.hipSetDevice.argtypes, lib.hipSetDevice.restype = [ctypes.c_int], ctypes.c_int
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    u = torch.randn((1, 2, 3, 4, 50), generator=gen, device="cuda") * 6
+    nu = -torch.arange(6, 0, -1, device="cuda", dtype=torch.float32)
+    want = u.clone()
+    slayerCuda.getSpikes(want, nu, 2.0, 1.0)
+    once, twice = u.clone(), want.clone()
+    slayerCuda.getSpikes(twice, nu, 2.0, 1.0)
+    assert not torch.equal(want, twice)
+    torch.cuda.synchronize()
+    assert lib.hipSetDevice(1 << 20) != 0
+    with pytest.raises(_lib.SlayerHipError, match="launch failed"):
+        slayerCuda.getSpikes(once, nu, 2.0, 1.0)
+    torch.cuda.synchronize()
+    assert torch.equal(once, want) and not torch.equal(once, u)
+    slayerCuda.getSpikes(once.copy_(u), nu, 2.0, 1.0)
+    assert torch.equal(once, want)
