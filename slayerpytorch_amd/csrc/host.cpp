@@ -15,6 +15,10 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/function_hook.h>
+#include <torch/csrc/autograd/graph_task.h>
+#include <torch/csrc/autograd/python_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 
@@ -640,6 +644,27 @@ SLAYER_HOST(unwrapped)
     Py_RETURN_TRUE;
 }
 
+// (ctx): whether someone looks at the gradient of this Function's first tensor argument in the backward pass that is running -
+// a hook on the tensor or on the node behind it, retain_grad, or the pass was asked for it - so that the gradient may not go
+// past that node.  True where there is no such pass.
+SLAYER_HOST(watched)
+{
+    using namespace torch::autograd;
+    HANDLE_TH_ERRORS
+    if (nargs != 1 || !THPFunction_Check(args[0])) Py_RETURN_TRUE;
+    const std::shared_ptr<PyNode> own = reinterpret_cast<THPFunction *>(args[0])->cdata.lock();
+    const auto *info = get_current_graph_task_exec_info();
+    if (!own || !info || own->num_outputs() == 0) Py_RETURN_TRUE;
+    Node *node = own->next_edge(0).function.get();
+    if (!node) Py_RETURN_FALSE;
+    const auto asked = info->find(node);
+    if (!node->pre_hooks().empty() || !node->tensor_pre_hooks().empty() || !node->retains_grad_hooks().empty() || !node->post_hooks().empty() ||
+        (asked != info->end() && asked->second.captures_ && !asked->second.captures_->empty()))
+        Py_RETURN_TRUE;
+    Py_RETURN_FALSE;
+    END_HANDLE_TH_ERRORS
+}
+
 #define SLAYER_METHOD(NAME, FN) {NAME, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(FN)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     SLAYER_METHOD("getSpikes", getSpikes),
@@ -668,6 +693,7 @@ PyMethodDef methods[] = {
     SLAYER_METHOD("denseThinGradInput", denseThinGradInput),
     SLAYER_METHOD("denseThinGradWeight", denseThinGradWeight),
     SLAYER_METHOD("unwrapped", unwrapped),
+    SLAYER_METHOD("watched", watched),
     {nullptr, nullptr, 0, nullptr},
 };
 

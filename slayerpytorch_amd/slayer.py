@@ -30,6 +30,7 @@ from torch.utils.weak import TensorWeakRef, WeakTensorKeyDictionary
 from . import slayerCuda
 from . import synapse
 from ._function import Function
+from ._lib import host
 
 
 # spikeLayer.psp filters with the alpha kernel as a recursion over time when the kernel has more taps than this
@@ -712,8 +713,8 @@ class _poolOfPspFunction(Function):
     ``membranePotential``.  Forward: the pooling.  Backward: pooling and the filter along time commute, so the gradient
     is correlated with the filter while it is still pooled - a KH KW-th of the samples - and goes to
     ``membranePotential`` directly, spread over the windows and multiplied by the spike function's surrogate gradient in
-    one kernel.  Where ``psp`` is still held by someone when the backward pass runs, who may ask for its gradient, it gets
-    it, and its own node does the rest."""
+    one kernel.  Where ``psp`` is still held by someone when the backward pass runs, or someone watches its gradient
+    (``host.watched``: hooks on a tensor that was let go are on its node), it gets it, and its own node does the rest."""
 
     @staticmethod
     def forward(ctx, psp, membranePotential, weight, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale):
@@ -727,7 +728,7 @@ class _poolOfPspFunction(Function):
     def backward(ctx, gradOutput):
         membranePotential, weight, filter = ctx.saved_tensors
         gradOutput = gradOutput.contiguous()
-        if ctx.psp() is not None:
+        if ctx.psp() is not None or host.watched(ctx):
             return (synapse.poolGradInput(gradOutput, weight, membranePotential.shape),) + (None,) * 8
         filtered = slayerCuda.pspAlpha(gradOutput, filter, ctx.alpha[0], ctx.alpha[1], ctx.Ts, causal=False)
         grad = synapse.poolGradInput(filtered, weight, membranePotential.shape, membranePotential, ctx.theta,
@@ -769,7 +770,7 @@ class PooledGradients:
 
 class _poolOfSpikesFunction(Function):
     """The pooling layer of spikes whose neuron takes pooled gradients.  Where the spikes are still held by someone when the
-    backward pass runs, who may ask for their gradient, they get it."""
+    backward pass runs, or someone watches their gradient (``host.watched``), they get it."""
 
     @staticmethod
     def forward(ctx, spikes, weight, node):
@@ -781,7 +782,7 @@ class _poolOfSpikesFunction(Function):
     def backward(ctx, gradOutput):
         (weight,) = ctx.saved_tensors
         gradOutput = gradOutput.contiguous()
-        if ctx.spikes() is not None:
+        if ctx.spikes() is not None or host.watched(ctx):
             return synapse.poolGradInput(gradOutput, weight, ctx.shape), None, None
         ctx.node.pooled.leave(gradOutput, weight, ctx.shape)
         return None, None, None

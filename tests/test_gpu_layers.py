@@ -1047,3 +1047,75 @@ def test_cpu_plumbing_configuration(scale):
     flips = float((s_gpu.cpu().numpy() != s_cpu).mean())
     assert 0.005 < float(s_cpu.mean()) < (0.5 if scale < 1 else 0.9)
     assert flips <= 1e-4, "spike flip rate %g" % flips
+
+
+def _pairs():
+    """name -> (the tensor in between, the result) of x: calls whose backward passes run as one."""
+    srm = snn.layer(neuron(), {"Ts": 1.0, "tSample": 300}).to(DEV)
+    chip = snn.loihi(loihi_neuron(), {"Ts": 1, "tSample": 300}).to(DEV)
+    pool, chipPool = srm.pool(2).to(DEV), chip.pool(2).to(DEV)
+
+    def pool_psp(x):
+        a = srm.psp(srm.spike(x))
+        return a, pool(a)
+
+    def pool_spikes(x):
+        s = chip.spikeLoihi(x)
+        return s, chipPool(s)
+
+    return {"pool of psp": pool_psp, "pool of Loihi spikes": pool_spikes}
+
+
+# ways of asking for the gradient of a tensor after its last use: (what `ask` returns is held, the tensor is let go)
+def _tensor_hook(t, seen):
+    t.register_hook(lambda g: (seen.append(g.clone()), g * 2)[1])
+
+
+def _node_prehook(t, seen):
+    t.grad_fn.register_prehook(lambda gs: (seen.append(gs[0].clone()), (gs[0] * 2,))[1])
+
+
+def _node_hook(t, seen):
+    t.grad_fn.register_hook(lambda gradIn, gradOut: seen.append(gradOut[0].clone()))
+
+
+def _retained(t, seen):
+    t.retain_grad()
+    return t
+
+
+@pytest.mark.parametrize("ask", [_tensor_hook, _node_prehook, _node_hook, _retained, "edge", "again"])
+@pytest.mark.parametrize("pair", ["pool of psp", "pool of Loihi spikes"])
+def test_a_gradient_that_is_asked_for_after_the_call_is_there(pair, ask, monkeypatch):
+    """A hook on the tensor between two paired calls, or on its node, registered after the second call on a tensor that is then
+    let go, sees and changes the gradient as with the Functions apart; so does autograd.grad for the tensor's edge."""
+    from slayerpytorch_amd import slayer as slayer_module
+    rng = np.random.default_rng(5)
+    x0 = dev((rng.integers(-3, 9, (2, 3, 4, 6, 300)) * 12).astype(np.float32))
+    calls = _pairs()[pair]
+
+    def run(paired):
+        monkeypatch.setattr(slayer_module, "PAIR_SPIKE_PSP", paired)
+        x = x0.clone().requires_grad_(True)
+        seen = []
+        between, y = calls(x * 1.0)
+        g = torch.linspace(-1.0, 2.0, y.numel(), device=DEV).reshape(y.shape)
+        if ask == "edge":
+            edge = torch.autograd.graph.get_gradient_edge(between)
+            del between
+            return list(torch.autograd.grad(y, [x, edge], g))
+        if ask == "again":                           # watched in one pass, and not in the next
+            handle = between.register_hook(lambda g: (seen.append(g.clone()), g * 2)[1])
+            del between
+            first = torch.autograd.grad(y, x, g, retain_graph=True)
+            handle.remove()
+            return [*first, *torch.autograd.grad(y, x, g), *seen]
+        held = ask(between, seen)
+        del between
+        (grad,) = torch.autograd.grad(y, x, g) if held is None else (y.backward(g), x.grad)[1:]
+        return [grad, *seen, *(() if held is None else (held.grad,))]
+
+    want, got = run(False), run(True)
+    assert len(want) == len(got) >= 2 and all(float(w.abs().sum()) > 0 for w in want)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and rel_err(host(a), host(b)) <= REL_TOL

@@ -392,3 +392,54 @@ def test_pooling_kernels_take_windows_that_lie_in_one_channel():
                         assert synapse.poolSupported(sizes, (1, 1, KH, KW)) == takes, (sizes, KH, KW)
                         assert lib.slayer_pool_f32(None, None, None, *sizes, KH, KW, None) == (1 if takes else 2)
                         assert lib.slayer_pool_grad_input_f32(None, None, None, None, 0.0, 1.0, 0.0, *sizes, KH, KW, None) == (1 if takes else 2)
+
+
+@pytest.mark.parametrize("how", ["nobody", "tensor hook", "node prehook", "node hook", "retain_grad", "asked for", "edge", "several"])
+def test_a_gradient_that_someone_watches_is_known_in_the_backward_pass(how):
+    """host.watched(ctx) for a Function that may send its gradient past its first argument: every way of looking at that
+    argument's gradient, registered after the call and with the tensor let go."""
+    answers, seen = [], []
+
+    class First(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            ctx.set_materialize_grads(False)
+            return x * 2
+
+        @staticmethod
+        def backward(ctx, g):
+            return None if g is None else g * 2
+
+    class Second(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, a, x):
+            return a * 3
+
+        @staticmethod
+        def backward(ctx, g):
+            answers.append(_lib.host.watched(ctx))
+            return (g * 3, None) if answers[-1] else (None, g * 6)
+
+    x = torch.ones(3, requires_grad=True)
+    a = First.apply(x)
+    y = Second.apply(a, x).sum()
+    wanted = [x]
+    if how == "tensor hook":
+        a.register_hook(lambda g: (seen.append(g), g * 2)[1])
+    elif how == "node prehook":
+        a.grad_fn.register_prehook(lambda gs: (seen.append(gs[0]), (gs[0] * 2,))[1])
+    elif how == "node hook":
+        a.grad_fn.register_hook(lambda gi, go: (seen.append(go[0]), (gi[0] * 2,))[1])
+    elif how == "retain_grad":
+        a.retain_grad()
+    elif how == "several":
+        torch.autograd.graph.register_multi_grad_hook([a], lambda gs: seen.append(gs[0]))
+    elif how in ("asked for", "edge"):
+        wanted = [x, a] if how == "asked for" else [x, torch.autograd.graph.get_gradient_edge(a)]
+    if how != "retain_grad":
+        del a
+    got = torch.autograd.grad(y, wanted)
+    assert answers == [how != "nobody"]
+    assert torch.equal(got[0], torch.full((3,), 12.0 if how in ("tensor hook", "node prehook", "node hook") else 6.0))
+    assert all(torch.equal(g, torch.full((3,), 3.0)) for g in (*seen, *got[1:]))
+    assert len(seen) == (how in ("tensor hook", "node prehook", "node hook", "several"))
