@@ -644,23 +644,31 @@ SLAYER_HOST(unwrapped)
     Py_RETURN_TRUE;
 }
 
-// (ctx): whether someone looks at the gradient of this Function's first tensor argument in the backward pass that is running -
-// a hook on the tensor or on the node behind it, retain_grad, or the pass was asked for it - so that the gradient may not go
-// past that node.  True where there is no such pass.
+// (ctx, nodes = 1): whether someone looks at the gradient of this Function's first tensor argument in the backward pass that is
+// running - a hook on the tensor or on the node behind it, retain_grad, or the pass was asked for it - so that the gradient
+// may not go past that node; with more `nodes`, at that of the node's first argument as well, and so on.  True where there is
+// no such pass.
 SLAYER_HOST(watched)
 {
     using namespace torch::autograd;
     HANDLE_TH_ERRORS
-    if (nargs != 1 || !THPFunction_Check(args[0])) Py_RETURN_TRUE;
+    const long nodes = nargs == 2 ? PyLong_AsLong(args[1]) : 1;
+    if (nargs < 1 || nargs > 2 || nodes < 1 || !THPFunction_Check(args[0])) {
+        PyErr_Clear();
+        Py_RETURN_TRUE;
+    }
     const std::shared_ptr<PyNode> own = reinterpret_cast<THPFunction *>(args[0])->cdata.lock();
     const auto *info = get_current_graph_task_exec_info();
-    if (!own || !info || own->num_outputs() == 0) Py_RETURN_TRUE;
-    Node *node = own->next_edge(0).function.get();
-    if (!node) Py_RETURN_FALSE;
-    const auto asked = info->find(node);
-    if (!node->pre_hooks().empty() || !node->tensor_pre_hooks().empty() || !node->retains_grad_hooks().empty() || !node->post_hooks().empty() ||
-        (asked != info->end() && asked->second.captures_ && !asked->second.captures_->empty()))
-        Py_RETURN_TRUE;
+    if (!own || !info) Py_RETURN_TRUE;
+    Node *node = own.get();
+    for (long i = 0; i < nodes; ++i) {
+        node = node->num_outputs() ? node->next_edge(0).function.get() : nullptr;
+        if (!node) Py_RETURN_FALSE;
+        const auto asked = info->find(node);
+        if (!node->pre_hooks().empty() || !node->tensor_pre_hooks().empty() || !node->retains_grad_hooks().empty() || !node->post_hooks().empty() ||
+            (asked != info->end() && asked->second.captures_ && !asked->second.captures_->empty()))
+            Py_RETURN_TRUE;
+    }
     Py_RETURN_FALSE;
     END_HANDLE_TH_ERRORS
 }

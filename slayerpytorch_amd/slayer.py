@@ -657,7 +657,8 @@ class _spikeOfPspFunction(Function):
     from ``pspInput`` with the alpha kernel as a recursion.  Forward: the spike function.  Backward: the gradient
     goes to ``pspInput`` directly - surrogate gradient, then the correlation of ``_pspFunction.backward``
     (src/slayer.py:888-893), in one kernel - and nothing to ``membranePotential``, whose producer then only
-    carries what reaches the potential from elsewhere."""
+    carries what reaches the potential from elsewhere; unless someone watches that gradient (``host.watched``): then
+    ``membranePotential`` gets it, and its producer does the rest."""
 
     @staticmethod
     def forward(ctx, membranePotential, pspInput, refractoryResponse, filter, neuron, Ts, alpha):
@@ -673,6 +674,10 @@ class _spikeOfPspFunction(Function):
     @staticmethod
     def backward(ctx, gradOutput):
         grad = None
+        if gradOutput is not None and host.watched(ctx):
+            membranePotential, _ = ctx.saved_tensors
+            return (slayerCuda.spikeBackward(gradOutput.contiguous(), membranePotential, ctx.theta, ctx.pdfTimeConstant,
+                                             ctx.pdfScale),) + (None,) * 6
         if gradOutput is not None and ctx.needs_input_grad[1]:
             membranePotential, filter = ctx.saved_tensors
             grad = slayerCuda.spikeBackwardPspAlpha(gradOutput.contiguous(), membranePotential, filter, ctx.alpha[0],
@@ -685,7 +690,7 @@ class _pspOfSpikeFunction(Function):
     ``membranePotential``, with the alpha kernel as a recursion.  Forward: the PSP filter.  Backward: the
     gradient goes to ``membranePotential`` directly - correlation, then the spike function's surrogate
     gradient (src/slayer.py:858-865), in one kernel - and nothing to ``spike``, whose own backward pass then
-    only carries what reaches the spikes from elsewhere."""
+    only carries what reaches the spikes from elsewhere; unless someone watches that gradient (``host.watched``)."""
 
     @staticmethod
     def forward(ctx, spike, membranePotential, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale):
@@ -701,6 +706,10 @@ class _pspOfSpikeFunction(Function):
     @staticmethod
     def backward(ctx, gradOutput):
         grad = None
+        if gradOutput is not None and host.watched(ctx):
+            _, filter = ctx.saved_tensors
+            return (slayerCuda.pspAlpha(gradOutput.contiguous(), filter, ctx.alpha[0], ctx.alpha[1], ctx.Ts,
+                                        causal=False),) + (None,) * 7
         if gradOutput is not None and ctx.needs_input_grad[1]:
             membranePotential, filter = ctx.saved_tensors
             grad = slayerCuda.pspSpikeBackwardAlpha(gradOutput.contiguous(), None, membranePotential, filter, ctx.alpha[0],
@@ -714,7 +723,8 @@ class _poolOfPspFunction(Function):
     is correlated with the filter while it is still pooled - a KH KW-th of the samples - and goes to
     ``membranePotential`` directly, spread over the windows and multiplied by the spike function's surrogate gradient in
     one kernel.  Where ``psp`` is still held by someone when the backward pass runs, or someone watches its gradient
-    (``host.watched``: hooks on a tensor that was let go are on its node), it gets it, and its own node does the rest."""
+    or that of the spikes (``host.watched``: hooks on a tensor that was let go are on its node), it gets it, and its own
+    node does the rest."""
 
     @staticmethod
     def forward(ctx, psp, membranePotential, weight, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale):
@@ -728,7 +738,7 @@ class _poolOfPspFunction(Function):
     def backward(ctx, gradOutput):
         membranePotential, weight, filter = ctx.saved_tensors
         gradOutput = gradOutput.contiguous()
-        if ctx.psp() is not None or host.watched(ctx):
+        if ctx.psp() is not None or host.watched(ctx, 2):     # (the psp signal, or the spikes that it was made from)
             return (synapse.poolGradInput(gradOutput, weight, membranePotential.shape),) + (None,) * 8
         filtered = slayerCuda.pspAlpha(gradOutput, filter, ctx.alpha[0], ctx.alpha[1], ctx.Ts, causal=False)
         grad = synapse.poolGradInput(filtered, weight, membranePotential.shape, membranePotential, ctx.theta,
@@ -881,8 +891,8 @@ class _delayOfSpikeFunction(Function):
     """``_delayFunction`` / ``_delayFunctionNoGradient`` (src/slayer.py:930-979) for a spike tensor that
     ``_spikeFunction`` has just produced from ``membranePotential``.  Forward: the shift.  Backward: the gradient
     goes to ``membranePotential`` directly - shifted back and multiplied by the spike function's surrogate gradient
-    (src/slayer.py:858-865) in one kernel - and nothing to ``spike``; a learnable delay table (``learn``) gets the
-    delay gradient as in ``_delayFunction``."""
+    (src/slayer.py:858-865) in one kernel - and nothing to ``spike``, unless someone watches that gradient
+    (``host.watched``); a learnable delay table (``learn``) gets the delay gradient as in ``_delayFunction``."""
 
     @staticmethod
     def forward(ctx, spike, membranePotential, delay, Ts, learn, theta, pdfTimeConstant, pdfScale):
@@ -903,6 +913,8 @@ class _delayOfSpikeFunction(Function):
         gradDelay = grad = None
         if ctx.learn and ctx.needs_input_grad[2]:
             gradDelay = slayerCuda.delayGrad(ctx.saved_tensors[1], gradOutput, ctx.Ts).reshape(ctx.delayShape)
+        if host.watched(ctx):
+            return (slayerCuda.shift(gradOutput, ctx.delay, ctx.Ts, sign=-1.0), None, gradDelay) + (None,) * 5
         if ctx.needs_input_grad[1]:
             grad = slayerCuda.spikeBackwardDelayed(gradOutput, membranePotential, ctx.theta, ctx.pdfTimeConstant,
                                                    ctx.pdfScale, ctx.delay, ctx.Ts)

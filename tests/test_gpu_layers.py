@@ -1063,7 +1063,29 @@ def _pairs():
         s = chip.spikeLoihi(x)
         return s, chipPool(s)
 
-    return {"pool of psp": pool_psp, "pool of Loihi spikes": pool_spikes}
+    def pool_psp_spike(x):
+        s = srm.spike(x)
+        return s, pool(srm.psp(s))
+
+    def spike_psp(x):
+        a = srm.psp(x)
+        return a, srm.spike(a)
+
+    def psp_spike(x):
+        s = srm.spike(x)
+        return s, srm.psp(s)
+
+    def delay_spike(x):
+        s = srm.spike(x)
+        return s, delay(s)
+
+    def shift_spike(x):
+        s = srm.spike(x)
+        return s, srm.delayShift(s, 3.0)
+
+    delay = srm.delay((3, 4, 6)).to(DEV)
+    return {"pool of psp": pool_psp, "pool of psp of spikes": pool_psp_spike, "pool of Loihi spikes": pool_spikes,
+            "spike of psp": spike_psp, "psp of spikes": psp_spike, "delay of spikes": delay_spike, "shift of spikes": shift_spike}
 
 
 # ways of asking for the gradient of a tensor after its last use: (what `ask` returns is held, the tensor is let go)
@@ -1085,7 +1107,8 @@ def _retained(t, seen):
 
 
 @pytest.mark.parametrize("ask", [_tensor_hook, _node_prehook, _node_hook, _retained, "edge", "again"])
-@pytest.mark.parametrize("pair", ["pool of psp", "pool of Loihi spikes"])
+@pytest.mark.parametrize("pair", ["pool of psp", "pool of psp of spikes", "pool of Loihi spikes", "spike of psp", "psp of spikes",
+                                  "delay of spikes", "shift of spikes"])
 def test_a_gradient_that_is_asked_for_after_the_call_is_there(pair, ask, monkeypatch):
     """A hook on the tensor between two paired calls, or on its node, registered after the second call on a tensor that is then
     let go, sees and changes the gradient as with the Functions apart; so does autograd.grad for the tensor's edge."""
