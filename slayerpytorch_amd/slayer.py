@@ -94,7 +94,7 @@ class spikeLayer(nn.Module):
         psp = _pspFunction.apply(spike, self.srmKernel, self.simulation["Ts"], alpha)
         if PAIR_SPIKE_PSP and alpha is not None and psp.requires_grad and _recursion_serves(spike):
             # for spike(): what this signal was filtered from, and that it has not been touched since
-            _pspNotes[psp] = (spike, self.srmKernel, alpha, psp._version)
+            _pspNotes[psp] = (spike, self.srmKernel, alpha, psp._version, self.srmKernel._version)
         return psp
 
     def _srmKernelIsAlpha(self):
@@ -121,7 +121,7 @@ class spikeLayer(nn.Module):
         updated in place with the refractory response, as in the reference."""
         origin = _pspNotes.pop(membranePotential, None) if PAIR_SPIKE_PSP else None   # (the note is what keeps x alive)
         if origin is not None and torch.is_grad_enabled() and membranePotential.requires_grad \
-                and membranePotential.is_contiguous() and membranePotential._version == origin[3] \
+                and membranePotential.is_contiguous() and membranePotential._version == origin[3] and origin[1]._version == origin[4] \
                 and isinstance(membranePotential.grad_fn, _pspFunction._backward_cls) \
                 and _unobserved(membranePotential) and origin[0].shape == membranePotential.shape:
             # spike(psp(x)), the ordering of the reference's MLP example: the spikes' gradient goes past the PSP
@@ -555,7 +555,7 @@ def _fresh_psp_of_spikes(psp, kH, kW):
             or not _unobserved(psp) or not psp.is_contiguous():
         return None
     membranePotential = _untouched(node.potential, node.potentialVersion, psp)
-    if membranePotential is None:
+    if membranePotential is None or node.filter._version != node.filterVersion:
         return None
     N, C, H, W, T = psp.shape
     pooled = N * C * ((H + H % kH) // kH) * ((W + W % kW) // kW) * T
@@ -567,7 +567,7 @@ def _fresh_psp_of_spikes(psp, kH, kW):
 # The pairing notes live beside the tensors, not on them: a tensor with Python attributes is pickled with them
 # (torch.save of a layer's output would carry the note, or fail on it), and an entry goes when its tensor does.  (What the
 # pooling layer goes by keeps nothing alive and lives on the node behind the psp signal.)
-_pspNotes = WeakTensorKeyDictionary()     # psp() output -> (its input, kernel, (tau, mult), version)
+_pspNotes = WeakTensorKeyDictionary()     # psp() output -> (its input, kernel, (tau, mult), versions)
 _spikeNotes = WeakTensorKeyDictionary()   # spike() output -> (weak potential, theta, pdf tau, pdf scale, versions)
 
 
@@ -700,7 +700,8 @@ class _pspOfSpikeFunction(Function):
         ctx.Ts, ctx.alpha = float(Ts), alpha
         ctx.theta, ctx.pdfTimeConstant, ctx.pdfScale = theta, pdfTimeConstant, pdfScale
         # for _fresh_psp_of_spikes (the filter is a buffer of the layer's)
-        ctx.potential, ctx.potentialVersion, ctx.filter = weakref.ref(membranePotential), membranePotential._version, filter
+        ctx.potential, ctx.potentialVersion = weakref.ref(membranePotential), membranePotential._version
+        ctx.filter, ctx.filterVersion = filter, filter._version
         return psp
 
     @staticmethod

@@ -1142,3 +1142,21 @@ def test_a_gradient_that_is_asked_for_after_the_call_is_there(pair, ask, monkeyp
     assert len(want) == len(got) >= 2 and all(float(w.abs().sum()) > 0 for w in want)
     for a, b in zip(got, want):
         assert a.shape == b.shape and rel_err(host(a), host(b)) <= REL_TOL
+
+
+@pytest.mark.parametrize("pair", ["pool of psp", "spike of psp"])
+@pytest.mark.parametrize("paired", [True, False])
+def test_a_filter_that_was_changed_in_place_between_the_calls_is_noticed(pair, paired, monkeypatch):
+    """The gradient belongs to the filter that the signal was made with: a filter that was changed in place since is an error
+    of the backward pass, as for any saved tensor, and not the filter of a paired kernel."""
+    from slayerpytorch_amd import slayer as slayer_module
+    monkeypatch.setattr(slayer_module, "PAIR_SPIKE_PSP", paired)
+    layer = snn.layer(neuron(), {"Ts": 1.0, "tSample": 300}).to(DEV)
+    pool = layer.pool(2).to(DEV)
+    x = torch.randn((2, 3, 4, 6, 300), device=DEV).mul_(9).requires_grad_(True)
+    a = layer.psp(layer.spike(x * 1.0)) if pair == "pool of psp" else layer.psp(x * 1.0)
+    layer.srmKernel.mul_(2.0)
+    y = pool(a) if pair == "pool of psp" else layer.spike(a)
+    del a
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
