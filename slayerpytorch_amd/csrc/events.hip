@@ -57,10 +57,11 @@ __device__ __forceinline__ void bin_event(float *tensor, const float *base, int 
 // One work-group per (sample, slice of its events).  The polarity of a sample's events is shifted so
 // that its minimum over the WHOLE sample is 0 (event.__init__, src/spikeFileIO.py:33), so every
 // work-group first scans the polarity field of all events of its sample - until it has seen a 0, below which there is
-// nothing, mostly among the first 256.  One event per lane: the events of a batch are few, and a launch is as long as one
-// work-group's chain of loads.  (12 samples of 5000 events on (2, 34, 34, 300): scanning all and eight events a lane 15.4 us,
-// this 6.5.)
+// nothing, mostly among the first 256; in what follows every lane has kScan loads on their way between two looks.  A launch
+// is as long as one work-group's chain of loads.
 // table[s] = {first byte of the sample in `bytes`, number of events, time shift in bins}.
+constexpr int kScan = 8;     // events whose polarities a lane has on their way at once
+
 template <int FORMAT>
 __global__ __launch_bounds__(256) void bin_packed_events_kernel(float *tensor, const float *base,
                                                                 const uint8_t *__restrict__ bytes,
@@ -75,11 +76,20 @@ __global__ __launch_bounds__(256) void bin_packed_events_kernel(float *tensor, c
     // a table entry that does not lie inside the byte buffer is skipped as a whole
     if (first < 0 || nEvents < 0 || nEvents > (nBytes - first) / kBytes || first > nBytes) return;
 
-    int pmin = 255;
-    for (int64_t e0 = 0; e0 < nEvents; e0 += 256) {
-        const int64_t e = e0 + threadIdx.x;
-        if (e < nEvents) pmin = min(pmin, static_cast<int>(FORMAT == 3 ? ev[e * kBytes + 3] : (ev[e * kBytes + 2] >> 7)));
-        if (__syncthreads_or(pmin == 0)) break;
+    auto polarity = [&](int64_t e) {                   // (behind the last event: the last again)
+        e = min(e, nEvents - 1);
+        return static_cast<int>(FORMAT == 3 ? ev[e * kBytes + 3] : (ev[e * kBytes + 2] >> 7));
+    };
+    int pmin = nEvents > 0 ? polarity(threadIdx.x) : 0;
+    if (!__syncthreads_or(pmin == 0)) {
+        for (int64_t e0 = 256; e0 < nEvents; e0 += 256 * kScan) {
+            int p[kScan];
+#pragma unroll
+            for (int k = 0; k < kScan; ++k) p[k] = polarity(e0 + k * 256 + static_cast<int>(threadIdx.x));
+#pragma unroll
+            for (int k = 0; k < kScan; ++k) pmin = min(pmin, p[k]);
+            if (e0 + 256 * kScan >= nEvents || __syncthreads_or(pmin == 0)) break;
+        }
     }
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) pmin = min(pmin, __shfl_xor(pmin, off, kWave));
@@ -133,10 +143,17 @@ extern "C" int slayer_bin_packed_events_f32(float *tensor, const float *base, co
     if (!tensor || !bytes || !sampleTable) return SLAYER_EINVAL;
     if (mode == 1 && (!base || base == tensor)) return SLAYER_EINVAL;
     if (!base) base = tensor;
-    // slices per sample: one event per lane up to 4096 work-groups
+    // Slices per sample: one event per lane, up to 1024 work-groups and 2^23 scanned events - where a sample has no event of
+    // polarity 0, each of its work-groups scans all of it - then 2048 events per slice.  us, random / no 0 at all, against 2048 per
+    // slice and a scan that looks at every event: 12 samples of 5000 9.4, 9.4 -> 5.7, 7.5, 64 of them 14, 14 -> 9, 12, 500 48, 49 -> 45,
+    // 49; one of 10^6 events 902, 899 -> 13, 443.  One event per lane up to 4096 work-groups: those of 5000 6, 13 and 9, 20 and 45, 74;
+    // 14, 4049.
     int64_t slices = ceil_div(maxEvents, 256);
-    const int64_t most = ceil_div(4096, nSamples);
+    const int64_t coarse = ceil_div(maxEvents, 2048), most = ceil_div(1024, nSamples), scanned = (1 << 23) / nSamples / maxEvents;
     if (slices > most) slices = most;
+    if (slices > scanned) slices = scanned;
+    if (slices < coarse) slices = coarse;
+    if (slices > 1024) slices = 1024;
     if (nSamples * slices >= (1LL << 31)) return SLAYER_EUNSUPPORTED;
     const dim3 grid(static_cast<unsigned>(nSamples * slices));
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -180,3 +180,34 @@ def test_binning_on_a_side_stream():
     ref = oracle_tensor(raw, 2, (2, 34, 34, 350), 1.0)
     for k in range(3):
         assert np.array_equal(out[k].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("fmt", [1, 2, 3])
+@pytest.mark.parametrize("mode", ["OR", "SUM"])
+def test_the_lowest_polarity_wherever_it_first_occurs(fmt, mode):
+    """Polarities count from the lowest of the whole sample: its first event lies at every edge of the trips in which the
+    work-groups look for it (256 lanes, 2048 events), in the last one, or a sample has but one polarity."""
+    rng = np.random.default_rng(7 + fmt)
+    C, H, W, T, Ts = (4 if fmt == 3 else 2), (1 if fmt == 1 else 9), 12, 40, 1.0
+    at = 3 if fmt == 3 else 2
+    raws = []
+    for n, first in ((5000, 255), (5000, 256), (5000, 2047), (5000, 2048), (5000, 4096), (5000, 4999), (2048, 2047), (2049, 2048), (1, None),
+                     (300, None), (2048, None), (70000, 69999), (70000, None)):
+        raw = random_events(rng, fmt, n, W, H, C, T * 1000).reshape(n, -1)
+        if fmt == 3:
+            raw[:, at] = rng.integers(1, C, n)
+            if first is not None:
+                raw[first, at] = 0
+        else:
+            raw[:, at] |= 0x80
+            if first is not None:
+                raw[first:, at] &= np.where(rng.random(n - first) < 0.5, 0x7F, 0xFF).astype(np.uint8)
+                raw[first, at] &= 0x7F
+        raws.append(raw.reshape(-1))
+    base = rng.standard_normal((len(raws), C, H, W, T)).astype(np.float32)
+    for some in ([*range(len(raws))], [5], [11], [12], [9]):     # as one batch and alone: different numbers of work-groups
+        got = snn.io.toSpikeTensorBatch([snn.io.event._fromBytes(raws[i], fmt) for i in some], torch.from_numpy(base[some]).cuda(), Ts,
+                                        False, mode)
+        for k, i in enumerate(some):
+            ref = oracle_tensor(raws[i], fmt, (C, H, W, T), Ts, 0, mode, base[i])
+            assert np.array_equal(got[k].cpu().numpy().view(np.uint32), ref.view(np.uint32)), "sample %d" % i
