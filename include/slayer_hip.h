@@ -55,7 +55,8 @@ const char *slayer_last_hip_error(void);
 /*
  * Debug/validation knob, process wide: 0 (default) = tiled LDS kernels wherever the sizes
  * allow; 1 = always use the generic one-thread-per-sample / one-thread-per-neuron kernels
- * (the ones that also serve sizes the tiled kernels do not cover).  Both produce the same
+ * (the ones that also serve sizes the tiled kernels do not cover); 2 = the 3x3 gathers of a synapse with
+ * their source rows in a ring wherever the sizes allow, also where another kernel is faster.  All produce the same
  * results.  Returns the previous value.  No counterpart in the reference.
  */
 int slayer_force_generic_kernels(int on);

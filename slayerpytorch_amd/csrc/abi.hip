@@ -27,7 +27,8 @@ int compute_units()
     return cus;
 }
 
-bool generic_forced() { return g_force_generic.load(std::memory_order_relaxed) != 0; }
+bool generic_forced() { return g_force_generic.load(std::memory_order_relaxed) == 1; }
+bool rings_forced() { return g_force_generic.load(std::memory_order_relaxed) == 2; }
 
 }  // namespace slayer
 
@@ -48,5 +49,5 @@ extern "C" const char *slayer_last_hip_error(void) { return slayer::g_last_error
 
 extern "C" int slayer_force_generic_kernels(int on)
 {
-    return slayer::g_force_generic.exchange(on ? 1 : 0);
+    return slayer::g_force_generic.exchange(on == 2 ? 2 : on ? 1 : 0);
 }

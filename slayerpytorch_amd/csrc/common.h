@@ -22,6 +22,7 @@ int compute_units();
 
 // True when slayer_force_generic_kernels(1) is in effect.
 bool generic_forced();
+bool rings_forced();
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

@@ -362,6 +362,59 @@ static int launch_ring_one(const RingArgs &g, unsigned blocks, hipStream_t st)
     return launch_status();
 }
 
+// What this kernel and the planes kernel take, in hundredths of a microsecond: a launch whose busiest work-group walks so many
+// rows and multiplies under all but two of a unit's, a wavefront as many pixels of each as the strip has for it; and one whose
+// busiest work-group makes so many pairs of a block of pixels and a step.  A walk has the longer start - the weights into
+// registers, three rows before the first product - and where a call is small or an image so narrow that strips are mostly
+// empty, the planes kernel wins: planes / this, us, (1, 300), 32 -> 64 channels of 8 x 8, forward, 14 / 19, 16 -> 16 of 16 x 5,
+// input gradient, 7 / 11; (8, 300), 16 -> 32 of 64 x 1, forward, 39 / 45; but 16 -> 32 of 16 x 16, (12, 300), forward, 87 / 76.
+// Fitted to 260 sizes (1 to 32 items, 1 to 24 pixels, 20 to 1450 samples, spikes and full samples, each instance by itself);
+// none of those sizes is more than 8 % slower this way than by the planes kernel, and none more than 15 % slower than by the
+// better of the two.
+struct RingCost {
+    int planes, pair, walk, row, pixel;
+};
+
+static RingCost ring_gather_cost(int P, int TW, int NT, bool two, bool backward)   // two: tiles of the planes kernel's work-group
+{
+    RingCost c{};
+    if (P == 1) {
+        c.planes = backward ? (two ? 385 : 421) : (two ? 581 : 466);
+        c.pair = backward ? (two ? 457 : 295) : (two ? 355 : 272);
+        if (TW == 1) { c.walk = backward ? 710 : 841; c.row = backward ? 52 : 65; c.pixel = backward ? 80 : 59; }
+        else { c.walk = backward ? 729 : 1281; c.row = backward ? 101 : 69; c.pixel = backward ? 129 : 104; }
+    } else {
+        c.planes = backward ? (two ? 565 : 449) : (two ? 752 : 491);
+        c.pair = backward ? (two ? 728 : 541) : (two ? 645 : 523);
+        if (NT == 1) { c.walk = backward ? 783 : 1139; c.row = 121; c.pixel = backward ? 36 : 33; }
+        else if (NT == 2) { c.walk = backward ? 892 : 1196; c.row = backward ? 75 : 81; c.pixel = backward ? 122 : 92; }
+        else { c.walk = backward ? 1000 : 1273; c.row = 64; c.pixel = backward ? 139 : 112; }
+    }
+    return c;
+}
+
+// Pairs of eight pixels of a row and a step that the planes kernel's busiest work-group makes (launch_gather_mfma).
+static int64_t planes_pairs(const RingGeom &s)
+{
+    const int64_t pairs = static_cast<int64_t>(s.N) * s.DH * ceil_div(s.DW, 8) * ((s.T + 31) / 32);
+    int64_t slices = 252 / (static_cast<int64_t>(s.groups) * ceil_div(s.Mg, s.Mg >= 32 ? 32 : 16));
+    if (slices < 1) slices = 1;
+    return ceil_div(pairs, slices < pairs ? slices : pairs);
+}
+
+// What the busiest work-group of a walk takes; `most`: pixels of a whole strip that a multiplying wavefront has
+static int64_t walk_cost(const RingArgs &g, const RingCost &c, int most)
+{
+    const int64_t units = ceil_div(g.units, g.workers), last = g.s.DW - static_cast<int64_t>(g.strips - 1) * ring_pixels(g.s.Qg / 16);
+    const int64_t pixels = static_cast<int64_t>(g.strips - 1) * most + (last < most ? last : most);   // of a row of the image
+    return c.walk + units * (g.segRows + 2) * c.row + units * g.segRows * c.pixel * pixels / g.strips;
+}
+
+static bool ring_pays(const RingArgs &g, const RingCost &c, int most, int64_t pairs)
+{
+    return walk_cost(g, c, most) < c.planes + pairs * c.pair;
+}
+
 template <bool BACKWARD>
 int launch_gather_ring(const RingGeom &s, hipStream_t st)
 {
@@ -377,10 +430,6 @@ int launch_gather_ring(const RingGeom &s, hipStream_t st)
     g.strips = static_cast<int>(ceil_div(s.DW, PX));
     const int64_t base = static_cast<int64_t>(s.groups) * g.oGroups;
     const int64_t columns = static_cast<int64_t>(s.N) * g.steps * g.strips;
-    // Few columns of the wide strips mean short segments, whose first rows are staged for nothing: the planes kernel then wins
-    // the forward pass, whose rows are long to multiply (columns: planes / this: (5, 14x18, 173), 90: 29 / 38 us; (8, 16x16,
-    // 300), 160: 55 / 58; (12, 16x16, 300), 240: 87 / 76), but not the input gradient (90: 34 / 30).
-    if (!BACKWARD && P == 1 && columns < 200) return SLAYER_EUNSUPPORTED;
     int64_t workers = compute_units() / base;
     if (workers < 1) workers = 1;
     // The units are columns of the image, cut into the number of segments with the fewest rows to walk for the work-group with
@@ -398,6 +447,7 @@ int launch_gather_ring(const RingGeom &s, hipStream_t st)
     g.units = static_cast<int>(units);
     if (workers > units) workers = units;
     g.workers = static_cast<int>(workers);
+    if (!rings_forced() && !ring_pays(g, ring_gather_cost(P, TW, NT, s.Mg >= 32, BACKWARD), PX * NT / kRgMul, planes_pairs(s))) return SLAYER_EUNSUPPORTED;
     const int64_t blocks = base * workers;
     if (blocks >= (1LL << 22)) return SLAYER_EUNSUPPORTED;
     g.byOGroups = make_fastdiv(static_cast<uint32_t>(g.oGroups));
@@ -673,6 +723,36 @@ __global__ __launch_bounds__(512) void synapse_wgrad_ring_kernel(RingArgs g, flo
     }
 }
 
+// The walk against the kernel with the patch of four pixels (plan_wgrad_lds), from 60 steps of a pixel per compute unit on, as in
+// the gather: full samples, spikes, patch against this, us: 15 steps, 32 -> 64 channels of 7 x 9, (5, 173), 38, 29 against 38,
+// 33; 17 x 17, 16 -> 32, (32, 64), 75, 72 against 66, 53; 16 x 16, 32 -> 96, (8, 100), 139, 97 against 124, 95; narrow images,
+// under which wavefronts stand by: 32 x 3, 16 -> 32, (4, 1450), 76, 51 against 77, 72; 64 x 2, 16 -> 16, (32, 100), 67, 53 against
+// 62, 58.  Both leave rows of sums, `add` the time of adding up a million of them.  A twentieth in favour of the patch.  It
+// does not take rows of less than 16 samples; the vector kernel against this, us: 16 -> 32 channels of 16 x 16, (64, 8), 97, 97
+// against 41, 35; of 32 x 32, (16, 4), 35, 35 against 41, 35.
+static bool ring_wgrad_pays(const RingArgs &g, int P, int OT)
+{
+    const RingGeom &s = g.s;
+    const int64_t base = static_cast<int64_t>(s.groups) * g.oGroups;
+    if (s.T < 8 || static_cast<int64_t>(s.N) * g.steps * s.DH * s.DW * base < 60 * 256) return false;
+    if (s.T < 16) return true;
+    struct Cost {
+        RingCost c;
+        int addPatch, addWalk;
+    };
+    const Cost c = P == 1 ? OT == 1 ? Cost{{545, 290, 790, 73, 45}, 1110, 880} : Cost{{585, 225, 935, 92, 82}, 620, 470}
+                          : OT == 1 ? Cost{{590, 330, 612, 119, 22}, 475, 543} : Cost{{730, 266, 962, 86, 85}, 405, 442};
+    // the patch kernel's column groups: at most nine tiles of 16 columns beside one tile of output channels, six beside two
+    const int64_t colGroups = P == 1 ? OT : OT + 1;
+    const int64_t pairs = static_cast<int64_t>(s.N) * s.DH * ceil_div(s.DW, 4) * g.steps, nW = static_cast<int64_t>(s.groups) * s.Mg * s.Qg * 9;
+    int64_t slices = 504 / (base * colGroups);
+    if (slices < 1) slices = 1;
+    if (slices > pairs) slices = pairs;
+    const int64_t patch = c.c.planes + ceil_div(pairs, slices) * c.c.pair + slices * nW * c.addPatch / 1000000;
+    const int64_t walk = walk_cost(g, c.c, ring_pixels(P) * P / kRgMul) + g.workers * nW * c.addWalk / 1000000;
+    return walk * 21 < patch * 20;
+}
+
 // Tiles and walk of the weight gradient; false where the kernel does not take the geometry.
 static bool plan_wgrad_ring(const RingGeom &s, RingArgs &g, int &P, int &OT)
 {
@@ -699,14 +779,10 @@ static bool plan_wgrad_ring(const RingGeom &s, RingArgs &g, int &P, int &OT)
     g.segs = static_cast<int>(ceil_div(s.DH, g.segRows));
     const int64_t units = columns * g.segs;
     if (units < 1 || units >= (1LL << 30) || base >= (1LL << 20)) return false;
-    // Work for the ring to pay: 60 steps of a pixel per compute unit.  Full samples, spikes, the kernel with the patch against
-    // this: 72 steps, 16 -> 32 channels of 17 x 17, (32, 64), 75, 72 against 66, 53 us; 96, 32 -> 96 of 16 x 16, (8, 100), 139, 97
-    // against 124, 95; 47, 16 -> 32 of 14 x 18, (8, 173), 53, 40 against 50, 42; 15, 32 -> 64 of 7 x 9, (5, 173), 38, 29
-    // against 38, 33.
-    if (static_cast<int64_t>(s.N) * g.steps * s.DH * s.DW * base < 60 * 256) return false;
     g.units = static_cast<int>(units);
     if (workers > units) workers = units;
     g.workers = static_cast<int>(workers);
+    if (!ring_wgrad_pays(g, P, OT)) return false;
     g.byOGroups = make_fastdiv(static_cast<uint32_t>(g.oGroups));
     g.byGroups = make_fastdiv(static_cast<uint32_t>(s.groups));
     g.bySteps = make_fastdiv(static_cast<uint32_t>(g.steps));

@@ -273,11 +273,13 @@ def test_rows_of_any_length_and_alignment(layer, T, impl):
 @pytest.mark.parametrize("H,T", [(19, 300), (6, 1001)])
 def test_tensors_beyond_the_last_level_cache_are_taken_in_bands(H, T):
     """Large tensors are walked in bands of four rows of pixels (the last one shorter), small ones image by image: the same
-    products in the same order per element, so every image of a large batch has the bits it has alone."""
-    N = 1 + (1 << 28) // (4 * T * (16 + 32) * H * 16)
+    products in the same order per element, so every image of a large batch has the bits it has alone.  (48 channels on either
+    side: three passes, which no kernel takes that keeps its source rows in a ring.)"""
+    C = 48
+    N = 1 + (1 << 28) // (4 * T * (C + C) * H * 16)
     gen = torch.Generator(device="cuda").manual_seed(3)
-    w = torch.randn((32, 16, 3, 3), device="cuda", generator=gen)
-    x = torch.randn((N, 16, H, 16, T), device="cuda", generator=gen)
+    w = torch.randn((C, C, 3, 3), device="cuda", generator=gen)
+    x = torch.randn((N, C, H, 16, T), device="cuda", generator=gen)
     y = synapse.conv(x, w, 1, 1)
     gx = synapse.convGradInput(y, w, x.shape, 1, 1)
     for n in (0, 1, N // 2, N - 1):
@@ -951,15 +953,52 @@ def test_dense_layer_with_few_outputs_keeps_what_torch_does_with_a_product(O, T)
             assert fc(x).dtype == torch.float16
 
 
+@pytest.fixture
+def rings():
+    """The 3x3 gathers with their source rows in a ring wherever they take the sizes, also where another kernel is faster."""
+    lib = _lib.load()
+    old = lib.slayer_force_generic_kernels(2)
+    yield
+    lib.slayer_force_generic_kernels(old)
+
+
+def test_small_and_narrow_images_leave_the_ring(rings):
+    """Gathers whose walk would be short, or whose strips of columns mostly empty, go by the planes kernel: 18 to 27 us where
+    the ring takes 1.4 to 1.6 times as long."""
+    def best(call):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        call()
+        times = []
+        for _ in range(5):
+            start.record()
+            for _ in range(40):
+                call()
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    lib = _lib.load()
+    for N, C, O_, H, W, T, backward in ((4, 16, 32, 1, 32, 1450, False), (4, 16, 32, 1, 32, 1450, True), (4, 32, 32, 1, 32, 1450, False)):
+        x, w = torch.zeros((N, C, H, W, T), device="cuda"), torch.ones((O_, C, 3, 3), device="cuda")
+        g = synapse.conv(x, w, 1, 1)
+        call = (lambda: synapse.convGradInput(g, w, x.shape, 1, 1)) if backward else (lambda: synapse.conv(x, w, 1, 1))
+        ring = best(call)
+        lib.slayer_force_generic_kernels(0)
+        assert best(call) < 0.92 * ring, (N, C, O_, H, W, T, backward)
+        lib.slayer_force_generic_kernels(2)
+
+
 @pytest.mark.parametrize("N,C,O,groups,H,W,T,pad,spikes", [
     (70, 16, 32, 1, 3, 9, 40, 1, False), (70, 16, 32, 1, 3, 9, 40, 1, True), (100, 16, 16, 1, 2, 3, 33, 1, False),
     (35, 32, 96, 2, 4, 17, 65, 2, False), (2, 32, 16, 1, 1, 4, 32, 1, False), (3, 32, 32, 1, 5, 7, 100, 0, False),
     (2, 32, 80, 1, 6, 5, 173, 3, True), (1, 64, 32, 2, 19, 6, 300, 1, False), (40, 16, 48, 1, 7, 8, 173, 1, False)])
-def test_gathers_with_the_source_rows_in_a_ring(N, C, O, groups, H, W, T, pad, spikes):
+def test_gathers_with_the_source_rows_in_a_ring(N, C, O, groups, H, W, T, pad, spikes, rings):
     """3x3 filters with 16 or 32 source channels per group: strips that end within the image and beyond it, one row, segments
     of a column, one unit per work-group and several, rows that are no whole vectors, paddings up to the filter's extent,
     tiles of channels that are partly there.  Forward pass and input gradient within SUM_TOL of the sum of their terms'
-    magnitudes, the latter also of a tensor with an infinity, which reaches what it reaches in a sum."""
+    magnitudes, both also of a tensor with an infinity, which reaches what it reaches in a sum, and the forward pass of one with
+    numbers next to the largest, whose sums are finite."""
     import torch.nn.functional as F
     from slayerpytorch_amd import synapse as S
     gen = torch.Generator().manual_seed(N + C + O + H + W + T)
@@ -970,6 +1009,21 @@ def test_gathers_with_the_source_rows_in_a_ring(N, C, O, groups, H, W, T, pad, s
     want, scale = F.conv3d(xd, wd, None, 1, pads, 1, groups), F.conv3d(x.double().abs(), wd.abs(), None, 1, pads, 1, groups)
     got = S.conv(x.cuda(), w.cuda(), 1, pad, 1, groups).cpu().double()
     assert bool(((got - want.detach()).abs() <= SUM_TOL * scale + 1e-30).all())
+    n, a, b, t = N - 1, H // 2, W - 1, T - 1          # an infinity in the last channel
+    odd = x.clone()
+    odd[n, C - 1, a, b, t] = float("inf")
+    got = S.conv(odd.cuda(), w.cuda(), 1, pad, 1, groups).cpu()
+    reached = torch.zeros(want.shape, dtype=torch.bool)
+    first = (groups - 1) * (O // groups)
+    reached[n, first:, max(0, a + pad - 2):a + pad + 1, max(0, b + pad - 2):b + pad + 1, t] = True
+    assert torch.equal(~torch.isfinite(got), reached)
+    assert bool(((got.double() - want.detach()).abs() <= SUM_TOL * scale + 1e-30)[~reached].all())
+    odd[n, C - 1, a, b, t], odd[0, 0, 0, 0, 0] = 3.4e38, -3.39e38
+    small = 0.01 * w
+    want2, scale2 = (F.conv3d(v, u, None, 1, pads, 1, groups) for v, u in ((odd.double(), small.double()[..., None]),
+                                                                          (odd.double().abs(), small.double().abs()[..., None])))
+    got = S.conv(odd.cuda(), small.cuda(), 1, pad, 1, groups).cpu().double()
+    assert bool(((got - want2).abs() <= SUM_TOL * scale2 + 1e-30).all())
     g = torch.randn(want.shape, generator=gen)
     (wantG,) = torch.autograd.grad(want, xd, g.double())
     xs = x.double().requires_grad_(True)
