@@ -518,7 +518,7 @@ int slayer_dense_rows_grad_weight_f32(float *gradW, const float *gradOut, const 
 
 /*
  * The same product and its two gradients for few outputs (O <= 32) and any other extents whose 16-byte vectors number
- * below 2^30: fp32 multiply-adds from tensors of any 4-byte alignment, sums of fixed order.  `workspace` of the product and
+ * below 2^30: fp32 arithmetic (the product on matrix instructions) on tensors of any 4-byte alignment, sums of fixed order.  `workspace` of the product and
  * of the weight gradient holds slayer_dense_thin_workspace_bytes bytes (gradWeight = 0 / 1; may be 0: NULL).
  */
 int slayer_dense_thin_supported(int64_t N, int64_t K, int64_t O, int64_t T);

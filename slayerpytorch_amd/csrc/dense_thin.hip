@@ -1,11 +1,12 @@
 // Fully connected synapse with few outputs (up to 32): the output layers of the reference's networks
 // (slayer._denseLayer, src/slayer.py:393-440), out[n][o][t] = sum_k W[o][k] x[n][k][t] and its two gradients.
 //
-// With O outputs a sample of x meets O multiply-adds: at O = 10 five operations a byte, far below what the vector ALUs
-// do in the time the byte takes to arrive, and the small layers are one launch's latency.  So plain fp32 multiply-adds
-// straight from memory, time on the lanes as everywhere (one 16-byte vector of samples each): no tiles of 16 outputs that
-// are partly empty, no transposed copies, and enough work-groups whatever the batch is, since the inputs k are split over
-// wavefronts and work-groups.  All sums are added in a fixed order.
+// With O outputs a sample of x meets O multiply-adds: at O = 10 five operations a byte, far below what the chip does in the
+// time the byte takes to arrive, and the small layers are one launch's latency.  So fp32 arithmetic straight from memory, time
+// on the lanes as everywhere (one 16-byte vector of samples each), no transposed copies, and enough work-groups whatever the
+// batch is, since the inputs k are split over wavefronts and work-groups: the product on fp32 matrix instructions (tiles of 16
+// outputs; those that are not there cost no memory), the gradients as multiply-adds of the vector ALUs.  All sums are added
+// in a fixed order.
 //
 // Rows that are not whole vectors: the last vector of a row starts at sample T - 4 and overlaps the one before; product and
 // input gradient store the shared samples twice with the same values, the weight gradient counts them once.
@@ -52,7 +53,9 @@ __device__ __forceinline__ int thin_start(int tv, int T) { return VEC == 4 ? min
 // with one 16-byte load, and the vector r of rows k + 4 h .. + 3 with four, which is 4 VEC instructions' worth of operands (a
 // vector's four samples are columns of four products).  Neither needs LDS, and two steps of loads are in flight while a
 // wavefront multiplies (four times as many: no faster, (64, 256, 2000) -> 8 27 -> 40 us).  A work-group owns 16 vectors (of any items) and a range of inputs, 16 at a time per
-// wavefront; the wavefronts' sums meet in LDS in three steps.  Vector instructions with the weights as broadcasts from LDS
+// wavefront; the wavefronts' sums meet in LDS in three steps.  Its pieces of the rows end within memory lines that the next
+// work-group reads too, so neighbours run on one die: in the order of their numbers 4096 -> 10 on (12, 300) 19 us, this 16;
+// 30000 -> 10 on (4, 300) 62, 32; 4096 -> 10 on (64, 300) 73, 66.  Vector instructions with the weights as broadcasts from LDS
 // or the scalar cache: 512 -> 11 on (8, 300) 10.2 us, 4096 -> 10 on (64, 300) 76.
 constexpr int kDtSteps = 1;                            // steps of 16 inputs in each of a wavefront's two sets of registers
 constexpr int kDtChunk = kDtWaves * kDtSteps * 16;     // inputs of a work-group's trip
@@ -63,8 +66,9 @@ __global__ __launch_bounds__(64 * kDtWaves) void dense_thin_kernel(ThinArgs p)
     typedef typename ThinVec<VEC>::V V;
     __shared__ __align__(16) f32x4 lds[kDtWaves / 2 * OT * VEC * 64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, h = lane >> 4;
-    const int split = static_cast<int>(fastdiv(blockIdx.x, p.byVecBlocks));
-    const int v = (static_cast<int>(blockIdx.x) - split * static_cast<int>(p.byVecBlocks.d)) * 16 + r;
+    const uint32_t block = xcd_contiguous(blockIdx.x, gridDim.x);   // neighbours share memory lines
+    const int split = static_cast<int>(fastdiv(block, p.byVecBlocks));
+    const int v = (static_cast<int>(block) - split * static_cast<int>(p.byVecBlocks.d)) * 16 + r;
     const bool live = v < p.vectors;
     const int n = static_cast<int>(fastdiv(static_cast<uint32_t>(live ? v : 0), p.byTV));
     const int t = thin_start<VEC>((live ? v : 0) - n * p.TV, p.T);
@@ -191,8 +195,9 @@ __global__ __launch_bounds__(512) void dense_thin_grad_input_kernel(ThinArgs p, 
     for (int k = k0; k < k1; k += KC) {
         const int kc = min(KC, k1 - k);
         __syncthreads();
-        for (int e = threadIdx.x; e < KC * OB; e += blockDim.x) {
-            const int o = e / KC, i = e - o * KC;
+        const int shift = kc <= 8 ? 3 : kc <= 16 ? 4 : 6;   // (a few inputs: a few weights)
+        for (int e = threadIdx.x; e < OB << shift; e += blockDim.x) {
+            const int o = e >> shift, i = e & ((1 << shift) - 1);
             lds[i * OB + o] = (o < p.O && i < kc) ? p.w[static_cast<int64_t>(o) * p.K + k + i] : 0.0f;
         }
         __syncthreads();
@@ -340,7 +345,7 @@ struct ThinPlan {
     int wSplits, wPerSplit, kBlocks;   // weight gradient, over the blocks of 64 vectors; blocks of inputs
 };
 
-constexpr int kDtKB = 4;
+constexpr int thin_inputs(int O) { return O <= 16 ? 4 : 1; }   // of a wavefront of the weight gradient
 constexpr int kDtOneLaunch = 1024, kDtBlocks = 2048;
 
 static bool thin_plan(int64_t N, int64_t K, int64_t O, int64_t T, ThinPlan &p)
@@ -354,7 +359,7 @@ static bool thin_plan(int64_t N, int64_t K, int64_t O, int64_t T, ThinPlan &p)
     p.vecBlocks = (p.vectors + 63) / 64;
     // The product: vectors of four samples unless there are so few that most compute units would stand by (one / four samples:
     // 512 -> 11 on (8, 300), 600 vectors, 4.0 / 6.2 us; 512 -> 10 on (12, 350), 1056, 5.6 / 6.2; 4096 -> 10 on (12, 300), 900,
-    // 29 / 20; 512 -> 16 on (32, 350) 12.7 / 7.6).  One work-group of eight wavefronts per 16 vectors while the inputs are few
+    // 29 / 20 (before neighbours shared a die); 512 -> 16 on (32, 350) 12.7 / 7.6).  One work-group of eight wavefronts per 16 vectors while the inputs are few
     // (a second launch costs more than a longer one), then as many ranges of inputs as give eight work-groups per compute unit.
     p.fwdVec = VEC == 4 && p.vectors >= 800 ? 4 : 1;
     p.fwdTV = p.fwdVec == 4 ? p.TV : static_cast<int>(T);
@@ -364,9 +369,10 @@ static bool thin_plan(int64_t N, int64_t K, int64_t O, int64_t T, ThinPlan &p)
     const int64_t per = ceil_div(ceil_div(K, splits), kDtChunk) * kDtChunk;
     p.perSplit = static_cast<int>(per);
     p.splits = static_cast<int>(ceil_div(K, per));
-    // The weight gradient: 32 inputs per work-group; as many ranges of vectors as give about 1024 work-groups, at least
+    // The weight gradient: 32 inputs per work-group, 8 where there are more than 16 outputs (a wavefront's sums, 32 per input,
+    // meet in one butterfly: 250 -> 25 at (1, 500) 9.8 -> 5.4 us, 512 -> 32 at (4, 500) 12.0 -> 7.9); as many ranges of vectors as give about 1024 work-groups, at least
     // two blocks of 64 vectors in each
-    p.kBlocks = static_cast<int>(ceil_div(K, kDtWaves * kDtKB));
+    p.kBlocks = static_cast<int>(ceil_div(K, kDtWaves * thin_inputs(static_cast<int>(O))));
     splits = ceil_div(1024, p.kBlocks);
     const int64_t mostW = ceil_div(p.vecBlocks, 2);
     splits = splits < 1 ? 1 : splits > mostW ? mostW : splits;
@@ -454,13 +460,14 @@ extern "C" int slayer_dense_thin_grad_input_f32(float *gradIn, const float *weig
     hipStream_t st = static_cast<hipStream_t>(stream);
     ThinArgs a = thin_args(p, N, K, O, T);
     a.w = weight; a.x = gradOut; a.out = gradIn;
-    // whole rows per work-group (as many items as 512 lanes hold, no more than give 256 work-groups their inputs), or pieces
-    // of 512 vectors of long ones; the inputs of a batch of few vectors are cut until there are about 1024 work-groups
+    // Whole rows per work-group (as many items as 512 lanes hold), or pieces of 512 vectors of long ones; the inputs of a
+    // batch of few vectors are cut until there are about 1024 work-groups or eight inputs in each, four where a lane has up to
+    // 32 outputs to multiply for each (250 -> 25 at (1, 500): 7.2 -> 4.5 us, with the weights read for those inputs alone).
     int vecs = 512;
     if (p.TV <= 512) vecs = static_cast<int>(p.TV * (512 / p.TV < N ? 512 / p.TV : N));
     const int vecBlocks = (p.vectors + vecs - 1) / vecs;
     int64_t splits = ceil_div(1024, vecBlocks);
-    const int64_t most = ceil_div(K, 8);
+    const int64_t most = ceil_div(K, O <= 16 ? 8 : 4);
     splits = splits < 1 ? 1 : splits > most ? most : splits;
     a.perSplit = static_cast<int>(ceil_div(K, splits));
     a.splits = static_cast<int>(ceil_div(K, a.perSplit));
@@ -488,7 +495,7 @@ extern "C" int slayer_dense_thin_grad_weight_f32(float *gradW, const float *grad
     a.byVecBlocks = make_fastdiv(static_cast<uint32_t>(p.kBlocks));
     const dim3 grid(static_cast<unsigned>(p.kBlocks * p.wSplits)), block(64 * kDtWaves);
     const bool vec = T >= 4;
-#define SLAYER_THIN_GW(OB, VEC, G, B, A) hipLaunchKernelGGL((dense_thin_wgrad_kernel<OB, kDtKB, VEC>), G, B, 0, st, A)
+#define SLAYER_THIN_GW(OB, VEC, G, B, A) hipLaunchKernelGGL((dense_thin_wgrad_kernel<OB, thin_inputs(OB), VEC>), G, B, 0, st, A)
     SLAYER_THIN(SLAYER_THIN_GW, grid, block, a);
 #undef SLAYER_THIN_GW
     const int status = launch_status();

@@ -627,13 +627,15 @@ def denseThinGradWeight(gradOutput, input):
 def denseThinPays(N, K, O, T):
     """Whether the layer's product (N, K, T) -> (N, O, T) is taken by the kernels for few outputs: up to 16, or up to 32 where
     the layer is so small that its launches count more than its work."""
-    # (us, ours / library: 4096 -> 10 at (1, 300) 6 / 14, (12, 300) 20 / 24, (64, 300) 75 / 82; 5760 -> 10 at (5, 173) 15 / 22;
-    # 512 -> 10 at (1, 350) 4.1 / 5.7, (12, 350) 6 / 8; 250 -> 25 at (1, 500) 4.3 / 5.9; 400 -> 25 at (32, 500) 18 / 9.
-    # Input gradient: 4096 -> 10 at (12, 300) 14 / 33, (64, 300) 66 / 134; 512 -> 10 at (12, 350) 5 / 12; 512 -> 11 at
-    # (4, 1450) 6 / 9; 256 -> 8 at (64, 2000) 23 / 58; 250 -> 25 at (1, 500) 7 / 5; 4096 -> 32 at (16, 300) 38 / 37.  Weight
-    # gradient: 4096 -> 10 at (12, 300) 18 / 27, (64, 300) 65 / 94; 512 -> 10 at (1, 350) 6 / 8, (12, 350) 8 / 12; 250 -> 25 at
-    # (1, 500) 10 / 25; 400 -> 25 at (32, 500) 24 / 20.  On the host a product of the library's and its gradients take 90 us,
-    # these 30.)
+    # (us on the GPU, the same tensors again and again, ours / library: 4096 -> 10 at (1, 300) 5.4 / 14, (12, 300) 16 / 24,
+    # (64, 300) 66 / 82, (256, 300) 250 / 228; 5760 -> 10 at (5, 173) 9.4 / 22; 512 -> 10 at (1, 350) 3.8 / 5.5, (12, 350) 5.9 /
+    # 8.2; 256 -> 8 at (64, 2000) 24 / 25; 2048 -> 16 at (64, 300) 34 / 40; 1024 -> 16 at (128, 1000) 105 / 93.  Input gradient: 4096 -> 10 at (12, 300) 13 / 32, (64, 300) 65 / 130;
+    # 512 -> 10 at (12, 350) 5.1 / 12; 512 -> 11 at (4, 1450) 5.6 / 9.0; 256 -> 8 at (64, 2000) 23 / 57.  Weight gradient: 4096 ->
+    # 10 at (12, 300) 19 / 27, (64, 300) 64 / 94; 512 -> 10 at (1, 350) 5.6 / 7.6, (12, 350) 8.3 / 12; 2048 -> 16 at (64, 300)
+    # 45 / 40.  More than 16 outputs, product; input gradient; weight gradient: 250 -> 25 at (1, 500) 3.7 / 5.7; 4.5 / 4.2; 5.4 /
+    # 25; 512 -> 32 at (4, 500) 5.0 / 6.5; 5.8 / 5.6; 7.9 / 8.4; 1024 -> 17 at (1, 300) 6.0 / 7.2; 4.6 / 4.6; 5.4 / 7.6; 4096 -> 32
+    # at (1, 250) 6.4 / 24; 5.5 / 6.0; 5.5 / 8.5; 300 -> 20 at (1, 37) 3.8 / 6.9; 4.8 / 4.1; 4.2 / 6.7: of 27 such sizes up to the
+    # limit none is slower in all three together.  On the host a product of the library's and its gradients take 90 us, these 30.)
     return (O <= 16 or (O <= 32 and N * K * T <= 1 << 20)) and bool(_lib.load().slayer_dense_thin_supported(N, K, O, T))
 
 
@@ -653,8 +655,6 @@ class _synapseDenseThinFunction(Function):
     @staticmethod
     def forward(ctx, input, weight):
         ctx.save_for_backward(input, weight)
-        N, K, T = input.shape
-        O = weight.shape[0]
         return denseThin(input, weight.contiguous())
 
     @staticmethod

@@ -884,7 +884,8 @@ def test_weight_gradient_sums_are_rounded_and_not_cut(N, C, O_, H, K, pad, T, ki
 
 @pytest.mark.parametrize("N,K,O,T", [(1, 1, 1, 1), (2, 3, 2, 3), (1, 25, 1, 500), (1, 250, 25, 501), (3, 65, 4, 4), (2, 513, 5, 37),
                                      (5, 129, 8, 130), (12, 512, 10, 350), (3, 1500, 12, 173), (1, 2100, 13, 300), (2, 700, 16, 2053),
-                                     (1, 100, 17, 9), (2, 600, 31, 66), (1, 520, 32, 1450)])
+                                     (1, 100, 17, 9), (2, 600, 31, 66), (1, 520, 32, 1450),
+                                     (70, 130, 20, 1030), (256, 70, 7, 1028), (87040, 130, 1, 3)])   # 9, 18, 64 + 1 inputs a group
 def test_dense_layers_with_few_outputs(N, K, O, T):
     """Product and gradients for few outputs against sums in double precision: every element within 1e-6 of the sum of its
     terms' magnitudes (chains of at most 16384 additions, split over wavefronts: each partial sum has at most 8 + 128
