@@ -642,7 +642,7 @@ def denseThinPays(N, K, O, T):
 def plainTensors(*tensors):
     """Whether nothing but autograd looks at operations on these tensors: no transform, no forward-mode derivative, no
     tracing or compiling, no autocast, no mode and no subclass that an autograd Function would hide the operation from."""
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+    return (host.unwrapped(*tensors)
             and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and not torch.is_autocast_enabled("cuda") and torch._C._get_tracing_state() is None
@@ -650,7 +650,8 @@ def plainTensors(*tensors):
 
 
 class _synapseDenseThinFunction(Function):
-    """The product and its gradients for few outputs.  A backward pass that is itself recorded (``create_graph``) is torch's."""
+    """The product and its gradients for few outputs.  A backward pass that is itself recorded (``create_graph``), or whose
+    gradients are not plain tensors (``is_grads_batched``), is torch's."""
 
     @staticmethod
     def forward(ctx, input, weight):
@@ -663,7 +664,7 @@ class _synapseDenseThinFunction(Function):
         gradInput = gradWeight = None
         N, K, T = input.shape
         O = weight.shape[0]
-        own = not torch.is_grad_enabled() and gradOutput.dtype == torch.float32
+        own = not torch.is_grad_enabled() and gradOutput.dtype == torch.float32 and plainTensors(gradOutput, input, weight)
         if own:
             gradOutput = gradOutput.contiguous()
         if ctx.needs_input_grad[0]:
@@ -673,7 +674,7 @@ class _synapseDenseThinFunction(Function):
                 gradInput = torch.bmm(weight.t().unsqueeze(0).expand(N, K, O), gradOutput)
         if ctx.needs_input_grad[1]:
             if own:
-                gradWeight = denseThinGradWeight(gradOutput, input)
+                gradWeight = denseThinGradWeight(gradOutput, input.contiguous())
             else:
                 gradWeight = torch.bmm(gradOutput, input.transpose(1, 2)).sum(0)
         return gradInput, gradWeight

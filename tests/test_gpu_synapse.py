@@ -943,6 +943,12 @@ def test_dense_layer_with_few_outputs_keeps_what_torch_does_with_a_product(O, T)
     gd = 2 * torch.einsum("ok,not->nkt", w.reshape(O, 600), yd)
     (want,) = torch.autograd.grad(gd.square().sum(), w)
     assert float((again.double() - want).norm() / want.norm()) < 1e-5
+    y = fc(x)
+    some = torch.randn((3,) + y.shape, device="cuda")
+    several = torch.autograd.grad(y, (x, fc.weight), some, is_grads_batched=True, retain_graph=True)
+    for k in range(3):
+        for got, one in zip(several, torch.autograd.grad(y, (x, fc.weight), some[k], retain_graph=True)):
+            assert got[k].shape == one.shape and float((got[k] - one).norm() / one.norm()) < 1e-6
     import torch.autograd.forward_ad as fwAD
     with fwAD.dual_level(), torch.no_grad():
         out = fwAD.unpack_dual(fc(fwAD.make_dual(x.detach(), torch.ones_like(x))))
