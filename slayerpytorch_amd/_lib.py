@@ -149,6 +149,8 @@ class _Host:
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_slayer_host", loader))
         loader.exec_module(module)
         self.__dict__.update((k, v) for k, v in vars(module).items() if not k.startswith("__"))
+        if name not in self.__dict__:
+            raise AttributeError("%s has no function %r" % (HOST_PATH, name))
         return self.__dict__[name]
 
 

@@ -283,6 +283,13 @@ def test_plans_are_kept_for_whole_numbers_only():
     assert synapse.outShape(a, w, (stride, 1)) == (1, 4, 4, 7, 8)
 
 
+def test_an_unknown_name_of_the_native_calls_is_an_attribute_error():
+    assert hasattr(_lib._Host(), "conv2d") and not hasattr(_lib._Host(), "conv4d")
+    assert getattr(_lib.host, "conv4d", None) is None
+    with pytest.raises(AttributeError, match="conv4d"):
+        _lib.host.conv4d
+
+
 def test_pool_layer_extends_odd_extents_by_zeros():
     """The pooled tensor and its gradient for odd heights and widths, against the extension that the layer stands for."""
     from slayerpytorch_amd import slayer, synapse
