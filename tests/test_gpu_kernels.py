@@ -1402,6 +1402,17 @@ def test_the_plain_case_of_a_call_equals_the_general_path(monkeypatch):
     assert host.conv(x, f, t(1)) is None and host.conv(x, f, True) is None and host.conv(x, f) is None
     assert host.spikeBackward(x, u[:1].contiguous(), 1.0, 1.0, 1.0) is None
     assert host.conv2d(x, w, -1, 0, 1, 1) is None and host.conv2d(x, w, 1, 0, 1, 2) is None
+    for shape, wShape, stride, pad, dil, groups in (((2, 6, 5, 7, 40), (4, 3, 3, 2), (2, 1), 1, 1, 2), ((1, 16, 6, 9, 33), (32, 16, 3, 3, 1), 1, (1, 0), 1, 1),
+                                                    ((2, 4, 9, 8, 13), (6, 2, 3, 3, 1), 1, 2, (2, 1), 2), ((3, 2, 8, 8, 20), (16, 2, 5, 5), (1, 1), (2, 2), (1, 1), 1)):
+        a, v = t(*shape), t(*wShape)
+        args = (stride, pad, dil, groups)
+        g = t(*synapse.outShape(a.shape, v.shape, *args))
+        for got, want in ((host.conv2dGradInput(g, v, a, *args), synapse.convGradInput(g, v, a.shape, *args)),
+                          (host.conv2dGradWeight(g, a, v, *args), synapse.convGradWeight(g, a, v.shape, *args))):
+            assert got.shape == want.shape and torch.equal(got, want)
+        for bad in (g[:, :, :, :-1].contiguous(), g[..., :-1], g.transpose(2, 3), g.double(), g[0], None):
+            assert host.conv2dGradInput(bad, v, a, *args) is None and host.conv2dGradWeight(bad, a, v, *args) is None
+        assert host.conv2dGradInput(g, v, a, stride, -1, dil, groups) is None and host.conv2dGradWeight(g, a, v, stride, pad, dil, 5) is None
     assert host.unwrapped(x, 3, None) and not host.unwrapped(torch.ones(2).as_subclass(type("Sub", (torch.Tensor,), {})))
 
 
