@@ -664,7 +664,9 @@ class _synapseDenseThinFunction(Function):
         gradInput = gradWeight = None
         N, K, T = input.shape
         O = weight.shape[0]
-        own = not torch.is_grad_enabled() and gradOutput.dtype == torch.float32 and plainTensors(gradOutput, input, weight)
+        # (of what plainTensors looks for, what can be there in a backward pass)
+        own = not torch.is_grad_enabled() and gradOutput.dtype == torch.float32 and host.unwrapped(gradOutput, input, weight) \
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
         if own:
             gradOutput = gradOutput.contiguous()
         if ctx.needs_input_grad[0]:
