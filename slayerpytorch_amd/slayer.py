@@ -702,11 +702,14 @@ class _pspOfSpikeFunction(Function):
         # for _fresh_psp_of_spikes (the filter is a buffer of the layer's)
         ctx.potential, ctx.potentialVersion = weakref.ref(membranePotential), membranePotential._version
         ctx.filter, ctx.filterVersion = filter, filter._version
+        ctx.passedIn = None                # the backward pass in which a pooling layer's gradient last went past this node
         return psp
 
     @staticmethod
     def backward(ctx, gradOutput):
         grad = None
+        if gradOutput is None and ctx.passedIn != torch._C._current_graph_task_id():
+            gradOutput = torch.zeros_like(ctx.saved_tensors[0])      # (whatever is behind the signal had none)
         if gradOutput is not None and host.watched(ctx):
             _, filter = ctx.saved_tensors
             return (slayerCuda.pspAlpha(gradOutput.contiguous(), filter, ctx.alpha[0], ctx.alpha[1], ctx.Ts,
@@ -744,6 +747,7 @@ class _poolOfPspFunction(Function):
         filtered = slayerCuda.pspAlpha(gradOutput, filter, ctx.alpha[0], ctx.alpha[1], ctx.Ts, causal=False)
         grad = synapse.poolGradInput(filtered, weight, membranePotential.shape, membranePotential, ctx.theta,
                                      ctx.pdfTimeConstant, ctx.pdfScale)
+        ctx.next_functions[0][0].passedIn = torch._C._current_graph_task_id()
         return (None, grad) + (None,) * 7
 
 

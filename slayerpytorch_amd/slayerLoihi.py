@@ -166,9 +166,9 @@ class _spike(Function):
     @staticmethod
     def backward(ctx, gradOutput):
         pooled = ctx.pooled.take()
-        if gradOutput is None and not pooled:
-            return None, None, None, None, None
         voltage, srmKernel = ctx.saved_tensors
+        if gradOutput is None and not pooled:
+            gradOutput = torch.zeros_like(voltage)       # (whatever is behind these spikes had none)
         if gradOutput is None and len(pooled) == 1:
             # the gradient of one pooling layer alone: spread over its windows by the kernel below, as well
             grad = synapse.poolSpikeBackwardDelayedCorr(pooled[0][0], pooled[0][1], voltage, srmKernel, ctx.delaySteps, ctx.theta,

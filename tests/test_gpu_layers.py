@@ -1160,3 +1160,32 @@ def test_a_filter_that_was_changed_in_place_between_the_calls_is_noticed(pair, p
     del a
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         y.sum().backward()
+
+
+@pytest.mark.parametrize("pair", ["pool of psp", "pool of Loihi spikes", "psp of spikes"])
+def test_a_signal_whose_users_send_no_gradient_sends_zeros(pair):
+    """A Function that answers None for the signal between the two calls, or for the result: zeros at the input, and what comes
+    by the other way where there is one."""
+    class Nothing(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, a):
+            return a.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    x = dev(np.random.default_rng(6).integers(-20, 90, (2, 3, 4, 6, 300)).astype(np.float32)).requires_grad_(True)
+    between, y = _pairs()[pair](x * 1.0)
+    if pair != "psp of spikes":                      # (the spike function by itself passes on that there is none)
+        (grad,) = torch.autograd.grad(Nothing.apply(between).sum(), x, retain_graph=True)
+        assert grad.shape == x.shape and not grad.any()
+    (grad,) = torch.autograd.grad(Nothing.apply(y).sum(), x, retain_graph=True)
+    assert not grad.any()
+    both = Nothing.apply(between).sum() + y.sum()
+    (want,) = torch.autograd.grad(y.sum(), x, retain_graph=True)
+    (grad,) = torch.autograd.grad(both, x, retain_graph=True)
+    assert want.any() and torch.equal(grad, want)
+    del between
+    (again,) = torch.autograd.grad(both, x)
+    assert float((again - want).norm()) <= 1e-5 * float(want.norm())
