@@ -3,13 +3,16 @@ import torch
 
 from ._lib import host
 
+_apply = torch.autograd.Function.apply.__func__
+
 
 class Function(torch.autograd.Function):
     """``apply`` straight to torch's binding where ``torch.autograd.Function.apply`` has nothing to add: no functorch
-    transform, and no tensor that one has left wrapped (its own look at that takes 2 us a call)."""
+    transform, no tensor that one has left wrapped (its own look at that takes 2 us a call), and no ``torch.compile``, which
+    knows that function and not the binding."""
 
     @classmethod
     def apply(cls, *args):
-        if not torch._C._are_functorch_transforms_active() and host.unwrapped(*args):
-            return super(torch.autograd.Function, cls).apply(*args)
-        return super().apply(*args)
+        if torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active() or not host.unwrapped(*args):
+            return _apply(cls, *args)
+        return super(torch.autograd.Function, cls).apply(*args)

@@ -450,3 +450,32 @@ def test_a_gradient_that_someone_watches_is_known_in_the_backward_pass(how):
     assert torch.equal(got[0], torch.full((3,), 12.0 if how in ("tensor hook", "node prehook", "node hook") else 6.0))
     assert all(torch.equal(g, torch.full((3,), 3.0)) for g in (*seen, *got[1:]))
     assert len(seen) == (how in ("tensor hook", "node prehook", "node hook", "several"))
+
+
+@pytest.mark.parametrize("traceable", [True, False])
+def test_a_function_of_this_package_can_be_compiled(traceable):
+    """torch.compile takes a model that calls one of the package's Functions: into its graph where it can follow the Function,
+    around it where it cannot (the kernels are called through ctypes and an extension module)."""
+    from slayerpytorch_amd._function import Function
+    _lib.host.unwrapped(torch.ones(1))               # the extension module is there, as in a model that has run before
+
+    class Scaled(Function):
+        @staticmethod
+        def forward(ctx, x, k):
+            ctx.k = k
+            return x * k if traceable else torch.from_numpy(x.detach().numpy() * (k if _lib.host.unwrapped(x) else 0.0))
+
+        @staticmethod
+        def backward(ctx, g):
+            return g * ctx.k, None
+
+    class Model(torch.nn.Module):
+        def forward(self, x):
+            return Scaled.apply(x + 1, 3.0) * 2
+
+    torch._dynamo.reset()
+    model = torch.compile(Model(), backend="eager", fullgraph=traceable)
+    x = torch.ones(3, requires_grad=True)
+    y = model(x)
+    (grad,) = torch.autograd.grad(y.sum(), x)
+    assert torch.equal(y, torch.full((3,), 12.0)) and torch.equal(grad, torch.full((3,), 6.0))
