@@ -550,7 +550,7 @@ def _untouched(potential, version, result):
 def _fresh_psp_of_spikes(psp, kH, kW):
     """(membranePotential, filter, Ts, alpha, theta, pdfTimeConstant, pdfScale) when ``psp`` is what ``spikeLayer.psp`` has
     just returned for the fresh spikes of that potential and the recursion serves the tensor pooled by kH x kW, else None."""
-    node = psp.grad_fn if PAIR_SPIKE_PSP else None
+    node = psp.grad_fn if PAIR_SPIKE_PSP and not torch.compiler.is_compiling() else None
     if type(node) is not _pspOfSpikeFunction._backward_cls or not torch.is_grad_enabled() or psp._version != 0 \
             or not _unobserved(psp) or not psp.is_contiguous():
         return None
@@ -753,8 +753,9 @@ class _poolOfPspFunction(Function):
 
 def _takes_pooled_gradients(spikes):
     """The node behind ``spikes`` when it is a neuron whose backward pass takes the gradient of a pooling layer as it is, still
-    pooled (``PooledGradients``), and these are its own output, untouched, with the graph being recorded - else None."""
-    node = spikes.grad_fn if PAIR_SPIKE_PSP else None
+    pooled (``PooledGradients``), and these are its own output, untouched, with the graph being recorded - else None (and under
+    ``torch.compile``, which follows no node)."""
+    node = spikes.grad_fn if PAIR_SPIKE_PSP and not torch.compiler.is_compiling() else None
     if not isinstance(getattr(node, "pooled", None), PooledGradients) or not torch.is_grad_enabled() or spikes._version != 0 \
             or not _unobserved(spikes) or not spikes.is_contiguous():
         return None

@@ -1189,3 +1189,25 @@ def test_a_signal_whose_users_send_no_gradient_sends_zeros(pair):
     del between
     (again,) = torch.autograd.grad(both, x)
     assert float((again - want).norm()) <= 1e-5 * float(want.norm())
+
+
+@pytest.mark.parametrize("pair", ["pool of Loihi spikes", "delay of spikes", "shift of spikes"])
+def test_paired_calls_in_a_compiled_model(pair):
+    """torch.compile around calls whose backward passes run as one: the values of the calls as they are, a second time as well.
+    (Not of ``psp``, whose look at its filter torch.compile does not take.)"""
+    call = _pairs()[pair]
+
+    class Model(torch.nn.Module):
+        def forward(self, x):
+            return call(x * 1.0)[1]
+
+    x = dev((np.random.default_rng(8).integers(-3, 9, (2, 3, 4, 6, 300)) * 12).astype(np.float32)).requires_grad_(True)
+    want = Model()(x)
+    g = torch.linspace(-1.0, 2.0, want.numel(), device=DEV).reshape(want.shape)
+    (wantGrad,) = torch.autograd.grad(want, x, g)
+    torch._dynamo.reset()
+    compiled = torch.compile(Model(), backend="eager")
+    for _ in range(2):
+        got = compiled(x)
+        (grad,) = torch.autograd.grad(got, x, g)
+        assert torch.equal(got, want) and rel_err(host(grad), host(wantGrad)) <= REL_TOL
