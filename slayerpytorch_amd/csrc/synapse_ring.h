@@ -14,12 +14,12 @@ struct RingGeom {
     int N, SC, SH, SW, DC, DH, DW, T, groups, Qg, Mg, Cg, Og, padH, padW;
 };
 
-// SLAYER_EUNSUPPORTED (nothing launched) for geometries that the kernel does not take: it takes 16 or 32 source and at least
-// 16 destination channels per group, rows of whole vectors or at least 32 samples.
+// SLAYER_EUNSUPPORTED (nothing launched) for geometries that the kernel does not take - it takes 16 or 32 source and at least
+// 16 destination channels per group, rows of whole vectors or at least 32 samples - and for sizes at which another is faster.
 template <bool BACKWARD> int launch_gather_ring(const RingGeom &s, hipStream_t st);
 
 // The weight gradient of the same geometry, src the input [N][SC][SH][SW][T], dst (read) the output gradient: rows of partial
-// sums [Og groups][Cg][9] in `workspace`, ring_wgrad_rows() of them (0: not a geometry for it), to be added up.
+// sums [Og groups][Cg][9] in `workspace`, ring_wgrad_rows() of them (0: not a geometry for it, or another kernel is faster), to be added up.
 int ring_wgrad_rows(const RingGeom &s);
 int launch_wgrad_ring(const RingGeom &s, float *workspace, hipStream_t st);
 
