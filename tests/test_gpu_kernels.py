@@ -1439,3 +1439,30 @@ def test_an_error_that_another_call_left_is_raised_once_and_nothing_is_launched_
     assert torch.equal(once, want) and not torch.equal(once, u)
     slayerCuda.getSpikes(once.copy_(u), nu, 2.0, 1.0)
     assert torch.equal(once, want)
+
+
+@pytest.mark.parametrize("tau", [4.0, 6.5, 10.0, 12.0])   # 31, 50, 77 and 92 taps: rows of r at every distance from a vector
+@pytest.mark.parametrize("T", [516, 860, 1148, 2000])
+def test_long_rows_of_many_neurons_through_the_recursion(T, tau):
+    """Thousands of rows in pieces, with every compute unit's memory queue full, have the bits of the same rows a few at a
+    time, in both directions and with the surrogate gradient on either side; and the sum over the taps to rounding."""
+    F = len(alphaKernel(tau, 1.0, 5000, 1.0))
+    f = dev(np.array(alphaKernel(tau, 1.0, 5000, 1.0), dtype=np.float32))
+    gen = torch.Generator(device="cuda").manual_seed(T + F)
+    x, u, more = (torch.randn((1, 8002, 1, 1, T), generator=gen, device="cuda") for _ in range(3))
+
+    def calls(x, u, more):
+        return [slayerCuda.pspAlpha(x, f, tau, 1.0, 1.0, True), slayerCuda.pspAlpha(x, f, tau, 1.0, 1.0, False),
+                slayerCuda.spikeBackwardPspAlpha(x, u, f, tau, 1.0, 1.0, 2.0, 1.0, 1.0),
+                slayerCuda.pspSpikeBackwardAlpha(x, None, u, f, tau, 1.0, 1.0, 2.0, 1.0, 1.0),
+                slayerCuda.pspSpikeBackwardAlpha(x, more, u, f, tau, 1.0, 1.0, 2.0, 1.0, 1.0)]
+
+    whole = calls(x, u, more)
+    for first in (0, 3004, 7940):
+        few = [t[:, first:first + 62].contiguous() for t in (x, u, more)]
+        assert all(torch.equal(a[:, first:first + 62], b) for a, b in zip(whole, calls(*few)))
+    gate = slayerCuda.spikeBackward(torch.ones_like(u), u, 1.0, 2.0, 1.0)
+    back = slayerCuda.corr(x, f, 1.0)
+    for got, want in zip(whole, (slayerCuda.conv(x, f, 1.0), back, slayerCuda.corr(x * gate, f, 1.0), back * gate, (back + more) * gate)):
+        # every output within 1e-5 of its terms' magnitudes: samples below 6, the gate below one half
+        assert float((got - want).abs().max()) <= 1e-5 * 6 * float(f.sum())
