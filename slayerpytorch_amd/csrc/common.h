@@ -182,8 +182,8 @@ __device__ __forceinline__ float4 buffer_load4(BufferRsrc b, int laneBytes, int 
 // reads its data registers after it has been issued, and an instruction of the vector ALUs that follows at once can overwrite
 // the first of them before that.  The compiler keeps the two apart, but not where the scalar offset is a register, which it
 // takes to be safe; it is not: with `buffer_store_dwordx4 v[2:5], v57, s[36:39], s33 offen` right before
-// `v_add_u32 v2, ..` one sample in a few thousand of a large tensor was the sum that v2 had become (alpha_psp_pieces_kernel,
-// whose stores were the only ones in the library that met such a neighbour).
+// `v_add_u32 v2, ..` one sample in a few thousand of a large tensor was the sum that v2 had become (alpha_psp_pieces_kernel;
+// no other store of the library whose data count had such a neighbour).
 template <int POLICY = kStream>
 __device__ __forceinline__ void buffer_store4(BufferRsrc b, int laneBytes, int uniformBytes, float4 v)
 {
